@@ -158,6 +158,19 @@ def test_path_any_tiling_of_the_positions(seed):
     assert np.array_equal(host(out), oracle.path(iteration, wall, src, out=np.full(cols, -1, np.int32), start=1, end=2))
 
 
+@pytest.mark.parametrize("cols", [1, 2, 3, 4, 5, 253, 257])
+@pytest.mark.parametrize("iteration", [1, 2, 3, 8, 9, 10, 17, 18, 127])
+def test_path_ring_of_rows_and_edges_of_the_grid(cols, iteration):
+    # rows around the depth of the ring of rows in flight, grids around a lane's 4 columns and the window's 256, negative
+    # costs; the wall is the whole allocation, so that the first and the last row lie at its ends
+    rng = np.random.default_rng(cols * 1000 + iteration)
+    wall = rng.integers(-1000, 1000, (iteration, cols), dtype=np.int32)
+    src = rng.integers(-1000, 1000, cols, dtype=np.int32)
+    out = torch.full((cols,), -1, dtype=torch.int32, device="cuda:0")
+    ta.gptb_path(iteration, dev(wall), dev(src), out)
+    assert np.array_equal(host(out), oracle.path(iteration, wall, src))
+
+
 def test_path_walks_a_grid_pyramid_by_pyramid():
     # Rodinia's host loop: the result of one pyramid is the source of the next
     cols, rows, height = 700, 61, 20
