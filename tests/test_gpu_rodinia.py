@@ -225,6 +225,23 @@ def test_lava_forms_match_the_oracle(boxes1d):
     assert ta.lava_blocks(boxes1d) == oracle.lava_blocks(boxes1d)
 
 
+@pytest.mark.parametrize("boxes1d,launch_grid", [(2, 1), (2, 8), (3, 40), (4, 64), (5, 256), (7, 300), (9, 700)])
+def test_lava_every_cut_of_the_boxes_gives_the_same_bits(boxes1d, launch_grid):
+    # how many wavefronts a launch has decides how a box's particles are dealt to them (7, 4, 2 or 1 a lane, whole rounds of
+    # boxes and what is left over): a particle's sum never changes
+    rv, qv = lava_inputs(boxes1d, seed=50 + boxes1d)
+    d_r, d_q = dev(rv), dev(qv)
+    out = [torch.zeros((rv.shape[0], 4), device="cuda:0") for _ in range(4)]
+    ta.gptb_lava(0.5, d_r, d_q, out[0])
+    ta.ori_lava(0.5, d_r, d_q, out[1])
+    ta.gptb_lava(0.5, d_r, d_q, out[2], launch_grid=launch_grid, launch_block=256)
+    ta.gptb_lava(0.5, d_r, d_q, out[3], launch_grid=launch_grid, launch_block=64)
+    for o in out[1:]:
+        assert np.array_equal(bits(o), bits(out[0]))
+    if boxes1d <= 4:
+        assert lava_close(host(out[0]), oracle.lava(0.5, boxes1d, rv, qv))
+
+
 def test_lava_box_list_is_the_oracles():
     for boxes1d in (1, 2, 5):
         want = oracle.lava_boxes(boxes1d)
