@@ -25,5 +25,5 @@ extern "C" __global__ void general_ptb_cutcp(
     (void)block_dimension_x;
     (void)block_dimension_y;
     (void)block_dimension_z;
-    tk::cutcp_role(binDim_x, binDim_y, binZeroAddr, h, cutoff2, inv_cutoff2, regionZeroAddr, grid_dimension_x, grid_dimension_y, grid_dimension_z, (int)blockIdx.x, ptb_iter_block_step, ptb_start_block_pos, ptb_end_block_pos, (int)threadIdx.x - thread_base, (int)blockDim.x);
+    tk::cutcp_role<4>(binDim_x, binDim_y, binZeroAddr, h, cutoff2, inv_cutoff2, regionZeroAddr, grid_dimension_x, grid_dimension_y, grid_dimension_z, (int)blockIdx.x, ptb_iter_block_step, ptb_start_block_pos, ptb_end_block_pos, (int)threadIdx.x - thread_base, (int)blockDim.x);
 }

@@ -5,15 +5,28 @@
 // The reference's block position is a region of 8 x 8 x 8 lattice points, given to a block of
 // 128 threads (8, 2, 8): thread (tx, ty, tz) owns the points (tx, ty + 2 e, tz), e = 0 .. 3, and all
 // threads walk the same atoms -- the bins the neighbour list names around the region's centre bin,
-// staged 32 bins at a time in shared memory between two block barriers.  Here the atoms of a bin are
-// the same for every lane of a wavefront, so they arrive by scalar loads (one bin = 128 bytes) and
-// there is nothing to stage or to wait for: a wavefront plays 64 of the 128 threads and serves
-// half a region on its own, which is what lets the role live in a fused kernel next to roles that
-// own the workgroup barrier.  Per lane the arithmetic and its order are the reference's:
-//   dx = ax - x; dz = az - z; dxdz2 = dx*dx + dz*dz; dy = ay - y; r2 = dy*dy + dxdz2;
-//   if (r2 < cutoff2) { s = 1 - r2 * inv_cutoff2; energy += aq * rsqrt(r2) * s * s; }  dy -= 2h; ...
-// with the hardware's reciprocal square root where the reference has CUDA's rsqrtf (both are
-// approximations of about one unit in the last place: results agree within rounding, not bit for bit).
+// staged 32 bins at a time in shared memory between two block barriers.  Here a wavefront serves a piece of
+// a region on its own -- 64 of the reference's threads, some or all of their four points each -- so the
+// role lives in a fused kernel next to roles that own the workgroup barrier.
+//   dx = ax - x; dz = az - z; dy = ay - y; r2 = dx dx + dy dy + dz dz;
+//   if (r2 < cutoff2) { s = 1 - r2 * inv_cutoff2; energy += aq * rsqrt(r2) * s * s; }
+// with the hardware's reciprocal square root where the reference has CUDA's rsqrtf and fused multiply-adds
+// (results agree within rounding, not bit for bit).
+//
+// What bounds it is VALU issue, so what counts is how many atoms are looked at and what an atom costs.
+//  * Atoms.  The neighbour list names every bin that may matter to some region: 335 bins, 1340 atoms at 4 an
+//    occupied bin, of which 450 are within 12 Angstroms of a point and 725 of some point of a half region.  A
+//    wavefront therefore looks at 64 slots (8 bins) at a time, a lane each: an atom that can reach none of the
+//    wavefront's points is dropped -- an exact zero is all it would have added -- and the others are packed, in
+//    order, into a list in LDS.
+//  * An atom.  It is read back from that list with one 16-byte broadcast read into vector registers (an
+//    instruction with a scalar register among its operands takes 4.4 cycles of a SIMD, one without 2.3), and a
+//    point takes 5 such instructions and the reciprocal square root: where inv_cutoff2 is 1 / cutoff2 the cutoff
+//    is the clamp of s to [0, 1], a modifier of the instruction that computes it, instead of a comparison and
+//    an execution mask.
+// The atoms' order, and so every point's sum, is the same in every form of the kernel.
+// 208^3 lattice, two layers of regions: 147 us, 26 layers 1.47 ms; 290 us and 3.07 ms with every atom of the list by scalar loads and
+// a branch for each point.
 #pragma once
 #include "role_common.h"
 #include "../header/cutcp_header.h"
@@ -25,166 +38,227 @@ __constant__ int NbrList[NBRLIST_MAXLEN][3];
 
 namespace tk {
 
-typedef __attribute__((address_space(4))) const float4_t cutcp_const_float4;
+typedef __attribute__((address_space(3))) float4_t cutcp_lds_float4;
 
-// half `half` of region (xr, yr, zr): the reference's threads 64 half + lane, over parts
-// [part_begin, part_end) of the neighbour list of `len` entries; part p of `parts` holds the entries
-// p, p + parts, p + 2 parts, ... (every part a sample of the whole neighbourhood, so that parts cost
-// the same wherever the atoms are).  A range that does not start with part 0 goes on from the
-// energies in memory, where the range before it left them (a float stored and reloaded is unchanged,
-// so consecutive ranges give the bits of one walk through all parts).
-//
-// AHEAD = false: the atoms of a bin by scalar loads, issued when the bin's turn comes -- the faster
-// form when the SIMD has other waves to run meanwhile (the plain kernel: 300 against 330 us).
-// AHEAD = true: the 32 floats of a bin in 32 lanes of one register, fetched with one vector load
-// while the bin before it is walked, the atoms handed out with v_readlane -- a wave that has its
-// SIMD almost to itself (a slice of positions next to a GEMM) does not wait for the L2 once per
-// bin.  The atoms' bits, and so the results, are the same either way.
-template <bool AHEAD>
-__device__ __forceinline__ void cutcp_half_region(int binDim_x, int binDim_y, const float *binZeroAddr, float h,
-                                                  float cutoff2, float inv_cutoff2, float *regionZeroAddr, int gdx,
-                                                  int gdy, int xr, int yr, int zr, int half, int lane, int part_begin,
-                                                  int part_end, int parts, int len)
+#define CUTCP_GROUP 4   // atoms read from the list at a time
+#define CUTCP_BATCH_BINS (TK_WAVE_SIZE / BIN_DEPTH)   // bins whose slots a wavefront looks at at a time
+
+// The neighbour list dealt to `parts` parts: part p holds the entries p, p + parts, p + 2 parts, ... (every part a
+// sample of the whole neighbourhood, so that parts cost the same wherever the atoms are).  Walked part by part
+// it is a sequence; these give the place in it where a part begins, and the entry at a place.
+struct CutcpWalk {
+    int len, parts, each, more;   // entries per part: each + 1 in the first `more` parts, each in the others
+    float inv_each, inv_each1;
+    __device__ __forceinline__ CutcpWalk(int len_, int parts_) : len(len_), parts(parts_)
+    {
+        each = len / parts;
+        more = len - each * parts;
+        inv_each = 1.0f / (float)max(each, 1);
+        inv_each1 = 1.0f / (float)(each + 1);
+    }
+    __device__ __forceinline__ int begin_of(int part) const { return part * each + min(part, more); }
+    __device__ __forceinline__ int entry_at(int place) const
+    {
+        // divisions of numbers below 2^12 by numbers below 2^11: exact with the half added
+        const int split = more * (each + 1);
+        const bool first = place < split;
+        const int f = first ? place : place - split;
+        const int part = (int)(((float)f + 0.5f) * (first ? inv_each1 : inv_each));
+        return part + (first ? 0 : more) + (f - part * (first ? each + 1 : each)) * parts;
+    }
+};
+
+// The piece `sub` of half `half` of region (xr, yr, zr): the reference's threads 64 half + lane, points e = PTS sub ..
+// PTS sub + PTS - 1 of each, over parts [part_begin, part_end) of the neighbour list.  A range that does not start
+// with part 0 goes on from the energies in memory, where the range before it left them (a float stored and reloaded
+// is unchanged, so consecutive ranges give the bits of one walk through all parts).  CLAMP: the cutoff is the clamp
+// of s.  stage: 64 x 16 bytes of LDS, this wavefront's own.
+template <int PTS, bool CLAMP>
+__device__ __forceinline__ void cutcp_piece(int binDim_x, int binDim_y, const float *binZeroAddr, float h, float cutoff2,
+                                            float inv_cutoff2, float *regionZeroAddr, int gdx, int gdy, int xr, int yr,
+                                            int zr, int half, int sub, int lane, int part_begin, int part_end,
+                                            const CutcpWalk walk, cutcp_lds_float4 *stage)
 {
     const int tid = 64 * half + lane;
     const int tx = tid & 7, ty = (tid >> 3) & 1, tz = tid >> 4;
     float *region = regionZeroAddr + (size_t)((zr * gdy + yr) * gdx + xr) * REGION_SIZE;
     const float x = (8 * xr + tx) * h;
-    const float y = (8 * yr + ty) * h;
     const float z = (8 * zr + tz) * h;
+    float y[PTS], energy[PTS];
+    float *mine = region + (tid >> 4) * 64 + (tid & 15) + 16 * PTS * sub;
+#pragma unroll
+    for (int e = 0; e < PTS; ++e) {
+        y[e] = (8 * yr + ty + 2 * (PTS * sub + e)) * h;
+        energy[e] = part_begin > 0 ? mine[16 * e] : 0.f;
+    }
     // bin of the region's centre
     const int bx = (int)floorf((8 * xr + 4) * h * BIN_INVLEN);
     const int by = (int)floorf((8 * yr + 4) * h * BIN_INVLEN);
     const int bz = (int)floorf((8 * zr + 4) * h * BIN_INVLEN);
-    const float two_h = 2.0f * h;
-    float *mine = region + (tid >> 4) * 64 + (tid & 15);
-    float energy0 = 0.f, energy1 = 0.f, energy2 = 0.f, energy3 = 0.f;
-    if (part_begin > 0) {
-        energy0 = mine[0];
-        energy1 = mine[16];
-        energy2 = mine[32];
-        energy3 = mine[48];
-    }
+    // the box around the wavefront's points, and how far from it an atom may lie (rounded outwards)
+    const float box_x0 = (8 * xr) * h, box_x1 = (8 * xr + 7) * h;
+    const float box_y0 = (8 * yr + 2 * PTS * sub) * h, box_y1 = (8 * yr + 2 * PTS * sub + 2 * PTS - 1) * h;
+    const float box_z0 = (8 * zr + 4 * half) * h, box_z1 = (8 * zr + 4 * half + 3) * h;
+    const float reach2 = cutoff2 * 1.0001f;
+    float inv = inv_cutoff2;
+    asm volatile("" : "+v"(inv));   // (in a vector register)
     const float4_t *bins = reinterpret_cast<const float4_t *>(binZeroAddr);
-    const auto bin_of = [&](int n) -> const float4_t * {
-        const int i = bx + NbrList[n][0];
-        const int j = by + NbrList[n][1];
-        const int k = bz + NbrList[n][2];
-        return bins + ((long long)(k * binDim_y + j) * binDim_x + i) * BIN_DEPTH;
+    const int end = walk.begin_of(part_end);
+    const int slot = lane & (BIN_DEPTH - 1);
+    // The batch that starts at `place`: the list's entry of this lane's bin, then the slot this lane looks at.  A place
+    // past the end is the last entry's and not used.  Entries are fetched two batches ahead, slots one.
+    struct Entry {
+        int i, j, k;
     };
-    const auto lane_of = [](float v, int l) -> float {
-        return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
+    const auto entry = [&](int place) -> Entry {
+        const int n = walk.entry_at(min(place + (lane >> 3), end - 1));
+        return Entry{NbrList[n][0], NbrList[n][1], NbrList[n][2]};
     };
-// one atom {ax_, ay_, az_, aq_} (wave-uniform) against the lane's four points
-#define CUTCP_ATOM(ax_, ay_, az_, aq_)                                                            \
-    {                                                                                             \
-        const float dx = (ax_) - x;                                                               \
-        const float dz = (az_) - z;                                                               \
-        const float dxdz2 = dx * dx + dz * dz;                                                    \
-        float dy = (ay_) - y;                                                                     \
-        float r2 = dy * dy + dxdz2;                                                               \
-        if (r2 < cutoff2) {                                                                       \
-            const float s = (1.f - r2 * inv_cutoff2);                                             \
-            energy0 += (aq_) * __builtin_amdgcn_rsqf(r2) * s * s;                                 \
-        }                                                                                         \
-        dy -= two_h;                                                                              \
-        r2 = dy * dy + dxdz2;                                                                     \
-        if (r2 < cutoff2) {                                                                       \
-            const float s = (1.f - r2 * inv_cutoff2);                                             \
-            energy1 += (aq_) * __builtin_amdgcn_rsqf(r2) * s * s;                                 \
-        }                                                                                         \
-        dy -= two_h;                                                                              \
-        r2 = dy * dy + dxdz2;                                                                     \
-        if (r2 < cutoff2) {                                                                       \
-            const float s = (1.f - r2 * inv_cutoff2);                                             \
-            energy2 += (aq_) * __builtin_amdgcn_rsqf(r2) * s * s;                                 \
-        }                                                                                         \
-        dy -= two_h;                                                                              \
-        r2 = dy * dy + dxdz2;                                                                     \
-        if (r2 < cutoff2) {                                                                       \
-            const float s = (1.f - r2 * inv_cutoff2);                                             \
-            energy3 += (aq_) * __builtin_amdgcn_rsqf(r2) * s * s;                                 \
-        }                                                                                         \
+    const auto fetch = [&](const Entry &n) -> float4_t {
+        return bins[((long long)((bz + n.k) * binDim_y + by + n.j) * binDim_x + bx + n.i) * BIN_DEPTH + slot];
+    };
+    int place = walk.begin_of(part_begin);
+    float4_t next = {0.f, 0.f, 0.f, 0.f};
+    Entry ahead = {0, 0, 0};
+    if (place < end) {
+        next = fetch(entry(place));
+        ahead = entry(place + CUTCP_BATCH_BINS);
     }
-    if (AHEAD) {
-        // entry of the walk after (part, n): n + parts, or the first entry of the next part
-        int part = part_begin, n = part_begin;
-        while (part < part_end && n >= len) n = ++part;   // parts beyond a short list are empty
-        float cur = part < part_end ? reinterpret_cast<const float *>(bin_of(n))[lane & 31] : 0.f;
-        while (part < part_end) {
-            int part_next = part, n_next = n + parts;
-            while (part_next < part_end && n_next >= len) n_next = ++part_next;
-            const float nxt = part_next < part_end ? reinterpret_cast<const float *>(bin_of(n_next))[lane & 31] : 0.f;
+    for (; place < end; place += CUTCP_BATCH_BINS) {
+        const float4_t a = next;
+        next = fetch(ahead);
+        ahead = entry(place + 2 * CUTCP_BATCH_BINS);
+        // a bin's atoms end with the first charge of zero
+        const unsigned long long zeros = __ballot(a.w == 0.f);
+        const unsigned before = (unsigned)(zeros >> (lane & ~(BIN_DEPTH - 1))) & (2u * (1u << slot) - 1u);
+        const float ex = fmaxf(fmaxf(box_x0 - a.x, a.x - box_x1), 0.f);
+        const float ey = fmaxf(fmaxf(box_y0 - a.y, a.y - box_y1), 0.f);
+        const float ez = fmaxf(fmaxf(box_z0 - a.z, a.z - box_z1), 0.f);
+        const float e2 = ex * ex + ey * ey + ez * ez;
+        const bool keep = before == 0u && e2 < reach2 && place + (lane >> 3) < end;
+        const unsigned long long kept = __ballot(keep);
+        const int count = __popcll(kept);
+        const int at = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(kept >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)kept, 0u));
+        // the wavefront's reads of the list before are behind it: LDS serves a wavefront in order
+        if (keep) stage[at] = a;
+        // ... and up to a whole number of groups, charges of zero out of everybody's reach
+        if (lane < (-count & (CUTCP_GROUP - 1))) stage[count + lane] = float4_t{1e18f, 1e18f, 1e18f, 0.f};
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        float4_t ga[CUTCP_GROUP], gb[CUTCP_GROUP];
+        const auto read = [&](float4_t (&g)[CUTCP_GROUP], int first) {
 #pragma unroll
-            for (int a = 0; a < BIN_DEPTH; ++a) {
-                const float aq = lane_of(cur, 4 * a + 3);
-                if (0.f == aq) break;   // no more atoms in this bin
-                CUTCP_ATOM(lane_of(cur, 4 * a), lane_of(cur, 4 * a + 1), lane_of(cur, 4 * a + 2), aq)
-            }
-            cur = nxt;
-            part = part_next;
-            n = n_next;
-        }
-    } else {
-        for (int part = part_begin; part < part_end; ++part) {
-            for (int n = part; n < len; n += parts) {
-                // wave-uniform address of read-only data: scalar loads
-                const cutcp_const_float4 *atoms = (const cutcp_const_float4 *)bin_of(n);
+            for (int u = 0; u < CUTCP_GROUP; ++u) g[u] = stage[(first & (TK_WAVE_SIZE - 1)) + u];
+            __builtin_amdgcn_sched_barrier(0);   // on its way while the group before it is used
+        };
+        const auto use = [&](const float4_t (&g)[CUTCP_GROUP]) {
 #pragma unroll
-                for (int a = 0; a < BIN_DEPTH; ++a) {
-                    const float4_t atom = atoms[a];
-                    const float aq = atom.w;
-                    if (0.f == aq) break;   // no more atoms in this bin
-                    CUTCP_ATOM(atom.x, atom.y, atom.z, aq)
+            for (int u = 0; u < CUTCP_GROUP; ++u) {
+                const float4_t c = g[u];
+                const float dx = c.x - x;
+                const float dz = c.z - z;
+                const float dxdz2 = __builtin_fmaf(dx, dx, dz * dz);
+#pragma unroll
+                for (int e = 0; e < PTS; ++e) {
+                    const float dy = c.y - y[e];
+                    const float r2 = __builtin_fmaf(dy, dy, dxdz2);
+                    float s = __builtin_fmaf(-r2, inv, 1.f);
+                    if (CLAMP) s = __builtin_amdgcn_fmed3f(s, 0.f, 1.f);
+                    const float add = __builtin_fmaf(c.w * __builtin_amdgcn_rsqf(r2), s * s, energy[e]);
+                    energy[e] = CLAMP || r2 < cutoff2 ? add : energy[e];
                 }
             }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        if (count > 0) read(ga, 0);
+        for (int i = 0; i < count; i += 2 * CUTCP_GROUP) {
+            read(gb, i + CUTCP_GROUP);
+            use(ga);
+            if (i + CUTCP_GROUP >= count) break;   // uniform
+            read(ga, i + 2 * CUTCP_GROUP);
+            use(gb);
         }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
     }
-#undef CUTCP_ATOM
-    mine[0] = energy0;
-    mine[16] = energy1;
-    mine[32] = energy2;
-    mine[48] = energy3;
+#pragma unroll
+    for (int e = 0; e < PTS; ++e) mine[16 * e] = energy[e];
 }
 
+// How the regions are cut into units of a wavefront each: half regions with all four points a thread, or pieces of
+// a quarter or a half of those.  A smaller piece is more wavefronts -- one that has its SIMD to itself issues at
+// half the rate of two -- and evener shares, and has fewer atoms in reach (725 of a half region, 620 of a quarter of
+// it); against it stand what a wavefront spends on looking for them, about 100 instructions for every 64 slots, and
+// the three instructions and the read an atom costs before its points.  Measured with 1, 2 and 4 points, us:
+// 128 regions 35 / 42 / 61, 288 47 / 50 / 64, 512 84 / 62 / 82, 676 86 / 77 / 75, 1352 150 / 147 / 160, 17576
+// 1501 / 1506 / 1466.
+struct CutcpPieces {
+    int pts, subs;
+    __device__ __forceinline__ CutcpPieces(int regions, int waves)
+    {
+        pts = regions * 8 <= min(waves, 2 * 4 * TK_CU_NUM) ? 1 : (regions <= 8 * TK_CU_NUM ? 2 : 4);
+        subs = 4 / pts;
+    }
+    __device__ __forceinline__ int first_of(int region) const { return region * 2 * subs; }
+};
+
 // One phase of a launch: regions [region_lo, region_hi) (in position order) each walk parts
-// [part_begin, part_end) of the neighbour list.  A wavefront serves the half regions it owns: first_owned,
+// [part_begin, part_end) of the neighbour list.  A wavefront serves the units it owns: first_owned,
 // first_owned + stride, ...
-template <bool AHEAD>
-__device__ __forceinline__ void cutcp_phase(int region_lo, int region_hi, int part_begin, int part_end, int parts,
-                                            int len, int binDim_x,
-                                            int binDim_y, const float *binZeroAddr, float h, float cutoff2,
-                                            float inv_cutoff2, float *regionZeroAddr, int gdx, int gdy, int gdz,
-                                            int first_owned, int stride, int lane)
+__device__ __forceinline__ void cutcp_phase(const CutcpPieces pieces, int region_lo, int region_hi, int part_begin, int part_end,
+                                            const CutcpWalk walk, int binDim_x, int binDim_y, const float *binZeroAddr,
+                                            float h, float cutoff2, float inv_cutoff2, float *regionZeroAddr, int gdx,
+                                            int gdy, int gdz, int first_owned, int stride, int lane,
+                                            cutcp_lds_float4 *stage)
 {
-    if (region_lo >= region_hi || part_begin >= part_end) return;
-    const int lo = 2 * region_lo, hi = 2 * region_hi;
+    // (1e-4: a shell where the two disagree has s below 1e-4 and adds less than 1e-8 of a term)
+    const bool clamp = fabsf(cutoff2 * inv_cutoff2 - 1.f) <= 1e-4f;
+    const int lo = pieces.first_of(region_lo), hi = pieces.first_of(region_hi);
     int c = first_owned;
     if (c < lo) c += (lo - c + stride - 1) / stride * stride;
     for (; c < hi; c += stride) {
-        const int cu = __builtin_amdgcn_readfirstlane(c);
-        const int r = cu >> 1;
+        const int unit = __builtin_amdgcn_readfirstlane(c);
+        const int sub = unit % pieces.subs, half = (unit / pieces.subs) & 1;
+        const int r = unit / (2 * pieces.subs);
         // region r of the reference's GPTB order, x slowest (src/gptb_kernel/cutcp_kernel.cu:61-63)
-        cutcp_half_region<AHEAD>(binDim_x, binDim_y, binZeroAddr, h, cutoff2, inv_cutoff2, regionZeroAddr, gdx, gdy,
-                                 r / (gdy * gdz), (r / gdz) % gdy, r % gdz, cu & 1, lane, part_begin, part_end, parts, len);
+#define CUTCP_PIECE(PTS_, CLAMP_, sub_)                                                                                 \
+    cutcp_piece<PTS_, CLAMP_>(binDim_x, binDim_y, binZeroAddr, h, cutoff2, inv_cutoff2, regionZeroAddr, gdx, gdy,       \
+                              r / (gdy * gdz), (r / gdz) % gdy, r % gdz, half, sub_, lane, part_begin, part_end, walk, stage)
+        if (clamp && pieces.pts == 4) CUTCP_PIECE(4, true, sub);
+        else if (clamp && pieces.pts == 2) CUTCP_PIECE(2, true, sub);
+        else if (clamp) CUTCP_PIECE(1, true, sub);
+        else CUTCP_PIECE(1, false, sub * pieces.pts);
+        if (!clamp)
+            for (int e = 1; e < pieces.pts; ++e) CUTCP_PIECE(1, false, sub * pieces.pts + e);
+#undef CUTCP_PIECE
     }
+}
+
+// the LDS of the role's wavefronts: 64 atoms each.  role_wave: the calling wavefront's number within the role
+template <int WAVES>
+__device__ __forceinline__ cutcp_lds_float4 *cutcp_stage_of_wave(int role_wave)
+{
+    __shared__ __align__(16) float4_t cutcp_stage[WAVES][TK_WAVE_SIZE];
+    return (cutcp_lds_float4 *)&cutcp_stage[role_wave][0];
 }
 
 // grid_dimension_x, _y: regions along x and y; grid_dimension_z: regions along z times the parts of
 // the neighbour list (ceil(NbrListLen / CUTCP_NBR_CHUNK) parts of at most CUTCP_NBR_CHUNK entries, dealt
 // round-robin; 1 part when the list is empty).  The position grid has the regions as columns and the
-// parts as rows: position p adds part (p / regions) % parts to region p % regions.  Every half region has one owner wavefront for the
-// whole launch, which walks the rows in order, so the parts of a region are added in ascending order
-// without any synchronisation, whole rows that follow each other are one run through their parts, and
+// parts as rows: position p adds part (p / regions) % parts to region p % regions.  Every unit has one owner
+// wavefront for the whole launch, which walks the rows in order, so the parts of a region are added in ascending
+// order without any synchronisation, whole rows that follow each other are one run through their parts, and
 // a range that runs past the grid wraps.
-template <bool AHEAD = false>
+// WAVES: wavefronts of the role in a workgroup, role_threads / 64 at least.
+template <int WAVES>
 __device__ __forceinline__ void cutcp_role(int binDim_x, int binDim_y, const float *binZeroAddr, float h, float cutoff2,
                                            float inv_cutoff2, float *regionZeroAddr, int grid_dimension_x,
                                            int grid_dimension_y, int grid_dimension_z, int role_block, int role_blocks,
                                            int start, int end, int tid, int role_threads)
 {
-    const int waves = role_threads / 64;
-    const int wave = tid / 64;
+    const int waves = role_threads / TK_WAVE_SIZE;
+    const int wave = tid / TK_WAVE_SIZE;
     if (wave >= waves || start >= end) return;
     const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
     const int len = NbrListLen;
@@ -194,32 +268,21 @@ __device__ __forceinline__ void cutcp_role(int binDim_x, int binDim_y, const flo
     if (gx <= 0) return;
     const int stride = role_blocks * waves;
     const int first_owned = wave * role_blocks + role_block;
-    const auto chunk_begin = [&](int row) { return row % gy; };
-    const auto chunk_end = [&](int row) { return row % gy + 1; };
-#define CUTCP_PHASE(lo_, hi_, pb_, pe_)                                                                          \
-    cutcp_phase<AHEAD>(lo_, hi_, pb_, pe_, gy, len, binDim_x, binDim_y, binZeroAddr, h, cutoff2, inv_cutoff2,           \
-                regionZeroAddr, grid_dimension_x, grid_dimension_y, gdz, first_owned, stride, lane)
-    const int first_row = start / gx;
-    const int last_row = (end - 1) / gx;
-    if (first_row == last_row) {
-        CUTCP_PHASE(start - first_row * gx, end - first_row * gx, chunk_begin(first_row), chunk_end(first_row));
-        return;
+    const CutcpWalk walk(len, gy);
+    const CutcpPieces pieces(gx, stride);
+    cutcp_lds_float4 *stage = cutcp_stage_of_wave<WAVES>(__builtin_amdgcn_readfirstlane(wave));
+    // the range as phases: a partial row, or whole rows that follow each other up to the last part
+    for (int pos = start; pos < end;) {
+        const int row = pos / gx;
+        const int part = row % gy;
+        const int lo = pos - row * gx;
+        int rows = 1;
+        const int hi = min(gx, lo + (end - pos));
+        if (lo == 0 && hi == gx) rows = min((end - pos) / gx, gy - part);
+        pos += rows == 1 ? hi - lo : rows * gx;
+        cutcp_phase(pieces, lo, hi, part, part + rows, walk, binDim_x, binDim_y, binZeroAddr, h, cutoff2, inv_cutoff2,
+                    regionZeroAddr, grid_dimension_x, grid_dimension_y, gdz, first_owned, stride, lane, stage);
     }
-    int row = first_row;
-    if (start != first_row * gx) {   // partial first row
-        CUTCP_PHASE(start - first_row * gx, gx, chunk_begin(row), chunk_end(row));
-        ++row;
-    }
-    const int whole_end = (end == (last_row + 1) * gx) ? last_row + 1 : last_row;   // whole rows [row, whole_end)
-    while (row < whole_end) {
-        // rows up to the next multiple of the part count are consecutive parts: one run
-        const int run_end = min(whole_end, (row / gy + 1) * gy);
-        CUTCP_PHASE(0, gx, chunk_begin(row), chunk_end(run_end - 1));
-        row = run_end;
-    }
-    if (whole_end == last_row)       // partial last row
-        CUTCP_PHASE(0, end - last_row * gx, chunk_begin(last_row), chunk_end(last_row));
-#undef CUTCP_PHASE
 }
 
 }  // namespace tk

@@ -107,7 +107,7 @@ extern "C" __global__ __launch_bounds__(64) void ori_sgemm(float *A, float *B, f
                      blockIdx.y * SGEMM_TILE_N, 0, NORMAL_K, (tk::sgemm_lds_float *)&stage[0]);
 }
 
-// grid (regions along x, y, z), block (8,2,8): a wavefront per half region
+// grid (regions along x, y, z), block (8,2,8): a wavefront per half region, all parts of the neighbour list
 // (src/ori_kernel/cutcp_kernel.cu:19-158; zRegionIndex_t is not read there either)
 extern "C" __global__ __launch_bounds__(CUTCP_BLOCK_THREADS) void ori_cutcp(int binDim_x, int binDim_y, float *binZeroAddr,
                                                                             float h, float cutoff2, float inv_cutoff2,
@@ -115,13 +115,12 @@ extern "C" __global__ __launch_bounds__(CUTCP_BLOCK_THREADS) void ori_cutcp(int 
 {
     (void)zRegionIndex_t;
     const int tid = (threadIdx.z * blockDim.y + threadIdx.y) * blockDim.x + threadIdx.x;
-    // the neighbour list in the order of the GPTB form's parts: entries p, p + parts, ... for p = 0, 1, ...
-    const int len = NbrListLen;
-    const int parts = max(1, (len + CUTCP_NBR_CHUNK - 1) / CUTCP_NBR_CHUNK);
-    tk::cutcp_half_region<false>(binDim_x, binDim_y, binZeroAddr, h, cutoff2, inv_cutoff2, regionZeroAddr, (int)gridDim.x,
-                          (int)gridDim.y, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z,
-                          __builtin_amdgcn_readfirstlane(tid >> 6),
-                          (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), 0, parts, parts, len);
+    const int parts = max(1, (NbrListLen + CUTCP_NBR_CHUNK - 1) / CUTCP_NBR_CHUNK);
+    const int regions = (int)(gridDim.x * gridDim.y * gridDim.z);
+    tk::cutcp_role<CUTCP_BLOCK_THREADS / TK_WAVE_SIZE>(
+        binDim_x, binDim_y, binZeroAddr, h, cutoff2, inv_cutoff2, regionZeroAddr, (int)gridDim.x, (int)gridDim.y,
+        (int)gridDim.z * parts, (int)((blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x), regions, 0,
+        regions * parts, tid, CUTCP_BLOCK_THREADS);
 }
 
 // grid (transforms), block 64: a wavefront per transform where the reference has a block of 128 threads

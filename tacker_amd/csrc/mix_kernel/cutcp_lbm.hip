@@ -43,7 +43,7 @@ extern "C" __global__ __launch_bounds__(256) void cutcp_lbm_mix_wg_1_1(
     (void)lbm1_ptb_iter_block_step;
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 1, 1);
     if (sp.role == 0) {
-        tk::cutcp_role(cutcp0_binDim_x, cutcp0_binDim_y, cutcp0_binZeroAddr, cutcp0_h, cutcp0_cutoff2, cutcp0_inv_cutoff2, cutcp0_regionZeroAddr, cutcp0_grid_dimension_x, cutcp0_grid_dimension_y, cutcp0_grid_dimension_z, sp.role_block, sp.role_blocks, cutcp0_ptb_start_block_pos, cutcp0_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::cutcp_role<4>(cutcp0_binDim_x, cutcp0_binDim_y, cutcp0_binZeroAddr, cutcp0_h, cutcp0_cutoff2, cutcp0_inv_cutoff2, cutcp0_regionZeroAddr, cutcp0_grid_dimension_x, cutcp0_grid_dimension_y, cutcp0_grid_dimension_z, sp.role_block, sp.role_blocks, cutcp0_ptb_start_block_pos, cutcp0_ptb_end_block_pos, (int)threadIdx.x, 256);
     } else {
         tk::lbm_role(lbm1_srcGrid, lbm1_dstGrid, lbm1_grid_dimension_x, lbm1_grid_dimension_y, lbm1_block_dimension_x, sp.role_block, sp.role_blocks, lbm1_ptb_start_block_pos, lbm1_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
@@ -91,7 +91,7 @@ extern "C" __global__ __launch_bounds__(256) void cutcp_lbm_mix_wg_1_2(
     (void)lbm1_ptb_iter_block_step;
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 1, 2);
     if (sp.role == 0) {
-        tk::cutcp_role(cutcp0_binDim_x, cutcp0_binDim_y, cutcp0_binZeroAddr, cutcp0_h, cutcp0_cutoff2, cutcp0_inv_cutoff2, cutcp0_regionZeroAddr, cutcp0_grid_dimension_x, cutcp0_grid_dimension_y, cutcp0_grid_dimension_z, sp.role_block, sp.role_blocks, cutcp0_ptb_start_block_pos, cutcp0_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::cutcp_role<4>(cutcp0_binDim_x, cutcp0_binDim_y, cutcp0_binZeroAddr, cutcp0_h, cutcp0_cutoff2, cutcp0_inv_cutoff2, cutcp0_regionZeroAddr, cutcp0_grid_dimension_x, cutcp0_grid_dimension_y, cutcp0_grid_dimension_z, sp.role_block, sp.role_blocks, cutcp0_ptb_start_block_pos, cutcp0_ptb_end_block_pos, (int)threadIdx.x, 256);
     } else {
         tk::lbm_role(lbm1_srcGrid, lbm1_dstGrid, lbm1_grid_dimension_x, lbm1_grid_dimension_y, lbm1_block_dimension_x, sp.role_block, sp.role_blocks, lbm1_ptb_start_block_pos, lbm1_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
@@ -139,7 +139,7 @@ extern "C" __global__ __launch_bounds__(256) void cutcp_lbm_mix_wg_2_1(
     (void)lbm1_ptb_iter_block_step;
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 2, 1);
     if (sp.role == 0) {
-        tk::cutcp_role(cutcp0_binDim_x, cutcp0_binDim_y, cutcp0_binZeroAddr, cutcp0_h, cutcp0_cutoff2, cutcp0_inv_cutoff2, cutcp0_regionZeroAddr, cutcp0_grid_dimension_x, cutcp0_grid_dimension_y, cutcp0_grid_dimension_z, sp.role_block, sp.role_blocks, cutcp0_ptb_start_block_pos, cutcp0_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::cutcp_role<4>(cutcp0_binDim_x, cutcp0_binDim_y, cutcp0_binZeroAddr, cutcp0_h, cutcp0_cutoff2, cutcp0_inv_cutoff2, cutcp0_regionZeroAddr, cutcp0_grid_dimension_x, cutcp0_grid_dimension_y, cutcp0_grid_dimension_z, sp.role_block, sp.role_blocks, cutcp0_ptb_start_block_pos, cutcp0_ptb_end_block_pos, (int)threadIdx.x, 256);
     } else {
         tk::lbm_role(lbm1_srcGrid, lbm1_dstGrid, lbm1_grid_dimension_x, lbm1_grid_dimension_y, lbm1_block_dimension_x, sp.role_block, sp.role_blocks, lbm1_ptb_start_block_pos, lbm1_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
@@ -188,7 +188,7 @@ extern "C" __global__ __launch_bounds__(256) void cutcp_lbm_mix_ord_1_1(
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 1, 1);
     for (int phase = 0; phase < 2; ++phase) {
         if ((sp.role ^ phase) == 0) {
-            tk::cutcp_role(cutcp0_binDim_x, cutcp0_binDim_y, cutcp0_binZeroAddr, cutcp0_h, cutcp0_cutoff2, cutcp0_inv_cutoff2, cutcp0_regionZeroAddr, cutcp0_grid_dimension_x, cutcp0_grid_dimension_y, cutcp0_grid_dimension_z, (int)blockIdx.x, (int)gridDim.x, cutcp0_ptb_start_block_pos, cutcp0_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::cutcp_role<4>(cutcp0_binDim_x, cutcp0_binDim_y, cutcp0_binZeroAddr, cutcp0_h, cutcp0_cutoff2, cutcp0_inv_cutoff2, cutcp0_regionZeroAddr, cutcp0_grid_dimension_x, cutcp0_grid_dimension_y, cutcp0_grid_dimension_z, (int)blockIdx.x, (int)gridDim.x, cutcp0_ptb_start_block_pos, cutcp0_ptb_end_block_pos, (int)threadIdx.x, 256);
         } else {
             tk::lbm_role(lbm1_srcGrid, lbm1_dstGrid, lbm1_grid_dimension_x, lbm1_grid_dimension_y, lbm1_block_dimension_x, (int)blockIdx.x, (int)gridDim.x, lbm1_ptb_start_block_pos, lbm1_ptb_end_block_pos, (int)threadIdx.x, 256);
         }
@@ -238,7 +238,7 @@ extern "C" __global__ __launch_bounds__(256) void cutcp_lbm_mix_ord_1_2(
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 1, 2);
     for (int phase = 0; phase < 2; ++phase) {
         if ((sp.role ^ phase) == 0) {
-            tk::cutcp_role(cutcp0_binDim_x, cutcp0_binDim_y, cutcp0_binZeroAddr, cutcp0_h, cutcp0_cutoff2, cutcp0_inv_cutoff2, cutcp0_regionZeroAddr, cutcp0_grid_dimension_x, cutcp0_grid_dimension_y, cutcp0_grid_dimension_z, (int)blockIdx.x, (int)gridDim.x, cutcp0_ptb_start_block_pos, cutcp0_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::cutcp_role<4>(cutcp0_binDim_x, cutcp0_binDim_y, cutcp0_binZeroAddr, cutcp0_h, cutcp0_cutoff2, cutcp0_inv_cutoff2, cutcp0_regionZeroAddr, cutcp0_grid_dimension_x, cutcp0_grid_dimension_y, cutcp0_grid_dimension_z, (int)blockIdx.x, (int)gridDim.x, cutcp0_ptb_start_block_pos, cutcp0_ptb_end_block_pos, (int)threadIdx.x, 256);
         } else {
             tk::lbm_role(lbm1_srcGrid, lbm1_dstGrid, lbm1_grid_dimension_x, lbm1_grid_dimension_y, lbm1_block_dimension_x, (int)blockIdx.x, (int)gridDim.x, lbm1_ptb_start_block_pos, lbm1_ptb_end_block_pos, (int)threadIdx.x, 256);
         }
@@ -288,7 +288,7 @@ extern "C" __global__ __launch_bounds__(256) void cutcp_lbm_mix_ord_2_1(
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 2, 1);
     for (int phase = 0; phase < 2; ++phase) {
         if ((sp.role ^ phase) == 0) {
-            tk::cutcp_role(cutcp0_binDim_x, cutcp0_binDim_y, cutcp0_binZeroAddr, cutcp0_h, cutcp0_cutoff2, cutcp0_inv_cutoff2, cutcp0_regionZeroAddr, cutcp0_grid_dimension_x, cutcp0_grid_dimension_y, cutcp0_grid_dimension_z, (int)blockIdx.x, (int)gridDim.x, cutcp0_ptb_start_block_pos, cutcp0_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::cutcp_role<4>(cutcp0_binDim_x, cutcp0_binDim_y, cutcp0_binZeroAddr, cutcp0_h, cutcp0_cutoff2, cutcp0_inv_cutoff2, cutcp0_regionZeroAddr, cutcp0_grid_dimension_x, cutcp0_grid_dimension_y, cutcp0_grid_dimension_z, (int)blockIdx.x, (int)gridDim.x, cutcp0_ptb_start_block_pos, cutcp0_ptb_end_block_pos, (int)threadIdx.x, 256);
         } else {
             tk::lbm_role(lbm1_srcGrid, lbm1_dstGrid, lbm1_grid_dimension_x, lbm1_grid_dimension_y, lbm1_block_dimension_x, (int)blockIdx.x, (int)gridDim.x, lbm1_ptb_start_block_pos, lbm1_ptb_end_block_pos, (int)threadIdx.x, 256);
         }

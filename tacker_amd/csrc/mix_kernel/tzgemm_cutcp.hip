@@ -72,7 +72,7 @@ extern "C" __global__ __launch_bounds__(384) void cutcp_tzgemm_mix_wave_128(
         const int be_block = apart ? (int)blockIdx.x - tz_busy : (int)blockIdx.x;
         const int be_blocks = apart ? launched - tz_busy : launched;
         if (be_block >= 0) {
-            tk::cutcp_role<true>(cutcp0_binDim_x, cutcp0_binDim_y, cutcp0_binZeroAddr, cutcp0_h, cutcp0_cutoff2, cutcp0_inv_cutoff2, cutcp0_regionZeroAddr, cutcp0_grid_dimension_x, cutcp0_grid_dimension_y, cutcp0_grid_dimension_z, be_block, be_blocks, cutcp0_ptb_start_block_pos, cutcp0_ptb_end_block_pos, (int)threadIdx.x - 256, 128);
+            tk::cutcp_role<2>(cutcp0_binDim_x, cutcp0_binDim_y, cutcp0_binZeroAddr, cutcp0_h, cutcp0_cutoff2, cutcp0_inv_cutoff2, cutcp0_regionZeroAddr, cutcp0_grid_dimension_x, cutcp0_grid_dimension_y, cutcp0_grid_dimension_z, be_block, be_blocks, cutcp0_ptb_start_block_pos, cutcp0_ptb_end_block_pos, (int)threadIdx.x - 256, 128);
         }
         tk::role_wave_done(tz_arrivals);
     }
@@ -148,7 +148,7 @@ extern "C" __global__ __launch_bounds__(512) void cutcp_tzgemm_mix_wave_256(
         const int be_block = apart ? (int)blockIdx.x - tz_busy : (int)blockIdx.x;
         const int be_blocks = apart ? launched - tz_busy : launched;
         if (be_block >= 0) {
-            tk::cutcp_role<true>(cutcp0_binDim_x, cutcp0_binDim_y, cutcp0_binZeroAddr, cutcp0_h, cutcp0_cutoff2, cutcp0_inv_cutoff2, cutcp0_regionZeroAddr, cutcp0_grid_dimension_x, cutcp0_grid_dimension_y, cutcp0_grid_dimension_z, be_block, be_blocks, cutcp0_ptb_start_block_pos, cutcp0_ptb_end_block_pos, (int)threadIdx.x - 256, 256);
+            tk::cutcp_role<4>(cutcp0_binDim_x, cutcp0_binDim_y, cutcp0_binZeroAddr, cutcp0_h, cutcp0_cutoff2, cutcp0_inv_cutoff2, cutcp0_regionZeroAddr, cutcp0_grid_dimension_x, cutcp0_grid_dimension_y, cutcp0_grid_dimension_z, be_block, be_blocks, cutcp0_ptb_start_block_pos, cutcp0_ptb_end_block_pos, (int)threadIdx.x - 256, 256);
         }
         tk::role_wave_done(tz_arrivals);
     }
@@ -224,7 +224,7 @@ extern "C" __global__ __launch_bounds__(640) void cutcp_tzgemm_mix_wave_384(
         const int be_block = apart ? (int)blockIdx.x - tz_busy : (int)blockIdx.x;
         const int be_blocks = apart ? launched - tz_busy : launched;
         if (be_block >= 0) {
-            tk::cutcp_role<true>(cutcp0_binDim_x, cutcp0_binDim_y, cutcp0_binZeroAddr, cutcp0_h, cutcp0_cutoff2, cutcp0_inv_cutoff2, cutcp0_regionZeroAddr, cutcp0_grid_dimension_x, cutcp0_grid_dimension_y, cutcp0_grid_dimension_z, be_block, be_blocks, cutcp0_ptb_start_block_pos, cutcp0_ptb_end_block_pos, (int)threadIdx.x - 256, 384);
+            tk::cutcp_role<6>(cutcp0_binDim_x, cutcp0_binDim_y, cutcp0_binZeroAddr, cutcp0_h, cutcp0_cutoff2, cutcp0_inv_cutoff2, cutcp0_regionZeroAddr, cutcp0_grid_dimension_x, cutcp0_grid_dimension_y, cutcp0_grid_dimension_z, be_block, be_blocks, cutcp0_ptb_start_block_pos, cutcp0_ptb_end_block_pos, (int)threadIdx.x - 256, 384);
         }
         tk::role_wave_done(tz_arrivals);
     }
@@ -300,7 +300,7 @@ extern "C" __global__ __launch_bounds__(768) void cutcp_tzgemm_mix_wave_512(
         const int be_block = apart ? (int)blockIdx.x - tz_busy : (int)blockIdx.x;
         const int be_blocks = apart ? launched - tz_busy : launched;
         if (be_block >= 0) {
-            tk::cutcp_role<true>(cutcp0_binDim_x, cutcp0_binDim_y, cutcp0_binZeroAddr, cutcp0_h, cutcp0_cutoff2, cutcp0_inv_cutoff2, cutcp0_regionZeroAddr, cutcp0_grid_dimension_x, cutcp0_grid_dimension_y, cutcp0_grid_dimension_z, be_block, be_blocks, cutcp0_ptb_start_block_pos, cutcp0_ptb_end_block_pos, (int)threadIdx.x - 256, 512);
+            tk::cutcp_role<8>(cutcp0_binDim_x, cutcp0_binDim_y, cutcp0_binZeroAddr, cutcp0_h, cutcp0_cutoff2, cutcp0_inv_cutoff2, cutcp0_regionZeroAddr, cutcp0_grid_dimension_x, cutcp0_grid_dimension_y, cutcp0_grid_dimension_z, be_block, be_blocks, cutcp0_ptb_start_block_pos, cutcp0_ptb_end_block_pos, (int)threadIdx.x - 256, 512);
         }
         tk::role_wave_done(tz_arrivals);
     }
@@ -359,7 +359,7 @@ extern "C" __global__ __launch_bounds__(256) void cutcp_tzgemm_mix_wg_1_1(
         tk::WorkgroupSync sync;
         tk::tzgemm_role<TZ_STAGES_WG, true>(tzgemm1_A, tzgemm1_B, tzgemm1_C, tzgemm1_NORMAL_M, tzgemm1_NORMAL_N, tzgemm1_NORMAL_K, tk::tz_workspace_of(tzgemm1_C, tzgemm1_NORMAL_M, tzgemm1_NORMAL_N, tzgemm1_NORMAL_K), sp.role_block, sp.role_blocks, tzgemm1_ptb_start_block_pos, tzgemm1_ptb_end_block_pos, (int)threadIdx.x, tz_lds, sync);
     } else {
-        tk::cutcp_role(cutcp0_binDim_x, cutcp0_binDim_y, cutcp0_binZeroAddr, cutcp0_h, cutcp0_cutoff2, cutcp0_inv_cutoff2, cutcp0_regionZeroAddr, cutcp0_grid_dimension_x, cutcp0_grid_dimension_y, cutcp0_grid_dimension_z, sp.role_block, sp.role_blocks, cutcp0_ptb_start_block_pos, cutcp0_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::cutcp_role<4>(cutcp0_binDim_x, cutcp0_binDim_y, cutcp0_binZeroAddr, cutcp0_h, cutcp0_cutoff2, cutcp0_inv_cutoff2, cutcp0_regionZeroAddr, cutcp0_grid_dimension_x, cutcp0_grid_dimension_y, cutcp0_grid_dimension_z, sp.role_block, sp.role_blocks, cutcp0_ptb_start_block_pos, cutcp0_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
 }
 
@@ -416,6 +416,6 @@ extern "C" __global__ __launch_bounds__(256) void cutcp_tzgemm_mix_wg_1_2(
         tk::WorkgroupSync sync;
         tk::tzgemm_role<TZ_STAGES_WG, true>(tzgemm1_A, tzgemm1_B, tzgemm1_C, tzgemm1_NORMAL_M, tzgemm1_NORMAL_N, tzgemm1_NORMAL_K, tk::tz_workspace_of(tzgemm1_C, tzgemm1_NORMAL_M, tzgemm1_NORMAL_N, tzgemm1_NORMAL_K), sp.role_block, sp.role_blocks, tzgemm1_ptb_start_block_pos, tzgemm1_ptb_end_block_pos, (int)threadIdx.x, tz_lds, sync);
     } else {
-        tk::cutcp_role(cutcp0_binDim_x, cutcp0_binDim_y, cutcp0_binZeroAddr, cutcp0_h, cutcp0_cutoff2, cutcp0_inv_cutoff2, cutcp0_regionZeroAddr, cutcp0_grid_dimension_x, cutcp0_grid_dimension_y, cutcp0_grid_dimension_z, sp.role_block, sp.role_blocks, cutcp0_ptb_start_block_pos, cutcp0_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::cutcp_role<4>(cutcp0_binDim_x, cutcp0_binDim_y, cutcp0_binZeroAddr, cutcp0_h, cutcp0_cutoff2, cutcp0_inv_cutoff2, cutcp0_regionZeroAddr, cutcp0_grid_dimension_x, cutcp0_grid_dimension_y, cutcp0_grid_dimension_z, sp.role_block, sp.role_blocks, cutcp0_ptb_start_block_pos, cutcp0_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
 }

@@ -72,9 +72,8 @@ extern "C" __global__ __launch_bounds__({threads}) void {name}(
 
 
 # Template arguments of a role inside a wave-split kernel, where few best-effort waves share the CU
-# with the GEMM: lbm takes two rows per wave to keep enough loads in flight, cutcp fetches every bin
-# of atoms a bin ahead instead of waiting for it.
-WAVE_SPLIT_EXTRA = {"lbm": "<2>", "cutcp": "<true>"}
+# with the GEMM: lbm takes two rows per wave to keep enough loads in flight.
+WAVE_SPLIT_EXTRA = {"lbm": "<2>"}
 
 
 def generate_wave_split(be, be_threads, tz_first=True, large=False):

@@ -105,6 +105,28 @@ def test_any_tiling_of_the_positions_gives_the_one_kernel(seed):
     assert np.array_equal(got == -3.0, want == -3.0) and close(got, want)
 
 
+@pytest.mark.parametrize("inv", [1 / 144.0, 0.0065, 0.008])
+@pytest.mark.parametrize("regions,natoms", [((1, 1, 1), 1), ((2, 1, 1), 64), ((1, 3, 2), 2000), ((9, 8, 3), 900), ((8, 9, 7), 1500)])
+def test_cut_of_the_regions_and_meaning_of_the_cutoff(inv, regions, natoms):
+    # the launch's wavefronts decide how regions are cut into pieces (1, 2 or 4 points a lane); inv_cutoff2 need not be
+    # 1 / cutoff2, and then the cutoff is a comparison; full bins, empty bins, a charge of zero inside a bin (it ends the bin)
+    nx, ny, nz = (8 * r for r in regions)
+    atoms = atoms_in_box(natoms, (min(nx, ny, nz) - 1) * H, seed=natoms)
+    inp = ta.CutcpInput(atoms, (0, 0, 0), nx, ny, nz, H, CUTOFF)
+    prep = oracle.cutcp_prepare(atoms, (0, 0, 0), nx, ny, nz, H, CUTOFF)
+    filled = np.argwhere(prep["bins"][..., 3] != 0)
+    for where in filled[::7]:
+        prep["bins"][tuple(where)][3] = 0.0
+    inp.bins.copy_(torch.from_numpy(prep["bins"]).cuda())
+    want = oracle.cutcp(prep, H, C2, inv, inp.regions, parts="chunks")
+    out = [torch.zeros_like(inp.energies) for _ in range(3)]
+    ta.gptb_cutcp(inp, C2, inv, out[0])
+    ta.gptb_cutcp(inp, C2, inv, out[1], launch_grid=1, launch_block=64)
+    ta.ori_cutcp(inp, C2, inv, out[2])
+    assert np.array_equal(bits(out[1]), bits(out[0])) and np.array_equal(bits(out[2]), bits(out[0]))
+    assert close(host(out[0]), want)
+
+
 @pytest.mark.parametrize("variant", [None, "wave_128", "wave_256", "wave_512", "wg_1_1", "wg_1_2"])
 def test_mix_tzgemm_cutcp(variant):
     M, N, K = 256, 256, 256
