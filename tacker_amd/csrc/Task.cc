@@ -61,9 +61,11 @@ tkGraphExec_t Task::captureQuery(cudaStream_t stream)
         for (auto &kernel : kernels) kernel->execute(stream);
     } catch (...) {   // a stream left recording would fail every later call on it
         tkStreamEndCapture(stream, &graph);
+        captured();
         if (graph) tkGraphExecDestroy(graph);
         throw;
     }
+    captured();
     TK_SAFE_CALL(tkStreamEndCapture(stream, &graph));
     return graph;
 }

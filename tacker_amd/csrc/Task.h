@@ -25,6 +25,8 @@ public:
     // kernel still has buffers to allocate, and the caller stages the input before each launch of
     // the graph.  The caller destroys the graph (tkGraphExecDestroy).
     tkGraphExec_t captureQuery(cudaStream_t stream);
+    // the kernels' execute() has been recorded, not run: what a task remembers of its last run no longer holds
+    virtual void captured() {}
 
     int taskId;
     std::string taskName;

@@ -5,6 +5,7 @@
 
 #include "../Creator.h"
 #include "../Logger.h"
+#include "direct.h"
 #include "../rng.h"
 
 extern Logger logger;
@@ -23,38 +24,122 @@ void launch1d(const char *key, long work, void **args, cudaStream_t stream)
     TK_SAFE_CALL(tkLaunchKernel(fmap.at(key), dim3((unsigned)blocks).raw(), dim3(256).raw(), args, 0, stream));
 }
 
-float *devAlloc(std::vector<void *> &freeList, size_t floats)
+// A task's device buffers, given back together.  The small ones -- four in five -- lie in slabs: tkFree waits for the device and
+// unmaps, 50 to 350 us a call, which made a task of one allocation a buffer 8 ms to give back.
+class Buffers {
+public:
+    ~Buffers()
+    {
+        for (void *p : slabs_) tkErrCheck(tkFree(p));
+    }
+    void *get(size_t bytes)
+    {
+        bytes = (bytes + 255) / 256 * 256;
+        void *p = nullptr;
+        if (bytes > left_) {
+            const bool own = bytes > SLAB / 2;
+            TK_SAFE_CALL(tkMalloc(&p, own ? bytes : SLAB));
+            slabs_.push_back(p);
+            if (own) return p;
+            next_ = (char *)p;
+            left_ = SLAB;
+        }
+        p = next_;
+        next_ += bytes;
+        left_ -= bytes;
+        return p;
+    }
+
+private:
+    static constexpr size_t SLAB = (size_t)64 << 20;
+    std::vector<void *> slabs_;
+    char *next_ = nullptr;
+    size_t left_ = 0;
+};
+
+void *zeroed(Buffers &buffers, size_t bytes)
 {
-    float *p = nullptr;
-    TK_SAFE_CALL(tkMalloc((void **)&p, floats * sizeof(float)));
-    TK_SAFE_CALL(tkMemset(p, 0, floats * sizeof(float)));
-    freeList.push_back(p);
+    void *p = buffers.get(bytes);
+    TK_SAFE_CALL(tkMemset(p, 0, bytes));
     return p;
 }
+float *devAlloc(Buffers &buffers, size_t floats) { return (float *)zeroed(buffers, floats * sizeof(float)); }
 
 // f16 [rows_pad][cols_pad] with uniform[-1,1]*scale in the top-left rows x cols, zero elsewhere
-void *randomHalfMatrix(std::vector<void *> &freeList, tk::Rng &rng, int rows, int cols, int rows_pad,
+void *randomHalfMatrix(Buffers &buffers, tk::Rng &rng, int rows, int cols, int rows_pad,
                        int cols_pad, float scale)
 {
     std::vector<uint16_t> host((size_t)rows_pad * cols_pad, 0);
     for (int r = 0; r < rows; ++r)
         for (int c = 0; c < cols; ++c)
             host[(size_t)r * cols_pad + c] = tk::float_to_half_bits(rng.uniform(-1.0f, 1.0f) * scale);
-    void *p = nullptr;
-    TK_SAFE_CALL(tkMalloc(&p, host.size() * 2));
+    void *p = buffers.get(host.size() * 2);
     TK_SAFE_CALL(tkMemcpy(p, host.data(), host.size() * 2, TK_MEMCPY_H2D));
-    freeList.push_back(p);
     return p;
 }
 
-float *randomBias(std::vector<void *> &freeList, tk::Rng &rng, int n, int n_pad)
+float *randomBias(Buffers &buffers, tk::Rng &rng, int n, int n_pad)
 {
     std::vector<float> host(n_pad, 0.0f);
     for (int i = 0; i < n; ++i) host[i] = rng.uniform(-0.1f, 0.1f);
-    float *p = devAlloc(freeList, n_pad);
+    float *p = devAlloc(buffers, n_pad);
     TK_SAFE_CALL(tkMemcpy(p, host.data(), (size_t)n_pad * sizeof(float), TK_MEMCPY_H2D));
     return p;
 }
+
+// The direct kernels (kernels/dnn_direct.hip) run a layer that has its launch to itself; a device layer without them
+// runs every layer through its operand builder and tzgemm, as a layer fused with a best-effort kernel always does.
+bool haveDirectKernels() { return fmap.count("conv3x3_image") != 0; }
+
+// The weights [rows][K] once more, in the order the direct kernels read them.
+void *weightFragments(Buffers &buffers, void *weights, int rows, int K)
+{
+    if (!haveDirectKernels()) return nullptr;
+    void *p = buffers.get((size_t)rows * K * 2);
+    void *args[] = {&weights, &p, &rows, &K};
+    launch1d("pack_weight_fragments", (long)rows * K / 8, args, nullptr);
+    return p;
+}
+
+// How tzgemm cuts the reduction of a (padded) GEMM: the segments' number -- 4 per part (tz_use_ksplit), or 1 -- and the
+// 64-k chunk each begins with.  Chunks from `real` on are padding: zeros, which nobody needs to add.
+int reductionCut(int M, int N, int K, int real, int begin[DNN_MAX_SEGMENTS + 1])
+{
+    const int chunks = K / TZ_BLOCK_K;
+    if (!tz_use_ksplit(M, N, K)) {
+        begin[0] = 0;
+        begin[1] = std::min(real, chunks);
+        return 1;
+    }
+    const int parts = tz_ksplit_parts(M, N, K), segments = 4 * parts;
+    static_assert(4 * TZ_KSPLIT_MAX_PARTS <= DNN_MAX_SEGMENTS, "the table holds every cut");
+    for (int i = 0; i <= segments; ++i) {   // as tzgemm_role_ksplit
+        const int part = i / 4, first = part * chunks / parts, count = (part + 1) * chunks / parts - first;
+        begin[i] = std::min(real, first + (i % 4) * count / 4);
+    }
+    begin[segments] = std::min(real, chunks);
+    return segments;
+}
+
+// d -> what dnn_div takes for a division by d
+unsigned reciprocal(int d) { return d == 1 ? 0u : (unsigned)((1ull << 32) / (unsigned)d + 1); }
+
+// A layer's activation as the next layer's direct kernel reads it: where it is, and whether it holds what the
+// layer's raw output holds (a layer that ran fused, or not through its direct kernel, has written only that).
+struct Activation {
+    DnnOutput out{};
+    int channels = 0;
+    bool fresh = false;
+    // bring it up to date, if it is not
+    void need(cudaStream_t stream)
+    {
+        if (fresh) return;
+        const int pixels = out.pool ? out.H * out.W / 4 : out.H * out.W;
+        void *args[] = {&out, &channels};
+        launch1d("dnn_activation", (long)pixels * (channels / 4), args, stream);
+        fresh = true;
+    }
+};
 
 // Shared GEMM machinery of conv and FC layers: persistent objects built once.
 class GemmLayer : public LcGemmKernel {
@@ -75,6 +160,7 @@ public:
 
 protected:
     virtual void before(cudaStream_t stream) = 0;   // operand staging (im2col / pack)
+    virtual void fused() {}                         // the layer's raw output is all this launch writes
     void executeImpl(cudaStream_t stream) override
     {
         before(stream);
@@ -85,11 +171,12 @@ public:
     void executeMixed(GPTBKernel *be, int be_start, int be_end, cudaStream_t stream,
                       const std::string &variant = "") override
     {
-        before(stream);
         if (be_end <= be_start) {
-            gptb_->execute(stream);
+            executeImpl(stream);
             return;
         }
+        before(stream);
+        fused();
         std::unique_ptr<MixKernel> mix(createTzgemmMix(be, gptb_.get(), be_start, be_end, 0, tiles_, variant, 0, 0));
         mix->execute(stream);
     }
@@ -117,7 +204,62 @@ public:
     // {n,c,h,w, k,c,kh,kw, pad,pad, stride,stride, dil,dil}
     std::vector<int> getArgs() override { return {1, C_, H_, W_, Cout_, C_, 3, 3, 1, 1, 1, 1, 1, 1}; }
 
+    // Run through the direct kernel from now on: `in` (null: the layer reads the image) to `out`, weights as
+    // fragments.  A workgroup's output channels are as many as still leave a workgroup for three CUs in four -- every
+    // workgroup reads its tile's input and its channels' weights once, so larger ones read less -- and, where tzgemm cuts
+    // the reduction, as many as 16 wavefronts serve with a segment each; a wavefront takes two 16-channel slices
+    // where 8 are left.  Segments that are too many for that are taken a part (four of them) a wavefront.
+    void useDirect(Activation *in, Activation *out, const void *fragments)
+    {
+        in_ = in;
+        next_ = out;
+        direct_.reset(new DnnConv{});
+        DnnConv &d = *direct_;
+        d.act = in ? in->out.act : nullptr;
+        d.weights = fragments;
+        d.out = out->out;
+        d.C = C_;
+        d.chunks = K_ / TZ_BLOCK_K;
+        d.tiles_x = (W_ + DNN_TILE - 1) / DNN_TILE;
+        d.tiles = d.tiles_x * ((H_ + DNN_TILE - 1) / DNN_TILE);
+        d.per_group = reciprocal(d.tiles);
+        d.per_row = reciprocal(d.tiles_x);
+        int ct = 8, slices = 1;
+        bool part = false;
+        if (in) {
+            const int segments = reductionCut(M_, N_, K_, 9 * C_ / TZ_BLOCK_K, d.segment_begin);
+            while (ct > 1 && (Cout_ % (16 * ct) != 0 || (segments > 1 && ct * segments > 16) ||
+                              (long)d.tiles * (Cout_ / (16 * ct)) * 4 < (long)cuCount() * 3))
+                ct /= 2;
+            slices = ct % 2 == 0 && ct / 2 * segments >= 8 ? 2 : 1;
+            part = segments > 16;
+            d.runs = part ? segments / 4 : segments;
+            key_ = std::string("conv3x3_direct_") + (slices == 2 ? "2" : "1") + (part ? "_1" : "_0");
+            lds_ = std::max((size_t)(C_ / 64) * DNN_PLANE_BYTES, (size_t)ct * d.runs * DNN_PARTIAL_BYTES);
+        } else {
+            ct = Cout_ / 16;
+            d.runs = 1;
+            key_ = "conv3x3_image";
+        }
+        d.ct_count = ct;
+        d.workgroups = d.tiles * (Cout_ / (16 * ct));
+        threads_ = in ? 64u * (unsigned)(ct / slices * d.runs) : 256u;
+        grid_ = (unsigned)(d.workgroups + TK_XCD_NUM - 1) / TK_XCD_NUM * TK_XCD_NUM;
+    }
+
 protected:
+    void fused() override
+    {
+        if (next_) next_->fresh = false;
+    }
+    void executeImpl(cudaStream_t stream) override
+    {
+        if (!direct_) return GemmLayer::executeImpl(stream);
+        if (in_) in_->need(stream);
+        void *args[] = {in_ ? (void *)direct_.get() : (void *)&act_, direct_.get()};
+        TK_SAFE_CALL(tkLaunchKernel(fmap.at(key_), dim3(grid_).raw(), dim3(threads_).raw(), args, lds_, stream));
+        next_->fresh = true;
+    }
     void before(cudaStream_t stream) override
     {
         int KH = 3, KW = 3, pad = 1, stride = 1, Ho = H_, Wo = W_, Kp = K_;
@@ -140,6 +282,11 @@ private:
     int pool_;
     int H_, W_, C_, cs_, Cout_;
     void *A_;
+    std::unique_ptr<DnnConv> direct_;
+    Activation *in_ = nullptr, *next_ = nullptr;
+    std::string key_;
+    unsigned grid_ = 0, threads_ = 0;
+    size_t lds_ = 0;
 };
 
 class FcKernel : public GemmLayer {
@@ -163,7 +310,40 @@ public:
     }
     std::vector<int> getArgs() override { return {M_, N_, K_}; }
 
+    // Run through the direct kernel from now on.  in, out: whether X's first row, and the next layer's (next_x), hold
+    // this layer's input and activation (out null: the last layer).
+    void useDirect(bool *in, bool *out, const void *fragments, float *raw, const float *bias, void *next_x)
+    {
+        inFresh_ = in;
+        outFresh_ = out;
+        direct_.reset(new DnnFc{});
+        direct_->x = X_;
+        direct_->weights = fragments;
+        direct_->raw = raw;
+        direct_->bias = bias;
+        direct_->act = next_x;
+        direct_->chunks = K_ / TZ_BLOCK_K;
+        direct_->segments = reductionCut(M_, N_, K_, direct_->chunks, direct_->segment_begin);
+        perWave_ = direct_->segments > 16 ? 2 : 1;
+    }
+
 protected:
+    void fused() override
+    {
+        if (inFresh_) *inFresh_ = true;   // before() packed it
+        if (outFresh_) *outFresh_ = false;
+    }
+    void executeImpl(cudaStream_t stream) override
+    {
+        if (!direct_) return GemmLayer::executeImpl(stream);
+        if (!*inFresh_) before(stream);
+        *inFresh_ = true;
+        void *args[] = {direct_.get()};
+        const int waves = (direct_->segments + perWave_ - 1) / perWave_;
+        TK_SAFE_CALL(tkLaunchKernel(fmap.at(perWave_ == 2 ? "fc_direct_2" : "fc_direct_1"), dim3((unsigned)(N_ / 16)).raw(),
+                                    dim3((unsigned)(64 * waves)).raw(), args, 0, stream));
+        if (outFresh_) *outFresh_ = true;
+    }
     void before(cudaStream_t stream) override
     {
         if (poolW_ > 0) {
@@ -182,17 +362,22 @@ private:
     int relu_, in_, out_;
     void *X_;
     int poolW_, poolLd_, poolC_;
+    std::unique_ptr<DnnFc> direct_;
+    bool *inFresh_ = nullptr, *outFresh_ = nullptr;
+    int perWave_ = 1;
 };
 
 }  // namespace
 
 struct VGG16::Impl {
-    std::vector<void *> freeList;
+    Buffers buffers;
     std::vector<float> hostInput;
     float *input = nullptr;
     std::vector<VGG16::Act> convOut;   // the 13 convolutions, then the 3 fully connected layers
     float *logits = nullptr;
     long logitsStride = 0;
+    Activation act[13];             // of the convolutions; the last one's is fc1's input
+    bool fcInput[3] = {};           // fc2's and fc3's input vectors hold the layer before's activation ([0] unused: act[12])
 };
 
 VGG16::VGG16(int taskId, const VGG16Options &o) : Task(taskId, "vgg16"), opt(o), impl(new Impl)
@@ -200,7 +385,7 @@ VGG16::VGG16(int taskId, const VGG16Options &o) : Task(taskId, "vgg16"), opt(o),
     taskType = LC;
     if (opt.height % 32 || opt.width % 32) logger.ERROR("vgg16: input resolution must be a multiple of 32");
     tk::Rng rng(opt.seed);
-    auto &fl = impl->freeList;
+    auto &fl = impl->buffers;
 
     int H = opt.height, W = opt.width, C = 3, ld = 3;
     impl->hostInput.resize((size_t)H * W * 3);
@@ -221,10 +406,10 @@ VGG16::VGG16(int taskId, const VGG16Options &o) : Task(taskId, "vgg16"), opt(o),
             c = p;
         }
     }
-    void *Abuf = nullptr;
-    TK_SAFE_CALL(tkMalloc(&Abuf, maxA * 2));
-    TK_SAFE_CALL(tkMemset(Abuf, 0, maxA * 2));
-    fl.push_back(Abuf);
+    void *Abuf = zeroed(fl, maxA * 2);
+
+    void *X1 = nullptr, *X2 = nullptr, *X3 = nullptr;   // the fully connected layers' operands
+    auto halfBuf = [&](void **p, size_t n) { *p = zeroed(fl, n * 2); };
 
     // A convolution leaves 1.1 * A * B^T in its output buffer; bias and ReLU are applied by
     // whatever reads that buffer next (the next layer's operand gather, or the pooling).
@@ -255,13 +440,29 @@ VGG16::VGG16(int taskId, const VGG16Options &o) : Task(taskId, "vgg16"), opt(o),
         float *bias = randomBias(fl, rng, Cout, Np);
         float *out = devAlloc(fl, (size_t)pad128(H * W) * Np);
         void *operand = Abuf;
-        if (C % 8 != 0) {   // gathered, and only its data columns rewritten: needs zeros nobody else disturbs
-            TK_SAFE_CALL(tkMalloc(&operand, (size_t)pad128(H * W) * Kp * 2));
-            TK_SAFE_CALL(tkMemset(operand, 0, (size_t)pad128(H * W) * Kp * 2));
-            fl.push_back(operand);
+        if (C % 8 != 0)   // gathered, and only its data columns rewritten: needs zeros nobody else disturbs
+            operand = zeroed(fl, (size_t)pad128(H * W) * Kp * 2);
+        auto *conv = new ConvKernel(id++, "Convolution_" + name, act, act_bias, pooled, H, W, C, ld, Cout, operand, Wt, out);
+        addKernel(conv);
+        if (haveDirectKernels()) {
+            // what the next layer reads: this layer's activation, pooled if a pooling follows, in a frame of
+            // zeros -- or, behind the last convolution, the classifier's input row
+            const int i = (int)impl->convOut.size();
+            Activation &a = impl->act[i];
+            a.channels = Cout;
+            a.out = DnnOutput{out, bias, nullptr, H, W, Np, 0, Cout, 0, plan[step + 1] < 0 ? 1 : 0};
+            const int ho = a.out.pool ? H / 2 : H, wo = a.out.pool ? W / 2 : W;
+            if (i < 12) {
+                a.out.border = 1;
+                a.out.act_pitch = wo + 2;
+                halfBuf(&a.out.act, (size_t)(ho + 2) * (wo + 2) * Cout);
+            } else {
+                a.out.act_pitch = wo;
+                halfBuf(&X1, (size_t)128 * pad128(ho * wo * Cout));
+                a.out.act = X1;
+            }
+            conv->useDirect(i == 0 ? nullptr : &impl->act[i - 1], &a, weightFragments(fl, Wt, Np, Kp));
         }
-        addKernel(new ConvKernel(id++, "Convolution_" + name, act, act_bias, pooled, H, W, C, ld, Cout, operand, Wt,
-                                 out));
         pooled = false;
         impl->convOut.push_back(Act{out, H, W, Cout, Np, Wt, bias, Np, Kp});
         act = out;
@@ -272,13 +473,7 @@ VGG16::VGG16(int taskId, const VGG16Options &o) : Task(taskId, "vgg16"), opt(o),
     // classifier: 512*(H/32)*(W/32) -> 4096 -> 4096 -> classes; activations travel as
     // row 0 of the previous FC output, bias+ReLU applied while packing the next input
     const int feat = H * W * C;   // NHWC flatten (ld == C == 512 here)
-    void *X1 = nullptr, *X2 = nullptr, *X3 = nullptr;
-    auto halfBuf = [&](void **p, size_t n) {
-        TK_SAFE_CALL(tkMalloc(p, n * 2));
-        TK_SAFE_CALL(tkMemset(*p, 0, n * 2));
-        fl.push_back(*p);
-    };
-    halfBuf(&X1, (size_t)128 * pad128(feat));
+    if (!X1) halfBuf(&X1, (size_t)128 * pad128(feat));
     halfBuf(&X2, (size_t)128 * 4096);
     halfBuf(&X3, (size_t)128 * 4096);
     void *W1 = randomHalfMatrix(fl, rng, 4096, feat, 4096, pad128(feat), std::sqrt(2.0f / feat));
@@ -288,9 +483,17 @@ VGG16::VGG16(int taskId, const VGG16Options &o) : Task(taskId, "vgg16"), opt(o),
     float *o1 = devAlloc(fl, (size_t)128 * 4096), *o2 = devAlloc(fl, (size_t)128 * 4096);
     float *o3 = devAlloc(fl, (size_t)128 * pad128(opt.classes));
     // act is conv5_3's raw output; its pooling, bias and ReLU happen while fc1's input is packed
-    addKernel(new FcKernel(id++, "Dot_fc1", act, 1, act_bias, 1, feat, 4096, W1, X1, o1, pooled ? unpooled_W : 0, ld, C));
-    addKernel(new FcKernel(id++, "Dot_fc2", o1, 1, b1, 1, 4096, 4096, W2, X2, o2));
-    addKernel(new FcKernel(id++, "Dot_fc3", o2, 1, b2, 1, 4096, opt.classes, W3, X3, o3));
+    auto *fc1 = new FcKernel(id++, "Dot_fc1", act, 1, act_bias, 1, feat, 4096, W1, X1, o1, pooled ? unpooled_W : 0, ld, C);
+    auto *fc2 = new FcKernel(id++, "Dot_fc2", o1, 1, b1, 1, 4096, 4096, W2, X2, o2);
+    auto *fc3 = new FcKernel(id++, "Dot_fc3", o2, 1, b2, 1, 4096, opt.classes, W3, X3, o3);
+    for (auto *fc : {fc1, fc2, fc3}) addKernel(fc);
+    if (haveDirectKernels()) {
+        bool *fresh = impl->fcInput;
+        fc1->useDirect(&impl->act[12].fresh, &fresh[1], weightFragments(fl, W1, 4096, pad128(feat)), o1, b1, X2);
+        fc2->useDirect(&fresh[1], &fresh[2], weightFragments(fl, W2, 4096, 4096), o2, b2, X3);
+        fc3->useDirect(&fresh[2], nullptr, weightFragments(fl, W3, pad128(opt.classes), 4096), o3, nullptr, nullptr);
+        TK_SAFE_CALL(tkDeviceSynchronize());   // the fragments are laid out before a kernel on any stream reads them
+    }
     impl->convOut.push_back(Act{o1, 1, 1, 4096, 4096, W1, b1, 4096, pad128(feat)});
     impl->convOut.push_back(Act{o2, 1, 1, 4096, 4096, W2, b2, 4096, 4096});
     impl->convOut.push_back(Act{o3, 1, 1, opt.classes, pad128(opt.classes), W3, nullptr, pad128(opt.classes), 4096});
@@ -298,10 +501,15 @@ VGG16::VGG16(int taskId, const VGG16Options &o) : Task(taskId, "vgg16"), opt(o),
     impl->logitsStride = 1;
 }
 
+void VGG16::captured()
+{
+    for (auto &a : impl->act) a.fresh = false;
+    for (bool &f : impl->fcInput) f = false;
+}
+
 VGG16::~VGG16()
 {
     for (auto *k : kernels) delete k;
-    for (void *p : impl->freeList) tkErrCheck(tkFree(p));
 }
 
 void VGG16::initExecution()

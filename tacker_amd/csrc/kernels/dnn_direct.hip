@@ -1,0 +1,447 @@
+// The layers of the latency-critical DNN task (VGG16, batch 1) as launches of their own: a convolution that reads
+// its input activation where it lies instead of an im2col operand in memory, and a fully connected layer as the
+// matrix-vector product it is.  They are what a layer runs when nothing is fused with it; a layer that shares its
+// launch with a best-effort kernel goes through im2col and the tzgemm role (dnn_kernels.h, the generated fused
+// kernels), and both give the same bits: every element of C is added up in the order of tzgemm_role --
+// v_mfma_f32_16x16x32_f16 over ascending k, and for the shapes whose reduction tzgemm cuts (tz_use_ksplit) the
+// same quarters of the same parts, ((w0 + w1) + w2) + w3, parts in order.
+//
+// Data.  An activation is f16 NHWC with a border of one zero pixel, [H + 2][W + 2][C], written by the layer before
+// with bias, ReLU and -- where a pooling follows -- the 2x2 maximum applied; beside it every layer leaves its raw
+// 1.1 * A * B^T in fp32 as the operand builders expect it.  Weights are laid out once, at the task's creation, in the
+// order the matrix instruction takes them (pack_weight_fragments): fragment (16 output channels, 32 k) is
+// 1 KiB in a row, lane l's 16 bytes at 16 l.
+#include <hip/hip_runtime.h>
+
+#include "../../../include/tacker_amd.h"
+#include "../header/tzgemm_header.h"
+#include "../dnn/direct.h"
+
+namespace tk {
+
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
+typedef float float4_t __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) char lds_char;
+typedef __attribute__((address_space(3))) const half8_t lds_half8;
+typedef __attribute__((address_space(3))) float4_t lds_float4;
+typedef __attribute__((address_space(3))) float lds_float;
+
+#define DNN_VMCNT_IMM(n) (((n) & 15) | (((n) >> 4) << 14) | 0x0F70)   // s_waitcnt vmcnt(n), nothing else
+
+// One LDS-direct load of 16 bytes per lane: scalar base + 32-bit lane offset, to LDS address + 16 lane.
+__device__ __forceinline__ void dnn_load_to_lds(const char *uniform_base, unsigned lane_offset, unsigned lds_address)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 :
+                 : "s"(lds_address), "v"(lane_offset), "s"(uniform_base)
+                 : "memory");
+}
+
+__device__ __forceinline__ half4_t dnn_activate(float4_t v, float4_t bias)
+{
+    v += bias;
+    half4_t h;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) h[i] = (_Float16)(v[i] < 0.0f ? 0.0f : v[i]);
+    return h;
+}
+
+// Where float4 q (channels 4 q ..) of pixel p of a tile of `quads` float4s a pixel lies in LDS, in units of 16 bytes: row p,
+// with a key that spreads a matrix instruction's result (16 pixels, one q) and a row's reads alike over all banks
+__device__ __forceinline__ int dnn_tile_at(int p, int q, int quads)
+{
+    return p * quads + (q ^ (quads >= 8 ? p & 7 : (p >> 1) & 3));
+}
+
+// The pixel p of an 8 x 8 tile: four 2x2 cells side by side per group of 16 (the rows of a matrix instruction), groups
+// two image rows apart
+__device__ __forceinline__ int dnn_tile_x(int p) { return 2 * ((p >> 2) & 3) + (p & 1); }
+__device__ __forceinline__ int dnn_tile_y(int p) { return 2 * (p >> 4) + ((p >> 1) & 1); }
+
+// n / d by the host's reciprocal (2^32 / d rounded up, 0 for d = 1): exact for the tile numbers of any image
+__device__ __forceinline__ int dnn_div(int n, unsigned reciprocal) { return reciprocal ? (int)__umulhi((unsigned)n, reciprocal) : n; }
+
+// A tile's results from LDS to memory.  `partials` tiles of [pixel][quads] lie in LDS, to be added in tzgemm's order
+// (parts of four segments, or -- parts_only -- sums of whole parts); n0: first channel.  Lanes take a pixel's channels
+// side by side, so that a pixel's row goes out in one piece: the raw value to C, the activation -- of the pixel, or of its
+// 2x2 cell -- to the next layer's input.
+__device__ __forceinline__ void dnn_finish(lds_float4 *tile, int partials, bool parts_only, int quads, int y0, int x0, int n0,
+                                           const DnnOutput &o)
+{
+    const int threads = (int)blockDim.x, quad_shift = __builtin_ctz(quads);
+    const int stride = DNN_TILE * DNN_TILE * quads;
+    for (int i = (int)threadIdx.x; i < stride; i += threads) {
+        const int p = i >> quad_shift, q = i & (quads - 1);
+        const int at = dnn_tile_at(p, q, quads);
+        float4_t v = tile[at];
+        if (parts_only) {
+            for (int s = 1; s < partials; ++s) v += tile[s * stride + at];
+        } else if (partials > 1) {
+            for (int s = 0; s < partials; s += 4) {
+                float4_t part = tile[s * stride + at];
+                part += tile[(s + 1) * stride + at];
+                part += tile[(s + 2) * stride + at];
+                part += tile[(s + 3) * stride + at];
+                v = s == 0 ? part : v + part;
+            }
+        }
+        v *= TZ_ALPHA;
+        const int y = y0 + dnn_tile_y(p), x = x0 + dnn_tile_x(p), n = n0 + 4 * q;
+        if (y < o.H && x < o.W) {
+            *reinterpret_cast<float4_t *>(o.raw + (size_t)(y * o.W + x) * o.ld + n) = v;
+            if (!o.pool)
+                *reinterpret_cast<half4_t *>(reinterpret_cast<_Float16 *>(o.act) +
+                                             (size_t)((y + o.border) * o.act_pitch + x + o.border) * o.act_C + n) =
+                    dnn_activate(v, *reinterpret_cast<const float4_t *>(o.bias + n));
+        }
+        if (o.pool) tile[at] = v;
+    }
+    if (!o.pool) return;
+    __syncthreads();
+    for (int i = (int)threadIdx.x; i < stride / 4; i += threads) {
+        const int cell = i >> quad_shift, q = i & (quads - 1);
+        float4_t v = tile[dnn_tile_at(4 * cell, q, quads)];
+#pragma unroll
+        for (int e = 1; e < 4; ++e) {
+            const float4_t w = tile[dnn_tile_at(4 * cell + e, q, quads)];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = fmaxf(v[j], w[j]);
+        }
+        const int y = y0 + dnn_tile_y(4 * cell), x = x0 + dnn_tile_x(4 * cell), n = n0 + 4 * q;
+        if (y < o.H && x < o.W)
+            *reinterpret_cast<half4_t *>(reinterpret_cast<_Float16 *>(o.act) +
+                                         (size_t)((y / 2 + o.border) * o.act_pitch + x / 2 + o.border) * o.act_C + n) =
+                dnn_activate(v, *reinterpret_cast<const float4_t *>(o.bias + n));
+    }
+}
+
+// workgroup -> (pixel tile, channel group): every XCD takes a contiguous run of the order "channel group, then pixel
+// tile", so that a group's weights come into few L2s
+__device__ __forceinline__ int dnn_tile_of(int block, int tiles)
+{
+    const int per = (tiles + TK_XCD_NUM - 1) / TK_XCD_NUM;
+    return (block % TK_XCD_NUM) * per + block / TK_XCD_NUM;
+}
+
+}  // namespace tk
+
+using namespace tk;
+
+// 3x3 / pad 1 / stride 1 convolution of an activation with C a multiple of 64 channels.  A workgroup computes an 8 x 8
+// pixel tile by 16 * ct_count output channels; wavefront (cp, kw) of it 16 * NT channels over a run of the reduction:
+// one segment, a whole part (PART: its four segments one after the other, added as tzgemm adds them), or all of it
+// where tzgemm does not cut it.
+//
+// The tile's input, 10 x 10 pixels x C, is brought into LDS once (im2col would read it nine times) and the k loop
+// runs without a barrier: a wavefront reads its 64 pixels' fragments from LDS at the tap's offset and its own
+// weights, which no other wavefront of the workgroup needs, straight from memory into registers, RING chunks ahead.
+// LDS rows are a pixel's 64 channels (128 bytes), one plane per 64 channels; 16-byte segment s of a pixel lies in
+// slot s ^ key, key = (x / 2 + 4 (y & 1)) & 7, which spreads the 16 pixels of a fragment read (8 x 2, at any
+// tap) over all banks.
+//
+// What bounds it is the rate at which a CU takes data in, 80 to 100 GB/s from the L2s: at 28 x 28, 512 -> 512 channels a
+// workgroup (64 pixels x 32 channels, one per CU) loads 104 KB of patch and 295 KB of weights, 4.4 us of a 9.1 us
+// kernel; launch and the first load's latency are 3 us, the last sums and stores 1.5.  So a workgroup takes as many
+// channels as leave every CU one, and two 16-channel slices a wavefront (NT = 2), which halves the fragment reads from
+// LDS, where eight wavefronts are left; the patch is asked for before the weights.  us a layer of VGG16 at 224 x
+// 224, against the operand in memory and tzgemm: conv1_2 38 -> 12, conv2_2 26 -> 10, conv3_2 21 -> 9.3, conv4_2 23 -> 9.1,
+// conv5_1 18 -> 8.0.
+template <int NT, bool PART>
+__device__ __forceinline__ void conv3x3_direct(const DnnConv &c, char *lds_generic)
+{
+    lds_char *const lds = (lds_char *)lds_generic;
+    const int lane = (int)threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int waves = (int)blockDim.x >> 6;
+    const int tile = dnn_tile_of((int)blockIdx.x, c.workgroups);
+    if (tile >= c.workgroups) return;
+    const int group = dnn_div(tile, c.per_group);
+    const int pixel_tile = tile - group * c.tiles;
+    const int tile_row = dnn_div(pixel_tile, c.per_row);
+    const int y0 = tile_row * DNN_TILE, x0 = (pixel_tile - tile_row * c.tiles_x) * DNN_TILE;
+    const int ct_shift = __builtin_ctz(c.ct_count / NT);
+    const int cp = wave & ((1 << ct_shift) - 1), kw = wave >> ct_shift;
+    const int n16 = group * c.ct_count + cp * NT;
+    const int H = c.out.H, W = c.out.W;
+    const int planes = c.C >> 6, plane_shift = __builtin_ctz(planes);
+
+    // this wavefront's chunks, and with PART where its second, third and fourth segment begin
+    const int *begin = c.segment_begin + (PART ? 4 * kw : kw);
+    const int first = begin[0], last = begin[PART ? 4 : 1];
+    const int second = PART ? begin[1] : last, third = PART ? begin[2] : last, fourth = PART ? begin[3] : last;
+
+    // the patch: 13 pieces of 8 pixels, every plane of a piece by one wavefront
+    const unsigned lds_base = (unsigned)(size_t)lds;
+    for (int piece = wave; piece < DNN_PATCH_LOADS; piece += waves) {
+        const int p = min(8 * piece + (lane >> 3), DNN_PATCH * DNN_PATCH - 1);
+        const int py = (p * 205) >> 11, px = p - py * DNN_PATCH;   // p / 10 for p < 1024
+        const int gy = min(y0 + py, H + 1), gx = min(x0 + px, W + 1);
+        const int key = ((px >> 1) + 4 * (py & 1)) & 7;
+        const unsigned at = (unsigned)((gy * (W + 2) + gx) * c.C + (((lane & 7) ^ key) << 3)) * 2u;
+        for (int plane = 0; plane < planes; ++plane)
+            dnn_load_to_lds(reinterpret_cast<const char *>(c.act) + plane * 128, at,
+                            lds_base + plane * DNN_PLANE_BYTES + piece * 1024);
+    }
+    // behind it the first chunks of the weights; the patch has landed when only they are still on their way
+    constexpr int RING = 3;
+    const half8_t *weights = reinterpret_cast<const half8_t *>(c.weights) + (size_t)n16 * c.chunks * 2 * 64 + lane;
+    half8_t b[RING][NT][2];
+    const auto fetch = [&](half8_t (&w)[NT][2], int chunk) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) w[t][h] = weights[(size_t)(t * c.chunks * 2 + 2 * chunk + h) * 64];
+    };
+#pragma unroll
+    for (int u = 0; u < RING; ++u) fetch(b[u], min(first + u, c.chunks - 1));
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(DNN_VMCNT_IMM(2 * NT * RING));
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+
+    const int r = lane & 15;
+    const int tx = dnn_tile_x(r), ty = dnn_tile_y(r);
+    float4_t acc[NT][4], sum[NT][4];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) acc[t][g] = sum[t][g] = float4_t{0.f, 0.f, 0.f, 0.f};
+
+    const auto multiply = [&](const half8_t (&w)[NT][2], int chunk) {
+        const int tap = chunk >> plane_shift, plane = chunk & (planes - 1);
+        const int kh = (tap * 11) >> 5, kx = tap - 3 * kh;   // tap / 3 for tap < 9
+        const int px = tx + kx, py = ty + kh;
+        const int key = ((px >> 1) + 4 * (py & 1)) & 7;
+        const unsigned at = (unsigned)(plane * DNN_PLANE_BYTES + (py * DNN_PATCH + px) * 128 + (((lane >> 4) ^ key) << 4));
+        half8_t a0[4], a1[4];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            a0[g] = *(lds_half8 *)(lds + at + g * (2 * DNN_PATCH * 128));
+            a1[g] = *(lds_half8 *)(lds + (at ^ 64u) + g * (2 * DNN_PATCH * 128));
+        }
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) acc[t][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[t][0], a0[g], acc[t][g], 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) acc[t][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[t][1], a1[g], acc[t][g], 0, 0, 0);
+    };
+    int segment = 1;
+    const auto segment_done = [&]() {   // ((w0 + w1) + w2) + w3
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                sum[t][g] = segment == 1 ? acc[t][g] : sum[t][g] + acc[t][g];
+                acc[t][g] = float4_t{0.f, 0.f, 0.f, 0.f};
+            }
+        ++segment;
+    };
+    const auto next_begins = [&]() -> int { return segment == 1 ? second : (segment == 2 ? third : (segment == 3 ? fourth : last)); };
+    for (int base = first; base < last; base += RING) {
+#pragma unroll
+        for (int u = 0; u < RING; ++u) {
+            const int chunk = base + u;
+            if (chunk < last) {   // uniform
+                if (PART)
+                    while (chunk == next_begins()) segment_done();
+                multiply(b[u], chunk);
+                fetch(b[u], min(chunk + RING, c.chunks - 1));
+            }
+        }
+    }
+    if (PART)
+        while (segment <= 4) segment_done();
+
+    // results to LDS, [run of the reduction][pixel][channels]; the patch is done with
+    __syncthreads();
+    lds_float4 *const results = (lds_float4 *)lds;
+    const int quads = 4 * c.ct_count;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+            results[kw * DNN_TILE * DNN_TILE * quads + dnn_tile_at(16 * g + r, 4 * (cp * NT + t) + (lane >> 4), quads)] =
+                PART ? sum[t][g] : acc[t][g];
+    __syncthreads();
+    dnn_finish(results, c.runs, PART, quads, y0, x0, group * c.ct_count * 16, c.out);
+}
+
+#define DNN_CONV_KERNEL(NT_, PART_, THREADS_)                                                                        \
+    extern "C" __global__ __launch_bounds__(THREADS_) void conv3x3_direct_##NT_##_##PART_(DnnConv c)                   \
+    {                                                                                                                 \
+        extern __shared__ __align__(16) char conv_lds[];                                                              \
+        conv3x3_direct<NT_, PART_ != 0>(c, conv_lds);                                                                  \
+    }
+DNN_CONV_KERNEL(1, 0, 1024)
+DNN_CONV_KERNEL(1, 1, 512)
+DNN_CONV_KERNEL(2, 0, 512)
+DNN_CONV_KERNEL(2, 1, 512)
+
+// The first convolution: the image, [H][W][3] fp32, 27 k in one matrix instruction.  A workgroup computes an 8 x 8 pixel
+// tile by 64 channels, wavefront g the pixel group g; a lane gathers its 8 k (of 32; the last 5 are padding) of its pixel.
+extern "C" __global__ __launch_bounds__(256) void conv3x3_image(const float *image, DnnConv c)
+{
+    __shared__ __align__(16) char image_lds[DNN_TILE * DNN_TILE * 64 * 4];
+    lds_float4 *const results = (lds_float4 *)(lds_char *)image_lds;
+    const int lane = (int)threadIdx.x & 63;
+    const int g = (int)threadIdx.x >> 6;
+    const int tile = dnn_tile_of((int)blockIdx.x, c.workgroups);
+    if (tile >= c.workgroups) return;
+    const int tile_row = dnn_div(tile, c.per_row);
+    const int y0 = tile_row * DNN_TILE, x0 = (tile - tile_row * c.tiles_x) * DNN_TILE;
+    const int H = c.out.H, W = c.out.W;
+    const int r = lane & 15;
+    const int x = x0 + dnn_tile_x(r), y = y0 + 2 * g + dnn_tile_y(r);
+    // all eight loads at once, from indices clamped to the image; what lies outside becomes zero afterwards
+    float v[8];
+    bool in[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const int k = 8 * (lane >> 4) + e;
+        const int tap = k / 3, ch = k - 3 * tap;
+        const int kh = tap / 3, kx = tap - 3 * kh;
+        const int yy = y + kh - 1, xx = x + kx - 1;
+        in[e] = k < 27 && yy >= 0 && yy < H && xx >= 0 && xx < W;
+        v[e] = image[(min(max(yy, 0), H - 1) * W + min(max(xx, 0), W - 1)) * 3 + ch];
+    }
+    const half8_t *weights = reinterpret_cast<const half8_t *>(c.weights) + lane;
+    half8_t w[4], a;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w[j] = weights[(size_t)(j * c.chunks * 2) * 64];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) a[e] = (_Float16)(in[e] ? v[e] : 0.0f);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const float4_t zero = {0.f, 0.f, 0.f, 0.f};
+        results[dnn_tile_at(16 * g + r, 4 * j + (lane >> 4), 16)] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[j], a, zero, 0, 0, 0);
+    }
+    __syncthreads();
+    dnn_finish(results, 1, false, 16, y0, x0, 0, c.out);
+}
+
+// A fully connected layer at batch 1: 16 outputs per workgroup, a wavefront takes SPW consecutive segments of the
+// reduction and streams their weights past the caches (nontemporal: a query reads each of them once).  All 16 rows of the
+// matrix instruction's other operand are the activation vector; its first row is the layer's.
+template <int SPW>
+__device__ __forceinline__ void fc_direct(const DnnFc &f)
+{
+    __shared__ float partial[16 * SPW][16];
+    const int lane = (int)threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const half8_t *weights = reinterpret_cast<const half8_t *>(f.weights) + ((size_t)blockIdx.x * f.chunks * 2) * 64 + lane;
+    const half8_t *x = reinterpret_cast<const half8_t *>(f.x) + (lane >> 4);
+#pragma unroll
+    for (int i = 0; i < SPW; ++i) {
+        const int s = wave * SPW + i;
+        if (s < f.segments) {
+            const int first = 2 * f.segment_begin[s], last = 2 * f.segment_begin[s + 1];
+            float4_t acc = {0.f, 0.f, 0.f, 0.f};
+            int k = first;   // in steps of 32
+            constexpr int U = 8;
+            for (; k + U <= last; k += U) {
+                half8_t w[U], a[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    w[u] = __builtin_nontemporal_load(weights + (size_t)(k + u) * 64);
+                    a[u] = x[4 * (k + u)];
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[u], a[u], acc, 0, 0, 0);
+            }
+            for (; k < last; k += 2) {
+                half8_t w[2], a[2];
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    w[u] = __builtin_nontemporal_load(weights + (size_t)(k + u) * 64);
+                    a[u] = x[4 * (k + u)];
+                }
+#pragma unroll
+                for (int u = 0; u < 2; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[u], a[u], acc, 0, 0, 0);
+            }
+            if ((lane & 15) == 0) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) partial[s][4 * (lane >> 4) + e] = acc[e];
+            }
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < 16) {
+        const int n = (int)blockIdx.x * 16 + (int)threadIdx.x;
+        float v = 0.0f;
+        for (int s = 0; s < f.segments; s += 4) {
+            float part = partial[s][threadIdx.x];
+            part += partial[s + 1][threadIdx.x];
+            part += partial[s + 2][threadIdx.x];
+            part += partial[s + 3][threadIdx.x];
+            v = s == 0 ? part : v + part;
+        }
+        v *= TZ_ALPHA;
+        f.raw[n] = v;
+        if (f.act) {
+            v += f.bias[n];
+            reinterpret_cast<_Float16 *>(f.act)[n] = (_Float16)(v < 0.0f ? 0.0f : v);
+        }
+    }
+}
+extern "C" __global__ __launch_bounds__(1024) void fc_direct_1(DnnFc f) { fc_direct<1>(f); }
+extern "C" __global__ __launch_bounds__(1024) void fc_direct_2(DnnFc f) { fc_direct<2>(f); }
+
+// The activation of a layer whose raw output another kernel wrote (a launch fused with a best-effort kernel), for a next
+// layer that runs by itself: a thread per four channels of a pixel, or of a 2x2 cell.
+extern "C" __global__ __launch_bounds__(256) void dnn_activation(DnnOutput o, int channels)
+{
+    const int Ho = o.pool ? o.H / 2 : o.H, Wo = o.pool ? o.W / 2 : o.W;
+    const int quads = channels / 4;
+    const int total = Ho * Wo * quads;
+    for (int i = (int)(blockIdx.x * blockDim.x + threadIdx.x); i < total; i += (int)(gridDim.x * blockDim.x)) {
+        const int p = i / quads, n = 4 * (i - p * quads);
+        const int y = p / Wo, x = p - y * Wo;
+        float4_t v;
+        if (o.pool) {
+            const float *at = o.raw + (size_t)(2 * y * o.W + 2 * x) * o.ld + n;
+            const float4_t a = *reinterpret_cast<const float4_t *>(at);
+            const float4_t b = *reinterpret_cast<const float4_t *>(at + o.ld);
+            const float4_t d = *reinterpret_cast<const float4_t *>(at + (size_t)o.W * o.ld);
+            const float4_t e = *reinterpret_cast<const float4_t *>(at + (size_t)o.W * o.ld + o.ld);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = fmaxf(fmaxf(a[j], b[j]), fmaxf(d[j], e[j]));
+        } else {
+            v = *reinterpret_cast<const float4_t *>(o.raw + (size_t)p * o.ld + n);
+        }
+        *reinterpret_cast<half4_t *>(reinterpret_cast<_Float16 *>(o.act) + (size_t)((y + o.border) * o.act_pitch + x + o.border) * o.act_C + n) =
+            dnn_activate(v, *reinterpret_cast<const float4_t *>(o.bias + n));
+    }
+}
+
+// [rows][K] f16 (rows a multiple of 16, K of 64) -> fragments: 16-byte segment (n, k / 8) to fragment (n / 16, k / 32),
+// lane n % 16 + 16 * (k / 8 % 4)
+extern "C" __global__ __launch_bounds__(256) void pack_weight_fragments(const void *src_, void *dst_, int rows, int K)
+{
+    const half8_t *src = reinterpret_cast<const half8_t *>(src_);
+    half8_t *dst = reinterpret_cast<half8_t *>(dst_);
+    const size_t per_row = (size_t)K / 8, total = (size_t)rows * per_row;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x) {
+        // i: destination segment, so that the writes are the contiguous side
+        const size_t fragment = i >> 6;
+        const int lane = (int)(i & 63);
+        const size_t n16 = fragment / (per_row / 4), step = fragment - n16 * (per_row / 4);
+        dst[i] = src[(n16 * 16 + (lane & 15)) * per_row + step * 4 + (lane >> 4)];
+    }
+}
+
+extern "C" void tk_register_dnn_kernels(tk_kernel_insert_fn insert, void *ctx)
+{
+    insert("conv3x3_direct_1_0", (const void *)conv3x3_direct_1_0, ctx);
+    insert("conv3x3_direct_1_1", (const void *)conv3x3_direct_1_1, ctx);
+    insert("conv3x3_direct_2_0", (const void *)conv3x3_direct_2_0, ctx);
+    insert("conv3x3_direct_2_1", (const void *)conv3x3_direct_2_1, ctx);
+    insert("conv3x3_image", (const void *)conv3x3_image, ctx);
+    insert("fc_direct_1", (const void *)fc_direct_1, ctx);
+    insert("fc_direct_2", (const void *)fc_direct_2, ctx);
+    insert("dnn_activation", (const void *)dnn_activation, ctx);
+    insert("pack_weight_fragments", (const void *)pack_weight_fragments, ctx);
+}

@@ -329,6 +329,7 @@ extern "C" __global__ void convertFp32ToFp16_(_Float16 *out, float *in, int n)
 
 // ------------------------------------------------------------------ registry
 extern "C" void tk_register_large_kernels(tk_kernel_insert_fn insert, void *ctx);   // tzgemm_large.hip
+extern "C" void tk_register_dnn_kernels(tk_kernel_insert_fn insert, void *ctx);     // dnn_direct.hip
 
 extern "C" TK_API int tk_register_kernels(tk_kernel_insert_fn insert, void *ctx)
 {
@@ -362,6 +363,7 @@ extern "C" TK_API int tk_register_kernels(tk_kernel_insert_fn insert, void *ctx)
     tk_register_gptb_kernels(insert, ctx);
     tk_register_mix_kernels(insert, ctx);
     tk_register_large_kernels(insert, ctx);
+    tk_register_dnn_kernels(insert, ctx);
     return TK_SUCCESS;
 }
 

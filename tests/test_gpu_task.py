@@ -390,3 +390,42 @@ def test_a_recorded_query_gives_the_eager_logits_on_every_replay():
     graph.close()
     assert l.tkStreamDestroy(stream) == 0
     task.close()
+
+
+@pytest.mark.parametrize("H,W", [(32, 32), (32, 160), (96, 32), (64, 224), (224, 224)])
+def test_a_layer_by_itself_gives_the_bits_of_its_operand_and_tzgemm(H, W):
+    # activations from 14 x 14 tiles of 8 x 8 pixels down to single pixels, whole and partial tiles, one segment of the
+    # reduction and up to 32, a wavefront a segment and a wavefront a part, one and two 16-channel slices: every
+    # layer of the query, which runs through its direct kernel, against im2col and tzgemm on the layer before's raw
+    # output.  The order of the additions is the same, so the bits are.
+    from gpu_util import launch
+    task = ta.LcTask("vgg16", H, W)
+    task.execute()
+    torch.cuda.synchronize()
+    i = C.c_int
+    raw, bias = dev(task.host_input().reshape(H, W, 3)), None
+    for idx in range(16):
+        ptr, (h, w_, cout, ld) = task.activation(idx)
+        w, b = task.conv_params(idx)
+        rows, Kp = (h * w_ if idx < 13 else 1), w.shape[1]
+        A = torch.zeros((-(-rows // 128) * 128, Kp), dtype=torch.float16, device="cuda:0")
+        ap, rp = C.c_void_p(A.data_ptr()), C.c_void_p(raw.data_ptr())
+        if idx == 0:
+            launch("im2col_nhwc_f16", 64, 256, [rp, i(H), i(W), i(3), i(3), i(3), i(3), i(1), i(1), i(h), i(w_), ap, i(Kp),
+                                                C.c_void_p(0), i(1), i(0)])
+        elif idx < 13:
+            launch("im2col3x3_scatter_nhwc_f16", 64, 256, [rp, i(h), i(w_), i(cin), i(raw.shape[2]), ap, i(Kp),
+                                                           C.c_void_p(bias.data_ptr()), i(1), i(int(raw.shape[0] != h))])
+        else:
+            x = torch.relu(raw + bias)
+            if idx == 13:
+                x = x.reshape(x.shape[0] // 2, 2, x.shape[1] // 2, 2, -1).amax(dim=(1, 3))
+            x = x.reshape(-1).half()
+            A[0, :x.numel()] = x
+        want = torch.empty((A.shape[0], w.shape[0]), dtype=torch.float32, device="cuda:0")
+        ta.gptb_tzgemm(A, dev(w), want)
+        torch.cuda.synchronize()
+        got = ta.device_to_host(ptr, (rows, ld), np.float32)
+        assert np.array_equal(got.view(np.uint32), host(want)[:rows].view(np.uint32)), idx
+        raw, bias, cin = dev(got.reshape((h, w_, ld) if idx < 13 else (ld,))), dev(b), cout
+    task.close()
