@@ -68,6 +68,9 @@ TK_API int tkFree(void *ptr);                                            /* cuda
  * No counterpart in the reference: a caller that must not allocate (stream capture, a serving
  * loop) reads it before and after a call to see that the library kept to that. */
 TK_API int tkAllocationCalls(long long *mallocs, long long *frees);
+/* cudaMallocHost / cudaFreeHost: page-locked host memory, which kernels can read too */
+TK_API int tkHostMalloc(void **ptr, size_t bytes);
+TK_API int tkHostFree(void *ptr);
 TK_API int tkMemcpy(void *dst, const void *src, size_t bytes, int kind); /* cudaMemcpy */
 TK_API int tkMemcpyAsync(void *dst, const void *src, size_t bytes, int kind, tkStream_t s);
 TK_API int tkMemset(void *ptr, int value, size_t bytes);                 /* cudaMemset */
@@ -80,6 +83,7 @@ TK_API int tkMemcpyToSymbol(const char *symbol, const void *src, size_t bytes, s
 TK_API int tkMemcpyFromSymbol(void *dst, const char *symbol, size_t bytes, size_t offset);
 
 TK_API int tkStreamCreate(tkStream_t *s);
+TK_API int tkStreamCreateNonBlocking(tkStream_t *s); /* not ordered with the null stream */
 TK_API int tkStreamDestroy(tkStream_t s);
 TK_API int tkStreamSynchronize(tkStream_t s);
 TK_API int tkDeviceSynchronize(void);

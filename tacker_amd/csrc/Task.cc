@@ -53,6 +53,12 @@ void Task::executeTask(ExecutionMode mode, cudaStream_t stream)
     if (mode == ExecutionMode::Aker) recorder.recordTask(taskId, taskName);
 }
 
+void Task::executeQuery(cudaStream_t stream)
+{
+    initExecution();
+    for (auto &kernel : kernels) kernel->execute(stream);
+}
+
 tkGraphExec_t Task::captureQuery(cudaStream_t stream)
 {
     tkGraphExec_t graph = nullptr;

@@ -20,6 +20,8 @@ public:
     void executeTask(ExecutionMode mode, int idx, cudaStream_t stream);
     // stage the job's input (host -> device copy for a DNN query)
     virtual void initExecution() = 0;
+    // the whole job: its input staged (the host's copy may change once this returns), every kernel launched on `stream`
+    virtual void executeQuery(cudaStream_t stream);
     // the job's launches recorded from `stream` (not the null stream) into one executable graph:
     // every kernel's execute() once, none of them run.  The job must have run before, so that no
     // kernel still has buffers to allocate, and the caller stages the input before each launch of

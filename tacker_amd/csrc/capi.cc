@@ -1391,8 +1391,7 @@ int tacker_task_execute(tacker_task_t h, tkStream_t stream)
     Task *t = static_cast<Task *>(h);
     if (!t) return fail(TK_ERROR_INVALID_VALUE, "null task");
     return guarded([&]() -> int {
-        t->initExecution();
-        for (auto *k : t->kernels) k->execute(stream);
+        t->executeQuery(stream);
         return TK_SUCCESS;
     });
 }

@@ -45,6 +45,7 @@ public:
     explicit VGG16(int taskId, const VGG16Options &opt = VGG16Options());
     ~VGG16() override;
     void initExecution() override;       // host -> device copy of the input image
+    void executeQuery(cudaStream_t stream) override;
     void captured() override;            // nothing of what was recorded has run: no activation is known to be up to date
     // device pointer / length of the logits (column 0 of the last GEMM's output, stride ld)
     const float *logits(long *stride) const;

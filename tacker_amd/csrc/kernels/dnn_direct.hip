@@ -283,7 +283,8 @@ DNN_CONV_KERNEL(2, 1, 512)
 
 // The first convolution: the image, [H][W][3] fp32, 27 k in one matrix instruction.  A workgroup computes an 8 x 8 pixel
 // tile by 64 channels, wavefront g the pixel group g; a lane gathers its 8 k (of 32; the last 5 are padding) of its pixel.
-extern "C" __global__ __launch_bounds__(256) void conv3x3_image(const float *image, DnnConv c)
+// keep: null, or where the image is stored as well.
+extern "C" __global__ __launch_bounds__(256) void conv3x3_image(const float *image, float *keep, DnnConv c)
 {
     __shared__ __align__(16) char image_lds[DNN_TILE * DNN_TILE * 64 * 4];
     lds_float4 *const results = (lds_float4 *)(lds_char *)image_lds;
@@ -294,6 +295,13 @@ extern "C" __global__ __launch_bounds__(256) void conv3x3_image(const float *ima
     const int tile_row = dnn_div(tile, c.per_row);
     const int y0 = tile_row * DNN_TILE, x0 = (tile - tile_row * c.tiles_x) * DNN_TILE;
     const int H = c.out.H, W = c.out.W;
+    if (keep && threadIdx.x < 3 * DNN_TILE * DNN_TILE) {
+        const int row = (int)threadIdx.x / (3 * DNN_TILE), column = (int)threadIdx.x - row * (3 * DNN_TILE);
+        if (y0 + row < H && 3 * x0 + column < 3 * W) {
+            const int at = ((y0 + row) * W + x0) * 3 + column;
+            keep[at] = image[at];
+        }
+    }
     const int r = lane & 15;
     const int x = x0 + dnn_tile_x(r), y = y0 + 2 * g + dnn_tile_y(r);
     // all eight loads at once, from indices clamped to the image; what lies outside becomes zero afterwards
@@ -321,6 +329,12 @@ extern "C" __global__ __launch_bounds__(256) void conv3x3_image(const float *ima
     }
     __syncthreads();
     dnn_finish(results, 1, false, 16, y0, x0, 0, c.out);
+}
+
+// The image from page-locked host memory, a float4 a thread: PCIe's latency once, everything under way at the same time.
+extern "C" __global__ __launch_bounds__(256) void stage_image(const float4_t *host, float4_t *image, int n)
+{
+    for (int i = (int)(blockIdx.x * blockDim.x + threadIdx.x); i < n; i += (int)(gridDim.x * blockDim.x)) image[i] = host[i];
 }
 
 // A fully connected layer at batch 1: 16 outputs per workgroup, a wavefront takes SPW consecutive segments of the
@@ -440,6 +454,7 @@ extern "C" void tk_register_dnn_kernels(tk_kernel_insert_fn insert, void *ctx)
     insert("conv3x3_direct_2_0", (const void *)conv3x3_direct_2_0, ctx);
     insert("conv3x3_direct_2_1", (const void *)conv3x3_direct_2_1, ctx);
     insert("conv3x3_image", (const void *)conv3x3_image, ctx);
+    insert("stage_image", (const void *)stage_image, ctx);
     insert("fc_direct_1", (const void *)fc_direct_1, ctx);
     insert("fc_direct_2", (const void *)fc_direct_2, ctx);
     insert("dnn_activation", (const void *)dnn_activation, ctx);

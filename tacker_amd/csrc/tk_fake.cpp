@@ -119,6 +119,8 @@ int tkFree(void *ptr)
     free(ptr);
     return TK_SUCCESS;
 }
+int tkHostMalloc(void **ptr, size_t bytes) { return (*ptr = calloc(1, bytes ? bytes : 1)) ? TK_SUCCESS : TK_ERROR_DEVICE; }
+int tkHostFree(void *ptr) { free(ptr); return TK_SUCCESS; }
 int tkMemcpy(void *dst, const void *src, size_t bytes, int)
 {
     touched(dst);
@@ -165,6 +167,7 @@ int tk_tzgemm_scratch(void **ptr, size_t *bytes)
     return TK_SUCCESS;
 }
 int tkStreamCreate(tkStream_t *s) { *s = malloc(1); return TK_SUCCESS; }
+int tkStreamCreateNonBlocking(tkStream_t *s) { return tkStreamCreate(s); }
 int tkStreamDestroy(tkStream_t s) { free(s); return TK_SUCCESS; }
 int tkStreamSynchronize(tkStream_t) { return TK_SUCCESS; }
 int tkDeviceSynchronize(void) { return TK_SUCCESS; }

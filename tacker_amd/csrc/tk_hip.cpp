@@ -113,6 +113,8 @@ int tkAllocationCalls(long long *mallocs, long long *frees)
     if (frees) *frees = g_free_calls.load();
     return TK_SUCCESS;
 }
+int tkHostMalloc(void **ptr, size_t bytes) { return FOLD(hipHostMalloc(ptr, bytes, hipHostMallocDefault)); }
+int tkHostFree(void *ptr) { return FOLD(hipHostFree(ptr)); }
 int tkMemcpy(void *dst, const void *src, size_t bytes, int kind)
 {
     return FOLD(hipMemcpy(dst, src, bytes, kind_of(kind)));
@@ -180,6 +182,7 @@ int tkMemcpyFromSymbol(void *dst, const char *symbol, size_t bytes, size_t offse
 }
 
 int tkStreamCreate(tkStream_t *s) { return FOLD(hipStreamCreate((hipStream_t *)s)); }
+int tkStreamCreateNonBlocking(tkStream_t *s) { return FOLD(hipStreamCreateWithFlags((hipStream_t *)s, hipStreamNonBlocking)); }
 int tkStreamDestroy(tkStream_t s) { return FOLD(hipStreamDestroy((hipStream_t)s)); }
 int tkStreamSynchronize(tkStream_t s) { return FOLD(hipStreamSynchronize((hipStream_t)s)); }
 int tkDeviceSynchronize(void) { return FOLD(hipDeviceSynchronize()); }

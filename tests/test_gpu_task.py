@@ -429,3 +429,45 @@ def test_a_layer_by_itself_gives_the_bits_of_its_operand_and_tzgemm(H, W):
         assert np.array_equal(got.view(np.uint32), host(want)[:rows].view(np.uint32)), idx
         raw, bias, cin = dev(got.reshape((h, w_, ld) if idx < 13 else (ld,))), dev(b), cout
     task.close()
+
+
+@pytest.mark.parametrize("H,W,own_stream", [(32, 32, False), (96, 64, True), (224, 224, True)])
+def test_an_image_may_change_as_soon_as_the_query_is_launched(H, W, own_stream):
+    # images are staged while the query before runs, into two device images in turn: the host's one is overwritten the
+    # moment execute() returns, nothing waits in between, and every query must still have seen its own
+    task = ta.LcTask("vgg16", H, W)
+    l, stream = ta.lib(), C.c_void_p(None)
+    if own_stream:
+        assert l.tkStreamCreate(C.byref(stream)) == 0
+    image = task.host_input()
+    rng = np.random.default_rng(H + W)
+    images = rng.random((5, image.size), dtype=np.float32)
+    p, stride, n = task.logits()
+    logits = lambda: ta.device_to_host(p, (n, stride), np.float32)[:, 0].copy()
+
+    def query(k):
+        image[:] = images[k]
+        task.execute(raw_stream=stream)
+        image[:] = np.nan
+    want = []
+    for k in range(5):
+        query(k)
+        torch.cuda.synchronize()
+        want.append(logits())
+        # ... and Input[0] is left holding the image: every layer again, from there
+        image[:] = 0
+        graph = task.capture(stream) if own_stream else None
+        if graph:
+            graph.launch(stream)
+            torch.cuda.synchronize()
+            assert np.array_equal(logits(), want[k])
+            graph.close()
+    assert np.isfinite(want).all() and all(np.abs(want[0] - w).max() > 0 for w in want[1:])
+    for last in (4, 3, 0):
+        for k in (0, 3, 1, 2, 4, 2, 1, last):
+            query(k)
+        torch.cuda.synchronize()
+        assert np.array_equal(logits(), want[last]), last
+    task.close()
+    if own_stream:
+        assert l.tkStreamDestroy(stream) == 0
