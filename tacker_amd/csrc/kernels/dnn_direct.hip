@@ -331,12 +331,6 @@ extern "C" __global__ __launch_bounds__(256) void conv3x3_image(const float *ima
     dnn_finish(results, 1, false, 16, y0, x0, 0, c.out);
 }
 
-// The image from page-locked host memory, a float4 a thread: PCIe's latency once, everything under way at the same time.
-extern "C" __global__ __launch_bounds__(256) void stage_image(const float4_t *host, float4_t *image, int n)
-{
-    for (int i = (int)(blockIdx.x * blockDim.x + threadIdx.x); i < n; i += (int)(gridDim.x * blockDim.x)) image[i] = host[i];
-}
-
 // A fully connected layer at batch 1: 16 outputs per workgroup, a wavefront takes SPW consecutive segments of the
 // reduction and streams their weights past the caches (nontemporal: a query reads each of them once).  All 16 rows of the
 // matrix instruction's other operand are the activation vector; its first row is the layer's.
@@ -454,7 +448,6 @@ extern "C" void tk_register_dnn_kernels(tk_kernel_insert_fn insert, void *ctx)
     insert("conv3x3_direct_2_0", (const void *)conv3x3_direct_2_0, ctx);
     insert("conv3x3_direct_2_1", (const void *)conv3x3_direct_2_1, ctx);
     insert("conv3x3_image", (const void *)conv3x3_image, ctx);
-    insert("stage_image", (const void *)stage_image, ctx);
     insert("fc_direct_1", (const void *)fc_direct_1, ctx);
     insert("fc_direct_2", (const void *)fc_direct_2, ctx);
     insert("dnn_activation", (const void *)dnn_activation, ctx);
