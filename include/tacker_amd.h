@@ -645,7 +645,8 @@ TK_API int tacker_task_activation(tacker_task_t task, int conv_index, float **pt
 TK_API int tacker_task_logits(tacker_task_t task, const float **ptr, long *stride, int *count);
 /* VGG16 only: weights (f16 [dims[0]][dims[1]] = [Cout padded][9*Cin padded], k =
  * (kh*3+kw)*Cin + c) and bias (f32 [dims[0]]) of convolution conv_index; 13..15: of the fully
- * connected layers ([out padded][in padded]; the last one has no bias: NULL) */
+ * connected layers ([out padded][in padded]; the last one has no bias: NULL).  Weights written there
+ * are those of every later query; a graph recorded before this call keeps the ones it was recorded with */
 TK_API int tacker_task_conv_params(tacker_task_t task, int conv_index, void **weights, float **bias,
                                    int dims[2]);
 TK_API int tacker_task_input(tacker_task_t task, float **host_ptr, int *bytes);

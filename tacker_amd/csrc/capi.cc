@@ -1452,6 +1452,7 @@ int tacker_task_conv_params(tacker_task_t h, int conv_index, void **weights, flo
     VGG16 *v = dynamic_cast<VGG16 *>(static_cast<Task *>(h));
     if (!v || conv_index < 0 || conv_index >= 16) return fail(TK_ERROR_INVALID_VALUE, "bad layer index");
     const VGG16::Act a = v->activation(conv_index);
+    v->weightsHandedOut(conv_index);
     *weights = a.weights;
     *bias = a.bias;
     dims[0] = a.Np;

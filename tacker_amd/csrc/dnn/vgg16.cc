@@ -158,10 +158,14 @@ public:
                                    dim3(TZ_THREADS, 1, 1), 0, tiles_));
     }
     std::vector<int> gemmDims() const override { return {M_, N_, K_}; }
+    // set whenever the layer is launched, whoever launches it
+    void noteLaunches(bool *flag) { launched_ = flag; }
+    // somebody may write the weights from now on, of which a direct kernel reads a copy: tzgemm reads them as they are
+    virtual void weightsHandedOut() {}
 
 protected:
     virtual void before(cudaStream_t stream) = 0;   // operand staging (im2col / pack)
-    virtual void fused() {}                         // the layer's raw output is all this launch writes
+    virtual void fused() {}                         // tzgemm runs the layer: its raw output is all this launch writes
     void executeImpl(cudaStream_t stream) override
     {
         before(stream);
@@ -176,6 +180,7 @@ public:
             executeImpl(stream);
             return;
         }
+        if (launched_) *launched_ = true;
         before(stream);
         fused();
         std::unique_ptr<MixKernel> mix(createTzgemmMix(be, gptb_.get(), be_start, be_end, 0, tiles_, variant, 0, 0));
@@ -184,6 +189,7 @@ public:
 
 protected:
     int M_, N_, K_, tiles_;
+    bool *launched_ = nullptr;
     std::unique_ptr<OriTZGEMMKernel> ori_;
     std::unique_ptr<GPTBKernel> gptb_;
 };
@@ -248,6 +254,8 @@ public:
         grid_ = (unsigned)(d.workgroups + TK_XCD_NUM - 1) / TK_XCD_NUM * TK_XCD_NUM;
     }
 
+    void weightsHandedOut() override { direct_.reset(); }
+    bool direct() const { return direct_ != nullptr; }
     // the first layer, its image read from `image` and stored where the layer has it as a rule
     void executeFrom(const float *image, float *keep, cudaStream_t stream) { launchDirect(image, keep, stream); }
 
@@ -258,7 +266,11 @@ protected:
     }
     void executeImpl(cudaStream_t stream) override
     {
-        if (!direct_) return GemmLayer::executeImpl(stream);
+        if (launched_) *launched_ = true;
+        if (!direct_) {
+            fused();
+            return GemmLayer::executeImpl(stream);
+        }
         if (in_) in_->need(stream);
         launchDirect(act_, nullptr, stream);
     }
@@ -335,6 +347,7 @@ public:
         direct_->segments = reductionCut(M_, N_, K_, direct_->chunks, direct_->segment_begin);
         perWave_ = direct_->segments > 16 ? 2 : 1;
     }
+    void weightsHandedOut() override { direct_.reset(); }
 
 protected:
     void fused() override
@@ -344,7 +357,11 @@ protected:
     }
     void executeImpl(cudaStream_t stream) override
     {
-        if (!direct_) return GemmLayer::executeImpl(stream);
+        if (launched_) *launched_ = true;
+        if (!direct_) {
+            fused();
+            return GemmLayer::executeImpl(stream);
+        }
         if (!*inFresh_) before(stream);
         *inFresh_ = true;
         void *args[] = {direct_.get()};
@@ -397,6 +414,7 @@ std::shared_ptr<StagingStream> stagingStream()
 
 struct VGG16::Impl {
     Buffers buffers;
+    bool direct = false;            // layers run through the direct kernels
     float *hostInput = nullptr;     // page-locked
     size_t pixels = 0;              // floats of it
     // executeQuery: two device images taken in turn, and an event behind the query that read each last
@@ -405,6 +423,10 @@ struct VGG16::Impl {
     tkEvent_t read[2] = {};
     bool used[2] = {};
     int turn = 0;
+    // what the next query would have to wait for besides its own stream: the stream of the last one, layers launched one by
+    // one since, and graphs that may be running
+    cudaStream_t lastStream = nullptr;
+    bool queried = false, launched = false, recorded = false;
     ~Impl()
     {
         for (tkEvent_t e : read)
@@ -434,7 +456,10 @@ VGG16::VGG16(int taskId, const VGG16Options &o) : Task(taskId, "vgg16"), opt(o),
     InputHost[0] = impl->hostInput;
     Input[0] = impl->input;
     InputSize[0] = (int)(impl->pixels * sizeof(float));
-    if (haveDirectKernels()) {
+    // A larger image's tile numbers times its tiles pass 2^32, where dnn_div's reciprocals stop being exact; it runs
+    // through the operand builders and tzgemm.
+    const bool direct = impl->direct = haveDirectKernels() && (long)H * W <= 2048L * 2048;
+    if (direct) {
         impl->staging = stagingStream();
         for (int i = 0; i < 2; ++i) {
             impl->image[i] = devAlloc(fl, impl->pixels);
@@ -491,7 +516,7 @@ VGG16::VGG16(int taskId, const VGG16Options &o) : Task(taskId, "vgg16"), opt(o),
             operand = zeroed(fl, (size_t)pad128(H * W) * Kp * 2);
         auto *conv = new ConvKernel(id++, "Convolution_" + name, act, act_bias, pooled, H, W, C, ld, Cout, operand, Wt, out);
         addKernel(conv);
-        if (haveDirectKernels()) {
+        if (direct) {
             // what the next layer reads: this layer's activation, pooled if a pooling follows, in a frame of
             // zeros -- or, behind the last convolution, the classifier's input row
             const int i = (int)impl->convOut.size();
@@ -534,7 +559,8 @@ VGG16::VGG16(int taskId, const VGG16Options &o) : Task(taskId, "vgg16"), opt(o),
     auto *fc2 = new FcKernel(id++, "Dot_fc2", o1, 1, b1, 1, 4096, 4096, W2, X2, o2);
     auto *fc3 = new FcKernel(id++, "Dot_fc3", o2, 1, b2, 1, 4096, opt.classes, W3, X3, o3);
     for (auto *fc : {fc1, fc2, fc3}) addKernel(fc);
-    if (haveDirectKernels()) {
+    for (auto *k : kernels) static_cast<GemmLayer *>(k)->noteLaunches(&impl->launched);
+    if (direct) {
         bool *fresh = impl->fcInput;
         fc1->useDirect(&impl->act[12].fresh, &fresh[1], weightFragments(fl, W1, 4096, pad128(feat)), o1, b1, X2);
         fc2->useDirect(&fresh[1], &fresh[2], weightFragments(fl, W2, 4096, 4096), o2, b2, X3);
@@ -552,6 +578,7 @@ void VGG16::captured()
 {
     for (auto &a : impl->act) a.fresh = false;
     for (bool &f : impl->fcInput) f = false;
+    impl->recorded = true;
 }
 
 // The image goes over PCIe while the query before is still running: on a stream of its own, into the device image which
@@ -559,11 +586,20 @@ void VGG16::captured()
 // waits for it, and the host's image may change as soon as this returns.  A copy on the query's stream waits for
 // the query before and leaves the GPU idle until the host has seen its end and launched again: 45 us of a 206 us query
 // at 224 x 224, 37 of 133 at 64 x 96.
+// All of a task's launches share its buffers.  What was launched on another stream than this query's -- a query, single
+// layers, a recorded graph -- is waited for by that copy on the null stream, so the query then takes that way.
 void VGG16::executeQuery(cudaStream_t stream)
 {
-    auto *first = haveDirectKernels() ? dynamic_cast<ConvKernel *>(kernels.front()) : nullptr;
-    if (!first) return Task::executeQuery(stream);
     Impl &m = *impl;
+    auto *first = m.direct ? dynamic_cast<ConvKernel *>(kernels.front()) : nullptr;
+    const bool alone = !m.recorded && !m.launched && (!m.queried || m.lastStream == stream);
+    m.queried = true;
+    m.lastStream = stream;
+    if (!first || !first->direct() || !alone) {
+        Task::executeQuery(stream);
+        m.launched = false;
+        return;
+    }
     const int slot = m.turn;
     m.turn ^= 1;
     if (m.used[slot]) TK_SAFE_CALL(tkEventSynchronize(m.read[slot]));
@@ -574,6 +610,7 @@ void VGG16::executeQuery(cudaStream_t stream)
     first->executeFrom(m.image[slot], m.input, stream);
     for (size_t i = 1; i < kernels.size(); ++i) kernels[i]->execute(stream);
     TK_SAFE_CALL(tkEventRecord(m.read[slot], stream));
+    m.launched = false;
 }
 
 VGG16::~VGG16()
@@ -591,6 +628,8 @@ const float *VGG16::logits(long *stride) const
     if (stride) *stride = impl->logitsStride;
     return impl->logits;
 }
+
+void VGG16::weightsHandedOut(int layer) { static_cast<GemmLayer *>(kernels.at(layer))->weightsHandedOut(); }
 
 VGG16::Act VGG16::activation(int conv_index) const { return impl->convOut.at(conv_index); }
 

@@ -46,6 +46,7 @@ public:
     ~VGG16() override;
     void initExecution() override;       // host -> device copy of the input image
     void executeQuery(cudaStream_t stream) override;
+    void weightsHandedOut(int layer);    // a caller has the address of layer 0 .. 15's weights and may write them
     void captured() override;            // nothing of what was recorded has run: no activation is known to be up to date
     // device pointer / length of the logits (column 0 of the last GEMM's output, stride ld)
     const float *logits(long *stride) const;

@@ -471,3 +471,64 @@ def test_an_image_may_change_as_soon_as_the_query_is_launched(H, W, own_stream):
     task.close()
     if own_stream:
         assert l.tkStreamDestroy(stream) == 0
+
+
+def test_queries_on_two_streams_run_one_after_the_other():
+    # a task's launches share its buffers: a query on another stream than the last one's (ordered with the null stream, as
+    # tkStreamCreate makes them), or behind a recorded query that still runs, waits for it
+    H, W = 224, 224
+    task = ta.LcTask("vgg16", H, W)
+    l = ta.lib()
+    streams = [C.c_void_p(None) for _ in range(2)]
+    for s in streams:
+        assert l.tkStreamCreate(C.byref(s)) == 0
+    image = task.host_input()
+    images = np.random.default_rng(7).random((2, image.size), dtype=np.float32)
+    p, stride, n = task.logits()
+    logits = lambda: ta.device_to_host(p, (n, stride), np.float32)[:, 0].copy()
+    want = []
+    for k in range(2):
+        image[:] = images[k]
+        task.execute(raw_stream=streams[0])
+        torch.cuda.synchronize()
+        want.append(logits())
+    for rounds in range(1, 8):
+        for k in range(rounds + 1):
+            image[:] = images[k % 2]
+            task.execute(raw_stream=streams[k % 2])
+        torch.cuda.synchronize()
+        assert np.array_equal(logits(), want[rounds % 2]), rounds
+    graph = task.capture(streams[0])
+    for _ in range(4):
+        image[:] = images[0]
+        task.stage_input()
+        graph.launch(streams[0])
+        image[:] = images[1]
+        task.execute(raw_stream=streams[1])
+        torch.cuda.synchronize()
+        assert np.array_equal(logits(), want[1])
+    graph.close()
+    task.close()
+    for s in streams:
+        assert l.tkStreamDestroy(s) == 0
+
+
+@pytest.mark.parametrize("layer", [0, 1, 6, 12, 13, 15])
+def test_weights_written_where_a_task_keeps_them_are_those_of_the_next_query(layer):
+    task = ta.LcTask("vgg16", 32, 64)
+    task.execute()
+    torch.cuda.synchronize()
+    before = read_act(task, layer)[0].copy()
+    w, b, dims = C.c_void_p(), C.c_void_p(), (C.c_int * 2)()
+    assert ta.lib().tacker_task_conv_params(task.h, layer, C.byref(w), C.byref(b), dims) == 0
+    halved = (ta.device_to_host(w.value, (dims[0], dims[1]), np.float16) * np.float16(0.5)).astype(np.float16)
+    src = dev(halved)
+    assert ta.lib().tkMemcpy(w, C.c_void_p(src.data_ptr()), halved.nbytes, 3) == 0
+    for _ in range(2):
+        task.execute()
+        torch.cuda.synchronize()
+        got = read_act(task, layer)[0]
+        # every product is halved exactly (the weights that rounding touched are below f16's smallest normal number / 2)
+        assert np.allclose(got, before / 2, rtol=0, atol=1e-5)
+        assert np.abs(got - before).max() > 1e-3
+    task.close()
