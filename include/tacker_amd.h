@@ -84,6 +84,7 @@ TK_API int tkMemcpyFromSymbol(void *dst, const char *symbol, size_t bytes, size_
 
 TK_API int tkStreamCreate(tkStream_t *s);
 TK_API int tkStreamCreateNonBlocking(tkStream_t *s); /* not ordered with the null stream */
+TK_API int tkStreamIsBlocking(tkStream_t s, unsigned *blocking); /* cudaStreamGetFlags: ordered with the null stream? */
 TK_API int tkStreamDestroy(tkStream_t s);
 TK_API int tkStreamSynchronize(tkStream_t s);
 TK_API int tkDeviceSynchronize(void);
@@ -91,6 +92,7 @@ TK_API int tkEventCreate(tkEvent_t *e);
 TK_API int tkEventDestroy(tkEvent_t e);
 TK_API int tkEventRecord(tkEvent_t e, tkStream_t s);
 TK_API int tkEventSynchronize(tkEvent_t e);
+TK_API int tkStreamWaitEvent(tkStream_t s, tkEvent_t e);   /* cudaStreamWaitEvent */
 TK_API int tkEventElapsedTime(float *ms, tkEvent_t start, tkEvent_t stop);
 
 /* A stream's work recorded once and launched as one graph afterwards (no counterpart in the

@@ -158,8 +158,6 @@ public:
                                    dim3(TZ_THREADS, 1, 1), 0, tiles_));
     }
     std::vector<int> gemmDims() const override { return {M_, N_, K_}; }
-    // set whenever the layer is launched, whoever launches it
-    void noteLaunches(bool *flag) { launched_ = flag; }
     // somebody may write the weights from now on, of which a direct kernel reads a copy: tzgemm reads them as they are
     virtual void weightsHandedOut() {}
 
@@ -180,7 +178,6 @@ public:
             executeImpl(stream);
             return;
         }
-        if (launched_) *launched_ = true;
         before(stream);
         fused();
         std::unique_ptr<MixKernel> mix(createTzgemmMix(be, gptb_.get(), be_start, be_end, 0, tiles_, variant, 0, 0));
@@ -189,7 +186,6 @@ public:
 
 protected:
     int M_, N_, K_, tiles_;
-    bool *launched_ = nullptr;
     std::unique_ptr<OriTZGEMMKernel> ori_;
     std::unique_ptr<GPTBKernel> gptb_;
 };
@@ -266,7 +262,6 @@ protected:
     }
     void executeImpl(cudaStream_t stream) override
     {
-        if (launched_) *launched_ = true;
         if (!direct_) {
             fused();
             return GemmLayer::executeImpl(stream);
@@ -357,7 +352,6 @@ protected:
     }
     void executeImpl(cudaStream_t stream) override
     {
-        if (launched_) *launched_ = true;
         if (!direct_) {
             fused();
             return GemmLayer::executeImpl(stream);
@@ -417,19 +411,16 @@ struct VGG16::Impl {
     bool direct = false;            // layers run through the direct kernels
     float *hostInput = nullptr;     // page-locked
     size_t pixels = 0;              // floats of it
-    // executeQuery: two device images taken in turn, and an event behind the query that read each last
+    // executeQuery: two device images taken in turn, and an event behind the last query of each turn
     std::shared_ptr<StagingStream> staging;
     float *image[2] = {};
-    tkEvent_t read[2] = {};
-    bool used[2] = {};
+    tkEvent_t over[2] = {};
     int turn = 0;
-    // what the next query would have to wait for besides its own stream: the stream of the last one, layers launched one by
-    // one since, and graphs that may be running
-    cudaStream_t lastStream = nullptr;
-    bool queried = false, launched = false, recorded = false;
+    cudaStream_t lastStream = nullptr;   // the last query's
+    tkEvent_t before = nullptr;          // recorded on the null stream for a query to wait for
     ~Impl()
     {
-        for (tkEvent_t e : read)
+        for (tkEvent_t e : {over[0], over[1], before})
             if (e) tkErrCheck(tkEventDestroy(e));
         if (hostInput) tkErrCheck(tkHostFree(hostInput));
     }
@@ -461,10 +452,12 @@ VGG16::VGG16(int taskId, const VGG16Options &o) : Task(taskId, "vgg16"), opt(o),
     const bool direct = impl->direct = haveDirectKernels() && (long)H * W <= 2048L * 2048;
     if (direct) {
         impl->staging = stagingStream();
-        for (int i = 0; i < 2; ++i) {
-            impl->image[i] = devAlloc(fl, impl->pixels);
-            TK_SAFE_CALL(tkEventCreate(&impl->read[i]));
-        }
+        for (float *&image : impl->image) image = devAlloc(fl, impl->pixels);
+    }
+    TK_SAFE_CALL(tkEventCreate(&impl->before));
+    for (tkEvent_t &e : impl->over) {
+        TK_SAFE_CALL(tkEventCreate(&e));
+        TK_SAFE_CALL(tkEventRecord(e, nullptr));   // nothing to wait for yet
     }
 
     // the largest im2col operand of the network, shared by every conv layer
@@ -559,7 +552,6 @@ VGG16::VGG16(int taskId, const VGG16Options &o) : Task(taskId, "vgg16"), opt(o),
     auto *fc2 = new FcKernel(id++, "Dot_fc2", o1, 1, b1, 1, 4096, 4096, W2, X2, o2);
     auto *fc3 = new FcKernel(id++, "Dot_fc3", o2, 1, b2, 1, 4096, opt.classes, W3, X3, o3);
     for (auto *fc : {fc1, fc2, fc3}) addKernel(fc);
-    for (auto *k : kernels) static_cast<GemmLayer *>(k)->noteLaunches(&impl->launched);
     if (direct) {
         bool *fresh = impl->fcInput;
         fc1->useDirect(&impl->act[12].fresh, &fresh[1], weightFragments(fl, W1, 4096, pad128(feat)), o1, b1, X2);
@@ -578,7 +570,6 @@ void VGG16::captured()
 {
     for (auto &a : impl->act) a.fresh = false;
     for (bool &f : impl->fcInput) f = false;
-    impl->recorded = true;
 }
 
 // The image goes over PCIe while the query before is still running: on a stream of its own, into the device image which
@@ -586,31 +577,45 @@ void VGG16::captured()
 // waits for it, and the host's image may change as soon as this returns.  A copy on the query's stream waits for
 // the query before and leaves the GPU idle until the host has seen its end and launched again: 45 us of a 206 us query
 // at 224 x 224, 37 of 133 at 64 x 96.
-// All of a task's launches share its buffers.  What was launched on another stream than this query's -- a query, single
-// layers, a recorded graph -- is waited for by that copy on the null stream, so the query then takes that way.
+//
+// All of a task's launches share its buffers, so a query comes after the last one, whichever stream that ran on, and after
+// what the null stream and the streams ordered with it have in front of them (a reader of the logits on a second stream, a
+// recorded graph, a bias written on the null stream) -- what a query whose image is copied on the null stream waits for.
+//  * On the null stream its launches wait for all that by themselves.
+//  * On a stream that is not ordered with it, the device waits for an event recorded there, which is over by the time the
+//    image is in place where the null stream is idle: 0 to 1 us a query.
+//  * On a stream that is, the host waits, after the image has been staged: 178 us a query at 224 x 224 where the null stream
+//    takes 163.  An event there, behind the stream's own last query, takes 315.
+// Graphs and single layers on a caller's stream that is not ordered with the null stream are the caller's to order
+// with a query on another stream.
 void VGG16::executeQuery(cudaStream_t stream)
 {
     Impl &m = *impl;
-    auto *first = m.direct ? dynamic_cast<ConvKernel *>(kernels.front()) : nullptr;
-    const bool alone = !m.recorded && !m.launched && (!m.queried || m.lastStream == stream);
-    m.queried = true;
-    m.lastStream = stream;
-    if (!first || !first->direct() || !alone) {
-        Task::executeQuery(stream);
-        m.launched = false;
-        return;
-    }
-    const int slot = m.turn;
+    const int turn = m.turn;
     m.turn ^= 1;
-    if (m.used[slot]) TK_SAFE_CALL(tkEventSynchronize(m.read[slot]));
-    // by the copy engine, 602 KB in 19 us; a kernel that reads the host's memory takes 23 and slows the one it runs beside
-    TK_SAFE_CALL(tkMemcpyAsync(m.image[slot], m.hostInput, (size_t)InputSize[0], TK_MEMCPY_H2D, m.staging->stream));
-    TK_SAFE_CALL(tkStreamSynchronize(m.staging->stream));
-    m.used[slot] = true;
-    first->executeFrom(m.image[slot], m.input, stream);
-    for (size_t i = 1; i < kernels.size(); ++i) kernels[i]->execute(stream);
-    TK_SAFE_CALL(tkEventRecord(m.read[slot], stream));
-    m.launched = false;
+    const tkEvent_t last = m.over[turn ^ 1];
+    auto *first = m.direct ? dynamic_cast<ConvKernel *>(kernels.front()) : nullptr;
+    if (!first || !first->direct()) {
+        // the copy on the null stream waits for the streams ordered with it; for the others the host does
+        TK_SAFE_CALL(tkEventSynchronize(last));
+        if (stream) TK_SAFE_CALL(tkStreamSynchronize(stream));
+        Task::executeQuery(stream);
+    } else {
+        unsigned ordered = 0;   // with the null stream
+        if (stream) TK_SAFE_CALL(tkStreamIsBlocking(stream, &ordered));
+        if (stream && !ordered) TK_SAFE_CALL(tkEventRecord(m.before, nullptr));
+        TK_SAFE_CALL(tkEventSynchronize(m.over[turn]));   // which read this image
+        // by the copy engine, 602 KB in 19 us; a kernel that reads the host's memory takes 23 and slows the one it runs beside
+        TK_SAFE_CALL(tkMemcpyAsync(m.image[turn], m.hostInput, (size_t)InputSize[0], TK_MEMCPY_H2D, m.staging->stream));
+        TK_SAFE_CALL(tkStreamSynchronize(m.staging->stream));
+        if (ordered) TK_SAFE_CALL(tkStreamSynchronize(nullptr));
+        else if (stream) TK_SAFE_CALL(tkStreamWaitEvent(stream, m.before));
+        if (stream || m.lastStream) TK_SAFE_CALL(tkStreamWaitEvent(stream, last));
+        first->executeFrom(m.image[turn], m.input, stream);
+        for (size_t i = 1; i < kernels.size(); ++i) kernels[i]->execute(stream);
+    }
+    TK_SAFE_CALL(tkEventRecord(m.over[turn], stream));
+    m.lastStream = stream;
 }
 
 VGG16::~VGG16()

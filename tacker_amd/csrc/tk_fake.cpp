@@ -168,6 +168,7 @@ int tk_tzgemm_scratch(void **ptr, size_t *bytes)
 }
 int tkStreamCreate(tkStream_t *s) { *s = malloc(1); return TK_SUCCESS; }
 int tkStreamCreateNonBlocking(tkStream_t *s) { return tkStreamCreate(s); }
+int tkStreamIsBlocking(tkStream_t, unsigned *blocking) { *blocking = 1; return TK_SUCCESS; }
 int tkStreamDestroy(tkStream_t s) { free(s); return TK_SUCCESS; }
 int tkStreamSynchronize(tkStream_t) { return TK_SUCCESS; }
 int tkDeviceSynchronize(void) { return TK_SUCCESS; }
@@ -175,6 +176,7 @@ int tkEventCreate(tkEvent_t *e) { *e = malloc(1); return TK_SUCCESS; }
 int tkEventDestroy(tkEvent_t e) { free(e); return TK_SUCCESS; }
 int tkEventRecord(tkEvent_t, tkStream_t) { return TK_SUCCESS; }
 int tkEventSynchronize(tkEvent_t) { return TK_SUCCESS; }
+int tkStreamWaitEvent(tkStream_t, tkEvent_t) { return TK_SUCCESS; }
 int tkEventElapsedTime(float *ms, tkEvent_t, tkEvent_t)
 {
     if (!g_event_queue.empty()) {

@@ -183,6 +183,12 @@ int tkMemcpyFromSymbol(void *dst, const char *symbol, size_t bytes, size_t offse
 
 int tkStreamCreate(tkStream_t *s) { return FOLD(hipStreamCreate((hipStream_t *)s)); }
 int tkStreamCreateNonBlocking(tkStream_t *s) { return FOLD(hipStreamCreateWithFlags((hipStream_t *)s, hipStreamNonBlocking)); }
+int tkStreamIsBlocking(tkStream_t s, unsigned *blocking)
+{
+    const int rc = FOLD(hipStreamGetFlags((hipStream_t)s, blocking));
+    *blocking = !(*blocking & hipStreamNonBlocking);
+    return rc;
+}
 int tkStreamDestroy(tkStream_t s) { return FOLD(hipStreamDestroy((hipStream_t)s)); }
 int tkStreamSynchronize(tkStream_t s) { return FOLD(hipStreamSynchronize((hipStream_t)s)); }
 int tkDeviceSynchronize(void) { return FOLD(hipDeviceSynchronize()); }
@@ -214,6 +220,7 @@ int tkGraphLaunch(tkGraphExec_t exec, tkStream_t s)
 int tkGraphExecDestroy(tkGraphExec_t exec) { return exec ? FOLD(hipGraphExecDestroy((hipGraphExec_t)exec)) : TK_SUCCESS; }
 int tkEventRecord(tkEvent_t e, tkStream_t s) { return FOLD(hipEventRecord((hipEvent_t)e, (hipStream_t)s)); }
 int tkEventSynchronize(tkEvent_t e) { return FOLD(hipEventSynchronize((hipEvent_t)e)); }
+int tkStreamWaitEvent(tkStream_t s, tkEvent_t e) { return FOLD(hipStreamWaitEvent((hipStream_t)s, (hipEvent_t)e, 0)); }
 int tkEventElapsedTime(float *ms, tkEvent_t start, tkEvent_t stop)
 {
     return FOLD(hipEventElapsedTime(ms, (hipEvent_t)start, (hipEvent_t)stop));

@@ -532,3 +532,81 @@ def test_weights_written_where_a_task_keeps_them_are_those_of_the_next_query(lay
         assert np.allclose(got, before / 2, rtol=0, atol=1e-5)
         assert np.abs(got - before).max() > 1e-3
     task.close()
+
+
+def own_stream(blocking):
+    """a raw stream handle, ordered with the null stream or not"""
+    s = C.c_void_p(None)
+    assert (ta.lib().tkStreamCreate if blocking else ta.lib().tkStreamCreateNonBlocking)(C.byref(s)) == 0
+    return s
+
+
+@pytest.mark.parametrize("kinds", [(False, False), (False, None), (None, False), (True, False)])
+@pytest.mark.parametrize("written", [False, True])
+def test_queries_on_streams_of_any_kind_run_one_after_the_other(kinds, written):
+    # streams ordered with the null stream (True), not ordered with it (False), and the null stream (None); written: the first
+    # layer's weights have been handed out, so that the image is copied on the null stream
+    task = ta.LcTask("vgg16", 224, 224)
+    if written:
+        task.conv_params(0)
+    streams = [C.c_void_p(None) if k is None else own_stream(k) for k in kinds]
+    image = task.host_input()
+    images = np.random.default_rng(11).random((2, image.size), dtype=np.float32)
+    p, stride, n = task.logits()
+    logits = lambda: ta.device_to_host(p, (n, stride), np.float32)[:, 0].copy()
+    want = []
+    for k in range(2):
+        image[:] = images[k]
+        task.execute(raw_stream=streams[0])
+        torch.cuda.synchronize()
+        want.append(logits())
+    assert np.abs(want[0] - want[1]).max() > 0
+    for rounds in range(1, 9):
+        for k in range(rounds + 1):
+            image[:] = images[k % 2]
+            task.execute(raw_stream=streams[k % 2])
+            image[:] = np.nan
+        torch.cuda.synchronize()
+        assert np.array_equal(logits(), want[rounds % 2]), rounds
+    task.close()
+    for s in streams:
+        assert not s or ta.lib().tkStreamDestroy(s) == 0
+
+
+@pytest.mark.parametrize("blocking", [False, True])
+def test_a_query_comes_after_what_the_null_stream_has_in_front_of_it(blocking):
+    # a bias written on the null stream behind 10 ms or more of waiting, and logits read on a blocking stream behind as much:
+    # a query on a stream of its own sees the one and leaves the other alone
+    task = ta.LcTask("vgg16", 64, 64)
+    stream, reader = own_stream(blocking), own_stream(True)
+    p, stride, n = task.logits()
+    logits = lambda: ta.device_to_host(p, (n, stride), np.float32)[:, 0].copy()
+    task.execute(raw_stream=stream)
+    torch.cuda.synchronize()
+    before = logits()
+    b, dims = C.c_void_p(), (C.c_int * 2)()
+    assert ta.lib().tacker_task_conv_params(task.h, 2, C.byref(C.c_void_p()), C.byref(b), dims) == 0
+    new = torch.full((dims[0],), 0.5, device="cuda:0")
+    torch.cuda.synchronize()
+    torch.cuda._sleep(10_000_000)
+    assert ta.lib().tkMemcpyAsync(b, C.c_void_p(new.data_ptr()), new.numel() * 4, 3, None) == 0
+    task.execute(raw_stream=stream)
+    torch.cuda.synchronize()
+    after = logits()
+    task.execute(raw_stream=stream)
+    torch.cuda.synchronize()
+    assert np.abs(after - before).max() > 0 and np.array_equal(logits(), after)
+
+    read = torch.zeros(n * stride, device="cuda:0")
+    image = task.host_input()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(torch.cuda.ExternalStream(reader.value)):
+        torch.cuda._sleep(10_000_000)
+    assert ta.lib().tkMemcpyAsync(C.c_void_p(read.data_ptr()), C.c_void_p(p), read.numel() * 4, 3, reader) == 0
+    image[:] = 0
+    task.execute(raw_stream=stream)
+    torch.cuda.synchronize()
+    assert np.array_equal(host(read)[::stride], after) and np.abs(logits() - after).max() > 0
+    task.close()
+    for s in (stream, reader):
+        assert ta.lib().tkStreamDestroy(s) == 0
