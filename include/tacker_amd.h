@@ -103,6 +103,7 @@ TK_API int tkEventElapsedTime(float *ms, tkEvent_t start, tkEvent_t stop);
 typedef void *tkGraphExec_t;
 TK_API int tkStreamBeginCapture(tkStream_t s);
 TK_API int tkStreamEndCapture(tkStream_t s, tkGraphExec_t *exec);
+TK_API int tkStreamIsCapturing(tkStream_t s, int *capturing);   /* cudaStreamIsCapturing; s: not the null stream */
 TK_API int tkGraphLaunch(tkGraphExec_t exec, tkStream_t s);
 TK_API int tkGraphExecDestroy(tkGraphExec_t exec);
 

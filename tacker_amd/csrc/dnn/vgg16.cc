@@ -2,6 +2,7 @@
 
 #include <cmath>
 #include <mutex>
+#include <stdexcept>
 #include <unordered_map>
 
 #include "../Creator.h"
@@ -591,6 +592,13 @@ void VGG16::captured()
 void VGG16::executeQuery(cudaStream_t stream)
 {
     Impl &m = *impl;
+    if (stream) {
+        // The copy on the null stream refuses to run while the stream is recorded.  The staged one would pass in a relaxed
+        // recording, and every launch of the graph would see the image of this moment.
+        int capturing = 0;
+        TK_SAFE_CALL(tkStreamIsCapturing(stream, &capturing));
+        if (capturing) throw std::runtime_error("vgg16: a query copies its image and cannot be recorded; captureQuery records its kernels");
+    }
     const int turn = m.turn;
     m.turn ^= 1;
     const tkEvent_t last = m.over[turn ^ 1];

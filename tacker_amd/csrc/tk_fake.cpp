@@ -227,6 +227,7 @@ int tkStreamEndCapture(tkStream_t s, tkGraphExec_t *exec)
     g_captured.clear();
     return TK_SUCCESS;
 }
+int tkStreamIsCapturing(tkStream_t s, int *capturing) { *capturing = s && s == g_capturing; return TK_SUCCESS; }
 int tkGraphLaunch(tkGraphExec_t exec, tkStream_t s)
 {
     if (!exec) return TK_ERROR_INVALID_VALUE;

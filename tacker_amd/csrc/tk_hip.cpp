@@ -212,6 +212,14 @@ int tkStreamEndCapture(tkStream_t s, tkGraphExec_t *exec)
     *exec = made;
     return TK_SUCCESS;
 }
+int tkStreamIsCapturing(tkStream_t s, int *capturing)
+{
+    if (!s || !capturing) return TK_ERROR_INVALID_VALUE;
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    const int rc = FOLD(hipStreamIsCapturing((hipStream_t)s, &status));
+    *capturing = status != hipStreamCaptureStatusNone;
+    return rc;
+}
 int tkGraphLaunch(tkGraphExec_t exec, tkStream_t s)
 {
     if (!exec) return TK_ERROR_INVALID_VALUE;

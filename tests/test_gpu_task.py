@@ -610,3 +610,35 @@ def test_a_query_comes_after_what_the_null_stream_has_in_front_of_it(blocking):
     task.close()
     for s in (stream, reader):
         assert ta.lib().tkStreamDestroy(s) == 0
+
+
+@pytest.mark.parametrize("mode", [1, 2])     # hipStreamCaptureModeThreadLocal, ...Relaxed
+def test_a_query_cannot_be_recorded_by_its_caller(mode):
+    # its image would be the recording's: refused in the mode that lets the staging pass, too, and the task goes on unharmed
+    l = ta.lib()
+    task, stream = ta.LcTask("vgg16", 64, 96), own_stream(False)
+    image = task.host_input()
+    images = np.random.default_rng(12).random((2, image.size), dtype=np.float32)
+    p, stride, n = task.logits()
+    logits = lambda: ta.device_to_host(p, (n, stride), np.float32)[:, 0].copy()
+    want = []
+    for k in (0, 1):
+        image[:] = images[k]
+        task.execute(raw_stream=stream)
+        torch.cuda.synchronize()
+        want.append(logits())
+    assert l.hipStreamBeginCapture(stream, C.c_int(mode)) == 0
+    try:
+        with pytest.raises(ta.TackerError, match="cannot be recorded"):
+            task.execute(raw_stream=stream)
+    finally:
+        graph = C.c_void_p()
+        assert l.hipStreamEndCapture(stream, C.byref(graph)) == 0
+        l.hipGraphDestroy(graph)
+    for k in (0, 1, 1, 0, 1, 0):
+        image[:] = images[k]
+        task.execute(raw_stream=stream)
+    torch.cuda.synchronize()
+    assert np.array_equal(logits(), want[0]) and np.abs(want[0] - want[1]).max() > 0
+    task.close()
+    assert l.tkStreamDestroy(stream) == 0
