@@ -390,8 +390,8 @@ __device__ __forceinline__ void fc_direct(const DnnFc &f)
     __syncthreads();
     if (threadIdx.x < 16) {
         const int n = (int)blockIdx.x * 16 + (int)threadIdx.x;
-        float v = 0.0f;
-        for (int s = 0; s < f.segments; s += 4) {
+        float v = partial[0][threadIdx.x];   // one segment (a reduction tzgemm does not cut) is its own sum
+        for (int s = 0; f.segments > 1 && s < f.segments; s += 4) {
             float part = partial[s][threadIdx.x];
             part += partial[s + 1][threadIdx.x];
             part += partial[s + 2][threadIdx.x];

@@ -642,3 +642,39 @@ def test_a_query_cannot_be_recorded_by_its_caller(mode):
     assert np.array_equal(logits(), want[0]) and np.abs(want[0] - want[1]).max() > 0
     task.close()
     assert l.tkStreamDestroy(stream) == 0
+
+
+class DnnFc(C.Structure):
+    """argument structure of fc_direct_1 / fc_direct_2 (dnn/direct.h)"""
+    _fields_ = [(k, C.c_void_p) for k in ("x", "weights", "raw", "bias", "act")] + \
+               [("chunks", C.c_int), ("segments", C.c_int), ("segment_begin", C.c_int * 33)]
+
+
+@pytest.mark.parametrize("segments", [1, 4, 8, 16, 32])
+@pytest.mark.parametrize("K", [64, 320, 2048])
+def test_a_fully_connected_layer_adds_the_segments_there_are(segments, K):
+    # reductions that tzgemm does not cut are one segment: what lies in LDS behind it is not part of the sum.  The launch of
+    # other, large values before fills the LDS.
+    from gpu_util import launch
+    rows, chunks = 16 * 512, K // 64
+    rng = np.random.default_rng(segments + K)
+    x, bias = rng.uniform(-1, 1, K).astype(np.float16), dev(rng.uniform(-1, 1, rows).astype(np.float32))
+    w = rng.uniform(-1, 1, (rows, K)).astype(np.float16)
+    d_w, fragments = dev(w), torch.empty((rows, K), dtype=torch.float16, device="cuda:0")
+    launch("pack_weight_fragments", 256, 256, [C.c_void_p(d_w.data_ptr()), C.c_void_p(fragments.data_ptr()), C.c_int(rows), C.c_int(K)])
+
+    def run(vector, cut):
+        d_x, raw = dev(vector), torch.zeros(rows, device="cuda:0")
+        act = torch.zeros(rows, dtype=torch.float16, device="cuda:0")
+        f = DnnFc(d_x.data_ptr(), fragments.data_ptr(), raw.data_ptr(), bias.data_ptr(), act.data_ptr(), chunks, cut)
+        for i in range(cut + 1):
+            f.segment_begin[i] = i * chunks // cut
+        per_wave = 2 if cut > 16 else 1
+        launch(f"fc_direct_{per_wave}", rows // 16, 64 * (cut // per_wave), [f])
+        return host(raw), host(act)
+    run((x * np.float16(1000)).astype(np.float16), 32)
+    raw, act = run(x, segments)
+    exact = float(np.float32(1.1)) * (w.astype(np.float64) @ x.astype(np.float64))
+    # a sum of K products below 1 in fp32, in any order: K roundings of a partial sum below K
+    assert np.abs(raw - exact).max() <= 1.1 * K * K * 2.0 ** -24 + 1e-6
+    assert np.array_equal(act, np.maximum(raw + host(bias), 0).astype(np.float16))
