@@ -250,14 +250,14 @@ __device__ __forceinline__ cutcp_lds_float4 *cutcp_stage_of_wave(int role_wave)
 // wavefront for the whole launch, which walks the rows in order, so the parts of a region are added in ascending
 // order without any synchronisation, whole rows that follow each other are one run through their parts, and
 // a range that runs past the grid wraps.
-// WAVES: wavefronts of the role in a workgroup, role_threads / 64 at least.
+// WAVES: wavefronts of a workgroup that there is LDS for; those of a larger workgroup leave the units to them.
 template <int WAVES>
 __device__ __forceinline__ void cutcp_role(int binDim_x, int binDim_y, const float *binZeroAddr, float h, float cutoff2,
                                            float inv_cutoff2, float *regionZeroAddr, int grid_dimension_x,
                                            int grid_dimension_y, int grid_dimension_z, int role_block, int role_blocks,
                                            int start, int end, int tid, int role_threads)
 {
-    const int waves = role_threads / TK_WAVE_SIZE;
+    const int waves = min(role_threads / TK_WAVE_SIZE, WAVES);
     const int wave = tid / TK_WAVE_SIZE;
     if (wave >= waves || start >= end) return;
     const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));

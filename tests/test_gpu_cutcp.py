@@ -4,13 +4,15 @@ bins within |d| <= 2e-4 + 2e-5 |ref| (the hardware's reciprocal square root here
 rsqrtf in the reference: approximations of an ulp each, summed over hundreds of atoms) and against the
 float64 sum over the atom list; the natural launch, the GPTB form over any tiling of its positions and
 every fused variant give the same bits as each other (positions = regions x parts of the neighbour list); the host's binning equals the oracle's exactly."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
 
 import oracle
 import tacker_amd as ta
-from gpu_util import dev, gemm_inputs, gemm_tolerance_ok, host, setup
+from gpu_util import dev, gemm_inputs, gemm_tolerance_ok, host, launch, setup
 
 pytestmark = pytest.mark.gpu
 H, CUTOFF = 0.5, 12.0
@@ -125,6 +127,23 @@ def test_cut_of_the_regions_and_meaning_of_the_cutoff(inv, regions, natoms):
     ta.ori_cutcp(inp, C2, inv, out[2])
     assert np.array_equal(bits(out[1]), bits(out[0])) and np.array_equal(bits(out[2]), bits(out[0]))
     assert close(host(out[0]), want)
+
+
+@pytest.mark.parametrize("threads", [64, 192, 256, 320, 512, 1024])
+@pytest.mark.parametrize("grid", [1, 3, 40])
+def test_workgroups_of_any_size_give_the_same_bits(threads, grid):
+    # the kernel launched by its handle: a workgroup has LDS for four wavefronts, further ones must not use any behind it
+    atoms, inp, prep = case(points=(40, 32, 16), natoms=700, seed=9)
+    want = torch.zeros_like(inp.energies)
+    ta.gptb_cutcp(inp, C2, INV_C2, want)
+    out = torch.zeros_like(want)
+    i, f, p = C.c_int, C.c_float, C.c_void_p
+    rx, ry, rz = inp.regions
+    parts = inp.blocks() // (rx * ry * rz)
+    launch("gptb_cutcp", grid, threads,
+           [i(inp.binDim[0]), i(inp.binDim[1]), p(inp.bin_zero), f(H), f(C2), f(INV_C2), p(out.data_ptr()), i(0), i(rx), i(ry),
+            i(rz * parts), i(8), i(2), i(8), i(0), i(grid), i(inp.blocks()), i(0)])
+    assert np.array_equal(bits(out), bits(want)) and np.abs(host(want)).max() > 0
 
 
 @pytest.mark.parametrize("variant", [None, "wave_128", "wave_256", "wave_512", "wg_1_1", "wg_1_2"])
