@@ -56,6 +56,7 @@ void Task::executeTask(ExecutionMode mode, cudaStream_t stream)
 void Task::executeQuery(cudaStream_t stream)
 {
     initExecution();
+    const WholeQuery whole(*this);
     for (auto &kernel : kernels) kernel->execute(stream);
 }
 
@@ -63,6 +64,7 @@ tkGraphExec_t Task::captureQuery(cudaStream_t stream)
 {
     tkGraphExec_t graph = nullptr;
     TK_SAFE_CALL(tkStreamBeginCapture(stream));
+    const WholeQuery whole(*this);
     try {
         for (auto &kernel : kernels) kernel->execute(stream);
     } catch (...) {   // a stream left recording would fail every later call on it

@@ -27,6 +27,13 @@ public:
     // kernel still has buffers to allocate, and the caller stages the input before each launch of
     // the graph.  The caller destroys the graph (tkGraphExecDestroy).
     tkGraphExec_t captureQuery(cudaStream_t stream);
+    // set while a query's kernels are launched one behind the other, with nobody in between
+    bool wholeQuery = false;
+    struct WholeQuery {
+        Task &task;
+        explicit WholeQuery(Task &t) : task(t) { task.wholeQuery = true; }
+        ~WholeQuery() { task.wholeQuery = false; }
+    };
     // the kernels' execute() has been recorded, not run: what a task remembers of its last run no longer holds
     virtual void captured() {}
 

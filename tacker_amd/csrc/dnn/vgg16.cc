@@ -126,20 +126,28 @@ int reductionCut(int M, int N, int K, int real, int begin[DNN_MAX_SEGMENTS + 1])
 // d -> what dnn_div takes for a division by d
 unsigned reciprocal(int d) { return d == 1 ? 0u : (unsigned)((1ull << 32) / (unsigned)d + 1); }
 
-// A layer's activation as the next layer's direct kernel reads it: where it is, and whether it holds what the
-// layer's raw output holds (a layer that ran fused, or not through its direct kernel, has written only that).
+// Whether the activation that a layer's direct kernel leaves for the next layer is what the layer's raw output and bias
+// give.  A layer that ran fused, or not through its direct kernel, has written only the raw output; and a caller who has
+// the raw output's or the bias's address may write there between two layers that are launched one by one.
+struct Fresh {
+    bool valid = false, exposed = false;
+    const bool *wholeQuery = nullptr;   // the layers follow each other, nobody writes in between
+    bool holds() const { return valid && (!exposed || *wholeQuery); }
+};
+
+// A layer's activation as the next layer's direct kernel reads it.
 struct Activation {
     DnnOutput out{};
     int channels = 0;
-    bool fresh = false;
+    Fresh fresh;
     // bring it up to date, if it is not
     void need(cudaStream_t stream)
     {
-        if (fresh) return;
+        if (fresh.holds()) return;
         const int pixels = out.pool ? out.H * out.W / 4 : out.H * out.W;
         void *args[] = {&out, &channels};
         launch1d("dnn_activation", (long)pixels * (channels / 4), args, stream);
-        fresh = true;
+        fresh.valid = true;
     }
 };
 
@@ -259,7 +267,7 @@ public:
 protected:
     void fused() override
     {
-        if (next_) next_->fresh = false;
+        if (next_) next_->fresh.valid = false;
     }
     void executeImpl(cudaStream_t stream) override
     {
@@ -275,7 +283,7 @@ protected:
         void *image_args[] = {&image, &keep, direct_.get()}, *act_args[] = {direct_.get()};
         void **args = in_ ? act_args : image_args;
         TK_SAFE_CALL(tkLaunchKernel(fmap.at(key_), dim3(grid_).raw(), dim3(threads_).raw(), args, lds_, stream));
-        next_->fresh = true;
+        next_->fresh.valid = true;
     }
     void before(cudaStream_t stream) override
     {
@@ -329,7 +337,7 @@ public:
 
     // Run through the direct kernel from now on.  in, out: whether X's first row, and the next layer's (next_x), hold
     // this layer's input and activation (out null: the last layer).
-    void useDirect(bool *in, bool *out, const void *fragments, float *raw, const float *bias, void *next_x)
+    void useDirect(Fresh *in, Fresh *out, const void *fragments, float *raw, const float *bias, void *next_x)
     {
         inFresh_ = in;
         outFresh_ = out;
@@ -348,8 +356,8 @@ public:
 protected:
     void fused() override
     {
-        if (inFresh_) *inFresh_ = true;   // before() packed it
-        if (outFresh_) *outFresh_ = false;
+        if (inFresh_) inFresh_->valid = true;   // before() packed it
+        if (outFresh_) outFresh_->valid = false;
     }
     void executeImpl(cudaStream_t stream) override
     {
@@ -357,13 +365,13 @@ protected:
             fused();
             return GemmLayer::executeImpl(stream);
         }
-        if (!*inFresh_) before(stream);
-        *inFresh_ = true;
+        if (!inFresh_->holds()) before(stream);
+        inFresh_->valid = true;
         void *args[] = {direct_.get()};
         const int waves = (direct_->segments + perWave_ - 1) / perWave_;
         TK_SAFE_CALL(tkLaunchKernel(fmap.at(perWave_ == 2 ? "fc_direct_2" : "fc_direct_1"), dim3((unsigned)(N_ / 16)).raw(),
                                     dim3((unsigned)(64 * waves)).raw(), args, 0, stream));
-        if (outFresh_) *outFresh_ = true;
+        if (outFresh_) outFresh_->valid = true;
     }
     void before(cudaStream_t stream) override
     {
@@ -384,7 +392,7 @@ private:
     void *X_;
     int poolW_, poolLd_, poolC_;
     std::unique_ptr<DnnFc> direct_;
-    bool *inFresh_ = nullptr, *outFresh_ = nullptr;
+    Fresh *inFresh_ = nullptr, *outFresh_ = nullptr;
     int perWave_ = 1;
 };
 
@@ -430,7 +438,7 @@ struct VGG16::Impl {
     float *logits = nullptr;
     long logitsStride = 0;
     Activation act[13];             // of the convolutions; the last one's is fc1's input
-    bool fcInput[3] = {};           // fc2's and fc3's input vectors hold the layer before's activation ([0] unused: act[12])
+    Fresh fcInput[3];               // fc2's and fc3's input vectors hold the layer before's activation ([0] unused: act[12])
 };
 
 VGG16::VGG16(int taskId, const VGG16Options &o) : Task(taskId, "vgg16"), opt(o), impl(new Impl)
@@ -554,7 +562,9 @@ VGG16::VGG16(int taskId, const VGG16Options &o) : Task(taskId, "vgg16"), opt(o),
     auto *fc3 = new FcKernel(id++, "Dot_fc3", o2, 1, b2, 1, 4096, opt.classes, W3, X3, o3);
     for (auto *fc : {fc1, fc2, fc3}) addKernel(fc);
     if (direct) {
-        bool *fresh = impl->fcInput;
+        for (auto &a : impl->act) a.fresh.wholeQuery = &wholeQuery;
+        Fresh *fresh = impl->fcInput;
+        fresh[1].wholeQuery = fresh[2].wholeQuery = &wholeQuery;
         fc1->useDirect(&impl->act[12].fresh, &fresh[1], weightFragments(fl, W1, 4096, pad128(feat)), o1, b1, X2);
         fc2->useDirect(&fresh[1], &fresh[2], weightFragments(fl, W2, 4096, 4096), o2, b2, X3);
         fc3->useDirect(&fresh[2], nullptr, weightFragments(fl, W3, pad128(opt.classes), 4096), o3, nullptr, nullptr);
@@ -569,8 +579,8 @@ VGG16::VGG16(int taskId, const VGG16Options &o) : Task(taskId, "vgg16"), opt(o),
 
 void VGG16::captured()
 {
-    for (auto &a : impl->act) a.fresh = false;
-    for (bool &f : impl->fcInput) f = false;
+    for (auto &a : impl->act) a.fresh.valid = false;
+    for (Fresh &f : impl->fcInput) f.valid = false;
 }
 
 // The image goes over PCIe while the query before is still running: on a stream of its own, into the device image which
@@ -619,6 +629,7 @@ void VGG16::executeQuery(cudaStream_t stream)
         if (ordered) TK_SAFE_CALL(tkStreamSynchronize(nullptr));
         else if (stream) TK_SAFE_CALL(tkStreamWaitEvent(stream, m.before));
         if (stream || m.lastStream) TK_SAFE_CALL(tkStreamWaitEvent(stream, last));
+        const WholeQuery whole(*this);
         first->executeFrom(m.image[turn], m.input, stream);
         for (size_t i = 1; i < kernels.size(); ++i) kernels[i]->execute(stream);
     }
@@ -644,7 +655,20 @@ const float *VGG16::logits(long *stride) const
 
 void VGG16::weightsHandedOut(int layer) { static_cast<GemmLayer *>(kernels.at(layer))->weightsHandedOut(); }
 
-VGG16::Act VGG16::activation(int conv_index) const { return impl->convOut.at(conv_index); }
+void VGG16::resultHandedOut(int layer)
+{
+    if (layer < 13) impl->act[layer].fresh.exposed = true;
+    else if (layer < 15) impl->fcInput[layer - 12].exposed = true;
+}
+
+const VGG16::Act &VGG16::layer(int idx) const { return impl->convOut.at(idx); }
+
+VGG16::Act VGG16::activation(int conv_index)
+{
+    resultHandedOut(conv_index);
+    weightsHandedOut(conv_index);
+    return layer(conv_index);
+}
 
 Task *createTask(const std::string &model)
 {

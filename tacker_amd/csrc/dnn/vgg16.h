@@ -47,14 +47,18 @@ public:
     void initExecution() override;       // host -> device copy of the input image
     void executeQuery(cudaStream_t stream) override;
     void weightsHandedOut(int layer);    // a caller has the address of layer 0 .. 15's weights and may write them
+    void resultHandedOut(int layer);     // ... of its raw output or its bias
     void captured() override;            // nothing of what was recorded has run: no activation is known to be up to date
     // device pointer / length of the logits (column 0 of the last GEMM's output, stride ld)
     const float *logits(long *stride) const;
     // output buffer of layer `idx` (0..12 the convolutions, 13..15 the fully connected layers; for
     // tests): device pointer, rows, channel stride.  It holds 1.1 * A * B^T; bias (returned here,
-    // none for the last layer) and ReLU are applied by the layer that reads it
+    // none for the last layer) and ReLU are applied by the layer that reads it.  A layer may be launched by itself,
+    // something written here, and the next one launched; the weights may be written, too: the layer goes through its operand
+    // and tzgemm from now on
     struct Act { float *ptr; int H, W, C, ld; void *weights; float *bias; int Np, Kp; };
-    Act activation(int conv_index) const;
+    Act activation(int conv_index);
+    const Act &layer(int idx) const;     // the same, handed to nobody
     VGG16Options opt;
     struct Impl;
     std::unique_ptr<Impl> impl;

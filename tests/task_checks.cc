@@ -1,0 +1,99 @@
+// Checks of the VGG16 task's C++ interface: what no C entry point reaches.  Usage: task_checks <check>; exit code 0 if it holds.
+#include <cstdio>
+#include <cstring>
+#include <vector>
+
+#include "dnn/vgg16.h"
+#include "../include/tacker_amd.h"
+
+namespace {
+
+std::vector<float> read(const float *p, size_t n)
+{
+    std::vector<float> host(n);
+    TK_SAFE_CALL(tkDeviceSynchronize());
+    TK_SAFE_CALL(tkMemcpy(host.data(), p, n * sizeof(float), TK_MEMCPY_D2H));
+    return host;
+}
+
+void write(float *p, const std::vector<float> &host)
+{
+    TK_SAFE_CALL(tkMemcpy(p, host.data(), host.size() * sizeof(float), TK_MEMCPY_H2D));
+    TK_SAFE_CALL(tkDeviceSynchronize());
+}
+
+bool same(const std::vector<float> &a, const std::vector<float> &b)
+{
+    return a.size() == b.size() && memcmp(a.data(), b.data(), a.size() * sizeof(float)) == 0;
+}
+
+size_t size_of(const VGG16::Act &a) { return (size_t)a.H * a.W * a.ld; }
+
+// the same network (weights and image come from the seed) with every layer through its operand and tzgemm
+void use_tzgemm(VGG16 &task)
+{
+    for (int i = 0; i < 16; ++i) task.weightsHandedOut(i);
+}
+
+// Layer `i` run by itself, its raw output or its bias written, layer i + 1 run by itself, twice: each run sees what was written last.
+bool written_between_layers(bool accessor, bool bias)
+{
+    VGG16Options opt;
+    opt.height = 64, opt.width = 96;
+    for (int i : {0, 1, 5, 9, 12, 13, 14}) {
+        VGG16 task(1, opt), plain(2, opt);
+        use_tzgemm(plain);
+        task.executeQuery(nullptr);
+        plain.executeQuery(nullptr);
+        std::vector<float> before = read(task.layer(i + 1).ptr, size_of(task.layer(i + 1)));
+        float *raw = nullptr;
+        int dims[4];
+        if (accessor) raw = task.activation(i).ptr;
+        else if (tacker_task_activation(static_cast<Task *>(&task), i, &raw, dims)) return false;
+        if (raw != task.layer(i).ptr) return false;
+        for (float factor : {0.5f, 3.0f}) {
+            for (VGG16 *t : {&task, &plain}) {
+                const VGG16::Act &a = t->layer(i);
+                std::vector<float> v = bias ? read(a.bias, a.C) : read(a.ptr, size_of(a));
+                for (float &x : v) x *= factor;
+                write(bias ? a.bias : a.ptr, v);
+                t->kernels[i + 1]->execute((cudaStream_t) nullptr);
+            }
+            const std::vector<float> got = read(task.layer(i + 1).ptr, size_of(task.layer(i + 1)));
+            if (!same(got, read(plain.layer(i + 1).ptr, size_of(plain.layer(i + 1)))) || same(got, before)) {
+                printf("layer %d, factor %g: not what was written\n", i, factor);
+                return false;
+            }
+            before = got;
+        }
+    }
+    return true;
+}
+
+// more classes than tzgemm cuts the last layer's reduction for
+bool many_classes(int classes)
+{
+    VGG16Options opt;
+    opt.height = opt.width = 32;
+    opt.classes = classes;
+    VGG16 task(1, opt), plain(2, opt);
+    use_tzgemm(plain);
+    task.executeQuery(nullptr);
+    plain.executeQuery(nullptr);
+    return same(read(task.logits(nullptr), classes), read(plain.logits(nullptr), classes));
+}
+
+}  // namespace
+
+int main(int argc, char **argv)
+{
+    const char *check = argc > 1 ? argv[1] : "";
+    if (tacker_init(0, nullptr)) return 2;
+    bool ok = false;
+    if (!strcmp(check, "raw")) ok = written_between_layers(false, false) && written_between_layers(true, false);
+    else if (!strcmp(check, "bias")) ok = written_between_layers(false, true) && written_between_layers(true, true);
+    else if (!strcmp(check, "classes")) ok = many_classes(1000) && many_classes(8192) && many_classes(9000);
+    else return 2;
+    printf("%s %s\n", check, ok ? "ok" : "FAILED");
+    return ok ? 0 : 1;
+}

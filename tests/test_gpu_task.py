@@ -1,6 +1,8 @@
 """GPU tests of the conv->GEMM helpers, the VGG16 latency-critical task and the
 TaskManager on the real device."""
 import ctypes as C
+import os
+import subprocess
 
 import numpy as np
 import pytest
@@ -678,3 +680,11 @@ def test_a_fully_connected_layer_adds_the_segments_there_are(segments, K):
     # a sum of K products below 1 in fp32, in any order: K roundings of a partial sum below K
     assert np.abs(raw - exact).max() <= 1.1 * K * K * 2.0 ** -24 + 1e-6
     assert np.array_equal(act, np.maximum(raw + host(bias), 0).astype(np.float16))
+
+
+@pytest.mark.parametrize("check", ["raw", "bias", "classes"])
+def test_checks_of_the_cxx_interface(check):
+    # raw, bias: written by a caller between two layers launched one by one; classes: up to 9000
+    program = os.path.join(os.path.dirname(ta.LIB_PATH), "task_checks")
+    p = subprocess.run([program, check], capture_output=True, text=True, timeout=100)
+    assert p.returncode == 0 and f"{check} ok" in p.stdout, p.stdout[-2000:] + p.stderr[-2000:]
