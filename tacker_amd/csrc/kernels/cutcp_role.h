@@ -28,6 +28,8 @@
 // 208^3 lattice, two layers of regions: 147 us, 26 layers 1.47 ms; 290 us and 3.07 ms with every atom of the list by scalar loads and
 // a branch for each point.
 #pragma once
+#include <type_traits>
+
 #include "role_common.h"
 #include "../header/cutcp_header.h"
 
@@ -135,7 +137,9 @@ __device__ __forceinline__ void cutcp_piece(int binDim_x, int binDim_y, const fl
         const float ey = fmaxf(fmaxf(box_y0 - a.y, a.y - box_y1), 0.f);
         const float ez = fmaxf(fmaxf(box_z0 - a.z, a.z - box_z1), 0.f);
         const float e2 = ex * ex + ey * ey + ez * ez;
-        const bool keep = before == 0u && e2 < reach2 && place + (lane >> 3) < end;
+        // (a coordinate that is no number is within no cutoff; the maxima above take it for nothing)
+        const float position = a.x + a.y + a.z;
+        const bool keep = before == 0u && e2 < reach2 && position == position && place + (lane >> 3) < end;
         const unsigned long long kept = __ballot(keep);
         const int count = __popcll(kept);
         const int at = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(kept >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)kept, 0u));
@@ -152,7 +156,7 @@ __device__ __forceinline__ void cutcp_piece(int binDim_x, int binDim_y, const fl
             for (int u = 0; u < CUTCP_GROUP; ++u) g[u] = stage[(first & (TK_WAVE_SIZE - 1)) + u];
             __builtin_amdgcn_sched_barrier(0);   // on its way while the group before it is used
         };
-        const auto use = [&](const float4_t (&g)[CUTCP_GROUP]) {
+        const auto use = [&](const float4_t (&g)[CUTCP_GROUP], auto compare) {
 #pragma unroll
             for (int u = 0; u < CUTCP_GROUP; ++u) {
                 const float4_t c = g[u];
@@ -166,19 +170,26 @@ __device__ __forceinline__ void cutcp_piece(int binDim_x, int binDim_y, const fl
                     float s = __builtin_fmaf(-r2, inv, 1.f);
                     if (CLAMP) s = __builtin_amdgcn_fmed3f(s, 0.f, 1.f);
                     const float add = __builtin_fmaf(c.w * __builtin_amdgcn_rsqf(r2), s * s, energy[e]);
-                    energy[e] = CLAMP || r2 < cutoff2 ? add : energy[e];
+                    energy[e] = !compare || r2 < cutoff2 ? add : energy[e];
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
         };
-        if (count > 0) read(ga, 0);
-        for (int i = 0; i < count; i += 2 * CUTCP_GROUP) {
-            read(gb, i + CUTCP_GROUP);
-            use(ga);
-            if (i + CUTCP_GROUP >= count) break;   // uniform
-            read(ga, i + 2 * CUTCP_GROUP);
-            use(gb);
-        }
+        const auto use_all = [&](auto compare) {
+            if (count > 0) read(ga, 0);
+            for (int i = 0; i < count; i += 2 * CUTCP_GROUP) {
+                read(gb, i + CUTCP_GROUP);
+                use(ga, compare);
+                if (i + CUTCP_GROUP >= count) break;   // uniform
+                read(ga, i + 2 * CUTCP_GROUP);
+                use(gb, compare);
+            }
+        };
+        // beyond a point's cutoff the clamp makes s zero, and the term with it unless the charge is infinite or no number:
+        // a batch with such a charge is compared
+        const bool compare = !CLAMP || __ballot(keep && !(__builtin_fabsf(a.w) < __builtin_inff())) != 0;
+        if (compare) use_all(std::true_type{});
+        else use_all(std::false_type{});
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
     }

@@ -129,6 +129,32 @@ def test_cut_of_the_regions_and_meaning_of_the_cutoff(inv, regions, natoms):
     assert close(host(out[0]), want)
 
 
+@pytest.mark.parametrize("inv", [1 / 144.0, 0.0069])
+@pytest.mark.parametrize("regions,natoms", [((1, 6, 2), 300), ((8, 9, 7), 3000)])
+@pytest.mark.parametrize("what", ["inf", "-inf", "nan", "both", "position"])
+def test_charges_and_positions_that_are_not_finite_reach_the_points_within_the_cutoff_only(inv, regions, natoms, what):
+    # an infinite charge, or one that is no number, shows at the points within its cutoff and nowhere else; an atom whose
+    # position is not finite shows nowhere.  0.0069: the cutoff is compared, and a term that rounding moves across it is
+    # below 1e-5
+    nx, ny, nz = (8 * r for r in regions)
+    atoms = atoms_in_box(natoms, (min(nx, ny, nz) - 1) * H, seed=natoms + 1)
+    inp = ta.CutcpInput(atoms, (0, 0, 0), nx, ny, nz, H, CUTOFF)
+    prep = oracle.cutcp_prepare(atoms, (0, 0, 0), nx, ny, nz, H, CUTOFF)
+    filled = np.argwhere(prep["bins"][..., 3] != 0)
+    values = {"inf": [np.inf], "-inf": [-np.inf], "nan": [np.nan], "both": [np.inf, -np.inf],
+              "position": [np.inf, -np.inf, np.nan]}[what]
+    for j, v in enumerate(values):
+        prep["bins"][tuple(filled[(3 * j) % len(filled)])][j if what == "position" else 3] = v
+    inp.bins.copy_(torch.from_numpy(prep["bins"]).cuda())
+    want = oracle.cutcp(prep, H, C2, inv, inp.regions, parts="chunks")
+    ta.gptb_cutcp(inp, C2, inv)
+    got = host(inp.energies)
+    ok = np.isfinite(want)
+    assert ok.any() and (what == "position") == ok.all()
+    assert np.array_equal(got[~ok], want[~ok], equal_nan=True)
+    assert np.isfinite(got[ok]).all() and close(got[ok], want[ok])
+
+
 @pytest.mark.parametrize("threads", [64, 192, 256, 320, 512, 1024])
 @pytest.mark.parametrize("grid", [1, 3, 40])
 def test_workgroups_of_any_size_give_the_same_bits(threads, grid):
