@@ -98,7 +98,8 @@ __device__ __forceinline__ void lava_box(const float scale, const box_str *d_box
         total[k] = fA[4 * in];
     }
     for (int part = part_begin; part < part_end; ++part) {
-        const long first_j = part == 0 ? first_i : boxes[bx].nei[part - 1].offset;
+        // (a neighbour is named by its number alone; its offset in the list is not read)
+        const long first_j = part == 0 ? first_i : boxes[boxes[bx].nei[part - 1].number].offset;
         const float4_t *rB = reinterpret_cast<const float4_t *>(d_rv_gpu + first_j) + row;
         const float *qB = d_qv_gpu + first_j + row;
         float4_t f[P];

@@ -5,13 +5,15 @@ hot3d_nn.cu, hot3d_path.cu, nn_path.cu, hot3d_lava.cu, lava_nn.cu, lava_path.cu)
 |d| <= 2e-3 + 2e-5 |ref| for lavaMD (the hardware's exponential against the C library's), for the natural
 launch, the GPTB form over any tiling of its positions, every fused variant with tzgemm and every fused pair
 among the four; every device form of the same lavaMD work gives the same bits as every other."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
 
 import oracle
 import tacker_amd as ta
-from gpu_util import dev, gemm_inputs, gemm_tolerance_ok, host, setup
+from gpu_util import dev, gemm_inputs, gemm_tolerance_ok, host, launch, setup
 
 pytestmark = pytest.mark.gpu
 
@@ -249,6 +251,36 @@ def test_lava_box_list_is_the_oracles():
         assert ta.lib().tacker_lava_boxes(boxes1d, got.ctypes.data, got.nbytes) == 0
         assert got.tobytes() == want.tobytes()
     assert ta.lib().tacker_lava_boxes(2, got.ctypes.data, 100) != 0        # buffer too small
+
+
+class ParStr(C.Structure):
+    _fields_ = [("alpha", C.c_float)]
+
+
+class DimStr(C.Structure):
+    _fields_ = [(k, C.c_int) for k in ("cur", "arch", "cores", "boxes1d")] + \
+               [(k, C.c_long) for k in ("number_boxes", "box_mem", "space_elem", "space_mem", "space_mem2")]
+
+
+def test_lava_a_neighbour_is_the_box_its_number_names():
+    # a caller's own list: boxes stored in another order than they are numbered, neighbours with a number and no offset
+    boxes1d, n = 3, 27
+    rv, qv = lava_inputs(boxes1d, seed=77)
+    want = torch.zeros((100 * n, 4), device="cuda:0")
+    ta.gptb_lava(0.5, dev(rv), dev(qv), want)
+    place = np.random.default_rng(5).permutation(n)          # box b's particles lie at 100 place[b]
+    boxes = oracle.lava_boxes(boxes1d)
+    boxes["nei"]["offset"] = 0
+    boxes["offset"] = 100 * place
+    r, q = np.empty_like(rv).reshape(n, 100, 4), np.empty_like(qv).reshape(n, 100)
+    r[place], q[place] = rv.reshape(n, 100, 4), qv.reshape(n, 100)
+    d_b, d_r, d_q = dev(boxes.view(np.uint8)), dev(r), dev(q)
+    out = torch.zeros((n, 100, 4), device="cuda:0")
+    i = C.c_int
+    launch("gptb_lava", 16, 256, [ParStr(0.5), DimStr(boxes1d=boxes1d, number_boxes=n)] +
+           [C.c_void_p(t.data_ptr()) for t in (d_b, d_r, d_q, out)] +
+           [i(v) for v in (n, 27, 1, 256, 1, 1, 0, 16, 27 * n, 0)])
+    assert np.array_equal(host(out)[place].view(np.uint32).reshape(-1), bits(want).reshape(-1))
 
 
 @pytest.mark.parametrize("seed", range(4))
