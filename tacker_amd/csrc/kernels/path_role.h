@@ -105,10 +105,12 @@ __device__ __forceinline__ void path_window(int iteration, const int *__restrict
         step(w_last);
     } else {
         // rows 0 .. middle - 1 go through the ring; a lane whole columns off the grid reads next to it.  Address:
-        // a row's pointer, the same for the whole wavefront, and an unsigned 32-bit lane offset.
+        // a pointer to the window's first column of a row, the same for the whole wavefront, and an unsigned 32-bit
+        // lane offset (from there, since a row may have 2^30 columns).
         const int middle = iteration - 1;
-        const unsigned at = (unsigned)(max(-(C - 1), min(x0, cols - 1)) + (C - 1)) * (unsigned)sizeof(int);
-        const char *ahead = reinterpret_cast<const char *>(first - (C - 1));   // the row the next fetch takes
+        const int window = min(max(blkX, 0), cols - 1);
+        const unsigned at = (unsigned)(max(-(C - 1), min(x0, cols - 1)) - window + (C - 1)) * (unsigned)sizeof(int);
+        const char *ahead = reinterpret_cast<const char *>(first + window - (C - 1));   // the row the next fetch takes
         int fetched = 0;
         int wall[AHEAD][C];
         const auto fetch = [&](int (&w)[C]) {

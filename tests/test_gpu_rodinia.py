@@ -173,6 +173,31 @@ def test_path_ring_of_rows_and_edges_of_the_grid(cols, iteration):
     assert np.array_equal(host(out), oracle.path(iteration, wall, src))
 
 
+def test_path_the_last_windows_of_a_very_wide_grid():
+    # rows of more than 2^30 columns (the kernel launched by its handle: the entry points take walls of less than 2^31
+    # cells): the last windows' columns, of which a byte offset from the row's start needs 33 bits
+    cols, rows, iteration, last = 2 ** 30 + 1003, 3, 3, 2000
+    small = 256 - 2 * iteration
+    rng = np.random.default_rng(8)
+    tail = rng.integers(0, 10, (rows, last), dtype=np.int32)
+    src_tail = rng.integers(0, 10, last, dtype=np.int32)
+    wall = torch.zeros((rows, cols), dtype=torch.int32, device="cuda:0")
+    src = torch.zeros(cols, dtype=torch.int32, device="cuda:0")
+    out = torch.full((cols,), -1, dtype=torch.int32, device="cuda:0")
+    wall[:, -last:], src[-last:] = dev(tail), dev(src_tail)
+    positions = -(-cols // small)
+    i, p = C.c_int, C.c_void_p
+    launch("gptb_path", 4, 64, [i(iteration), p(wall.data_ptr()), p(src.data_ptr()), p(out.data_ptr()), i(cols), i(rows + 1), i(0),
+                                i(iteration)] + [i(v) for v in (positions, 1, 1, 256, 1, 1, positions - 4, 4, positions, 0)])
+    cur = src_tail.astype(np.int64)
+    for r in range(rows):
+        left, right = np.concatenate(([0], cur[:-1])), np.concatenate((cur[1:], [cur[-1]]))
+        cur = tail[r] + np.minimum(np.minimum(left, cur), right)
+    begin = small * (positions - 4)
+    got = host(out[begin - 10:])
+    assert np.all(got[:10] == -1) and np.array_equal(got[10:], cur[begin - cols:])
+
+
 def test_path_walks_a_grid_pyramid_by_pyramid():
     # Rodinia's host loop: the result of one pyramid is the source of the next
     cols, rows, height = 700, 61, 20
