@@ -110,7 +110,7 @@ def test_any_tiling_of_the_positions_gives_the_one_kernel(seed):
 @pytest.mark.parametrize("inv", [1 / 144.0, 0.0065, 0.008])
 @pytest.mark.parametrize("regions,natoms", [((1, 1, 1), 1), ((2, 1, 1), 64), ((1, 3, 2), 2000), ((9, 8, 3), 900), ((8, 9, 7), 1500)])
 def test_cut_of_the_regions_and_meaning_of_the_cutoff(inv, regions, natoms):
-    # the launch's wavefronts decide how regions are cut into pieces (1, 2 or 4 points a lane); inv_cutoff2 need not be
+    # the launch's wavefronts decide how regions are cut into pieces (1 or 2 points a lane); inv_cutoff2 need not be
     # 1 / cutoff2, and then the cutoff is a comparison; full bins, empty bins, a charge of zero inside a bin (it ends the bin)
     nx, ny, nz = (8 * r for r in regions)
     atoms = atoms_in_box(natoms, (min(nx, ny, nz) - 1) * H, seed=natoms)
@@ -127,6 +127,26 @@ def test_cut_of_the_regions_and_meaning_of_the_cutoff(inv, regions, natoms):
     ta.ori_cutcp(inp, C2, inv, out[2])
     assert np.array_equal(bits(out[1]), bits(out[0])) and np.array_equal(bits(out[2]), bits(out[0]))
     assert close(host(out[0]), want)
+
+
+@pytest.mark.parametrize("inv", [1 / 144.0, 0.0069])
+def test_four_points_a_lane_give_the_bits_of_one_and_two(inv):
+    # more than 2048 regions take four points a lane, one layer of them takes one and twelve take two; 0.0069: the cutoff is
+    # compared, point by point, and a term that rounding moves across it is below 1e-5
+    n = 8 * 13
+    atoms = atoms_in_box(1500, (n - 1) * H, seed=13)
+    prep = oracle.cutcp_prepare(atoms, (0, 0, 0), n, n, n, H, CUTOFF)
+    got = {}
+    for layers in (13, 12, 1):
+        inp = ta.CutcpInput(atoms, (0, 0, 0), n, n, n, H, CUTOFF, regions=(13, 13, layers))
+        out = [torch.zeros_like(inp.energies) for _ in range(2)]
+        ta.gptb_cutcp(inp, C2, inv, out[0])
+        ta.ori_cutcp(inp, C2, inv, out[1])
+        assert np.array_equal(bits(out[0]), bits(out[1]))
+        got[layers] = host(out[0])
+    for layers in (12, 1):
+        assert np.array_equal(got[layers].view(np.uint32), got[13][:layers].view(np.uint32))
+    assert close(got[13], oracle.cutcp(prep, H, C2, inv, (13, 13, 13), parts="chunks"))
 
 
 @pytest.mark.parametrize("inv", [1 / 144.0, 0.0069])

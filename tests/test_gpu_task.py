@@ -433,7 +433,7 @@ def test_a_layer_by_itself_gives_the_bits_of_its_operand_and_tzgemm(H, W):
     task.close()
 
 
-@pytest.mark.parametrize("H,W,own_stream", [(32, 32, False), (96, 64, True), (224, 224, True)])
+@pytest.mark.parametrize("H,W,own_stream", [(32, 32, False), (224, 224, False), (96, 64, True), (224, 224, True)])
 def test_an_image_may_change_as_soon_as_the_query_is_launched(H, W, own_stream):
     # images are staged while the query before runs, into two device images in turn: the host's one is overwritten the
     # moment execute() returns, nothing waits in between, and every query must still have seen its own
