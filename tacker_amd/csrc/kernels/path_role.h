@@ -108,7 +108,7 @@ __device__ __forceinline__ void path_window(int iteration, const int *__restrict
         // a pointer to the window's first column of a row, the same for the whole wavefront, and an unsigned 32-bit
         // lane offset (from there, since a row may have 2^30 columns).
         const int middle = iteration - 1;
-        const int window = min(max(blkX, 0), cols - 1);
+        const int window = __builtin_amdgcn_readfirstlane(min(max(blkX, 0), cols - 1));
         const unsigned at = (unsigned)(max(-(C - 1), min(x0, cols - 1)) - window + (C - 1)) * (unsigned)sizeof(int);
         const char *ahead = reinterpret_cast<const char *>(first + window - (C - 1));   // the row the next fetch takes
         int fetched = 0;
