@@ -7,7 +7,6 @@
 #define DNN_PATCH_LOADS ((DNN_PATCH * DNN_PATCH + 7) / 8)   // LDS-direct loads (8 pixels x 64 channels) per 64 channels
 #define DNN_PLANE_BYTES (DNN_PATCH_LOADS * 1024)
 #define DNN_PARTIAL_BYTES (DNN_TILE * DNN_TILE * 16 * 4)    // one segment's partial tile of 16 channels
-#define DNN_MAX_PARTIALS 32                            // partial tiles a workgroup keeps in LDS
 
 // where a layer's result goes
 typedef struct DnnOutput {

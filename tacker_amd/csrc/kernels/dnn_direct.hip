@@ -290,7 +290,6 @@ __device__ __forceinline__ void conv3x3_direct(const DnnConv &c, char *lds_gener
 DNN_CONV_KERNEL(1, 0, 1024)
 DNN_CONV_KERNEL(1, 1, 512)
 DNN_CONV_KERNEL(2, 0, 512)
-DNN_CONV_KERNEL(2, 1, 512)
 
 // The first convolution: the image, [H][W][3] fp32, 27 k in one matrix instruction.  A workgroup computes an 8 x 8 pixel
 // tile by 64 channels, wavefront g the pixel group g; a lane gathers its 8 k (of 32; the last 5 are padding) of its pixel.
@@ -457,7 +456,6 @@ extern "C" void tk_register_dnn_kernels(tk_kernel_insert_fn insert, void *ctx)
     insert("conv3x3_direct_1_0", (const void *)conv3x3_direct_1_0, ctx);
     insert("conv3x3_direct_1_1", (const void *)conv3x3_direct_1_1, ctx);
     insert("conv3x3_direct_2_0", (const void *)conv3x3_direct_2_0, ctx);
-    insert("conv3x3_direct_2_1", (const void *)conv3x3_direct_2_1, ctx);
     insert("conv3x3_image", (const void *)conv3x3_image, ctx);
     insert("fc_direct_1", (const void *)fc_direct_1, ctx);
     insert("fc_direct_2", (const void *)fc_direct_2, ctx);
