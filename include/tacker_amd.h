@@ -649,7 +649,11 @@ TK_API int tacker_task_logits(tacker_task_t task, const float **ptr, long *strid
 /* VGG16 only: weights (f16 [dims[0]][dims[1]] = [Cout padded][9*Cin padded], k =
  * (kh*3+kw)*Cin + c) and bias (f32 [dims[0]]) of convolution conv_index; 13..15: of the fully
  * connected layers ([out padded][in padded]; the last one has no bias: NULL).  Weights written there
- * are those of every later query; a graph recorded before this call keeps the ones it was recorded with */
+ * are those of every later query; a graph recorded before this call keeps the ones it was recorded with.
+ * From this call on the layer reads its weights as they lie there, through its operand builder and
+ * tzgemm, for as long as the task lives: 163 us a query at 224 x 224 become 173 with layer 5 handed
+ * out, 178 with layer 13, 206 with layer 0 (the query's image is then copied on the null stream) and
+ * 361 with all of them */
 TK_API int tacker_task_conv_params(tacker_task_t task, int conv_index, void **weights, float **bias,
                                    int dims[2]);
 TK_API int tacker_task_input(tacker_task_t task, float **host_ptr, int *bytes);

@@ -142,7 +142,8 @@ using namespace tk;
 //
 // What bounds it is the rate at which a CU takes data in, 80 to 100 GB/s from the L2s: at 28 x 28, 512 -> 512 channels a
 // workgroup (64 pixels x 32 channels, one per CU) loads 104 KB of patch and 295 KB of weights, 4.4 us of a 9.1 us
-// kernel; launch and the first load's latency are 3 us, the last sums and stores 1.5.  So a workgroup takes as many
+// kernel; launch and the first load's latency are 3 us, the last sums and stores 1.5 (by counters 97 MB asked of the L2s
+// there, matrix pipes busy 0.25 of the time, vector units 0.20, LDS bank conflicts 0.08).  So a workgroup takes as many
 // channels as leave every CU one, and two 16-channel slices a wavefront (NT = 2), which halves the fragment reads from
 // LDS, where eight wavefronts are left; the patch is asked for before the weights.  us a layer of VGG16 at 224 x
 // 224, against the operand in memory and tzgemm: conv1_2 38 -> 12, conv2_2 26 -> 10, conv3_2 21 -> 9.3, conv4_2 23 -> 9.1,
@@ -252,7 +253,8 @@ __device__ __forceinline__ void conv3x3_direct(const DnnConv &c, char *lds_gener
     // need; with the end's condition inside the loop the compiler has to allow for a fetch left out, and waited for all of
     // them every third chunk.  A query of one image over and over takes 163 instead of 167.5 us at 224 x 224, 106
     // instead of 113 at 64 x 96, 129 instead of 137 at 128 x 160.  More chunks in flight lose: 6 (9 with parts or two slices) 171 us and 113, 4 (5) 166 and
-    // 107 to 112, presumably by their longer code, which every launch of 5 to 10 us reads anew.
+    // 107 to 112.  (Why is not known.  It is not the longer code: 0.1 to 0.7 % of the instruction fetches of these launches
+    // miss.)
     int base = first;
     for (; base + RING < last; base += RING) {
 #pragma unroll

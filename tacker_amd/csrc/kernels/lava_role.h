@@ -23,9 +23,10 @@
 //    serves seven pairs.
 // A pair is 12 such instructions and the exponential.  At the end of a part the four rows' sums are added,
 // (g0 + g2) + (g1 + g3), by lane swaps that add two values at once, which leaves component v, y, x, z of the
-// total in row 0, 1, 2, 3; the total goes on from the output array.  24^3 boxes: 1.32 ms, 32^3: 3.1 ms (52 cycles a SIMD
+// total in row 0, 1, 2, 3; the total goes on from the output array.  24^3 boxes: 1.31 ms, 32^3: 3.1 ms (52 cycles a SIMD
 // and step of 64 slots); 2.86 and 5.35 ms with neighbours by scalar loads, two particles a lane, 25
-// instructions a pair.
+// instructions a pair.  (By counters the vector units issue all the time: 1.30 in the units in which a kernel that keeps all
+// SIMDs busy reads 1.)
 //
 // Few boxes: a box is then split over several wavefronts (P home particles a lane instead of 7, every particle
 // summed exactly as before), see LavaUnits.
