@@ -602,6 +602,9 @@ void VGG16::captured()
 void VGG16::executeQuery(cudaStream_t stream)
 {
     Impl &m = *impl;
+    // The null stream by its other name, hipStreamLegacy: kernels and events take it, but a question about it
+    // (its flags, whether it is recorded) is answered for the handles of streams that were created only.
+    if (stream == reinterpret_cast<cudaStream_t>(1)) stream = nullptr;
     if (stream) {
         // The copy on the null stream refuses to run while the stream is recorded.  The staged one would pass in a relaxed
         // recording, and every launch of the graph would see the image of this moment.

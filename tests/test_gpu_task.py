@@ -575,6 +575,35 @@ def test_queries_on_streams_of_any_kind_run_one_after_the_other(kinds, written):
         assert not s or ta.lib().tkStreamDestroy(s) == 0
 
 
+@pytest.mark.parametrize("handle", [1, 2])     # hipStreamLegacy, hipStreamPerThread
+@pytest.mark.parametrize("written", [False, True])
+def test_queries_on_the_streams_that_nobody_creates(handle, written):
+    # the runtime's constants for the null stream and the thread's own are streams like any other: images in turn, beside
+    # queries on the null stream; written: as above
+    task = ta.LcTask("vgg16", 64, 96)
+    if written:
+        task.conv_params(0)
+    image = task.host_input()
+    images = np.random.default_rng(14).random((2, image.size), dtype=np.float32)
+    p, stride, n = task.logits()
+    logits = lambda: ta.device_to_host(p, (n, stride), np.float32)[:, 0].copy()
+    want = []
+    for k in range(2):
+        image[:] = images[k]
+        task.execute(raw_stream=None)
+        torch.cuda.synchronize()
+        want.append(logits())
+    assert np.abs(want[0] - want[1]).max() > 0
+    for queries in (1, 2, 5, 8):
+        for k in range(queries):
+            image[:] = images[k % 2]
+            task.execute(raw_stream=None if k % 3 == 2 else C.c_void_p(handle))
+            image[:] = np.nan
+        torch.cuda.synchronize()
+        assert np.array_equal(logits(), want[(queries - 1) % 2]), queries
+    task.close()
+
+
 @pytest.mark.parametrize("blocking", [False, True])
 def test_a_query_comes_after_what_the_null_stream_has_in_front_of_it(blocking):
     # a bias written on the null stream behind 10 ms or more of waiting, and logits read on a blocking stream behind as much:
