@@ -25,10 +25,12 @@
 //    is the clamp of s to [0, 1], a modifier of the instruction that computes it, instead of a comparison and
 //    an execution mask.
 // The atoms' order, and so every point's sum, is the same in every form of the kernel.
-// 208^3 lattice, two layers of regions: 138 us, 26 layers 1.47 ms; 290 us and 3.07 ms with every atom of the list by scalar loads and
-// a branch for each point.  Where inv_cutoff2 is not 1 / cutoff2 every point walks the list by itself: 187 us, 2.06 ms.
+// 208^3 lattice, two layers of regions: 136 us, 26 layers 1.46 ms; 290 us and 3.07 ms with every atom of the list by scalar loads and
+// a branch for each point.  Where inv_cutoff2 is not 1 / cutoff2 every point walks the list by itself: 185 us, 2.05 ms.
 // (By counters the vector units issue all the time, 1.16 in the units in which a kernel that keeps all SIMDs busy reads 1.)
 #pragma once
+#include <cfloat>
+
 #include "role_common.h"
 #include "../header/cutcp_header.h"
 
@@ -124,10 +126,10 @@ __device__ __forceinline__ void cutcp_piece(int binDim_x, int binDim_y, const fl
         const unsigned before = (unsigned)(zeros >> (lane & ~(BIN_DEPTH - 1))) & (2u * (1u << slot) - 1u);
         return __ballot(before == 0u) & __ballot(place + (lane >> 3) < end);
     };
-    // ... and those it is finite and of ordinary size in
-    const auto finite = [](const float4_t &a) -> unsigned long long { return __ballot(__builtin_fabsf((a.x + a.y) + (a.z + a.w)) < 1e38f); };
+    // ... and those whose charge is a finite number
+    const auto finite = [](const float4_t &a) -> unsigned long long { return __ballot(__builtin_fabsf(a.w) <= FLT_MAX); };
     const int begin = walk.begin_of(part_begin);
-    unsigned long long all = ~0ull;   // slots looked at were finite
+    unsigned long long all = ~0ull;   // the lanes that have met finite charges only
     float4_t next = {0.f, 0.f, 0.f, 0.f};
     Entry ahead = {0, 0, 0};
     if (begin < end) {
@@ -138,12 +140,12 @@ __device__ __forceinline__ void cutcp_piece(int binDim_x, int binDim_y, const fl
         const float4_t a = next;
         next = fetch(ahead);
         ahead = entry(place + 2 * CUTCP_BATCH_BINS);
-        const float ex = fmaxf(fmaxf(box_x0 - a.x, a.x - box_x1), 0.f);
-        const float ey = fmaxf(fmaxf(box_y0 - a.y, a.y - box_y1), 0.f);
-        const float ez = fmaxf(fmaxf(box_z0 - a.z, a.z - box_z1), 0.f);
+        // how far the atom is from the box (no number, and so out of reach, where a coordinate is none)
+        const float ex = a.x - __builtin_amdgcn_fmed3f(a.x, box_x0, box_x1);
+        const float ey = a.y - __builtin_amdgcn_fmed3f(a.y, box_y0, box_y1);
+        const float ez = a.z - __builtin_amdgcn_fmed3f(a.z, box_z0, box_z1);
         const float e2 = ex * ex + ey * ey + ez * ez;
-        // beyond a point's cutoff the clamp makes s zero, and the term with it unless the charge is infinite or no number;
-        // and a coordinate that is no number is within no cutoff, where the maxima above take it for nothing
+        // beyond a point's cutoff the clamp makes s zero, and the term with it unless the charge is infinite or no number
         // (whole masks, so that no branch and no mask made into numbers and back comes of it)
         const unsigned long long usable = CLAMP ? finite(a) : ~0ull;
         all &= usable;
@@ -196,7 +198,7 @@ __device__ __forceinline__ void cutcp_piece(int binDim_x, int binDim_y, const fl
     }
     // The atoms left out are compared with the cutoff, on a walk of their own: a sum they are part of is infinite or no
     // number whenever they are added.  (As a second form of the loop above, chosen for every 64 slots, this cost 1.5 us of
-    // 26 at 36 regions and 2.3 of 45 at 361; now the check costs nothing there, and 0.7 of 138 at 1352.)
+    // 26 at 36 regions and 2.3 of 45 at 361.)
     if (CLAMP && all != ~0ull) {   // uniform
         for (int place = begin; place < end; place += CUTCP_BATCH_BINS) {
             const float4_t a = fetch(entry(place));
