@@ -165,12 +165,12 @@ extern "C" __global__ __launch_bounds__(TK_WAVE_SIZE) void ori_path(int iteratio
 
 // grid (boxes), block 64: a wavefront per home box, all 27 parts of its work, where the reference
 // launches 128 threads (src/ori_kernel/lava_kernel.cu:9-141)
-extern "C" __global__ __launch_bounds__(TK_WAVE_SIZE) void ori_lava(par_str d_par_gpu, dim_str d_dim_gpu,
-                                                                    box_str *d_box_gpu, FOUR_VECTOR *d_rv_gpu,
-                                                                    float *d_qv_gpu, FOUR_VECTOR *d_fv_gpu)
+extern "C" __global__ __launch_bounds__(TK_WAVE_SIZE, 4) void ori_lava(par_str d_par_gpu, dim_str d_dim_gpu,
+                                                                       box_str *d_box_gpu, FOUR_VECTOR *d_rv_gpu,
+                                                                       float *d_qv_gpu, FOUR_VECTOR *d_fv_gpu)
 {
-    tk::lava_role(d_par_gpu, d_dim_gpu, d_box_gpu, d_rv_gpu, d_qv_gpu, d_fv_gpu, (int)gridDim.x, (int)blockIdx.x,
-                  (int)gridDim.x, 0, (int)gridDim.x * LAVA_PARTS, (int)threadIdx.x, TK_WAVE_SIZE);
+    tk::lava_role<1>(d_par_gpu, d_dim_gpu, d_box_gpu, d_rv_gpu, d_qv_gpu, d_fv_gpu, (int)gridDim.x, (int)blockIdx.x,
+                     (int)gridDim.x, 0, (int)gridDim.x * LAVA_PARTS, (int)threadIdx.x, TK_WAVE_SIZE);
 }
 
 // Values that depend on (index, seed) only, for the default instances of the large kernels.

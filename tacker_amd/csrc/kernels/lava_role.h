@@ -8,27 +8,32 @@
 // Replaces ori_lava / general_ptb_lava (src/ori_kernel/lava_kernel.cu:9-141,
 // src/gptb_kernel/lava_kernel.cu:3-140 of the reference).  The reference gives a home box to a
 // block of 128 threads and stages the home and the neighbour particles in shared memory between
-// block barriers.  Here wavefronts serve a box without LDS and without a barrier.  fp32; the exponential is
+// block barriers.  Here wavefronts serve a box without a barrier, each with LDS of its own.  fp32; the exponential is
 // the hardware's 2^x of -r2 a2 log2(e) where the reference calls CUDA's expf, and multiply-adds are fused:
 // results agree within a tolerance, not bit for bit.
 //
-// What bounds it is VALU issue, so two things count.
-//  * Which registers an instruction reads: with all operands in vector registers a 32-bit multiply, add or
-//    fused multiply-add takes about 2.3 cycles of a SIMD with two or more waves at work, with a scalar
-//    register among them 4.4 (measured; the exponential 8.5 either way).  Neighbour particles are the same
-//    for many lanes, but they arrive by vector loads (one address for 16 lanes), not by scalar ones.
-//  * How full the lanes are: 100 particles on 64 lanes, one neighbour at a time, leave 22 % of the slots
-//    empty.  The wavefront is four rows of 16 lanes: row g takes neighbours g, g + 4, g + 8, ... (25 of the
-//    100), a lane LAVA_MAX_P = 7 home particles (112 slots for 100) -- 89 % of the slots work, and a load
-//    serves seven pairs.
-// A pair is 12 such instructions and the exponential.  At the end of a part the four rows' sums are added,
+// What bounds it is VALU issue (measured, cycles of a SIMD an instruction with two or more wavefronts at work: 32-bit
+// add, multiply, fused multiply-add 2.5 to 2.8 with all operands in vector registers and 4.4 with a scalar one, the
+// exponential 8.4, and MFMAs take the same slots), so three things count.
+//  * How many instructions a pair takes.  The force on i is a sum of w (xi - xj), w = qj vij; it is computed as
+//    (xi - c) sum w - sum vij [qj (xj - c)], which leaves four multiply-adds a pair (v and the force together)
+//    where the difference, its product and the sum of w took eight instructions.  c is about the middle of the home box (lava_centre),
+//    so that the two terms are of the size of the force and nothing cancels: against 64 bits the result is as far off as with
+//    the differences (2-norm of the whole output, 2^3 / 5^3 / 9^3 / 24^3 boxes: 5.0 / 7.3 / 7.6 / 7.9e-8 both ways; of
+//    the forces alone 5.4 / 7.3 / 7.7 / 7.9e-8 against 5.2 / 7.3 / 7.6 / 7.9e-8).
+//  * What is computed per neighbour and not per pair.  A wavefront prepares the 100 neighbours of a part once, a lane
+//    each: {scale v, -scale x, -scale y, -scale z} and {q, q (x - cx), q (y - cy), q (z - cz)} go to LDS and
+//    come back as two 16-byte broadcast reads a step.  (By a vector load for every step and row of lanes, and four multiplies
+//    behind it, this was a tenth of the time.)
+//  * How full the lanes are.  The wavefront is four rows of 16 lanes: row g takes neighbours g, g + 4, g + 8, ... (25 of the
+//    100), a lane LAVA_MAX_P = 6 of the first 96 home particles: 150 steps without an empty slot.  The last four
+//    particles are four lanes side by side, 16 neighbours at a time: 7 steps, where a seventh particle a lane would take 25.
+// A pair is 8 such instructions and the exponential.  At the end of a part the four rows' sums are added,
 // (g0 + g2) + (g1 + g3), by lane swaps that add two values at once, which leaves component v, y, x, z of the
-// total in row 0, 1, 2, 3; the total goes on from the output array.  24^3 boxes: 1.31 ms, 32^3: 3.1 ms (52 cycles a SIMD
-// and step of 64 slots); 2.86 and 5.35 ms with neighbours by scalar loads, two particles a lane, 25
-// instructions a pair.  (By counters the vector units issue all the time: 1.30 in the units in which a kernel that keeps all
-// SIMDs busy reads 1.)
+// total in row 0, 1, 2, 3; the total goes on from the output array.  24^3 boxes: 837 us (35 cycles a SIMD and step of 64 pairs), where twelve instructions
+// a pair, neighbours by vector loads and seven particles a lane took 1325; 18^3 372 / 577, 9^3 78 / 116, 3^3 36.5 / 46.
 //
-// Few boxes: a box is then split over several wavefronts (P home particles a lane instead of 7, every particle
+// Few boxes: a box is then split over several wavefronts (P home particles a lane instead of 6, every particle
 // summed exactly as before), see LavaUnits.
 //
 // Block positions.  A box through its 27 boxes is 270 000 pair interactions, 180 us of one
@@ -39,6 +44,8 @@
 // rows of the grid in order, so a box's parts are added in ascending order without any
 // synchronisation and whole rows that follow each other are one run through their parts.
 #pragma once
+#include <cfloat>
+
 #include "role_common.h"
 #include "../header/lava_header.h"
 
@@ -48,14 +55,24 @@ typedef __attribute__((address_space(4))) const box_str lava_const_box;
 
 #define LAVA_ROWS 4                                     // rows of 16 lanes: neighbours are dealt to them in turn
 #define LAVA_LANES 16                                   // home particles side by side in a row
-#define LAVA_MAX_P 7                                    // home particles per lane when one wavefront serves a box
+#define LAVA_MAX_P 6                                    // home particles per lane when one wavefront serves a box
 #define LAVA_WAVES_PER_SIMD 4                           // wavefronts of this role a SIMD holds (registers)
 #define LAVA_STEPS (NUMBER_PAR_PER_BOX / LAVA_ROWS)     // neighbours a row takes per box
-// of them in flight: a step of a lane with many particles outlasts a load by itself, and the registers of
-// more would cost a wavefront of the SIMD
-#define LAVA_AHEAD(P_) ((P_) >= 4 ? 1 : 5)
-static_assert(NUMBER_PAR_PER_BOX % LAVA_ROWS == 0 && LAVA_STEPS % 5 == 0, "rows and fetches come out even");
-static_assert(LAVA_LANES * LAVA_MAX_P >= NUMBER_PAR_PER_BOX, "a wavefront holds a box");
+#define LAVA_REST 4                                     // home particles behind the lanes' own ...
+#define LAVA_REST_FROM (NUMBER_PAR_PER_BOX - LAVA_REST)
+#define LAVA_REST_STEP (TK_WAVE_SIZE / LAVA_REST)       // ... and the neighbours they take a step
+static_assert(NUMBER_PAR_PER_BOX % LAVA_ROWS == 0 && LAVA_LANES * LAVA_MAX_P == LAVA_REST_FROM, "rows and lanes come out even");
+static_assert(NUMBER_PAR_PER_BOX > TK_WAVE_SIZE && NUMBER_PAR_PER_BOX <= 2 * TK_WAVE_SIZE, "two neighbours a lane are staged");
+
+typedef __attribute__((address_space(3))) float4_t lava_lds_float4;
+
+// the LDS of the role's wavefronts: two float4s a neighbour, and the last home particles.  role_wave: the calling wavefront's number within the role
+template <int WAVES>
+__device__ __forceinline__ lava_lds_float4 *lava_stage_of_wave(int role_wave)
+{
+    __shared__ __align__(16) float4_t lava_stage[WAVES][2 * NUMBER_PAR_PER_BOX + LAVA_REST];
+    return (lava_lds_float4 *)&lava_stage[role_wave][0];
+}
 
 // the halves of a wavefront, and the rows of its halves, exchanged between two registers: after it a holds
 // the lower half (even rows) of both, b the upper half (odd rows)
@@ -70,14 +87,43 @@ __device__ __forceinline__ float lava_fold_rows(float a, float b)
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);   // even rows: sum of a's pair, odd rows: of b's
 }
 
-// box `bx`, parts [part_begin, part_end) of its list, for the 16 P home particles from 16 P `sub` on, by one
-// wavefront.  scale = -a2 log2(e).
+// v plus the value n lanes further along the row of 16 (around its end)
+template <int N>
+__device__ __forceinline__ float lava_add_along_row(float v)
+{
+    return v + __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x120 + N, 0xf, 0xf, false));
+}
+
+// About the middle of the home box, the same for every wavefront that serves a part of it: the median of three thirds' means,
+// which one particle far away -- or one that is no number -- does not move, and 0 where that is not finite either.
+__device__ __forceinline__ void lava_centre(const float4_t *rA, int lane, float (&centre)[3])
+{
+    const float4_t lo = rA[lane], hi = rA[min(lane + TK_WAVE_SIZE, NUMBER_PAR_PER_BOX - 1)];
+    const bool two = lane + TK_WAVE_SIZE < NUMBER_PAR_PER_BOX;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        float v = lo[c + 1] + (two ? hi[c + 1] : 0.f);
+        v = lava_add_along_row<8>(v);
+        v = lava_add_along_row<4>(v);
+        v = lava_add_along_row<2>(v);
+        v = lava_add_along_row<1>(v);
+        float row[LAVA_ROWS];
+#pragma unroll
+        for (int g = 0; g < LAVA_ROWS; ++g)
+            row[g] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), LAVA_LANES * g));
+        // particles 0 - 15 and 64 - 79, 16 - 31 and 80 - 95, 32 - 63 and 96 - 99
+        const float m = __builtin_amdgcn_fmed3f(row[0] * (1.f / 32), row[1] * (1.f / 32), (row[2] + row[3]) * (1.f / 36));
+        centre[c] = __builtin_fabsf(m) <= FLT_MAX ? m : 0.f;
+    }
+}
+
+// box `bx`, parts [part_begin, part_end) of its list, for the 16 P home particles from 16 P `sub` on -- and the last four,
+// if `rest` -- by one wavefront.  scale = -a2 log2(e).  stage: this wavefront's LDS.
 template <int P>
 __device__ __forceinline__ void lava_box(const float scale, const box_str *d_box_gpu, const FOUR_VECTOR *d_rv_gpu,
-                                         const float *d_qv_gpu, FOUR_VECTOR *d_fv_gpu, int bx, int sub, int part_begin,
-                                         int part_end, int lane)
+                                         const float *d_qv_gpu, FOUR_VECTOR *d_fv_gpu, int bx, int sub, bool rest,
+                                         int part_begin, int part_end, int lane, lava_lds_float4 *stage)
 {
-    constexpr int AHEAD = LAVA_AHEAD(P);
     const lava_const_box *boxes = (const lava_const_box *)d_box_gpu;
     const long first_i = boxes[bx].offset;
     const int neighbours = boxes[bx].nn;
@@ -89,92 +135,133 @@ __device__ __forceinline__ void lava_box(const float scale, const box_str *d_box
     const float4_t *rA = reinterpret_cast<const float4_t *>(d_rv_gpu + first_i);
     float *fA = reinterpret_cast<float *>(d_fv_gpu + first_i) + component;
     float4_t home[P];   // {scale v, x, y, z}
-    float total[P];
+    float total[P], last_total;
 #pragma unroll
     for (int k = 0; k < P; ++k) {
         const int i = (sub * P + k) * LAVA_LANES + (lane & (LAVA_LANES - 1));
-        const int in = i < NUMBER_PAR_PER_BOX ? i : 0;   // slots past the box compute along and are not stored
-        home[k] = rA[in];
+        home[k] = rA[i];
         home[k][0] *= scale;
-        total[k] = fA[4 * in];
+        total[k] = fA[4 * i];
     }
-    // A neighbour is named by its number alone (its offset in the list is not read): two loads behind one another.  The
-    // first is issued two parts ahead, the second one; where there is no such part, the home box's own are read.  Both at
-    // the part's start took 1347 us at 24^3 boxes and 403 at 14^3, this 1315 and 379.
+    lava_lds_float4 *rest_home = stage + 2 * NUMBER_PAR_PER_BOX;
+    if (lane < LAVA_REST) {
+        float4_t r = rA[LAVA_REST_FROM + lane];
+        r[0] *= scale;
+        rest_home[lane] = r;
+    }
+    last_total = fA[4 * (LAVA_REST_FROM + (lane & (LAVA_REST - 1)))];
+    float centre[3];
+    lava_centre(rA, lane, centre);
+    // A neighbour is named by its number alone (its offset in the list is not read): two loads behind one another, and the
+    // particles behind them.  The number is fetched three parts ahead, the offset two, the particles one; where there is no such part,
+    // the home box's own are read.
     const auto box_of = [&](int part) -> int { return part == 0 || part >= part_end ? bx : boxes[bx].nei[part - 1].number; };
-    long next_j = boxes[box_of(part_begin)].offset;
-    int after_next = box_of(part_begin + 1);
+    const int second = min(lane + TK_WAVE_SIZE, NUMBER_PAR_PER_BOX - 1);   // a lane's second neighbour (past the last: not used)
+    float4_t r0, r1;
+    float q0, q1;
+    const auto fetch = [&](long first_j) {
+        const float4_t *rB = reinterpret_cast<const float4_t *>(d_rv_gpu + first_j);
+        const float *qB = d_qv_gpu + first_j;
+        r0 = rB[lane];
+        r1 = rB[second];
+        q0 = qB[lane];
+        q1 = qB[second];
+    };
+    fetch(boxes[box_of(part_begin)].offset);
+    long next_j = boxes[box_of(part_begin + 1)].offset;
+    int after_next = box_of(part_begin + 2);
     for (int part = part_begin; part < part_end; ++part) {
-        const long first_j = next_j;
+        const auto put = [&](int j, const float4_t &r, float q) {
+            stage[2 * j] = float4_t{scale * r[0], -scale * r[1], -scale * r[2], -scale * r[3]};
+            stage[2 * j + 1] = float4_t{q, q * (r[1] - centre[0]), q * (r[2] - centre[1]), q * (r[3] - centre[2])};
+        };
+        // the wavefront's reads of the part before are behind it: LDS serves a wavefront in order
+        put(lane, r0, q0);
+        if (lane < NUMBER_PAR_PER_BOX - TK_WAVE_SIZE) put(lane + TK_WAVE_SIZE, r1, q1);
+        fetch(next_j);
         next_j = boxes[after_next].offset;
-        after_next = box_of(part + 2);
-        const float4_t *rB = reinterpret_cast<const float4_t *>(d_rv_gpu + first_j) + row;
-        const float *qB = d_qv_gpu + first_j + row;
-        float4_t f[P];
+        after_next = box_of(part + 3);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+
+        float4_t f[P];   // sums of w, and of vij q (x - c) component by component
 #pragma unroll
         for (int k = 0; k < P; ++k) f[k] = float4_t{0.f, 0.f, 0.f, 0.f};
-        float4_t rb[AHEAD];
-        float qb[AHEAD];
+        const lava_lds_float4 *at = stage + 2 * row;
+        float4_t a = at[0], b = at[1];
+        // Six particles a lane are chains enough for the compiler to interleave as it likes (24^3 boxes 829 us, with the step's
+        // read held in front of it 871); with fewer, the reads stay in front of a step's work and every step is written out (3^3 boxes
+        // 36.5 us; 42.1 in a loop of five steps, 43.2 as the compiler likes).
+#pragma unroll P < LAVA_MAX_P ? LAVA_STEPS : 5
+        for (int t = 0; t < LAVA_STEPS; ++t) {
+            at += 2 * LAVA_ROWS;
+            const lava_lds_float4 *next = t + 1 < LAVA_STEPS ? at : stage;   // (the last read is not used)
+            const float4_t na = next[0], nb = next[1];
+            if (P < LAVA_MAX_P) __builtin_amdgcn_sched_barrier(0);
+            // scale (vi + vj - (xi xj + yi yj + zi zj)) = -r2 a2 log2(e), stage by stage over the lane's
+            // particles: their chains are independent, and in this order none waits for its own last result
+            float w[P];
 #pragma unroll
-        for (int u = 0; u < AHEAD; ++u) {
-            rb[u] = rB[LAVA_ROWS * u];
-            qb[u] = qB[LAVA_ROWS * u];
-        }
-        for (int t = 0; t < LAVA_STEPS; t += AHEAD) {
-            const int next = t + AHEAD < LAVA_STEPS ? t + AHEAD : 0;   // (the last fetch is not used)
+            for (int k = 0; k < P; ++k) w[k] = home[k][0] + a[0];
 #pragma unroll
-            for (int u = 0; u < AHEAD; ++u) {
-                const float4_t b = rb[u];
-                const float q = qb[u];
-                rb[u] = rB[LAVA_ROWS * (next + u)];
-                qb[u] = qB[LAVA_ROWS * (next + u)];
-                // scale (vi + vj - (xi xj + yi yj + zi zj)) = -r2 a2 log2(e), stage by stage over the lane's
-                // particles: their chains are independent, and in this order none waits for its own last result
-                const float4_t sb = {scale * b[0], -scale * b[1], -scale * b[2], -scale * b[3]};
-                float w[P];
+            for (int c = 1; c < 4; ++c)
 #pragma unroll
-                for (int k = 0; k < P; ++k) w[k] = home[k][0] + sb[0];
+                for (int k = 0; k < P; ++k) w[k] = __builtin_fmaf(home[k][c], a[c], w[k]);
 #pragma unroll
-                for (int c = 1; c < 4; ++c)
+            for (int k = 0; k < P; ++k) w[k] = __builtin_amdgcn_exp2f(w[k]);
 #pragma unroll
-                    for (int k = 0; k < P; ++k) w[k] = __builtin_fmaf(home[k][c], sb[c], w[k]);
+            for (int c = 0; c < 4; ++c)
 #pragma unroll
-                for (int k = 0; k < P; ++k) w[k] = __builtin_amdgcn_exp2f(w[k]);
-#pragma unroll
-                for (int k = 0; k < P; ++k) w[k] *= q;
-#pragma unroll
-                for (int k = 0; k < P; ++k) f[k][0] += w[k];
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int c = 1; c < 4; ++c) {
-                    float d[P];
-#pragma unroll
-                    for (int k = 0; k < P; ++k) d[k] = home[k][c] - b[c];
-#pragma unroll
-                    for (int k = 0; k < P; ++k) f[k][c] = __builtin_fmaf(w[k], d[k], f[k][c]);
-                    __builtin_amdgcn_sched_barrier(0);   // (fewer differences alive at a time)
-                }
-            }
+                for (int k = 0; k < P; ++k) f[k][c] = __builtin_fmaf(w[k], b[c], f[k][c]);
+            if (P < LAVA_MAX_P) __builtin_amdgcn_sched_barrier(0);
+            a = na;
+            b = nb;
         }
 #pragma unroll
-        for (int k = 0; k < P; ++k)
+        for (int k = 0; k < P; ++k) {
+#pragma unroll
+            for (int c = 1; c < 4; ++c) f[k][c] = __builtin_fmaf(home[k][c] - centre[c - 1], f[k][0], -f[k][c]);
             total[k] += twice * lava_fold_rows(lava_fold_halves(f[k][0], f[k][1]), lava_fold_halves(f[k][2], f[k][3]));
+        }
+        if (rest) {   // uniform
+            const float4_t last = rest_home[lane & (LAVA_REST - 1)];
+            float4_t g = {0.f, 0.f, 0.f, 0.f};
+            const auto pair = [&](int j) {
+                const float4_t a = stage[2 * j], b = stage[2 * j + 1];
+                float w = last[0] + a[0];
+#pragma unroll
+                for (int c = 1; c < 4; ++c) w = __builtin_fmaf(last[c], a[c], w);
+                w = __builtin_amdgcn_exp2f(w);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) g[c] = __builtin_fmaf(w, b[c], g[c]);
+            };
+            const int from = lane / LAVA_REST;
+#pragma unroll
+            for (int j = 0; j + LAVA_REST_STEP <= NUMBER_PAR_PER_BOX; j += LAVA_REST_STEP) pair(j + from);
+            if (from < NUMBER_PAR_PER_BOX % LAVA_REST_STEP) pair(NUMBER_PAR_PER_BOX / LAVA_REST_STEP * LAVA_REST_STEP + from);
+#pragma unroll
+            for (int c = 1; c < 4; ++c) g[c] = __builtin_fmaf(last[c] - centre[c - 1], g[0], -g[c]);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) g[c] = lava_add_along_row<4>(lava_add_along_row<8>(g[c]));
+            last_total += twice * lava_fold_rows(lava_fold_halves(g[0], g[1]), lava_fold_halves(g[2], g[3]));
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
     }
 #pragma unroll
-    for (int k = 0; k < P; ++k) {
-        const int i = (sub * P + k) * LAVA_LANES + (lane & (LAVA_LANES - 1));
-        if (i < NUMBER_PAR_PER_BOX) fA[4 * i] = total[k];
-    }
+    for (int k = 0; k < P; ++k) fA[4 * ((sub * P + k) * LAVA_LANES + (lane & (LAVA_LANES - 1)))] = total[k];
+    if (rest && (lane & (LAVA_LANES - 1)) < LAVA_REST) fA[4 * (LAVA_REST_FROM + (lane & (LAVA_REST - 1)))] = last_total;
 }
 
 // wavefronts a box is split over with P home particles a lane
 __device__ __forceinline__ constexpr int lava_subs(int P)
 {
-    return (NUMBER_PAR_PER_BOX + LAVA_LANES * P - 1) / (LAVA_LANES * P);
+    return LAVA_REST_FROM / (LAVA_LANES * P);
 }
 
 // Which wavefront takes what.  A unit is a box, or a part of its home particles: the first `whole` boxes are one
-// unit each (7 particles a lane), the boxes behind them `subs` units each of 16 P particles.  A wavefront serves
+// unit each (6 particles a lane), the boxes behind them `subs` units each of 16 P particles.  A wavefront serves
 // the units it owns -- first_owned, first_owned + stride, ... -- through all phases of a launch.
 struct LavaUnits {
     int whole;   // boxes of one unit each
@@ -182,19 +269,23 @@ struct LavaUnits {
     int subs;    // units each of them makes
 
     // `waves` wavefronts serve `boxes` boxes.  Whole rounds of as many boxes as wavefronts are at work at a time
-    // take a box each; what is left over -- all of it when the domain is small -- is cut as fine as makes no more
-    // units than those wavefronts: a box is 0.1 to 0.4 ms of one wavefront, with up to 4 of them on a SIMD, and a
-    // last round of few boxes would leave most of the chip idle that long.  (Cut finer throughout, lanes are
-    // emptier -- 78 % of the slots work with 2 and 4 particles a lane -- and a load serves fewer pairs.)
-    // Measured against one unit a box throughout: 24^3 boxes (three rounds and 1536 boxes) 1.32 against 1.62 ms, 18^3
-    // 0.58 / 0.74; against the kernel without any split 8^3 0.10 / 0.30, 3^3 0.05 / 0.30, 2^3 0.016 / 0.093 ms.
+    // take a box each; what is left over -- all of it when the domain is small -- is cut: a box is 0.1 to 0.3 ms of
+    // one wavefront, with up to 4 of them on a SIMD, and a last round of few boxes would leave most of the chip idle that
+    // long.  Finer cuts spread better, but every wavefront prepares the neighbours again and a read serves fewer pairs.  us
+    // with everything left over in units of 6 / 3 / 2 / 1 particles a lane, in a launch of more wavefronts than are at work
+    // at a time, which the dispatcher evens out:
+    //     8^3 (512 boxes) 117 / 63 / 66 / 60,  9^3 (729) 116 / 86 / 79 / 70,  11^3 (1331) 160 / 120 / 120 / 113,
+    //     12^3 (1728) 163 / 153 / 137 / 140,  13^3 (2197) 218 / 149 / 157 / 172,  15^3 (3375) 296 / 229 / 224 / 255,
+    //     24^3 (3 x 4096 + 1536) 833 / 823 / 818 / 829.
+    // In a launch of fewer, whose wavefronts each have their units from the start, the finest cut that gives nobody two.
     __device__ __forceinline__ LavaUnits(int boxes, int waves)
     {
         const int at_once = min(waves, LAVA_WAVES_PER_SIMD * 4 * TK_CU_NUM);
+        const bool evened = waves > at_once;
         whole = boxes / at_once * at_once;
         const int left = boxes - whole;
-        p = left * lava_subs(1) <= at_once * 3 / 4 ? 1 : (left * lava_subs(2) <= at_once ? 2 : (left * lava_subs(4) <= at_once ? 4 : LAVA_MAX_P));
-        subs = p == 1 ? lava_subs(1) : (p == 2 ? lava_subs(2) : (p == 4 ? lava_subs(4) : 1));
+        p = left * (evened ? 3 : lava_subs(1)) <= at_once ? 1 : (left * (evened ? 2 : lava_subs(2)) <= at_once ? 2 : (evened || left * lava_subs(3) <= at_once ? 3 : LAVA_MAX_P));
+        subs = p == 1 ? lava_subs(1) : (p == 2 ? lava_subs(2) : (p == 3 ? lava_subs(3) : 1));
     }
     __device__ __forceinline__ int first_of(int box) const { return box <= whole ? box : whole + (box - whole) * subs; }
 };
@@ -203,7 +294,7 @@ struct LavaUnits {
 __device__ __forceinline__ void lava_phase(const LavaUnits units, int box_lo, int box_hi, int part_begin, int part_end,
                                            const float scale, const box_str *d_box_gpu, const FOUR_VECTOR *d_rv_gpu,
                                            const float *d_qv_gpu, FOUR_VECTOR *d_fv_gpu, int first_owned, int stride,
-                                           int lane)
+                                           int lane, lava_lds_float4 *stage)
 {
     const int lo = units.first_of(box_lo), hi = units.first_of(box_hi);
     int c = first_owned;
@@ -214,9 +305,10 @@ __device__ __forceinline__ void lava_phase(const LavaUnits units, int box_lo, in
         const int box = left < 0 ? unit : units.whole + left / units.subs;
         const int sub = left < 0 ? 0 : left % units.subs;
         const int p = left < 0 ? LAVA_MAX_P : units.p;
-#define LAVA_BOX(P_) lava_box<P_>(scale, d_box_gpu, d_rv_gpu, d_qv_gpu, d_fv_gpu, box, sub, part_begin, part_end, lane)
+        const bool rest = left < 0 || sub == units.subs - 1;
+#define LAVA_BOX(P_) lava_box<P_>(scale, d_box_gpu, d_rv_gpu, d_qv_gpu, d_fv_gpu, box, sub, rest, part_begin, part_end, lane, stage)
         if (p == LAVA_MAX_P) LAVA_BOX(LAVA_MAX_P);
-        else if (p == 4) LAVA_BOX(4);
+        else if (p == 3) LAVA_BOX(3);
         else if (p == 2) LAVA_BOX(2);
         else LAVA_BOX(1);
 #undef LAVA_BOX
@@ -225,14 +317,17 @@ __device__ __forceinline__ void lava_phase(const LavaUnits units, int box_lo, in
 
 // grid_dimension_x: boxes (the reference's grid); the position grid has the boxes as columns and the
 // LAVA_PARTS parts as rows.  A range that runs past the grid wraps.
+// WAVES: wavefronts of a workgroup that there is LDS for; those of a larger workgroup leave the units to them.
+template <int WAVES>
 __device__ __forceinline__ void lava_role(par_str d_par_gpu, dim_str d_dim_gpu, const box_str *d_box_gpu,
                                           const FOUR_VECTOR *d_rv_gpu, const float *d_qv_gpu, FOUR_VECTOR *d_fv_gpu,
                                           int grid_dimension_x, int role_block, int role_blocks, int start, int end,
                                           int tid, int role_threads)
 {
-    const int waves = role_threads / TK_WAVE_SIZE;
+    const int waves = min(role_threads / TK_WAVE_SIZE, WAVES);
     const int wave = tid / TK_WAVE_SIZE;
     if (wave >= waves || start >= end) return;
+    lava_lds_float4 *stage = lava_stage_of_wave<WAVES>(__builtin_amdgcn_readfirstlane(wave));
     const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
     // boxes past number_boxes do nothing in the reference (src/ori_kernel/lava_kernel.cu:21)
     const int gx = (long)grid_dimension_x < d_dim_gpu.number_boxes ? grid_dimension_x : (int)d_dim_gpu.number_boxes;
@@ -257,7 +352,7 @@ __device__ __forceinline__ void lava_role(par_str d_par_gpu, dim_str d_dim_gpu, 
         const int last = min(hi, gx);
         if (lo >= last) continue;
         lava_phase(units, lo, last, part, part + rows, scale, d_box_gpu, d_rv_gpu, d_qv_gpu, d_fv_gpu, first_owned, stride,
-                   lane);
+                   lane, stage);
     }
 }
 

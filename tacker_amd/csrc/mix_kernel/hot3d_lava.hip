@@ -55,7 +55,7 @@ extern "C" __global__ __launch_bounds__(256) void hot3d_lava_mix_wg_1_1(
     if (sp.role == 0) {
         tk::hot3d_role(hot3d0_p, hot3d0_tIn, hot3d0_tOut, hot3d0_sdc, hot3d0_nx, hot3d0_ny, hot3d0_nz, hot3d0_ce, hot3d0_cw, hot3d0_cn, hot3d0_cs, hot3d0_ct, hot3d0_cb, hot3d0_cc, hot3d0_grid_dimension_x, hot3d0_grid_dimension_y, hot3d0_block_dimension_x, hot3d0_block_dimension_y, sp.role_block, sp.role_blocks, hot3d0_ptb_start_block_pos, hot3d0_ptb_end_block_pos, (int)threadIdx.x, 256);
     } else {
-        tk::lava_role(lava1_d_par_gpu, lava1_d_dim_gpu, lava1_d_box_gpu, lava1_d_rv_gpu, lava1_d_qv_gpu, lava1_d_fv_gpu, lava1_grid_dimension_x, sp.role_block, sp.role_blocks, lava1_ptb_start_block_pos, lava1_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::lava_role<4>(lava1_d_par_gpu, lava1_d_dim_gpu, lava1_d_box_gpu, lava1_d_rv_gpu, lava1_d_qv_gpu, lava1_d_fv_gpu, lava1_grid_dimension_x, sp.role_block, sp.role_blocks, lava1_ptb_start_block_pos, lava1_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
 }
 
@@ -113,7 +113,7 @@ extern "C" __global__ __launch_bounds__(256) void hot3d_lava_mix_wg_1_2(
     if (sp.role == 0) {
         tk::hot3d_role(hot3d0_p, hot3d0_tIn, hot3d0_tOut, hot3d0_sdc, hot3d0_nx, hot3d0_ny, hot3d0_nz, hot3d0_ce, hot3d0_cw, hot3d0_cn, hot3d0_cs, hot3d0_ct, hot3d0_cb, hot3d0_cc, hot3d0_grid_dimension_x, hot3d0_grid_dimension_y, hot3d0_block_dimension_x, hot3d0_block_dimension_y, sp.role_block, sp.role_blocks, hot3d0_ptb_start_block_pos, hot3d0_ptb_end_block_pos, (int)threadIdx.x, 256);
     } else {
-        tk::lava_role(lava1_d_par_gpu, lava1_d_dim_gpu, lava1_d_box_gpu, lava1_d_rv_gpu, lava1_d_qv_gpu, lava1_d_fv_gpu, lava1_grid_dimension_x, sp.role_block, sp.role_blocks, lava1_ptb_start_block_pos, lava1_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::lava_role<4>(lava1_d_par_gpu, lava1_d_dim_gpu, lava1_d_box_gpu, lava1_d_rv_gpu, lava1_d_qv_gpu, lava1_d_fv_gpu, lava1_grid_dimension_x, sp.role_block, sp.role_blocks, lava1_ptb_start_block_pos, lava1_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
 }
 
@@ -171,7 +171,7 @@ extern "C" __global__ __launch_bounds__(256) void hot3d_lava_mix_wg_2_1(
     if (sp.role == 0) {
         tk::hot3d_role(hot3d0_p, hot3d0_tIn, hot3d0_tOut, hot3d0_sdc, hot3d0_nx, hot3d0_ny, hot3d0_nz, hot3d0_ce, hot3d0_cw, hot3d0_cn, hot3d0_cs, hot3d0_ct, hot3d0_cb, hot3d0_cc, hot3d0_grid_dimension_x, hot3d0_grid_dimension_y, hot3d0_block_dimension_x, hot3d0_block_dimension_y, sp.role_block, sp.role_blocks, hot3d0_ptb_start_block_pos, hot3d0_ptb_end_block_pos, (int)threadIdx.x, 256);
     } else {
-        tk::lava_role(lava1_d_par_gpu, lava1_d_dim_gpu, lava1_d_box_gpu, lava1_d_rv_gpu, lava1_d_qv_gpu, lava1_d_fv_gpu, lava1_grid_dimension_x, sp.role_block, sp.role_blocks, lava1_ptb_start_block_pos, lava1_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::lava_role<4>(lava1_d_par_gpu, lava1_d_dim_gpu, lava1_d_box_gpu, lava1_d_rv_gpu, lava1_d_qv_gpu, lava1_d_fv_gpu, lava1_grid_dimension_x, sp.role_block, sp.role_blocks, lava1_ptb_start_block_pos, lava1_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
 }
 
@@ -230,7 +230,7 @@ extern "C" __global__ __launch_bounds__(256) void hot3d_lava_mix_ord_1_1(
         if ((sp.role ^ phase) == 0) {
             tk::hot3d_role(hot3d0_p, hot3d0_tIn, hot3d0_tOut, hot3d0_sdc, hot3d0_nx, hot3d0_ny, hot3d0_nz, hot3d0_ce, hot3d0_cw, hot3d0_cn, hot3d0_cs, hot3d0_ct, hot3d0_cb, hot3d0_cc, hot3d0_grid_dimension_x, hot3d0_grid_dimension_y, hot3d0_block_dimension_x, hot3d0_block_dimension_y, (int)blockIdx.x, (int)gridDim.x, hot3d0_ptb_start_block_pos, hot3d0_ptb_end_block_pos, (int)threadIdx.x, 256);
         } else {
-            tk::lava_role(lava1_d_par_gpu, lava1_d_dim_gpu, lava1_d_box_gpu, lava1_d_rv_gpu, lava1_d_qv_gpu, lava1_d_fv_gpu, lava1_grid_dimension_x, (int)blockIdx.x, (int)gridDim.x, lava1_ptb_start_block_pos, lava1_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::lava_role<4>(lava1_d_par_gpu, lava1_d_dim_gpu, lava1_d_box_gpu, lava1_d_rv_gpu, lava1_d_qv_gpu, lava1_d_fv_gpu, lava1_grid_dimension_x, (int)blockIdx.x, (int)gridDim.x, lava1_ptb_start_block_pos, lava1_ptb_end_block_pos, (int)threadIdx.x, 256);
         }
     }
 }
@@ -290,7 +290,7 @@ extern "C" __global__ __launch_bounds__(256) void hot3d_lava_mix_ord_1_2(
         if ((sp.role ^ phase) == 0) {
             tk::hot3d_role(hot3d0_p, hot3d0_tIn, hot3d0_tOut, hot3d0_sdc, hot3d0_nx, hot3d0_ny, hot3d0_nz, hot3d0_ce, hot3d0_cw, hot3d0_cn, hot3d0_cs, hot3d0_ct, hot3d0_cb, hot3d0_cc, hot3d0_grid_dimension_x, hot3d0_grid_dimension_y, hot3d0_block_dimension_x, hot3d0_block_dimension_y, (int)blockIdx.x, (int)gridDim.x, hot3d0_ptb_start_block_pos, hot3d0_ptb_end_block_pos, (int)threadIdx.x, 256);
         } else {
-            tk::lava_role(lava1_d_par_gpu, lava1_d_dim_gpu, lava1_d_box_gpu, lava1_d_rv_gpu, lava1_d_qv_gpu, lava1_d_fv_gpu, lava1_grid_dimension_x, (int)blockIdx.x, (int)gridDim.x, lava1_ptb_start_block_pos, lava1_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::lava_role<4>(lava1_d_par_gpu, lava1_d_dim_gpu, lava1_d_box_gpu, lava1_d_rv_gpu, lava1_d_qv_gpu, lava1_d_fv_gpu, lava1_grid_dimension_x, (int)blockIdx.x, (int)gridDim.x, lava1_ptb_start_block_pos, lava1_ptb_end_block_pos, (int)threadIdx.x, 256);
         }
     }
 }
@@ -350,7 +350,7 @@ extern "C" __global__ __launch_bounds__(256) void hot3d_lava_mix_ord_2_1(
         if ((sp.role ^ phase) == 0) {
             tk::hot3d_role(hot3d0_p, hot3d0_tIn, hot3d0_tOut, hot3d0_sdc, hot3d0_nx, hot3d0_ny, hot3d0_nz, hot3d0_ce, hot3d0_cw, hot3d0_cn, hot3d0_cs, hot3d0_ct, hot3d0_cb, hot3d0_cc, hot3d0_grid_dimension_x, hot3d0_grid_dimension_y, hot3d0_block_dimension_x, hot3d0_block_dimension_y, (int)blockIdx.x, (int)gridDim.x, hot3d0_ptb_start_block_pos, hot3d0_ptb_end_block_pos, (int)threadIdx.x, 256);
         } else {
-            tk::lava_role(lava1_d_par_gpu, lava1_d_dim_gpu, lava1_d_box_gpu, lava1_d_rv_gpu, lava1_d_qv_gpu, lava1_d_fv_gpu, lava1_grid_dimension_x, (int)blockIdx.x, (int)gridDim.x, lava1_ptb_start_block_pos, lava1_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::lava_role<4>(lava1_d_par_gpu, lava1_d_dim_gpu, lava1_d_box_gpu, lava1_d_rv_gpu, lava1_d_qv_gpu, lava1_d_fv_gpu, lava1_grid_dimension_x, (int)blockIdx.x, (int)gridDim.x, lava1_ptb_start_block_pos, lava1_ptb_end_block_pos, (int)threadIdx.x, 256);
         }
     }
 }

@@ -45,7 +45,7 @@ extern "C" __global__ __launch_bounds__(256) void lava_nn_mix_wg_1_1(
     (void)nn1_ptb_iter_block_step;
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 1, 1);
     if (sp.role == 0) {
-        tk::lava_role(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, sp.role_block, sp.role_blocks, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::lava_role<4>(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, sp.role_block, sp.role_blocks, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x, 256);
     } else {
         tk::nn_role(nn1_d_locations, nn1_d_distances, nn1_numRecords, nn1_lat, nn1_lng, nn1_grid_dimension_x, nn1_grid_dimension_y, nn1_block_dimension_x, sp.role_block, sp.role_blocks, nn1_ptb_start_block_pos, nn1_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
@@ -95,7 +95,7 @@ extern "C" __global__ __launch_bounds__(256) void lava_nn_mix_wg_1_2(
     (void)nn1_ptb_iter_block_step;
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 1, 2);
     if (sp.role == 0) {
-        tk::lava_role(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, sp.role_block, sp.role_blocks, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::lava_role<4>(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, sp.role_block, sp.role_blocks, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x, 256);
     } else {
         tk::nn_role(nn1_d_locations, nn1_d_distances, nn1_numRecords, nn1_lat, nn1_lng, nn1_grid_dimension_x, nn1_grid_dimension_y, nn1_block_dimension_x, sp.role_block, sp.role_blocks, nn1_ptb_start_block_pos, nn1_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
@@ -145,7 +145,7 @@ extern "C" __global__ __launch_bounds__(256) void lava_nn_mix_wg_2_1(
     (void)nn1_ptb_iter_block_step;
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 2, 1);
     if (sp.role == 0) {
-        tk::lava_role(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, sp.role_block, sp.role_blocks, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::lava_role<4>(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, sp.role_block, sp.role_blocks, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x, 256);
     } else {
         tk::nn_role(nn1_d_locations, nn1_d_distances, nn1_numRecords, nn1_lat, nn1_lng, nn1_grid_dimension_x, nn1_grid_dimension_y, nn1_block_dimension_x, sp.role_block, sp.role_blocks, nn1_ptb_start_block_pos, nn1_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
@@ -196,7 +196,7 @@ extern "C" __global__ __launch_bounds__(256) void lava_nn_mix_ord_1_1(
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 1, 1);
     for (int phase = 0; phase < 2; ++phase) {
         if ((sp.role ^ phase) == 0) {
-            tk::lava_role(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, (int)blockIdx.x, (int)gridDim.x, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::lava_role<4>(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, (int)blockIdx.x, (int)gridDim.x, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x, 256);
         } else {
             tk::nn_role(nn1_d_locations, nn1_d_distances, nn1_numRecords, nn1_lat, nn1_lng, nn1_grid_dimension_x, nn1_grid_dimension_y, nn1_block_dimension_x, (int)blockIdx.x, (int)gridDim.x, nn1_ptb_start_block_pos, nn1_ptb_end_block_pos, (int)threadIdx.x, 256);
         }
@@ -248,7 +248,7 @@ extern "C" __global__ __launch_bounds__(256) void lava_nn_mix_ord_1_2(
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 1, 2);
     for (int phase = 0; phase < 2; ++phase) {
         if ((sp.role ^ phase) == 0) {
-            tk::lava_role(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, (int)blockIdx.x, (int)gridDim.x, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::lava_role<4>(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, (int)blockIdx.x, (int)gridDim.x, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x, 256);
         } else {
             tk::nn_role(nn1_d_locations, nn1_d_distances, nn1_numRecords, nn1_lat, nn1_lng, nn1_grid_dimension_x, nn1_grid_dimension_y, nn1_block_dimension_x, (int)blockIdx.x, (int)gridDim.x, nn1_ptb_start_block_pos, nn1_ptb_end_block_pos, (int)threadIdx.x, 256);
         }
@@ -300,7 +300,7 @@ extern "C" __global__ __launch_bounds__(256) void lava_nn_mix_ord_2_1(
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 2, 1);
     for (int phase = 0; phase < 2; ++phase) {
         if ((sp.role ^ phase) == 0) {
-            tk::lava_role(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, (int)blockIdx.x, (int)gridDim.x, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::lava_role<4>(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, (int)blockIdx.x, (int)gridDim.x, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x, 256);
         } else {
             tk::nn_role(nn1_d_locations, nn1_d_distances, nn1_numRecords, nn1_lat, nn1_lng, nn1_grid_dimension_x, nn1_grid_dimension_y, nn1_block_dimension_x, (int)blockIdx.x, (int)gridDim.x, nn1_ptb_start_block_pos, nn1_ptb_end_block_pos, (int)threadIdx.x, 256);
         }

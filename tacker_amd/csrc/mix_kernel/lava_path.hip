@@ -52,7 +52,7 @@ extern "C" __global__ __launch_bounds__(256) void lava_path_mix_wg_1_1(
     (void)path1_ptb_iter_block_step;
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 1, 1);
     if (sp.role == 0) {
-        tk::lava_role(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, sp.role_block, sp.role_blocks, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::lava_role<4>(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, sp.role_block, sp.role_blocks, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x, 256);
     } else {
         tk::path_role(path1_iteration, path1_gpuWall, path1_gpuSrc, path1_gpuResults, path1_cols, path1_startStep, path1_border, sp.role_block, sp.role_blocks, path1_ptb_start_block_pos, path1_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
@@ -109,7 +109,7 @@ extern "C" __global__ __launch_bounds__(256) void lava_path_mix_wg_1_2(
     (void)path1_ptb_iter_block_step;
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 1, 2);
     if (sp.role == 0) {
-        tk::lava_role(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, sp.role_block, sp.role_blocks, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::lava_role<4>(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, sp.role_block, sp.role_blocks, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x, 256);
     } else {
         tk::path_role(path1_iteration, path1_gpuWall, path1_gpuSrc, path1_gpuResults, path1_cols, path1_startStep, path1_border, sp.role_block, sp.role_blocks, path1_ptb_start_block_pos, path1_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
@@ -166,7 +166,7 @@ extern "C" __global__ __launch_bounds__(256) void lava_path_mix_wg_2_1(
     (void)path1_ptb_iter_block_step;
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 2, 1);
     if (sp.role == 0) {
-        tk::lava_role(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, sp.role_block, sp.role_blocks, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::lava_role<4>(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, sp.role_block, sp.role_blocks, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x, 256);
     } else {
         tk::path_role(path1_iteration, path1_gpuWall, path1_gpuSrc, path1_gpuResults, path1_cols, path1_startStep, path1_border, sp.role_block, sp.role_blocks, path1_ptb_start_block_pos, path1_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
@@ -224,7 +224,7 @@ extern "C" __global__ __launch_bounds__(256) void lava_path_mix_ord_1_1(
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 1, 1);
     for (int phase = 0; phase < 2; ++phase) {
         if ((sp.role ^ phase) == 0) {
-            tk::lava_role(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, (int)blockIdx.x, (int)gridDim.x, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::lava_role<4>(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, (int)blockIdx.x, (int)gridDim.x, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x, 256);
         } else {
             tk::path_role(path1_iteration, path1_gpuWall, path1_gpuSrc, path1_gpuResults, path1_cols, path1_startStep, path1_border, (int)blockIdx.x, (int)gridDim.x, path1_ptb_start_block_pos, path1_ptb_end_block_pos, (int)threadIdx.x, 256);
         }
@@ -283,7 +283,7 @@ extern "C" __global__ __launch_bounds__(256) void lava_path_mix_ord_1_2(
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 1, 2);
     for (int phase = 0; phase < 2; ++phase) {
         if ((sp.role ^ phase) == 0) {
-            tk::lava_role(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, (int)blockIdx.x, (int)gridDim.x, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::lava_role<4>(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, (int)blockIdx.x, (int)gridDim.x, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x, 256);
         } else {
             tk::path_role(path1_iteration, path1_gpuWall, path1_gpuSrc, path1_gpuResults, path1_cols, path1_startStep, path1_border, (int)blockIdx.x, (int)gridDim.x, path1_ptb_start_block_pos, path1_ptb_end_block_pos, (int)threadIdx.x, 256);
         }
@@ -342,7 +342,7 @@ extern "C" __global__ __launch_bounds__(256) void lava_path_mix_ord_2_1(
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 2, 1);
     for (int phase = 0; phase < 2; ++phase) {
         if ((sp.role ^ phase) == 0) {
-            tk::lava_role(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, (int)blockIdx.x, (int)gridDim.x, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::lava_role<4>(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, (int)blockIdx.x, (int)gridDim.x, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x, 256);
         } else {
             tk::path_role(path1_iteration, path1_gpuWall, path1_gpuSrc, path1_gpuResults, path1_cols, path1_startStep, path1_border, (int)blockIdx.x, (int)gridDim.x, path1_ptb_start_block_pos, path1_ptb_end_block_pos, (int)threadIdx.x, 256);
         }

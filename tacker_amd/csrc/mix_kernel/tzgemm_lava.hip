@@ -71,7 +71,7 @@ extern "C" __global__ __launch_bounds__(512) void lava_tzgemm_mix_wave_256(
         const int be_block = apart ? (int)blockIdx.x - tz_busy : (int)blockIdx.x;
         const int be_blocks = apart ? launched - tz_busy : launched;
         if (be_block >= 0) {
-            tk::lava_role(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, be_block, be_blocks, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x - 256, 256);
+            tk::lava_role<4>(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, be_block, be_blocks, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x - 256, 256);
         }
         tk::role_wave_done(tz_arrivals);
     }
@@ -146,7 +146,7 @@ extern "C" __global__ __launch_bounds__(768) void lava_tzgemm_mix_wave_512(
         const int be_block = apart ? (int)blockIdx.x - tz_busy : (int)blockIdx.x;
         const int be_blocks = apart ? launched - tz_busy : launched;
         if (be_block >= 0) {
-            tk::lava_role(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, be_block, be_blocks, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x - 256, 512);
+            tk::lava_role<8>(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, be_block, be_blocks, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x - 256, 512);
         }
         tk::role_wave_done(tz_arrivals);
     }
@@ -204,7 +204,7 @@ extern "C" __global__ __launch_bounds__(256) void lava_tzgemm_mix_wg_1_1(
         tk::WorkgroupSync sync;
         tk::tzgemm_role<TZ_STAGES_WG, true>(tzgemm1_A, tzgemm1_B, tzgemm1_C, tzgemm1_NORMAL_M, tzgemm1_NORMAL_N, tzgemm1_NORMAL_K, tk::tz_workspace_of(tzgemm1_C, tzgemm1_NORMAL_M, tzgemm1_NORMAL_N, tzgemm1_NORMAL_K), sp.role_block, sp.role_blocks, tzgemm1_ptb_start_block_pos, tzgemm1_ptb_end_block_pos, (int)threadIdx.x, tz_lds, sync);
     } else {
-        tk::lava_role(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, sp.role_block, sp.role_blocks, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::lava_role<4>(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, sp.role_block, sp.role_blocks, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
 }
 
@@ -260,6 +260,6 @@ extern "C" __global__ __launch_bounds__(256) void lava_tzgemm_mix_wg_1_2(
         tk::WorkgroupSync sync;
         tk::tzgemm_role<TZ_STAGES_WG, true>(tzgemm1_A, tzgemm1_B, tzgemm1_C, tzgemm1_NORMAL_M, tzgemm1_NORMAL_N, tzgemm1_NORMAL_K, tk::tz_workspace_of(tzgemm1_C, tzgemm1_NORMAL_M, tzgemm1_NORMAL_N, tzgemm1_NORMAL_K), sp.role_block, sp.role_blocks, tzgemm1_ptb_start_block_pos, tzgemm1_ptb_end_block_pos, (int)threadIdx.x, tz_lds, sync);
     } else {
-        tk::lava_role(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, sp.role_block, sp.role_blocks, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::lava_role<4>(lava0_d_par_gpu, lava0_d_dim_gpu, lava0_d_box_gpu, lava0_d_rv_gpu, lava0_d_qv_gpu, lava0_d_fv_gpu, lava0_grid_dimension_x, sp.role_block, sp.role_blocks, lava0_ptb_start_block_pos, lava0_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
 }

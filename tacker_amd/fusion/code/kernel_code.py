@@ -125,11 +125,11 @@ ROLES = {
     },
     "lava": {
         "gptb": {"symbol": "general_ptb_lava", "cite": "src/gptb_kernel/lava_kernel.cu:3-140",
-                 "attributes": "__launch_bounds__(256)"},
+                 "attributes": "__launch_bounds__(256, 4)"},
         "params": [("par_str", "d_par_gpu"), ("dim_str", "d_dim_gpu"), ("box_str*", "d_box_gpu"),
                    ("FOUR_VECTOR*", "d_rv_gpu"), ("float*", "d_qv_gpu"), ("FOUR_VECTOR*", "d_fv_gpu")],
         "needs_sync": False,
-        "call": ("tk::lava_role({p}d_par_gpu, {p}d_dim_gpu, {p}d_box_gpu, {p}d_rv_gpu, {p}d_qv_gpu, {p}d_fv_gpu, "
+        "call": ("tk::lava_role<{waves}>({p}d_par_gpu, {p}d_dim_gpu, {p}d_box_gpu, {p}d_rv_gpu, {p}d_qv_gpu, {p}d_fv_gpu, "
                  "{p}grid_dimension_x, {block}, {blocks}, {p}ptb_start_block_pos, {p}ptb_end_block_pos, {tid}, "
                  "{threads});"),
     },

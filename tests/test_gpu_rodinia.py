@@ -254,7 +254,7 @@ def test_lava_forms_match_the_oracle(boxes1d):
 
 @pytest.mark.parametrize("boxes1d,launch_grid", [(2, 1), (2, 8), (3, 40), (4, 64), (5, 256), (7, 300), (9, 700)])
 def test_lava_every_cut_of_the_boxes_gives_the_same_bits(boxes1d, launch_grid):
-    # how many wavefronts a launch has decides how a box's particles are dealt to them (7, 4, 2 or 1 a lane, whole rounds of
+    # how many wavefronts a launch has decides how a box's particles are dealt to them (6, 3, 2 or 1 a lane, whole rounds of
     # boxes and what is left over): a particle's sum never changes
     rv, qv = lava_inputs(boxes1d, seed=50 + boxes1d)
     d_r, d_q = dev(rv), dev(qv)
@@ -306,6 +306,46 @@ def test_lava_a_neighbour_is_the_box_its_number_names():
            [C.c_void_p(t.data_ptr()) for t in (d_b, d_r, d_q, out)] +
            [i(v) for v in (n, 27, 1, 256, 1, 1, 0, 16, 27 * n, 0)])
     assert np.array_equal(host(out)[place].view(np.uint32).reshape(-1), bits(want).reshape(-1))
+
+
+def lava_float64(boxes1d, rv, qv):
+    """v and forces in 64 bits, without the particles whose v is infinite (they are out of everybody's reach)"""
+    r, q = rv.astype(np.float64).reshape(-1, 100, 4), qv.astype(np.float64).reshape(-1, 100)
+    out = np.zeros_like(r)
+    for b in oracle.lava_boxes(boxes1d):
+        A = r[b["number"]]
+        for other in [b["number"]] + b["nei"][:b["nn"]]["number"].tolist():
+            there = np.isfinite(r[other, :, 0])
+            B, w = r[other][there], q[other][there]
+            w = w * np.exp(-0.5 * (A[:, None, 0] + B[None, :, 0] - A[:, 1:] @ B[:, 1:].T))
+            out[b["number"], :, 0] += w.sum(1)
+            out[b["number"], :, 1:] += 2 * (w[..., None] * (A[:, None, 1:] - B[None, :, 1:])).sum(1)
+    return out.reshape(-1, 4)
+
+
+@pytest.mark.parametrize("boxes1d,offset,far", [(2, 0, None), (5, 0, None), (2, -3, None), (2, 0, 0), (2, 0, 70), (2, 0, 97)])
+def test_lava_forces_against_64_bits(boxes1d, offset, far):
+    # coordinates around 0.5 and away from the origin (v = |x|^2 / 2 there, which keeps the exponent small); one particle of
+    # every box, of the lanes' own ones and of the last four, far away in x with an infinite v: no force comes from it, and it
+    # does not cost the others their precision
+    rng = np.random.default_rng(900 + boxes1d)
+    n = 100 * boxes1d ** 3
+    rv = rng.uniform(0.1, 1, (n, 4)).astype(np.float32)
+    qv = rng.uniform(0.1, 1, n).astype(np.float32)
+    if offset:
+        rv[:, 1:] += np.float32(offset)
+        rv[:, 0] = (rv[:, 1:].astype(np.float64) ** 2).sum(1) / 2
+    if far is not None:
+        rv[far::100, 0], rv[far::100, 1] = np.inf, 1e30
+    out = torch.zeros((n, 4), device="cuda:0")
+    ta.gptb_lava(0.5, dev(rv), dev(qv), out)
+    keep = np.isfinite(rv[:, 0])
+    got, want = host(out).astype(np.float64)[keep], lava_float64(boxes1d, rv, qv)[keep]
+    # 25 + 2 additions of a part and 27 parts, each rounded to 2^-24 of a sum: in the 2-norm, where roundings are independent,
+    # sqrt(54) 2^-24 = 4.4e-7; an exponent of up to |x|^2 / 2 = 14 is itself rounded to 2^-24 of it, five times over
+    bound = 4.4e-7 + (5 * 14 * 2.0 ** -24 if offset else 0)
+    for part in (slice(0, 1), slice(1, 4)):
+        assert np.linalg.norm(got[:, part] - want[:, part]) <= bound * np.linalg.norm(want[:, part])
 
 
 @pytest.mark.parametrize("seed", range(4))
