@@ -25,5 +25,5 @@ extern "C" __global__ void general_ptb_mrif(
     (void)block_dimension_x;
     (void)block_dimension_y;
     (void)block_dimension_z;
-    tk::mrif_role(numK, x, y, z, outR, outI, grid_dimension_x, grid_dimension_y, (int)blockIdx.x, ptb_iter_block_step, ptb_start_block_pos, ptb_end_block_pos, (int)threadIdx.x - thread_base, (int)blockDim.x);
+    tk::mrif_role<16>(numK, x, y, z, outR, outI, grid_dimension_x, grid_dimension_y, (int)blockIdx.x, ptb_iter_block_step, ptb_start_block_pos, ptb_end_block_pos, (int)threadIdx.x - thread_base, (int)blockDim.x);
 }

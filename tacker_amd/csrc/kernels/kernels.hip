@@ -70,7 +70,8 @@ extern "C" __global__ __launch_bounds__(256) void ori_mriq(int numK, int kGlobal
                                                            float *y, float *z, float *Qr, float *Qi)
 {
     (void)kGlobalIndex;
-    tk::mriq_voxel(numK, x, y, z, Qr, Qi, blockIdx.x * KERNEL_Q_THREADS_PER_BLOCK + threadIdx.x);
+    tk::mriq_voxel<KERNEL_Q_THREADS_PER_BLOCK / TK_WAVE_SIZE>(
+        numK, x, y, z, Qr, Qi, blockIdx.x * KERNEL_Q_THREADS_PER_BLOCK + threadIdx.x, threadIdx.x);
 }
 
 extern "C" __global__ void ComputeRhoPhiGPU(int numK, float *phiR, float *phiI, float *dR, float *dI,
@@ -93,7 +94,8 @@ extern "C" __global__ __launch_bounds__(256) void ori_mrif(int numK, int kGlobal
                                                            float *y, float *z, float *outR, float *outI)
 {
     (void)kGlobalIndex;
-    tk::mrif_voxel(numK, x, y, z, outR, outI, blockIdx.x * KERNEL_FH_THREADS_PER_BLOCK + threadIdx.x);
+    tk::mriq_voxel<KERNEL_FH_THREADS_PER_BLOCK / TK_WAVE_SIZE, tk::MrifBody>(
+        numK, x, y, z, outR, outI, blockIdx.x * KERNEL_FH_THREADS_PER_BLOCK + threadIdx.x, threadIdx.x);
 }
 
 // grid (M/128, N/16), block (16,4): one wavefront where the reference has 128 threads, a lane owning the

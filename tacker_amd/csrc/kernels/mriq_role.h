@@ -10,16 +10,17 @@
 // with k ascending.  The reference's loop "for QGrid < 1" handles only the first
 // 1024-sample chunk; here all numK samples held in the table are used.
 //
-// gfx950: the table index is wave-uniform, so the compiler fetches each record
-// with one scalar 16-byte load; the work is VALU/transcendental bound.  The
-// hardware sine and cosine take their argument in revolutions, so the phase
-// k.x is used as it is (reduced with v_fract) instead of being scaled by 2 pi
-// and reduced again in software: cos(2 pi p) = v_cos(fract(p)).  The dot product and
-// the two accumulations are fused multiply-adds in the reference's order
-// (((Kx*x) + Ky*y) + Kz*z; Q + PhiMag*c) -- what nvcc makes of the reference's source
-// with its default -fmad=true -- 8 instructions per (k, x) pair instead of 13.  The
-// result differs from a float64 evaluation by about 1e-6 per term, far inside the
-// 1e-3 + 1e-4 |Q| bar.
+// gfx950: what bounds it is VALU issue.  The hardware sine and cosine take their argument in revolutions and reduce
+// it themselves, at any size: the phase k.x goes to them as it is, cos(2 pi p) = v_cos(p).  (Over the whole range of
+// floats they are within 1.3e-7 of sine and cosine; behind a v_fract, which rounds a negative phase to a whole turn's
+// last bit, within 2.7e-7 at |p| < 300 and the same above.)  The dot product and the two accumulations are fused
+// multiply-adds in the reference's order (((Kx*x) + Ky*y) + Kz*z; Q + PhiMag*c) -- what nvcc makes of the reference's
+// source with its default -fmad=true -- so a (k, x) pair is 5 such instructions and the two transcendentals.  The five
+// take 2.5 to 2.8 cycles of a SIMD with two wavefronts at work if all their operands are vector registers and 4.4 with a
+// scalar one (v_fract 4.3, sine and cosine 8.5 each), so a wavefront brings the records, 64 at a time, through LDS of its
+// own and reads each back with one 16-byte broadcast.  2048 records and 262144 voxels: 130 us alone, 145 beside tzgemm
+// 2048^3; 153 and 161 with the records in scalar registers and a v_fract.  (Without the v_fract alone: 152 and 153.)
+// The result differs from a float64 evaluation by about 1e-6 per term, far inside the 1e-3 + 1e-4 |Q| bar.
 #pragma once
 #include "role_common.h"
 #include "../header/mriq_header.h"
@@ -28,17 +29,43 @@ __constant__ mriq_kValues ck[MRIQ_MAX_K];
 
 namespace tk {
 
+template <int N>
+struct mriq_count {
+    static constexpr int value = N;
+};
+
+typedef __attribute__((address_space(3))) float4_t mriq_lds_float4;
+
+// the LDS of the role's wavefronts, QUADS float4s each.  role_wave: the calling wavefront's number within the role
+template <int WAVES, int QUADS>
+__device__ __forceinline__ mriq_lds_float4 *mriq_stage_of_wave(int role_wave)
+{
+    __shared__ __align__(16) float4_t mriq_stage[WAVES][QUADS];
+    return (mriq_lds_float4 *)&mriq_stage[role_wave][0];
+}
+
+// what a wavefront wrote to its own LDS is there for all its lanes (LDS serves a wavefront in order), and what it read is read
+__device__ __forceinline__ void mriq_stage_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+__device__ __forceinline__ int mriq_lane() { return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
+
 // V voxels per thread at once, k records [k_begin, k_end).  The k loop is a chain of
-// dependent operations per voxel (dot product, fract, sin/cos, accumulate) and a fused
+// dependent operations per voxel (dot product, sin/cos, accumulate) and a fused
 // launch leaves the role at most two waves per SIMD, so the independent work that hides
 // instruction latency has to come from inside the thread; V voxels also share each
-// scalar load of a k record.
+// read of a k record.  stage: this wavefront's LDS.
 template <int V>
 __device__ __forceinline__ void mriq_voxels(int k_begin, int k_end, const float *__restrict__ x,
                                             const float *__restrict__ y, const float *__restrict__ z,
                                             float *__restrict__ Qr, float *__restrict__ Qi,
-                                            const int (&xIndex)[V])
+                                            const int (&xIndex)[V], mriq_lds_float4 *stage)
 {
+    if (k_begin >= k_end) return;
     float sX[V], sY[V], sZ[V], sQr[V], sQi[V];
 #pragma unroll
     for (int v = 0; v < V; ++v) {
@@ -49,51 +76,64 @@ __device__ __forceinline__ void mriq_voxels(int k_begin, int k_end, const float 
         sQr[v] = Qr[i];
         sQi[v] = Qi[i];
     }
+    const int lane = mriq_lane();
+    const float4_t *table = reinterpret_cast<const float4_t *>(ck);
+    constexpr int U = 4;
     // U records at a time, written stage by stage (all phases, then all sines and cosines,
     // then the accumulation in ascending k): the U * V chains are independent until the last
     // stage, and the order of the source is already the interleaved one -- the compiler's
     // scheduler does not have to find it (for one of the instances in a fused kernel it did
-    // not, and that loop ran one dependent chain at a time).  The scalar loads of the U
-    // records are issued together: one record per iteration would put a scalar-cache round
-    // trip on every step.
-    constexpr int U = V >= 4 ? 4 : 8;
-    int kIndex = k_begin;
-    for (; kIndex + U <= k_end; kIndex += U) {
-        mriq_kValues k[U];
+    // not, and that loop ran one dependent chain at a time).
+    const auto add = [&](const float4_t *k, auto records) {
+        constexpr int N = decltype(records)::value;
+        float c[N][V], s[N][V];
 #pragma unroll
-        for (int u = 0; u < U; ++u) k[u] = ck[kIndex + u];
-        float c[U][V], s[U][V];
+        for (int u = 0; u < N; ++u)
 #pragma unroll
-        for (int u = 0; u < U; ++u)
+            for (int v = 0; v < V; ++v)   // revolutions
+                c[u][v] = __builtin_fmaf(k[u].z, sZ[v], __builtin_fmaf(k[u].y, sY[v], k[u].x * sX[v]));
 #pragma unroll
-            for (int v = 0; v < V; ++v) {
-                const float phase = __builtin_fmaf(k[u].Kz, sZ[v], __builtin_fmaf(k[u].Ky, sY[v], k[u].Kx * sX[v]));
-                c[u][v] = __builtin_amdgcn_fractf(phase);   // revolutions
-            }
-#pragma unroll
-        for (int u = 0; u < U; ++u)
+        for (int u = 0; u < N; ++u)
 #pragma unroll
             for (int v = 0; v < V; ++v) {
                 s[u][v] = __builtin_amdgcn_sinf(c[u][v]);
                 c[u][v] = __builtin_amdgcn_cosf(c[u][v]);
             }
 #pragma unroll
-        for (int u = 0; u < U; ++u)
+        for (int u = 0; u < N; ++u)
 #pragma unroll
             for (int v = 0; v < V; ++v) {
-                sQr[v] = __builtin_fmaf(k[u].PhiMag, c[u][v], sQr[v]);
-                sQi[v] = __builtin_fmaf(k[u].PhiMag, s[u][v], sQi[v]);
+                sQr[v] = __builtin_fmaf(k[u].w, c[u][v], sQr[v]);
+                sQi[v] = __builtin_fmaf(k[u].w, s[u][v], sQi[v]);
             }
-    }
-    for (; kIndex < k_end; ++kIndex) {
-        const mriq_kValues k = ck[kIndex];
+    };
+    float4_t ahead = table[min(k_begin + lane, k_end - 1)];
+    for (int k0 = k_begin; k0 < k_end; k0 += TK_WAVE_SIZE) {
+        stage[lane] = ahead;
+        ahead = table[min(k0 + TK_WAVE_SIZE + lane, k_end - 1)];
+        mriq_stage_fence();
+        const int count = min(TK_WAVE_SIZE, k_end - k0);
+        const auto read = [&](float4_t (&r)[U], int first) {
 #pragma unroll
-        for (int v = 0; v < V; ++v) {
-            const float turn = __builtin_amdgcn_fractf(
-                __builtin_fmaf(k.Kz, sZ[v], __builtin_fmaf(k.Ky, sY[v], k.Kx * sX[v])));
-            sQr[v] = __builtin_fmaf(k.PhiMag, __builtin_amdgcn_cosf(turn), sQr[v]);
-            sQi[v] = __builtin_fmaf(k.PhiMag, __builtin_amdgcn_sinf(turn), sQi[v]);
+            for (int u = 0; u < U; ++u) r[u] = stage[(first & (TK_WAVE_SIZE - 1)) + u];
+            __builtin_amdgcn_sched_barrier(0);   // on its way while the records before it are used
+        };
+        float4_t ka[U], kb[U];
+        read(ka, 0);
+        int i = 0;
+        for (; i + 2 * U <= count; i += 2 * U) {
+            read(kb, i + U);
+            add(ka, mriq_count<U>());
+            __builtin_amdgcn_sched_barrier(0);
+            read(ka, i + 2 * U);
+            add(kb, mriq_count<U>());
+            __builtin_amdgcn_sched_barrier(0);
         }
+        for (; i < count; ++i) {   // (the table's last records)
+            const float4_t one[1] = {stage[i]};
+            add(one, mriq_count<1>());
+        }
+        mriq_stage_fence();
     }
 #pragma unroll
     for (int v = 0; v < V; ++v) {
@@ -102,29 +142,32 @@ __device__ __forceinline__ void mriq_voxels(int k_begin, int k_end, const float 
     }
 }
 
-// the natural kernel's thread: one voxel, every record
-__device__ __forceinline__ void mriq_voxel(int numK, const float *__restrict__ x,
-                                           const float *__restrict__ y, const float *__restrict__ z,
-                                           float *__restrict__ Qr, float *__restrict__ Qi, int xIndex)
-{
-    const int one[1] = {xIndex};
-    mriq_voxels<1>(0, numK, x, y, z, Qr, Qi, one);
-}
-
 // What a thread does for V voxels and a run of k records: the part of the kernel that the
 // walk over block positions below does not know about.  MRI-FHD (mrif_role.h) walks the
 // same position grid with another body.
 struct MriqBody {
+    static constexpr int STAGE_QUADS = TK_WAVE_SIZE;   // float4s of LDS a wavefront needs
     static __device__ __forceinline__ int chunk() { return MRIQ_K_CHUNK; }
     template <int V>
     static __device__ __forceinline__ void voxels(int k_begin, int k_end, const float *__restrict__ x,
                                                   const float *__restrict__ y, const float *__restrict__ z,
                                                   float *__restrict__ Qr, float *__restrict__ Qi,
-                                                  const int (&xIndex)[V])
+                                                  const int (&xIndex)[V], mriq_lds_float4 *stage)
     {
-        mriq_voxels<V>(k_begin, k_end, x, y, z, Qr, Qi, xIndex);
+        mriq_voxels<V>(k_begin, k_end, x, y, z, Qr, Qi, xIndex, stage);
     }
 };
+
+// the natural kernel's thread: one voxel, every record.  tid: thread of the workgroup, of WAVES wavefronts
+template <int WAVES, class Body = MriqBody>
+__device__ __forceinline__ void mriq_voxel(int numK, const float *__restrict__ x,
+                                           const float *__restrict__ y, const float *__restrict__ z,
+                                           float *__restrict__ Qr, float *__restrict__ Qi, int xIndex, int tid)
+{
+    const int one[1] = {xIndex};
+    Body::template voxels<1>(0, numK, x, y, z, Qr, Qi, one,
+                             mriq_stage_of_wave<WAVES, Body::STAGE_QUADS>(__builtin_amdgcn_readfirstlane(tid / TK_WAVE_SIZE)));
+}
 
 // One phase of a launch: voxel blocks [block_lo, block_hi) each take records
 // [k_begin, k_end).  A thread serves the blocks it owns -- first_owned, first_owned +
@@ -134,7 +177,8 @@ template <class Body>
 __device__ __forceinline__ void mriq_phase(int block_lo, int block_hi, int k_begin, int k_end,
                                            const float *__restrict__ x, const float *__restrict__ y,
                                            const float *__restrict__ z, float *__restrict__ Qr,
-                                           float *__restrict__ Qi, int first_owned, int stride, int t)
+                                           float *__restrict__ Qi, int first_owned, int stride, int t,
+                                           mriq_lds_float4 *stage)
 {
     constexpr int V = MRIQ_VOXELS_PER_THREAD;
     if (block_lo >= block_hi || k_begin >= k_end) return;
@@ -150,15 +194,15 @@ __device__ __forceinline__ void mriq_phase(int block_lo, int block_hi, int k_beg
             idx[v] = (bv < block_hi ? bv : b) * KERNEL_Q_THREADS_PER_BLOCK + t;
         }
         if (count == V) {
-            Body::template voxels<V>(k_begin, k_end, x, y, z, Qr, Qi, idx);
+            Body::template voxels<V>(k_begin, k_end, x, y, z, Qr, Qi, idx, stage);
         } else {
             if (count >= 2) {
                 const int two[2] = {idx[0], idx[1]};
-                Body::template voxels<2>(k_begin, k_end, x, y, z, Qr, Qi, two);
+                Body::template voxels<2>(k_begin, k_end, x, y, z, Qr, Qi, two, stage);
             }
             if (count & 1) {
                 const int one[1] = {idx[count - 1]};
-                Body::template voxels<1>(k_begin, k_end, x, y, z, Qr, Qi, one);
+                Body::template voxels<1>(k_begin, k_end, x, y, z, Qr, Qi, one, stage);
             }
         }
     }
@@ -180,17 +224,19 @@ __device__ __forceinline__ void mriq_phase(int block_lo, int block_hi, int k_beg
 // and the owner walks the three parts in order: the chunks of a voxel are added in
 // ascending position order without any synchronisation between threads.  Whole rows that
 // follow each other are one run of the k loop.
-template <class Body = MriqBody>
+// WAVES: wavefronts of a workgroup that there is LDS for; those of a larger workgroup leave the blocks to them.
+template <int WAVES, class Body = MriqBody>
 __device__ __forceinline__ void mriq_role(int numK, const float *__restrict__ x,
                                           const float *__restrict__ y, const float *__restrict__ z,
                                           float *__restrict__ Qr, float *__restrict__ Qi,
                                           int grid_dimension_x, int grid_dimension_y, int role_block,
                                           int role_blocks, int start, int end, int tid, int role_threads)
 {
-    const int blocks_at_once = role_threads / KERNEL_Q_THREADS_PER_BLOCK;
+    const int blocks_at_once = min(role_threads, WAVES * TK_WAVE_SIZE) / KERNEL_Q_THREADS_PER_BLOCK;
     const int slot = tid / KERNEL_Q_THREADS_PER_BLOCK;
     const int t = tid % KERNEL_Q_THREADS_PER_BLOCK;
     if (slot >= blocks_at_once || start >= end) return;
+    mriq_lds_float4 *stage = mriq_stage_of_wave<WAVES, Body::STAGE_QUADS>(__builtin_amdgcn_readfirstlane(tid / TK_WAVE_SIZE));
     const int gx = grid_dimension_x;
     const int gy = grid_dimension_y;
     const int stride = role_blocks * blocks_at_once;
@@ -202,25 +248,25 @@ __device__ __forceinline__ void mriq_role(int numK, const float *__restrict__ x,
     const int last_row = (end - 1) / gx;   // row of the last position
     if (first_row == last_row) {
         mriq_phase<Body>(start - first_row * gx, end - first_row * gx, chunk_begin(first_row), chunk_end(first_row),
-                   x, y, z, Qr, Qi, first_owned, stride, t);
+                   x, y, z, Qr, Qi, first_owned, stride, t, stage);
         return;
     }
     int row = first_row;
     if (start != first_row * gx) {   // partial first row
         mriq_phase<Body>(start - first_row * gx, gx, chunk_begin(row), chunk_end(row), x, y, z, Qr, Qi,
-                   first_owned, stride, t);
+                   first_owned, stride, t, stage);
         ++row;
     }
     const int whole_end = (end == (last_row + 1) * gx) ? last_row + 1 : last_row;   // whole rows [row, whole_end)
     while (row < whole_end) {
         // rows up to the next multiple of grid_dimension_y are consecutive chunks
         const int run_end = min(whole_end, (row / gy + 1) * gy);
-        mriq_phase<Body>(0, gx, chunk_begin(row), chunk_end(run_end - 1), x, y, z, Qr, Qi, first_owned, stride, t);
+        mriq_phase<Body>(0, gx, chunk_begin(row), chunk_end(run_end - 1), x, y, z, Qr, Qi, first_owned, stride, t, stage);
         row = run_end;
     }
     if (whole_end == last_row)       // partial last row
         mriq_phase<Body>(0, end - last_row * gx, chunk_begin(last_row), chunk_end(last_row), x, y, z, Qr, Qi,
-                   first_owned, stride, t);
+                   first_owned, stride, t, stage);
 }
 
 }  // namespace tk

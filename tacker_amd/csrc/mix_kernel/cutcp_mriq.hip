@@ -52,7 +52,7 @@ extern "C" __global__ __launch_bounds__(256) void cutcp_mriq_mix_wg_1_1(
     if (sp.role == 0) {
         tk::cutcp_role<4>(cutcp0_binDim_x, cutcp0_binDim_y, cutcp0_binZeroAddr, cutcp0_h, cutcp0_cutoff2, cutcp0_inv_cutoff2, cutcp0_regionZeroAddr, cutcp0_grid_dimension_x, cutcp0_grid_dimension_y, cutcp0_grid_dimension_z, sp.role_block, sp.role_blocks, cutcp0_ptb_start_block_pos, cutcp0_ptb_end_block_pos, (int)threadIdx.x, 256);
     } else {
-        tk::mriq_role(mriq1_numK, mriq1_x, mriq1_y, mriq1_z, mriq1_Qr, mriq1_Qi, mriq1_grid_dimension_x, mriq1_grid_dimension_y, sp.role_block, sp.role_blocks, mriq1_ptb_start_block_pos, mriq1_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::mriq_role<4>(mriq1_numK, mriq1_x, mriq1_y, mriq1_z, mriq1_Qr, mriq1_Qi, mriq1_grid_dimension_x, mriq1_grid_dimension_y, sp.role_block, sp.role_blocks, mriq1_ptb_start_block_pos, mriq1_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
 }
 
@@ -107,7 +107,7 @@ extern "C" __global__ __launch_bounds__(256) void cutcp_mriq_mix_wg_1_2(
     if (sp.role == 0) {
         tk::cutcp_role<4>(cutcp0_binDim_x, cutcp0_binDim_y, cutcp0_binZeroAddr, cutcp0_h, cutcp0_cutoff2, cutcp0_inv_cutoff2, cutcp0_regionZeroAddr, cutcp0_grid_dimension_x, cutcp0_grid_dimension_y, cutcp0_grid_dimension_z, sp.role_block, sp.role_blocks, cutcp0_ptb_start_block_pos, cutcp0_ptb_end_block_pos, (int)threadIdx.x, 256);
     } else {
-        tk::mriq_role(mriq1_numK, mriq1_x, mriq1_y, mriq1_z, mriq1_Qr, mriq1_Qi, mriq1_grid_dimension_x, mriq1_grid_dimension_y, sp.role_block, sp.role_blocks, mriq1_ptb_start_block_pos, mriq1_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::mriq_role<4>(mriq1_numK, mriq1_x, mriq1_y, mriq1_z, mriq1_Qr, mriq1_Qi, mriq1_grid_dimension_x, mriq1_grid_dimension_y, sp.role_block, sp.role_blocks, mriq1_ptb_start_block_pos, mriq1_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
 }
 
@@ -162,7 +162,7 @@ extern "C" __global__ __launch_bounds__(256) void cutcp_mriq_mix_wg_2_1(
     if (sp.role == 0) {
         tk::cutcp_role<4>(cutcp0_binDim_x, cutcp0_binDim_y, cutcp0_binZeroAddr, cutcp0_h, cutcp0_cutoff2, cutcp0_inv_cutoff2, cutcp0_regionZeroAddr, cutcp0_grid_dimension_x, cutcp0_grid_dimension_y, cutcp0_grid_dimension_z, sp.role_block, sp.role_blocks, cutcp0_ptb_start_block_pos, cutcp0_ptb_end_block_pos, (int)threadIdx.x, 256);
     } else {
-        tk::mriq_role(mriq1_numK, mriq1_x, mriq1_y, mriq1_z, mriq1_Qr, mriq1_Qi, mriq1_grid_dimension_x, mriq1_grid_dimension_y, sp.role_block, sp.role_blocks, mriq1_ptb_start_block_pos, mriq1_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::mriq_role<4>(mriq1_numK, mriq1_x, mriq1_y, mriq1_z, mriq1_Qr, mriq1_Qi, mriq1_grid_dimension_x, mriq1_grid_dimension_y, sp.role_block, sp.role_blocks, mriq1_ptb_start_block_pos, mriq1_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
 }
 
@@ -218,7 +218,7 @@ extern "C" __global__ __launch_bounds__(256) void cutcp_mriq_mix_ord_1_1(
         if ((sp.role ^ phase) == 0) {
             tk::cutcp_role<4>(cutcp0_binDim_x, cutcp0_binDim_y, cutcp0_binZeroAddr, cutcp0_h, cutcp0_cutoff2, cutcp0_inv_cutoff2, cutcp0_regionZeroAddr, cutcp0_grid_dimension_x, cutcp0_grid_dimension_y, cutcp0_grid_dimension_z, (int)blockIdx.x, (int)gridDim.x, cutcp0_ptb_start_block_pos, cutcp0_ptb_end_block_pos, (int)threadIdx.x, 256);
         } else {
-            tk::mriq_role(mriq1_numK, mriq1_x, mriq1_y, mriq1_z, mriq1_Qr, mriq1_Qi, mriq1_grid_dimension_x, mriq1_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mriq1_ptb_start_block_pos, mriq1_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::mriq_role<4>(mriq1_numK, mriq1_x, mriq1_y, mriq1_z, mriq1_Qr, mriq1_Qi, mriq1_grid_dimension_x, mriq1_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mriq1_ptb_start_block_pos, mriq1_ptb_end_block_pos, (int)threadIdx.x, 256);
         }
     }
 }
@@ -275,7 +275,7 @@ extern "C" __global__ __launch_bounds__(256) void cutcp_mriq_mix_ord_1_2(
         if ((sp.role ^ phase) == 0) {
             tk::cutcp_role<4>(cutcp0_binDim_x, cutcp0_binDim_y, cutcp0_binZeroAddr, cutcp0_h, cutcp0_cutoff2, cutcp0_inv_cutoff2, cutcp0_regionZeroAddr, cutcp0_grid_dimension_x, cutcp0_grid_dimension_y, cutcp0_grid_dimension_z, (int)blockIdx.x, (int)gridDim.x, cutcp0_ptb_start_block_pos, cutcp0_ptb_end_block_pos, (int)threadIdx.x, 256);
         } else {
-            tk::mriq_role(mriq1_numK, mriq1_x, mriq1_y, mriq1_z, mriq1_Qr, mriq1_Qi, mriq1_grid_dimension_x, mriq1_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mriq1_ptb_start_block_pos, mriq1_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::mriq_role<4>(mriq1_numK, mriq1_x, mriq1_y, mriq1_z, mriq1_Qr, mriq1_Qi, mriq1_grid_dimension_x, mriq1_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mriq1_ptb_start_block_pos, mriq1_ptb_end_block_pos, (int)threadIdx.x, 256);
         }
     }
 }
@@ -332,7 +332,7 @@ extern "C" __global__ __launch_bounds__(256) void cutcp_mriq_mix_ord_2_1(
         if ((sp.role ^ phase) == 0) {
             tk::cutcp_role<4>(cutcp0_binDim_x, cutcp0_binDim_y, cutcp0_binZeroAddr, cutcp0_h, cutcp0_cutoff2, cutcp0_inv_cutoff2, cutcp0_regionZeroAddr, cutcp0_grid_dimension_x, cutcp0_grid_dimension_y, cutcp0_grid_dimension_z, (int)blockIdx.x, (int)gridDim.x, cutcp0_ptb_start_block_pos, cutcp0_ptb_end_block_pos, (int)threadIdx.x, 256);
         } else {
-            tk::mriq_role(mriq1_numK, mriq1_x, mriq1_y, mriq1_z, mriq1_Qr, mriq1_Qi, mriq1_grid_dimension_x, mriq1_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mriq1_ptb_start_block_pos, mriq1_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::mriq_role<4>(mriq1_numK, mriq1_x, mriq1_y, mriq1_z, mriq1_Qr, mriq1_Qi, mriq1_grid_dimension_x, mriq1_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mriq1_ptb_start_block_pos, mriq1_ptb_end_block_pos, (int)threadIdx.x, 256);
         }
     }
 }

@@ -46,7 +46,7 @@ extern "C" __global__ __launch_bounds__(256) void fft_mrif_mix_wg_1_1(
     if (sp.role == 0) {
         tk::fft_role<4>(fft0_data, fft0_grid_dimension_x, sp.role_block, sp.role_blocks, fft0_ptb_start_block_pos, fft0_ptb_end_block_pos, (int)threadIdx.x, 256);
     } else {
-        tk::mrif_role(mrif1_numK, mrif1_x, mrif1_y, mrif1_z, mrif1_outR, mrif1_outI, mrif1_grid_dimension_x, mrif1_grid_dimension_y, sp.role_block, sp.role_blocks, mrif1_ptb_start_block_pos, mrif1_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::mrif_role<4>(mrif1_numK, mrif1_x, mrif1_y, mrif1_z, mrif1_outR, mrif1_outI, mrif1_grid_dimension_x, mrif1_grid_dimension_y, sp.role_block, sp.role_blocks, mrif1_ptb_start_block_pos, mrif1_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
 }
 
@@ -95,7 +95,7 @@ extern "C" __global__ __launch_bounds__(256) void fft_mrif_mix_wg_1_2(
     if (sp.role == 0) {
         tk::fft_role<4>(fft0_data, fft0_grid_dimension_x, sp.role_block, sp.role_blocks, fft0_ptb_start_block_pos, fft0_ptb_end_block_pos, (int)threadIdx.x, 256);
     } else {
-        tk::mrif_role(mrif1_numK, mrif1_x, mrif1_y, mrif1_z, mrif1_outR, mrif1_outI, mrif1_grid_dimension_x, mrif1_grid_dimension_y, sp.role_block, sp.role_blocks, mrif1_ptb_start_block_pos, mrif1_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::mrif_role<4>(mrif1_numK, mrif1_x, mrif1_y, mrif1_z, mrif1_outR, mrif1_outI, mrif1_grid_dimension_x, mrif1_grid_dimension_y, sp.role_block, sp.role_blocks, mrif1_ptb_start_block_pos, mrif1_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
 }
 
@@ -144,7 +144,7 @@ extern "C" __global__ __launch_bounds__(256) void fft_mrif_mix_wg_2_1(
     if (sp.role == 0) {
         tk::fft_role<4>(fft0_data, fft0_grid_dimension_x, sp.role_block, sp.role_blocks, fft0_ptb_start_block_pos, fft0_ptb_end_block_pos, (int)threadIdx.x, 256);
     } else {
-        tk::mrif_role(mrif1_numK, mrif1_x, mrif1_y, mrif1_z, mrif1_outR, mrif1_outI, mrif1_grid_dimension_x, mrif1_grid_dimension_y, sp.role_block, sp.role_blocks, mrif1_ptb_start_block_pos, mrif1_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::mrif_role<4>(mrif1_numK, mrif1_x, mrif1_y, mrif1_z, mrif1_outR, mrif1_outI, mrif1_grid_dimension_x, mrif1_grid_dimension_y, sp.role_block, sp.role_blocks, mrif1_ptb_start_block_pos, mrif1_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
 }
 
@@ -194,7 +194,7 @@ extern "C" __global__ __launch_bounds__(256) void fft_mrif_mix_ord_1_1(
         if ((sp.role ^ phase) == 0) {
             tk::fft_role<4>(fft0_data, fft0_grid_dimension_x, (int)blockIdx.x, (int)gridDim.x, fft0_ptb_start_block_pos, fft0_ptb_end_block_pos, (int)threadIdx.x, 256);
         } else {
-            tk::mrif_role(mrif1_numK, mrif1_x, mrif1_y, mrif1_z, mrif1_outR, mrif1_outI, mrif1_grid_dimension_x, mrif1_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mrif1_ptb_start_block_pos, mrif1_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::mrif_role<4>(mrif1_numK, mrif1_x, mrif1_y, mrif1_z, mrif1_outR, mrif1_outI, mrif1_grid_dimension_x, mrif1_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mrif1_ptb_start_block_pos, mrif1_ptb_end_block_pos, (int)threadIdx.x, 256);
         }
     }
 }
@@ -245,7 +245,7 @@ extern "C" __global__ __launch_bounds__(256) void fft_mrif_mix_ord_1_2(
         if ((sp.role ^ phase) == 0) {
             tk::fft_role<4>(fft0_data, fft0_grid_dimension_x, (int)blockIdx.x, (int)gridDim.x, fft0_ptb_start_block_pos, fft0_ptb_end_block_pos, (int)threadIdx.x, 256);
         } else {
-            tk::mrif_role(mrif1_numK, mrif1_x, mrif1_y, mrif1_z, mrif1_outR, mrif1_outI, mrif1_grid_dimension_x, mrif1_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mrif1_ptb_start_block_pos, mrif1_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::mrif_role<4>(mrif1_numK, mrif1_x, mrif1_y, mrif1_z, mrif1_outR, mrif1_outI, mrif1_grid_dimension_x, mrif1_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mrif1_ptb_start_block_pos, mrif1_ptb_end_block_pos, (int)threadIdx.x, 256);
         }
     }
 }
@@ -296,7 +296,7 @@ extern "C" __global__ __launch_bounds__(256) void fft_mrif_mix_ord_2_1(
         if ((sp.role ^ phase) == 0) {
             tk::fft_role<4>(fft0_data, fft0_grid_dimension_x, (int)blockIdx.x, (int)gridDim.x, fft0_ptb_start_block_pos, fft0_ptb_end_block_pos, (int)threadIdx.x, 256);
         } else {
-            tk::mrif_role(mrif1_numK, mrif1_x, mrif1_y, mrif1_z, mrif1_outR, mrif1_outI, mrif1_grid_dimension_x, mrif1_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mrif1_ptb_start_block_pos, mrif1_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::mrif_role<4>(mrif1_numK, mrif1_x, mrif1_y, mrif1_z, mrif1_outR, mrif1_outI, mrif1_grid_dimension_x, mrif1_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mrif1_ptb_start_block_pos, mrif1_ptb_end_block_pos, (int)threadIdx.x, 256);
         }
     }
 }

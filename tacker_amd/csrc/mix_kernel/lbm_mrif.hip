@@ -45,7 +45,7 @@ extern "C" __global__ __launch_bounds__(256) void lbm_mrif_mix_wg_1_1(
     if (sp.role == 0) {
         tk::lbm_role(lbm0_srcGrid, lbm0_dstGrid, lbm0_grid_dimension_x, lbm0_grid_dimension_y, lbm0_block_dimension_x, sp.role_block, sp.role_blocks, lbm0_ptb_start_block_pos, lbm0_ptb_end_block_pos, (int)threadIdx.x, 256);
     } else {
-        tk::mrif_role(mrif1_numK, mrif1_x, mrif1_y, mrif1_z, mrif1_outR, mrif1_outI, mrif1_grid_dimension_x, mrif1_grid_dimension_y, sp.role_block, sp.role_blocks, mrif1_ptb_start_block_pos, mrif1_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::mrif_role<4>(mrif1_numK, mrif1_x, mrif1_y, mrif1_z, mrif1_outR, mrif1_outI, mrif1_grid_dimension_x, mrif1_grid_dimension_y, sp.role_block, sp.role_blocks, mrif1_ptb_start_block_pos, mrif1_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
 }
 
@@ -93,7 +93,7 @@ extern "C" __global__ __launch_bounds__(256) void lbm_mrif_mix_wg_1_2(
     if (sp.role == 0) {
         tk::lbm_role(lbm0_srcGrid, lbm0_dstGrid, lbm0_grid_dimension_x, lbm0_grid_dimension_y, lbm0_block_dimension_x, sp.role_block, sp.role_blocks, lbm0_ptb_start_block_pos, lbm0_ptb_end_block_pos, (int)threadIdx.x, 256);
     } else {
-        tk::mrif_role(mrif1_numK, mrif1_x, mrif1_y, mrif1_z, mrif1_outR, mrif1_outI, mrif1_grid_dimension_x, mrif1_grid_dimension_y, sp.role_block, sp.role_blocks, mrif1_ptb_start_block_pos, mrif1_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::mrif_role<4>(mrif1_numK, mrif1_x, mrif1_y, mrif1_z, mrif1_outR, mrif1_outI, mrif1_grid_dimension_x, mrif1_grid_dimension_y, sp.role_block, sp.role_blocks, mrif1_ptb_start_block_pos, mrif1_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
 }
 
@@ -141,7 +141,7 @@ extern "C" __global__ __launch_bounds__(256) void lbm_mrif_mix_wg_2_1(
     if (sp.role == 0) {
         tk::lbm_role(lbm0_srcGrid, lbm0_dstGrid, lbm0_grid_dimension_x, lbm0_grid_dimension_y, lbm0_block_dimension_x, sp.role_block, sp.role_blocks, lbm0_ptb_start_block_pos, lbm0_ptb_end_block_pos, (int)threadIdx.x, 256);
     } else {
-        tk::mrif_role(mrif1_numK, mrif1_x, mrif1_y, mrif1_z, mrif1_outR, mrif1_outI, mrif1_grid_dimension_x, mrif1_grid_dimension_y, sp.role_block, sp.role_blocks, mrif1_ptb_start_block_pos, mrif1_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::mrif_role<4>(mrif1_numK, mrif1_x, mrif1_y, mrif1_z, mrif1_outR, mrif1_outI, mrif1_grid_dimension_x, mrif1_grid_dimension_y, sp.role_block, sp.role_blocks, mrif1_ptb_start_block_pos, mrif1_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
 }
 
@@ -190,7 +190,7 @@ extern "C" __global__ __launch_bounds__(256) void lbm_mrif_mix_ord_1_1(
         if ((sp.role ^ phase) == 0) {
             tk::lbm_role(lbm0_srcGrid, lbm0_dstGrid, lbm0_grid_dimension_x, lbm0_grid_dimension_y, lbm0_block_dimension_x, (int)blockIdx.x, (int)gridDim.x, lbm0_ptb_start_block_pos, lbm0_ptb_end_block_pos, (int)threadIdx.x, 256);
         } else {
-            tk::mrif_role(mrif1_numK, mrif1_x, mrif1_y, mrif1_z, mrif1_outR, mrif1_outI, mrif1_grid_dimension_x, mrif1_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mrif1_ptb_start_block_pos, mrif1_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::mrif_role<4>(mrif1_numK, mrif1_x, mrif1_y, mrif1_z, mrif1_outR, mrif1_outI, mrif1_grid_dimension_x, mrif1_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mrif1_ptb_start_block_pos, mrif1_ptb_end_block_pos, (int)threadIdx.x, 256);
         }
     }
 }
@@ -240,7 +240,7 @@ extern "C" __global__ __launch_bounds__(256) void lbm_mrif_mix_ord_1_2(
         if ((sp.role ^ phase) == 0) {
             tk::lbm_role(lbm0_srcGrid, lbm0_dstGrid, lbm0_grid_dimension_x, lbm0_grid_dimension_y, lbm0_block_dimension_x, (int)blockIdx.x, (int)gridDim.x, lbm0_ptb_start_block_pos, lbm0_ptb_end_block_pos, (int)threadIdx.x, 256);
         } else {
-            tk::mrif_role(mrif1_numK, mrif1_x, mrif1_y, mrif1_z, mrif1_outR, mrif1_outI, mrif1_grid_dimension_x, mrif1_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mrif1_ptb_start_block_pos, mrif1_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::mrif_role<4>(mrif1_numK, mrif1_x, mrif1_y, mrif1_z, mrif1_outR, mrif1_outI, mrif1_grid_dimension_x, mrif1_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mrif1_ptb_start_block_pos, mrif1_ptb_end_block_pos, (int)threadIdx.x, 256);
         }
     }
 }
@@ -290,7 +290,7 @@ extern "C" __global__ __launch_bounds__(256) void lbm_mrif_mix_ord_2_1(
         if ((sp.role ^ phase) == 0) {
             tk::lbm_role(lbm0_srcGrid, lbm0_dstGrid, lbm0_grid_dimension_x, lbm0_grid_dimension_y, lbm0_block_dimension_x, (int)blockIdx.x, (int)gridDim.x, lbm0_ptb_start_block_pos, lbm0_ptb_end_block_pos, (int)threadIdx.x, 256);
         } else {
-            tk::mrif_role(mrif1_numK, mrif1_x, mrif1_y, mrif1_z, mrif1_outR, mrif1_outI, mrif1_grid_dimension_x, mrif1_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mrif1_ptb_start_block_pos, mrif1_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::mrif_role<4>(mrif1_numK, mrif1_x, mrif1_y, mrif1_z, mrif1_outR, mrif1_outI, mrif1_grid_dimension_x, mrif1_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mrif1_ptb_start_block_pos, mrif1_ptb_end_block_pos, (int)threadIdx.x, 256);
         }
     }
 }

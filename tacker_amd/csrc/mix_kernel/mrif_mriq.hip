@@ -50,9 +50,9 @@ extern "C" __global__ __launch_bounds__(256) void mrif_mriq_mix_wg_1_1(
     (void)mriq1_ptb_iter_block_step;
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 1, 1);
     if (sp.role == 0) {
-        tk::mrif_role(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, sp.role_block, sp.role_blocks, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::mrif_role<4>(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, sp.role_block, sp.role_blocks, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
     } else {
-        tk::mriq_role(mriq1_numK, mriq1_x, mriq1_y, mriq1_z, mriq1_Qr, mriq1_Qi, mriq1_grid_dimension_x, mriq1_grid_dimension_y, sp.role_block, sp.role_blocks, mriq1_ptb_start_block_pos, mriq1_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::mriq_role<4>(mriq1_numK, mriq1_x, mriq1_y, mriq1_z, mriq1_Qr, mriq1_Qi, mriq1_grid_dimension_x, mriq1_grid_dimension_y, sp.role_block, sp.role_blocks, mriq1_ptb_start_block_pos, mriq1_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
 }
 
@@ -105,9 +105,9 @@ extern "C" __global__ __launch_bounds__(256) void mrif_mriq_mix_wg_1_2(
     (void)mriq1_ptb_iter_block_step;
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 1, 2);
     if (sp.role == 0) {
-        tk::mrif_role(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, sp.role_block, sp.role_blocks, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::mrif_role<4>(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, sp.role_block, sp.role_blocks, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
     } else {
-        tk::mriq_role(mriq1_numK, mriq1_x, mriq1_y, mriq1_z, mriq1_Qr, mriq1_Qi, mriq1_grid_dimension_x, mriq1_grid_dimension_y, sp.role_block, sp.role_blocks, mriq1_ptb_start_block_pos, mriq1_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::mriq_role<4>(mriq1_numK, mriq1_x, mriq1_y, mriq1_z, mriq1_Qr, mriq1_Qi, mriq1_grid_dimension_x, mriq1_grid_dimension_y, sp.role_block, sp.role_blocks, mriq1_ptb_start_block_pos, mriq1_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
 }
 
@@ -160,9 +160,9 @@ extern "C" __global__ __launch_bounds__(256) void mrif_mriq_mix_wg_2_1(
     (void)mriq1_ptb_iter_block_step;
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 2, 1);
     if (sp.role == 0) {
-        tk::mrif_role(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, sp.role_block, sp.role_blocks, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::mrif_role<4>(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, sp.role_block, sp.role_blocks, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
     } else {
-        tk::mriq_role(mriq1_numK, mriq1_x, mriq1_y, mriq1_z, mriq1_Qr, mriq1_Qi, mriq1_grid_dimension_x, mriq1_grid_dimension_y, sp.role_block, sp.role_blocks, mriq1_ptb_start_block_pos, mriq1_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::mriq_role<4>(mriq1_numK, mriq1_x, mriq1_y, mriq1_z, mriq1_Qr, mriq1_Qi, mriq1_grid_dimension_x, mriq1_grid_dimension_y, sp.role_block, sp.role_blocks, mriq1_ptb_start_block_pos, mriq1_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
 }
 
@@ -216,9 +216,9 @@ extern "C" __global__ __launch_bounds__(256) void mrif_mriq_mix_ord_1_1(
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 1, 1);
     for (int phase = 0; phase < 2; ++phase) {
         if ((sp.role ^ phase) == 0) {
-            tk::mrif_role(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::mrif_role<4>(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
         } else {
-            tk::mriq_role(mriq1_numK, mriq1_x, mriq1_y, mriq1_z, mriq1_Qr, mriq1_Qi, mriq1_grid_dimension_x, mriq1_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mriq1_ptb_start_block_pos, mriq1_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::mriq_role<4>(mriq1_numK, mriq1_x, mriq1_y, mriq1_z, mriq1_Qr, mriq1_Qi, mriq1_grid_dimension_x, mriq1_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mriq1_ptb_start_block_pos, mriq1_ptb_end_block_pos, (int)threadIdx.x, 256);
         }
     }
 }
@@ -273,9 +273,9 @@ extern "C" __global__ __launch_bounds__(256) void mrif_mriq_mix_ord_1_2(
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 1, 2);
     for (int phase = 0; phase < 2; ++phase) {
         if ((sp.role ^ phase) == 0) {
-            tk::mrif_role(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::mrif_role<4>(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
         } else {
-            tk::mriq_role(mriq1_numK, mriq1_x, mriq1_y, mriq1_z, mriq1_Qr, mriq1_Qi, mriq1_grid_dimension_x, mriq1_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mriq1_ptb_start_block_pos, mriq1_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::mriq_role<4>(mriq1_numK, mriq1_x, mriq1_y, mriq1_z, mriq1_Qr, mriq1_Qi, mriq1_grid_dimension_x, mriq1_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mriq1_ptb_start_block_pos, mriq1_ptb_end_block_pos, (int)threadIdx.x, 256);
         }
     }
 }
@@ -330,9 +330,9 @@ extern "C" __global__ __launch_bounds__(256) void mrif_mriq_mix_ord_2_1(
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 2, 1);
     for (int phase = 0; phase < 2; ++phase) {
         if ((sp.role ^ phase) == 0) {
-            tk::mrif_role(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::mrif_role<4>(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
         } else {
-            tk::mriq_role(mriq1_numK, mriq1_x, mriq1_y, mriq1_z, mriq1_Qr, mriq1_Qi, mriq1_grid_dimension_x, mriq1_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mriq1_ptb_start_block_pos, mriq1_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::mriq_role<4>(mriq1_numK, mriq1_x, mriq1_y, mriq1_z, mriq1_Qr, mriq1_Qi, mriq1_grid_dimension_x, mriq1_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mriq1_ptb_start_block_pos, mriq1_ptb_end_block_pos, (int)threadIdx.x, 256);
         }
     }
 }

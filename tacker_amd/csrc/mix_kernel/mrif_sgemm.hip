@@ -47,7 +47,7 @@ extern "C" __global__ __launch_bounds__(256) void mrif_sgemm_mix_wg_1_1(
     (void)sgemm1_ptb_iter_block_step;
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 1, 1);
     if (sp.role == 0) {
-        tk::mrif_role(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, sp.role_block, sp.role_blocks, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::mrif_role<4>(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, sp.role_block, sp.role_blocks, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
     } else {
         tk::sgemm_role(sgemm1_A, sgemm1_B, sgemm1_C, sgemm1_NORMAL_M, sgemm1_NORMAL_N, sgemm1_NORMAL_K, sgemm1_grid_dimension_x, sgemm1_grid_dimension_y, sgemm1_grid_dimension_z, sp.role_block, sp.role_blocks, sgemm1_ptb_start_block_pos, sgemm1_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
@@ -99,7 +99,7 @@ extern "C" __global__ __launch_bounds__(256) void mrif_sgemm_mix_wg_1_2(
     (void)sgemm1_ptb_iter_block_step;
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 1, 2);
     if (sp.role == 0) {
-        tk::mrif_role(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, sp.role_block, sp.role_blocks, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::mrif_role<4>(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, sp.role_block, sp.role_blocks, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
     } else {
         tk::sgemm_role(sgemm1_A, sgemm1_B, sgemm1_C, sgemm1_NORMAL_M, sgemm1_NORMAL_N, sgemm1_NORMAL_K, sgemm1_grid_dimension_x, sgemm1_grid_dimension_y, sgemm1_grid_dimension_z, sp.role_block, sp.role_blocks, sgemm1_ptb_start_block_pos, sgemm1_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
@@ -151,7 +151,7 @@ extern "C" __global__ __launch_bounds__(256) void mrif_sgemm_mix_wg_2_1(
     (void)sgemm1_ptb_iter_block_step;
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 2, 1);
     if (sp.role == 0) {
-        tk::mrif_role(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, sp.role_block, sp.role_blocks, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::mrif_role<4>(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, sp.role_block, sp.role_blocks, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
     } else {
         tk::sgemm_role(sgemm1_A, sgemm1_B, sgemm1_C, sgemm1_NORMAL_M, sgemm1_NORMAL_N, sgemm1_NORMAL_K, sgemm1_grid_dimension_x, sgemm1_grid_dimension_y, sgemm1_grid_dimension_z, sp.role_block, sp.role_blocks, sgemm1_ptb_start_block_pos, sgemm1_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
@@ -204,7 +204,7 @@ extern "C" __global__ __launch_bounds__(256) void mrif_sgemm_mix_ord_1_1(
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 1, 1);
     for (int phase = 0; phase < 2; ++phase) {
         if ((sp.role ^ phase) == 0) {
-            tk::mrif_role(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::mrif_role<4>(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
         } else {
             tk::sgemm_role(sgemm1_A, sgemm1_B, sgemm1_C, sgemm1_NORMAL_M, sgemm1_NORMAL_N, sgemm1_NORMAL_K, sgemm1_grid_dimension_x, sgemm1_grid_dimension_y, sgemm1_grid_dimension_z, (int)blockIdx.x, (int)gridDim.x, sgemm1_ptb_start_block_pos, sgemm1_ptb_end_block_pos, (int)threadIdx.x, 256);
         }
@@ -258,7 +258,7 @@ extern "C" __global__ __launch_bounds__(256) void mrif_sgemm_mix_ord_1_2(
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 1, 2);
     for (int phase = 0; phase < 2; ++phase) {
         if ((sp.role ^ phase) == 0) {
-            tk::mrif_role(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::mrif_role<4>(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
         } else {
             tk::sgemm_role(sgemm1_A, sgemm1_B, sgemm1_C, sgemm1_NORMAL_M, sgemm1_NORMAL_N, sgemm1_NORMAL_K, sgemm1_grid_dimension_x, sgemm1_grid_dimension_y, sgemm1_grid_dimension_z, (int)blockIdx.x, (int)gridDim.x, sgemm1_ptb_start_block_pos, sgemm1_ptb_end_block_pos, (int)threadIdx.x, 256);
         }
@@ -312,7 +312,7 @@ extern "C" __global__ __launch_bounds__(256) void mrif_sgemm_mix_ord_2_1(
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 2, 1);
     for (int phase = 0; phase < 2; ++phase) {
         if ((sp.role ^ phase) == 0) {
-            tk::mrif_role(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::mrif_role<4>(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
         } else {
             tk::sgemm_role(sgemm1_A, sgemm1_B, sgemm1_C, sgemm1_NORMAL_M, sgemm1_NORMAL_N, sgemm1_NORMAL_K, sgemm1_grid_dimension_x, sgemm1_grid_dimension_y, sgemm1_grid_dimension_z, (int)blockIdx.x, (int)gridDim.x, sgemm1_ptb_start_block_pos, sgemm1_ptb_end_block_pos, (int)threadIdx.x, 256);
         }

@@ -48,7 +48,7 @@ extern "C" __global__ __launch_bounds__(256) void mrif_stencil_mix_wg_1_1(
     (void)stencil1_ptb_iter_block_step;
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 1, 1);
     if (sp.role == 0) {
-        tk::mrif_role(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, sp.role_block, sp.role_blocks, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::mrif_role<4>(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, sp.role_block, sp.role_blocks, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
     } else {
         tk::stencil_role(stencil1_c0, stencil1_c1, stencil1_A0, stencil1_Anext, stencil1_nx, stencil1_ny, stencil1_nz, stencil1_grid_dimension_x, stencil1_grid_dimension_y, stencil1_grid_dimension_z, sp.role_block, sp.role_blocks, stencil1_ptb_start_block_pos, stencil1_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
@@ -101,7 +101,7 @@ extern "C" __global__ __launch_bounds__(256) void mrif_stencil_mix_wg_1_2(
     (void)stencil1_ptb_iter_block_step;
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 1, 2);
     if (sp.role == 0) {
-        tk::mrif_role(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, sp.role_block, sp.role_blocks, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::mrif_role<4>(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, sp.role_block, sp.role_blocks, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
     } else {
         tk::stencil_role(stencil1_c0, stencil1_c1, stencil1_A0, stencil1_Anext, stencil1_nx, stencil1_ny, stencil1_nz, stencil1_grid_dimension_x, stencil1_grid_dimension_y, stencil1_grid_dimension_z, sp.role_block, sp.role_blocks, stencil1_ptb_start_block_pos, stencil1_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
@@ -154,7 +154,7 @@ extern "C" __global__ __launch_bounds__(256) void mrif_stencil_mix_wg_2_1(
     (void)stencil1_ptb_iter_block_step;
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 2, 1);
     if (sp.role == 0) {
-        tk::mrif_role(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, sp.role_block, sp.role_blocks, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::mrif_role<4>(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, sp.role_block, sp.role_blocks, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
     } else {
         tk::stencil_role(stencil1_c0, stencil1_c1, stencil1_A0, stencil1_Anext, stencil1_nx, stencil1_ny, stencil1_nz, stencil1_grid_dimension_x, stencil1_grid_dimension_y, stencil1_grid_dimension_z, sp.role_block, sp.role_blocks, stencil1_ptb_start_block_pos, stencil1_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
@@ -208,7 +208,7 @@ extern "C" __global__ __launch_bounds__(256) void mrif_stencil_mix_ord_1_1(
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 1, 1);
     for (int phase = 0; phase < 2; ++phase) {
         if ((sp.role ^ phase) == 0) {
-            tk::mrif_role(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::mrif_role<4>(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
         } else {
             tk::stencil_role(stencil1_c0, stencil1_c1, stencil1_A0, stencil1_Anext, stencil1_nx, stencil1_ny, stencil1_nz, stencil1_grid_dimension_x, stencil1_grid_dimension_y, stencil1_grid_dimension_z, (int)blockIdx.x, (int)gridDim.x, stencil1_ptb_start_block_pos, stencil1_ptb_end_block_pos, (int)threadIdx.x, 256);
         }
@@ -263,7 +263,7 @@ extern "C" __global__ __launch_bounds__(256) void mrif_stencil_mix_ord_1_2(
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 1, 2);
     for (int phase = 0; phase < 2; ++phase) {
         if ((sp.role ^ phase) == 0) {
-            tk::mrif_role(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::mrif_role<4>(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
         } else {
             tk::stencil_role(stencil1_c0, stencil1_c1, stencil1_A0, stencil1_Anext, stencil1_nx, stencil1_ny, stencil1_nz, stencil1_grid_dimension_x, stencil1_grid_dimension_y, stencil1_grid_dimension_z, (int)blockIdx.x, (int)gridDim.x, stencil1_ptb_start_block_pos, stencil1_ptb_end_block_pos, (int)threadIdx.x, 256);
         }
@@ -318,7 +318,7 @@ extern "C" __global__ __launch_bounds__(256) void mrif_stencil_mix_ord_2_1(
     const tk::WgSplit sp = tk::wg_split((int)blockIdx.x, (int)gridDim.x, 2, 1);
     for (int phase = 0; phase < 2; ++phase) {
         if ((sp.role ^ phase) == 0) {
-            tk::mrif_role(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
+            tk::mrif_role<4>(mrif0_numK, mrif0_x, mrif0_y, mrif0_z, mrif0_outR, mrif0_outI, mrif0_grid_dimension_x, mrif0_grid_dimension_y, (int)blockIdx.x, (int)gridDim.x, mrif0_ptb_start_block_pos, mrif0_ptb_end_block_pos, (int)threadIdx.x, 256);
         } else {
             tk::stencil_role(stencil1_c0, stencil1_c1, stencil1_A0, stencil1_Anext, stencil1_nx, stencil1_ny, stencil1_nz, stencil1_grid_dimension_x, stencil1_grid_dimension_y, stencil1_grid_dimension_z, (int)blockIdx.x, (int)gridDim.x, stencil1_ptb_start_block_pos, stencil1_ptb_end_block_pos, (int)threadIdx.x, 256);
         }

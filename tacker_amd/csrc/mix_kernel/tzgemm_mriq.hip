@@ -72,7 +72,7 @@ extern "C" __global__ __launch_bounds__(512) void mriq_tzgemm_mix_wave_256(
         const int be_block = apart ? (int)blockIdx.x - tz_busy : (int)blockIdx.x;
         const int be_blocks = apart ? launched - tz_busy : launched;
         if (be_block >= 0) {
-            tk::mriq_role(mriq0_numK, mriq0_x, mriq0_y, mriq0_z, mriq0_Qr, mriq0_Qi, mriq0_grid_dimension_x, mriq0_grid_dimension_y, be_block, be_blocks, mriq0_ptb_start_block_pos, mriq0_ptb_end_block_pos, (int)threadIdx.x - 256, 256);
+            tk::mriq_role<4>(mriq0_numK, mriq0_x, mriq0_y, mriq0_z, mriq0_Qr, mriq0_Qi, mriq0_grid_dimension_x, mriq0_grid_dimension_y, be_block, be_blocks, mriq0_ptb_start_block_pos, mriq0_ptb_end_block_pos, (int)threadIdx.x - 256, 256);
         }
         tk::role_wave_done(tz_arrivals);
     }
@@ -148,7 +148,7 @@ extern "C" __global__ __launch_bounds__(768) void mriq_tzgemm_mix_wave_512(
         const int be_block = apart ? (int)blockIdx.x - tz_busy : (int)blockIdx.x;
         const int be_blocks = apart ? launched - tz_busy : launched;
         if (be_block >= 0) {
-            tk::mriq_role(mriq0_numK, mriq0_x, mriq0_y, mriq0_z, mriq0_Qr, mriq0_Qi, mriq0_grid_dimension_x, mriq0_grid_dimension_y, be_block, be_blocks, mriq0_ptb_start_block_pos, mriq0_ptb_end_block_pos, (int)threadIdx.x - 256, 512);
+            tk::mriq_role<8>(mriq0_numK, mriq0_x, mriq0_y, mriq0_z, mriq0_Qr, mriq0_Qi, mriq0_grid_dimension_x, mriq0_grid_dimension_y, be_block, be_blocks, mriq0_ptb_start_block_pos, mriq0_ptb_end_block_pos, (int)threadIdx.x - 256, 512);
         }
         tk::role_wave_done(tz_arrivals);
     }
@@ -207,7 +207,7 @@ extern "C" __global__ __launch_bounds__(256) void mriq_tzgemm_mix_wg_1_1(
         tk::WorkgroupSync sync;
         tk::tzgemm_role<TZ_STAGES_WG, true>(tzgemm1_A, tzgemm1_B, tzgemm1_C, tzgemm1_NORMAL_M, tzgemm1_NORMAL_N, tzgemm1_NORMAL_K, tk::tz_workspace_of(tzgemm1_C, tzgemm1_NORMAL_M, tzgemm1_NORMAL_N, tzgemm1_NORMAL_K), sp.role_block, sp.role_blocks, tzgemm1_ptb_start_block_pos, tzgemm1_ptb_end_block_pos, (int)threadIdx.x, tz_lds, sync);
     } else {
-        tk::mriq_role(mriq0_numK, mriq0_x, mriq0_y, mriq0_z, mriq0_Qr, mriq0_Qi, mriq0_grid_dimension_x, mriq0_grid_dimension_y, sp.role_block, sp.role_blocks, mriq0_ptb_start_block_pos, mriq0_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::mriq_role<4>(mriq0_numK, mriq0_x, mriq0_y, mriq0_z, mriq0_Qr, mriq0_Qi, mriq0_grid_dimension_x, mriq0_grid_dimension_y, sp.role_block, sp.role_blocks, mriq0_ptb_start_block_pos, mriq0_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
 }
 
@@ -264,7 +264,7 @@ extern "C" __global__ __launch_bounds__(256) void mriq_tzgemm_mix_wg_1_2(
         tk::WorkgroupSync sync;
         tk::tzgemm_role<TZ_STAGES_WG, true>(tzgemm1_A, tzgemm1_B, tzgemm1_C, tzgemm1_NORMAL_M, tzgemm1_NORMAL_N, tzgemm1_NORMAL_K, tk::tz_workspace_of(tzgemm1_C, tzgemm1_NORMAL_M, tzgemm1_NORMAL_N, tzgemm1_NORMAL_K), sp.role_block, sp.role_blocks, tzgemm1_ptb_start_block_pos, tzgemm1_ptb_end_block_pos, (int)threadIdx.x, tz_lds, sync);
     } else {
-        tk::mriq_role(mriq0_numK, mriq0_x, mriq0_y, mriq0_z, mriq0_Qr, mriq0_Qi, mriq0_grid_dimension_x, mriq0_grid_dimension_y, sp.role_block, sp.role_blocks, mriq0_ptb_start_block_pos, mriq0_ptb_end_block_pos, (int)threadIdx.x, 256);
+        tk::mriq_role<4>(mriq0_numK, mriq0_x, mriq0_y, mriq0_z, mriq0_Qr, mriq0_Qi, mriq0_grid_dimension_x, mriq0_grid_dimension_y, sp.role_block, sp.role_blocks, mriq0_ptb_start_block_pos, mriq0_ptb_end_block_pos, (int)threadIdx.x, 256);
     }
 }
 
@@ -341,7 +341,7 @@ extern "C" __global__ __launch_bounds__(512) void mriq_tzgemm_mix_wave_256_large
         const int be_block = apart ? (int)blockIdx.x - tz_busy : (int)blockIdx.x;
         const int be_blocks = apart ? launched - tz_busy : launched;
         if (be_block >= 0) {
-            tk::mriq_role(mriq0_numK, mriq0_x, mriq0_y, mriq0_z, mriq0_Qr, mriq0_Qi, mriq0_grid_dimension_x, mriq0_grid_dimension_y, be_block, be_blocks, mriq0_ptb_start_block_pos, mriq0_ptb_end_block_pos, (int)threadIdx.x - 256, 256);
+            tk::mriq_role<4>(mriq0_numK, mriq0_x, mriq0_y, mriq0_z, mriq0_Qr, mriq0_Qi, mriq0_grid_dimension_x, mriq0_grid_dimension_y, be_block, be_blocks, mriq0_ptb_start_block_pos, mriq0_ptb_end_block_pos, (int)threadIdx.x - 256, 256);
         }
         tk::role_wave_done(tz_arrivals);
     }

@@ -218,7 +218,7 @@ def generate_gptb(name):
     role = ROLES[name]
     sig = gptb_signature(name)
     call = role["call"].format(p="", block="(int)blockIdx.x", blocks="ptb_iter_block_step",
-                               tid="(int)threadIdx.x - thread_base", threads="(int)blockDim.x", waves=GPTB_MAX_WAVES,
+                               tid="(int)threadIdx.x - thread_base", threads="(int)blockDim.x", waves=role["gptb"].get("waves", GPTB_MAX_WAVES),
                                extra="",
                                stages="TZ_STAGES", stream_c="true")
     symbol = role["gptb"]["symbol"]

@@ -13,7 +13,8 @@ device functions.
                without the 10-int GPTB trailer.
 ``gptb``     -- the plain GPTB kernel of the role: its symbol (the reference's names,
                src/main.cu:108-125: ``g_general_ptb_`` for mriq and cp), attributes in front
-               of ``void`` and the reference file that holds its counterpart.
+               of ``void``, the reference file that holds its counterpart and, where its
+               launches may have more than GPTB_MAX_WAVES wavefronts that use LDS, how many.
 ``call``     -- format string of the role call; ``{p}`` is the parameter prefix,
                ``{block}``, ``{blocks}`` the role-local persistent-workgroup id
                and count, ``{tid}`` the role-local thread id, ``{threads}`` the
@@ -56,20 +57,20 @@ ROLES = {
                  "{p}ptb_end_block_pos, {tid}, {threads});"),
     },
     "mriq": {
-        "gptb": {"symbol": "g_general_ptb_mriq", "cite": "src/gptb_kernel/mriq_kernel.cu:3-70", "attributes": ""},
+        "gptb": {"symbol": "g_general_ptb_mriq", "cite": "src/gptb_kernel/mriq_kernel.cu:3-70", "attributes": "", "waves": 16},
         "params": [("int", "numK"), ("int", "kGlobalIndex"), ("float*", "x"), ("float*", "y"),
                    ("float*", "z"), ("float*", "Qr"), ("float*", "Qi")],
         "needs_sync": False,
-        "call": ("tk::mriq_role({p}numK, {p}x, {p}y, {p}z, {p}Qr, {p}Qi, {p}grid_dimension_x, "
+        "call": ("tk::mriq_role<{waves}>({p}numK, {p}x, {p}y, {p}z, {p}Qr, {p}Qi, {p}grid_dimension_x, "
                  "{p}grid_dimension_y, {block}, {blocks}, {p}ptb_start_block_pos, {p}ptb_end_block_pos, {tid}, "
                  "{threads});"),
     },
     "mrif": {
-        "gptb": {"symbol": "general_ptb_mrif", "cite": "src/gptb_kernel/mrif_kernel.cu:6-93", "attributes": ""},
+        "gptb": {"symbol": "general_ptb_mrif", "cite": "src/gptb_kernel/mrif_kernel.cu:6-93", "attributes": "", "waves": 16},
         "params": [("int", "numK"), ("int", "kGlobalIndex"), ("float*", "x"), ("float*", "y"),
                    ("float*", "z"), ("float*", "outR"), ("float*", "outI")],
         "needs_sync": False,
-        "call": ("tk::mrif_role({p}numK, {p}x, {p}y, {p}z, {p}outR, {p}outI, {p}grid_dimension_x, "
+        "call": ("tk::mrif_role<{waves}>({p}numK, {p}x, {p}y, {p}z, {p}outR, {p}outI, {p}grid_dimension_x, "
                  "{p}grid_dimension_y, {block}, {blocks}, {p}ptb_start_block_pos, {p}ptb_end_block_pos, {tid}, "
                  "{threads});"),
     },

@@ -506,6 +506,36 @@ def test_mriq_closed_forms_and_ranges():
     assert np.array_equal(pr[256:768], fr[256:768]) and np.all(pr[:256] == 0) and np.all(pr[768:] == 0)
 
 
+@pytest.mark.parametrize("kernel", ["mriq", "mrif"])
+@pytest.mark.parametrize("numK", [1, 7, 8, 9, 63, 64, 65, 71, 127, 129, 200])
+def test_mri_record_counts_signs_and_large_phases(kernel, numK):
+    # records come 64 at a time and 8 a step: every remainder, in a launch with one and with several voxel blocks a
+    # thread and in the natural one; phases of both signs, below and far above a revolution
+    rng = np.random.default_rng(numK)
+    numX = 1280
+    kv = rng.uniform(-1, 1, (numK, 4 if kernel == "mriq" else 5)).astype(np.float32)
+    xyz = rng.uniform(-1, 1, (3, numX)).astype(np.float32)
+    xyz[:, ::3] *= 400
+    phase = kv[:, :3].astype(np.float64) @ xyz.astype(np.float64)
+    turn = np.exp(2j * np.pi * phase)
+    amplitude = kv[:, 3].astype(np.float64) + (1j * kv[:, 4].astype(np.float64) if kernel == "mrif" else 0)
+    want = amplitude @ turn
+    (ta.mriq_set_kvalues if kernel == "mriq" else ta.mrif_set_kvalues)(kv)
+    d = [dev(v) for v in xyz]
+    # a phase is three products and two sums, each rounded to 2^-24 of at most |K||x|; sine and cosine are within 2e-7;
+    # a sum of numK terms of at most sqrt(2) is rounded numK times
+    reach = np.abs(kv[:, :3]).astype(np.float64) @ np.abs(xyz).astype(np.float64)
+    bound = (np.abs(amplitude)[:, None] * (2 * np.pi * 3 * 2.0 ** -24 * reach + 4e-7)).sum(0) + numK * numK * 1.5 * 2.0 ** -24
+    first = None
+    for form, kw in (("ori", {}), ("gptb", {}), ("gptb", {"launch_grid": 1}), ("gptb", {"launch_grid": 2})):
+        re, im = torch.zeros(numX, device="cuda:0"), torch.zeros(numX, device="cuda:0")
+        getattr(ta, f"{form}_{kernel}")(numK, *d, re, im, **kw)
+        got = host(re), host(im)
+        assert np.all(np.abs(got[0] - want.real) <= bound) and np.all(np.abs(got[1] - want.imag) <= bound)
+        first = first or got
+        assert np.array_equal(got[0], first[0]) and np.array_equal(got[1], first[1])
+
+
 def test_mriq_block_positions_are_voxel_blocks_by_k_chunks():
     # numK 300 -> chunks of 128, 128 and 44 records; 4 voxel blocks -> 12 block positions
     numK, numX = 300, 1024
