@@ -247,6 +247,14 @@ public:
             part = segments > 16;
             d.runs = part ? segments / 4 : segments;
             key_ = std::string("conv3x3_direct_") + (slices == 2 ? "2" : "1") + (part ? "_1" : "_0");
+            // Tiles of four rows where an image has no more, and where those of eight make workgroups for half of the CUs or
+            // fewer: us with tiles of eight and four rows, conv5_1 at 224 x 224 (128 workgroups of 8 x 8) 8.0 / 6.7, conv4_2 at
+            // 64 x 96 (64) 9.0 / 7.3, conv3_2 there (96) 6.2 / 5.2.
+            if (slices == 1 && (H_ <= DNN_TILE / 2 || (ct == 1 && 2L * d.tiles * (Cout_ / 16) <= cuCount()))) {
+                key_ += "_low";
+                d.tiles = d.tiles_x * ((H_ + DNN_TILE / 2 - 1) / (DNN_TILE / 2));
+                d.per_group = reciprocal(d.tiles);
+            }
             lds_ = std::max((size_t)(C_ / 64) * DNN_PLANE_BYTES, (size_t)ct * d.runs * DNN_PARTIAL_BYTES);
         } else {
             ct = Cout_ / 16;

@@ -29,6 +29,11 @@ typedef __attribute__((address_space(3))) float lds_float;
 
 #define DNN_VMCNT_IMM(n) (((n) & 15) | (((n) >> 4) << 14) | 0x0F70)   // s_waitcnt vmcnt(n), nothing else
 
+template <int N>
+struct dnn_int {
+    static constexpr int value = N;
+};
+
 // One LDS-direct load of 16 bytes per lane: scalar base + 32-bit lane offset, to LDS address + 16 lane.
 __device__ __forceinline__ void dnn_load_to_lds(const char *uniform_base, unsigned lane_offset, unsigned lds_address)
 {
@@ -62,16 +67,17 @@ __device__ __forceinline__ int dnn_tile_y(int p) { return 2 * (p >> 4) + ((p >> 
 // n / d by the host's reciprocal (2^32 / d rounded up, 0 for d = 1): exact for the tile numbers of any image
 __device__ __forceinline__ int dnn_div(int n, unsigned reciprocal) { return reciprocal ? (int)__umulhi((unsigned)n, reciprocal) : n; }
 
-// A tile's results from LDS to memory.  `partials` tiles of [pixel][quads] lie in LDS, to be added in tzgemm's order
+// A tile's results from LDS to memory, of its first 16 GROUPS pixels.  `partials` tiles of [pixel][quads] lie in LDS, to be added in tzgemm's order
 // (parts of four segments, or -- parts_only -- sums of whole parts); n0: first channel.  Lanes take a pixel's channels
 // side by side, so that a pixel's row goes out in one piece: the raw value to C, the activation -- of the pixel, or of its
 // 2x2 cell -- to the next layer's input.
+template <int GROUPS>
 __device__ __forceinline__ void dnn_finish(lds_float4 *tile, int partials, bool parts_only, int quads, int y0, int x0, int n0,
-                                           const DnnOutput &o)
+                                           const float4_t bias, const DnnOutput &o)
 {
     const int threads = (int)blockDim.x, quad_shift = __builtin_ctz(quads);
     const int stride = DNN_TILE * DNN_TILE * quads;
-    for (int i = (int)threadIdx.x; i < stride; i += threads) {
+    for (int i = (int)threadIdx.x; i < 16 * GROUPS * quads; i += threads) {
         const int p = i >> quad_shift, q = i & (quads - 1);
         const int at = dnn_tile_at(p, q, quads);
         float4_t v = tile[at];
@@ -93,13 +99,13 @@ __device__ __forceinline__ void dnn_finish(lds_float4 *tile, int partials, bool 
             if (!o.pool)
                 *reinterpret_cast<half4_t *>(reinterpret_cast<_Float16 *>(o.act) +
                                              (size_t)((y + o.border) * o.act_pitch + x + o.border) * o.act_C + n) =
-                    dnn_activate(v, *reinterpret_cast<const float4_t *>(o.bias + n));
+                    dnn_activate(v, bias);
         }
         if (o.pool) tile[at] = v;
     }
     if (!o.pool) return;
     __syncthreads();
-    for (int i = (int)threadIdx.x; i < stride / 4; i += threads) {
+    for (int i = (int)threadIdx.x; i < 4 * GROUPS * quads; i += threads) {
         const int cell = i >> quad_shift, q = i & (quads - 1);
         float4_t v = tile[dnn_tile_at(4 * cell, q, quads)];
 #pragma unroll
@@ -112,8 +118,15 @@ __device__ __forceinline__ void dnn_finish(lds_float4 *tile, int partials, bool 
         if (y < o.H && x < o.W)
             *reinterpret_cast<half4_t *>(reinterpret_cast<_Float16 *>(o.act) +
                                          (size_t)((y / 2 + o.border) * o.act_pitch + x / 2 + o.border) * o.act_C + n) =
-                dnn_activate(v, *reinterpret_cast<const float4_t *>(o.bias + n));
+                dnn_activate(v, bias);
     }
+}
+
+// The bias of the channels a thread finishes, float4 threadIdx.x of the tile's `quads` a pixel (which divide the threads).
+// Asked for as the kernel starts: where it is needed it would be one more trip to memory, at the end of a short kernel.
+__device__ __forceinline__ float4_t dnn_bias(const DnnOutput &o, int n0, int quads)
+{
+    return *reinterpret_cast<const float4_t *>(o.bias + n0 + 4 * ((int)threadIdx.x & (quads - 1)));
 }
 
 // workgroup -> (pixel tile, channel group): every XCD takes a contiguous run of the order "channel group, then pixel
@@ -140,15 +153,17 @@ using namespace tk;
 // slot s ^ key, key = (x / 2 + 4 (y & 1)) & 7, which spreads the 16 pixels of a fragment read (8 x 2, at any
 // tap) over all banks.
 //
-// What bounds it is the rate at which a CU takes data in, 80 to 100 GB/s from the L2s: at 28 x 28, 512 -> 512 channels a
-// workgroup (64 pixels x 32 channels, one per CU) loads 104 KB of patch and 295 KB of weights, 4.4 us of a 9.1 us
-// kernel; launch and the first load's latency are 3 us, the last sums and stores 1.5 (by counters 97 MB asked of the L2s
-// there, matrix pipes busy 0.25 of the time, vector units 0.20, LDS bank conflicts 0.08).  So a workgroup takes as many
-// channels as leave every CU one, and two 16-channel slices a wavefront (NT = 2), which halves the fragment reads from
-// LDS, where eight wavefronts are left; the patch is asked for before the weights.  us a layer of VGG16 at 224 x
-// 224, against the operand in memory and tzgemm: conv1_2 38 -> 12, conv2_2 26 -> 10, conv3_2 21 -> 9.3, conv4_2 23 -> 9.1,
-// conv5_1 18 -> 8.0.
-template <int NT, bool PART>
+// What bounds it is a chain of short things one after the other.  Of the 9.2 us of 28 x 28, 512 -> 512 channels (a workgroup
+// is 64 pixels x 32 channels, one per CU, and loads 104 KB of patch and 295 KB of weights) 4.1 are left where the patch
+// and all chunks but one are left out -- launch, first load, barrier, last sums and stores --, 2 are the k loop where its
+// loads are left out, 1.6 the patch and 1.5 the weights.  So a workgroup takes as many channels as leave every CU one,
+// and two 16-channel slices a wavefront (NT = 2), which halves the fragment reads from LDS, where eight wavefronts are left (four
+// are too few: conv2_2 10.3 -> 11.2 us); where there are workgroups for half of the CUs or fewer, tiles have four rows (GROUPS = 2
+// pairs of rows instead of 4); the bias is asked for first, then the patch, then the weights; and a step's
+// fragments are read from LDS while the matrix units work on those of the step before.  us a layer of VGG16 at 224 x 224,
+// first through the operand in memory and tzgemm, then reading its fragments where it uses them, now: conv2_2 26, 10.5, 9.5,
+// conv3_2 21, 9.5, 8.8, conv4_2 23, 9.7, 9.1, conv5_1 18, 8.4, 6.6; at 64 x 96 conv4_2 8.6, 6.8, conv5_1 8.2, 6.3 (the last two each).
+template <int NT, bool PART, int GROUPS>
 __device__ __forceinline__ void conv3x3_direct(const DnnConv &c, char *lds_generic)
 {
     lds_char *const lds = (lds_char *)lds_generic;
@@ -160,7 +175,7 @@ __device__ __forceinline__ void conv3x3_direct(const DnnConv &c, char *lds_gener
     const int group = dnn_div(tile, c.per_group);
     const int pixel_tile = tile - group * c.tiles;
     const int tile_row = dnn_div(pixel_tile, c.per_row);
-    const int y0 = tile_row * DNN_TILE, x0 = (pixel_tile - tile_row * c.tiles_x) * DNN_TILE;
+    const int y0 = tile_row * (2 * GROUPS), x0 = (pixel_tile - tile_row * c.tiles_x) * DNN_TILE;
     const int ct_shift = __builtin_ctz(c.ct_count / NT);
     const int cp = wave & ((1 << ct_shift) - 1), kw = wave >> ct_shift;
     const int n16 = group * c.ct_count + cp * NT;
@@ -172,9 +187,12 @@ __device__ __forceinline__ void conv3x3_direct(const DnnConv &c, char *lds_gener
     const int first = begin[0], last = begin[PART ? 4 : 1];
     const int second = PART ? begin[1] : last, third = PART ? begin[2] : last, fourth = PART ? begin[3] : last;
 
-    // the patch: 13 pieces of 8 pixels, every plane of a piece by one wavefront
+    const int quads = 4 * c.ct_count;
+    const float4_t bias = dnn_bias(c.out, group * c.ct_count * 16, quads);
+    // the patch: pieces of 8 pixels, every plane of a piece by one wavefront; what lies below the image's border is left out
+    const int pieces = (min(2 * GROUPS + 2, H + 2 - y0) * DNN_PATCH + 7) >> 3;
     const unsigned lds_base = (unsigned)(size_t)lds;
-    for (int piece = wave; piece < DNN_PATCH_LOADS; piece += waves) {
+    for (int piece = wave; piece < pieces; piece += waves) {
         const int p = min(8 * piece + (lane >> 3), DNN_PATCH * DNN_PATCH - 1);
         const int py = (p * 205) >> 11, px = p - py * DNN_PATCH;   // p / 10 for p < 1024
         const int gy = min(y0 + py, H + 1), gx = min(x0 + px, W + 1);
@@ -185,7 +203,8 @@ __device__ __forceinline__ void conv3x3_direct(const DnnConv &c, char *lds_gener
                             lds_base + plane * DNN_PLANE_BYTES + piece * 1024);
     }
     // behind it the first chunks of the weights; the patch has landed when only they are still on their way
-    constexpr int RING = 3;
+    constexpr int RING = 2;
+    static_assert(RING % 2 == 0, "a step's fragments are read into the set the step before does not use");
     const half8_t *weights = reinterpret_cast<const half8_t *>(c.weights) + (size_t)n16 * c.chunks * 2 * 64 + lane;
     half8_t b[RING][NT][2];
     const int final_chunk = max(last - 1, 0);   // an empty run fetches the first chunk, which is there
@@ -204,95 +223,98 @@ __device__ __forceinline__ void conv3x3_direct(const DnnConv &c, char *lds_gener
 
     const int r = lane & 15;
     const int tx = dnn_tile_x(r), ty = dnn_tile_y(r);
-    float4_t acc[NT][4], sum[NT][4];
+    float4_t acc[NT][GROUPS], sum[NT][GROUPS];
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int g = 0; g < 4; ++g) acc[t][g] = sum[t][g] = float4_t{0.f, 0.f, 0.f, 0.f};
+        for (int g = 0; g < GROUPS; ++g) acc[t][g] = sum[t][g] = float4_t{0.f, 0.f, 0.f, 0.f};
 
-    const auto multiply = [&](const half8_t (&w)[NT][2], int chunk) {
+    half8_t a[2][2][GROUPS];   // the pixels' fragments of this step and the next, both halves of their 64 k
+    const auto read = [&](half8_t (&to)[2][GROUPS], int chunk) {
         const int tap = chunk >> plane_shift, plane = chunk & (planes - 1);
         const int kh = (tap * 11) >> 5, kx = tap - 3 * kh;   // tap / 3 for tap < 9
         const int px = tx + kx, py = ty + kh;
         const int key = ((px >> 1) + 4 * (py & 1)) & 7;
         const unsigned at = (unsigned)(plane * DNN_PLANE_BYTES + (py * DNN_PATCH + px) * 128 + (((lane >> 4) ^ key) << 4));
-        half8_t a0[4], a1[4];
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            a0[g] = *(lds_half8 *)(lds + at + g * (2 * DNN_PATCH * 128));
-            a1[g] = *(lds_half8 *)(lds + (at ^ 64u) + g * (2 * DNN_PATCH * 128));
-        }
+        for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
+            for (int g = 0; g < GROUPS; ++g) to[h][g] = *(lds_half8 *)(lds + (at ^ (64u * h)) + g * (2 * DNN_PATCH * 128));
+    };
+    const auto multiply = [&](const half8_t (&w)[NT][2], const half8_t (&p)[2][GROUPS]) {
 #pragma unroll
-            for (int g = 0; g < 4; ++g) acc[t][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[t][0], a0[g], acc[t][g], 0, 0, 0);
+        for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
+            for (int t = 0; t < NT; ++t)
 #pragma unroll
-            for (int g = 0; g < 4; ++g) acc[t][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[t][1], a1[g], acc[t][g], 0, 0, 0);
+                for (int g = 0; g < GROUPS; ++g) acc[t][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[t][h], p[h][g], acc[t][g], 0, 0, 0);
     };
     int segment = 1;
     const auto segment_done = [&]() {   // ((w0 + w1) + w2) + w3
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
+            for (int g = 0; g < GROUPS; ++g) {
                 sum[t][g] = segment == 1 ? acc[t][g] : sum[t][g] + acc[t][g];
                 acc[t][g] = float4_t{0.f, 0.f, 0.f, 0.f};
             }
         ++segment;
     };
     const auto next_begins = [&]() -> int { return segment == 1 ? second : (segment == 2 ? third : (segment == 3 ? fourth : last)); };
-    const auto step = [&](const half8_t (&w)[NT][2], int chunk) {
+    const auto step = [&](const half8_t (&w)[NT][2], const half8_t (&now)[2][GROUPS], half8_t (&next)[2][GROUPS], int chunk) {
         if (PART)
             while (chunk == next_begins()) segment_done();
-        multiply(w, chunk);
+        read(next, min(chunk + 1, final_chunk));   // (behind the run the last ones again)
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(w, now);
+        __builtin_amdgcn_sched_barrier(0);
     };
     // A run is 9 chunks in most layers.  Its last RING chunks are told apart from the rest: nothing behind the run is
     // fetched (that was a third more weights than it has), and the loop's waits count exactly the loads behind the one they
-    // need; with the end's condition inside the loop the compiler has to allow for a fetch left out, and waited for all of
-    // them every third chunk.  A query of one image over and over takes 163 instead of 167.5 us at 224 x 224, 106
-    // instead of 113 at 64 x 96, 129 instead of 137 at 128 x 160.  More chunks in flight lose: 6 (9 with parts or two slices) 171 us and 113, 4 (5) 166 and
-    // 107 to 112.  (Why is not known.  It is not the longer code: 0.1 to 0.7 % of the instruction fetches of these launches
-    // miss.)
+    // need; with the end's condition inside the loop the compiler has to allow for a fetch left out, and waits for all of
+    // them every time round.  More chunks in flight lose: with 4 a query takes 145.7 instead of 142.4 us at 224 x 224 and 90.7
+    // instead of 89.1 at 64 x 96 (what is in front of the barrier, the patch, is what the wavefronts wait for).
+    read(a[0], min(first, final_chunk));
     int base = first;
     for (; base + RING < last; base += RING) {
 #pragma unroll
         for (int u = 0; u < RING; ++u) {
-            step(b[u], base + u);
+            step(b[u], a[u & 1], a[(u + 1) & 1], base + u);
             fetch(b[u], min(base + u + RING, final_chunk));
         }
     }
 #pragma unroll
     for (int u = 0; u < RING; ++u)
-        if (base + u < last) step(b[u], base + u);   // uniform
+        if (base + u < last) step(b[u], a[u & 1], a[(u + 1) & 1], base + u);   // uniform
     if (PART)
         while (segment <= 4) segment_done();
 
     // results to LDS, [run of the reduction][pixel][channels]; the patch is done with
     __syncthreads();
     lds_float4 *const results = (lds_float4 *)lds;
-    const int quads = 4 * c.ct_count;
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int g = 0; g < 4; ++g)
+        for (int g = 0; g < GROUPS; ++g)
             results[kw * DNN_TILE * DNN_TILE * quads + dnn_tile_at(16 * g + r, 4 * (cp * NT + t) + (lane >> 4), quads)] =
                 PART ? sum[t][g] : acc[t][g];
     __syncthreads();
-    dnn_finish(results, c.runs, PART, quads, y0, x0, group * c.ct_count * 16, c.out);
+    dnn_finish<GROUPS>(results, c.runs, PART, quads, y0, x0, group * c.ct_count * 16, bias, c.out);
 }
 
-#define DNN_CONV_KERNEL(NT_, PART_, THREADS_)                                                                        \
-    extern "C" __global__ __launch_bounds__(THREADS_) void conv3x3_direct_##NT_##_##PART_(DnnConv c)                   \
+#define DNN_CONV_KERNEL(NAME_, NT_, PART_, GROUPS_, THREADS_)                                                          \
+    extern "C" __global__ __launch_bounds__(THREADS_) void NAME_(DnnConv c)                                            \
     {                                                                                                                 \
         extern __shared__ __align__(16) char conv_lds[];                                                              \
-        conv3x3_direct<NT_, PART_ != 0>(c, conv_lds);                                                                  \
+        conv3x3_direct<NT_, PART_, GROUPS_>(c, conv_lds);                                                              \
     }
-DNN_CONV_KERNEL(1, 0, 1024)
-DNN_CONV_KERNEL(1, 1, 512)
-DNN_CONV_KERNEL(2, 0, 512)
-
+DNN_CONV_KERNEL(conv3x3_direct_1_0, 1, false, 4, 1024)
+DNN_CONV_KERNEL(conv3x3_direct_1_1, 1, true, 4, 512)
+DNN_CONV_KERNEL(conv3x3_direct_2_0, 2, false, 4, 512)
+// Tiles of four rows instead of eight, for layers of few workgroups: half the reads from LDS and matrix instructions, 62 instead of
+// 104 KB of patch at 512 channels, twice the workgroups (conv5_1 at 224 x 224 8.0 -> 6.7 us, conv4_2 at 64 x 96 9.0 -> 7.3).
+DNN_CONV_KERNEL(conv3x3_direct_1_0_low, 1, false, 2, 1024)
+DNN_CONV_KERNEL(conv3x3_direct_1_1_low, 1, true, 2, 512)
 // The first convolution: the image, [H][W][3] fp32, 27 k in one matrix instruction.  A workgroup computes an 8 x 8 pixel
 // tile by 64 channels, wavefront g the pixel group g; a lane gathers its 8 k (of 32; the last 5 are padding) of its pixel.
 // keep: null, or where the image is stored as well.
@@ -307,6 +329,7 @@ extern "C" __global__ __launch_bounds__(256) void conv3x3_image(const float *ima
     const int tile_row = dnn_div(tile, c.per_row);
     const int y0 = tile_row * DNN_TILE, x0 = (tile - tile_row * c.tiles_x) * DNN_TILE;
     const int H = c.out.H, W = c.out.W;
+    const float4_t bias = dnn_bias(c.out, 0, 16);
     if (keep && threadIdx.x < 3 * DNN_TILE * DNN_TILE) {
         const int row = (int)threadIdx.x / (3 * DNN_TILE), column = (int)threadIdx.x - row * (3 * DNN_TILE);
         if (y0 + row < H && 3 * x0 + column < 3 * W) {
@@ -340,51 +363,71 @@ extern "C" __global__ __launch_bounds__(256) void conv3x3_image(const float *ima
         results[dnn_tile_at(16 * g + r, 4 * j + (lane >> 4), 16)] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[j], a, zero, 0, 0, 0);
     }
     __syncthreads();
-    dnn_finish(results, 1, false, 16, y0, x0, 0, c.out);
+    dnn_finish<4>(results, 1, false, 16, y0, x0, 0, bias, c.out);
 }
 
 // A fully connected layer at batch 1: 16 outputs per workgroup, a wavefront takes SPW consecutive segments of the
 // reduction and streams their weights past the caches (nontemporal: a query reads each of them once).  All 16 rows of the
 // matrix instruction's other operand are the activation vector; its first row is the layer's.
+//
+// A segment is a few steps to a few dozen, and it is up to 8 steps' loads at a time, the last ones as well: a trip to
+// memory is 1 to 2 us, and a segment of 6 steps (3072 -> 4096), or two of 4 (4096 -> 1000), two steps at a time made three or four
+// of them.
 template <int SPW>
 __device__ __forceinline__ void fc_direct(const DnnFc &f)
 {
     __shared__ float partial[16 * SPW][16];
+    const float bias = f.act ? f.bias[blockIdx.x * 16 + (threadIdx.x & 15)] : 0.0f;   // (asked for first, as dnn_bias)
     const int lane = (int)threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const half8_t *weights = reinterpret_cast<const half8_t *>(f.weights) + ((size_t)blockIdx.x * f.chunks * 2) * 64 + lane;
     const half8_t *x = reinterpret_cast<const half8_t *>(f.x) + (lane >> 4);
+    half8_t w[8], a[8];
+    const auto load = [&](auto steps, int k) {   // steps of 32 k
 #pragma unroll
-    for (int i = 0; i < SPW; ++i) {
-        const int s = wave * SPW + i;
-        if (s < f.segments) {
-            const int first = 2 * f.segment_begin[s], last = 2 * f.segment_begin[s + 1];
-            float4_t acc = {0.f, 0.f, 0.f, 0.f};
-            int k = first;   // in steps of 32
-            constexpr int U = 8;
-            for (; k + U <= last; k += U) {
-                half8_t w[U], a[U];
+        for (int u = 0; u < decltype(steps)::value; ++u) {
+            w[u] = __builtin_nontemporal_load(weights + (size_t)(k + u) * 64);
+            a[u] = x[4 * (k + u)];
+        }
+    };
+    const auto multiply = [&](auto from, auto to, float4_t &acc) {
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    w[u] = __builtin_nontemporal_load(weights + (size_t)(k + u) * 64);
-                    a[u] = x[4 * (k + u)];
-                }
+        for (int u = decltype(from)::value; u < decltype(to)::value; ++u)
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[u], a[u], acc, 0, 0, 0);
+    };
+    const auto store = [&](int s, const float4_t &acc) {
+        if ((lane & 15) == 0) {
 #pragma unroll
-                for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[u], a[u], acc, 0, 0, 0);
-            }
-            for (; k < last; k += 2) {
-                half8_t w[2], a[2];
+            for (int e = 0; e < 4; ++e) partial[s][4 * (lane >> 4) + e] = acc[e];
+        }
+    };
+    const int s0 = wave * SPW;
+    if (SPW == 2 && s0 + 1 < f.segments && f.segment_begin[s0 + 1] - f.segment_begin[s0] == 2 &&
+        f.segment_begin[s0 + 2] - f.segment_begin[s0 + 1] == 2) {   // two of four steps: at once
+        float4_t acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = acc0;
+        load(dnn_int<8>(), 2 * f.segment_begin[s0]);
+        multiply(dnn_int<0>(), dnn_int<4>(), acc0);
+        multiply(dnn_int<4>(), dnn_int<8>(), acc1);
+        store(s0, acc0);
+        store(s0 + 1, acc1);
+    } else {
 #pragma unroll
-                for (int u = 0; u < 2; ++u) {
-                    w[u] = __builtin_nontemporal_load(weights + (size_t)(k + u) * 64);
-                    a[u] = x[4 * (k + u)];
-                }
-#pragma unroll
-                for (int u = 0; u < 2; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[u], a[u], acc, 0, 0, 0);
-            }
-            if ((lane & 15) == 0) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) partial[s][4 * (lane >> 4) + e] = acc[e];
+        for (int i = 0; i < SPW; ++i) {
+            const int s = s0 + i;
+            if (s < f.segments) {
+                int k = 2 * f.segment_begin[s];
+                const int last = 2 * f.segment_begin[s + 1];
+                float4_t acc = {0.f, 0.f, 0.f, 0.f};
+                const auto step = [&](auto steps) {
+                    load(steps, k);
+                    multiply(dnn_int<0>(), steps, acc);
+                    k += decltype(steps)::value;
+                };
+                while (k + 8 <= last) step(dnn_int<8>());
+                if (k + 6 <= last) step(dnn_int<6>());
+                else if (k + 4 <= last) step(dnn_int<4>());
+                else if (k + 2 <= last) step(dnn_int<2>());
+                store(s, acc);
             }
         }
     }
@@ -402,7 +445,7 @@ __device__ __forceinline__ void fc_direct(const DnnFc &f)
         v *= TZ_ALPHA;
         f.raw[n] = v;
         if (f.act) {
-            v += f.bias[n];
+            v += bias;
             reinterpret_cast<_Float16 *>(f.act)[n] = (_Float16)(v < 0.0f ? 0.0f : v);
         }
     }
@@ -458,6 +501,8 @@ extern "C" void tk_register_dnn_kernels(tk_kernel_insert_fn insert, void *ctx)
     insert("conv3x3_direct_1_0", (const void *)conv3x3_direct_1_0, ctx);
     insert("conv3x3_direct_1_1", (const void *)conv3x3_direct_1_1, ctx);
     insert("conv3x3_direct_2_0", (const void *)conv3x3_direct_2_0, ctx);
+    insert("conv3x3_direct_1_0_low", (const void *)conv3x3_direct_1_0_low, ctx);
+    insert("conv3x3_direct_1_1_low", (const void *)conv3x3_direct_1_1_low, ctx);
     insert("conv3x3_image", (const void *)conv3x3_image, ctx);
     insert("fc_direct_1", (const void *)fc_direct_1, ctx);
     insert("fc_direct_2", (const void *)fc_direct_2, ctx);

@@ -433,6 +433,12 @@ def test_a_layer_by_itself_gives_the_bits_of_its_operand_and_tzgemm(H, W):
     task.close()
 
 
+@pytest.mark.parametrize("H,W", [(64, 96), (32, 224), (160, 64)])
+def test_a_layer_in_tiles_of_four_rows_gives_the_bits_of_its_operand_and_tzgemm(H, W):
+    # layers with workgroups for half of the CUs or fewer, and those of four rows and fewer: 1, 2, 4, 5, 8 and 10 rows
+    test_a_layer_by_itself_gives_the_bits_of_its_operand_and_tzgemm(H, W)
+
+
 @pytest.mark.parametrize("H,W,own_stream", [(32, 32, False), (224, 224, False), (96, 64, True), (224, 224, True)])
 def test_an_image_may_change_as_soon_as_the_query_is_launched(H, W, own_stream):
     # images are staged while the query before runs, into two device images in turn: the host's one is overwritten the
@@ -709,6 +715,12 @@ def test_a_fully_connected_layer_adds_the_segments_there_are(segments, K):
     # a sum of K products below 1 in fp32, in any order: K roundings of a partial sum below K
     assert np.abs(raw - exact).max() <= 1.1 * K * K * 2.0 ** -24 + 1e-6
     assert np.array_equal(act, np.maximum(raw + host(bias), 0).astype(np.float16))
+
+
+@pytest.mark.parametrize("segments,K", [(32, 4096), (32, 4160), (16, 3072), (16, 1280), (16, 5120), (4, 3136)])
+def test_a_fully_connected_layer_whose_segments_are_a_few_steps(segments, K):
+    # steps of 32 k, eight at a time: two segments of four a wavefront, one of four and one of six, six, two and four, ten, and 24 and 26
+    test_a_fully_connected_layer_adds_the_segments_there_are(segments, K)
 
 
 @pytest.mark.parametrize("check", ["raw", "bias", "classes"])
