@@ -643,7 +643,10 @@ TK_API int tacker_task_kernel_info(tacker_task_t task, int index, char *name, in
 /* VGG16 only: the buffer layer conv_index writes (0..12 the convolutions, 13..15 the three fully
  * connected layers, whose result is one row: H = W = 1): device pointer and dims = {H, W, channels,
  * channel stride}.  It holds the raw GEMM output 1.1 * A * B^T; the layer that reads it adds the bias
- * and rectifies.  logits = the first `count` floats of the last layer's buffer */
+ * and rectifies.  A whole query after a whole query leaves the convolutions' buffers out as long as nobody has
+ * asked for an address here or below: the first call behind such a query runs its convolutions once more, with
+ * them, and waits (0.2 ms), and from then on every query writes them (141 -> 152 us at 224 x 224).
+ * logits = the first `count` floats of the last layer's buffer */
 TK_API int tacker_task_activation(tacker_task_t task, int conv_index, float **ptr, int dims[4]);
 TK_API int tacker_task_logits(tacker_task_t task, const float **ptr, long *stride, int *count);
 /* VGG16 only: weights (f16 [dims[0]][dims[1]] = [Cout padded][9*Cin padded], k =
@@ -651,9 +654,9 @@ TK_API int tacker_task_logits(tacker_task_t task, const float **ptr, long *strid
  * connected layers ([out padded][in padded]; the last one has no bias: NULL).  Weights written there
  * are those of every later query; a graph recorded before this call keeps the ones it was recorded with.
  * From this call on the layer reads its weights as they lie there, through its operand builder and
- * tzgemm, for as long as the task lives: 163 us a query at 224 x 224 become 173 with layer 5 handed
- * out, 178 with layer 13, 206 with layer 0 (the query's image is then copied on the null stream) and
- * 361 with all of them */
+ * tzgemm, for as long as the task lives: 141 us a query at 224 x 224 become 163 with layer 5 handed
+ * out, 167 with layer 13, 197 with layer 0 (the query's image is then copied on the null stream) and
+ * 360 with all of them */
 TK_API int tacker_task_conv_params(tacker_task_t task, int conv_index, void **weights, float **bias,
                                    int dims[2]);
 TK_API int tacker_task_input(tacker_task_t task, float **host_ptr, int *bytes);

@@ -1441,25 +1441,29 @@ int tacker_task_activation(tacker_task_t h, int conv_index, float **ptr, int dim
 {
     VGG16 *v = dynamic_cast<VGG16 *>(static_cast<Task *>(h));
     if (!v || conv_index < 0 || conv_index >= 16) return fail(TK_ERROR_INVALID_VALUE, "bad activation index");
-    const VGG16::Act &a = v->layer(conv_index);
-    v->resultHandedOut(conv_index);
-    *ptr = a.ptr;
-    dims[0] = a.H; dims[1] = a.W; dims[2] = a.C; dims[3] = a.ld;
-    return TK_SUCCESS;
+    return guarded([&]() -> int {
+        const VGG16::Act &a = v->layer(conv_index);
+        v->resultHandedOut(conv_index);
+        *ptr = a.ptr;
+        dims[0] = a.H; dims[1] = a.W; dims[2] = a.C; dims[3] = a.ld;
+        return TK_SUCCESS;
+    });
 }
 
 int tacker_task_conv_params(tacker_task_t h, int conv_index, void **weights, float **bias, int dims[2])
 {
     VGG16 *v = dynamic_cast<VGG16 *>(static_cast<Task *>(h));
     if (!v || conv_index < 0 || conv_index >= 16) return fail(TK_ERROR_INVALID_VALUE, "bad layer index");
-    const VGG16::Act &a = v->layer(conv_index);
-    v->weightsHandedOut(conv_index);
-    v->resultHandedOut(conv_index);
-    *weights = a.weights;
-    *bias = a.bias;
-    dims[0] = a.Np;
-    dims[1] = a.Kp;
-    return TK_SUCCESS;
+    return guarded([&]() -> int {
+        const VGG16::Act &a = v->layer(conv_index);
+        v->weightsHandedOut(conv_index);
+        v->resultHandedOut(conv_index);
+        *weights = a.weights;
+        *bias = a.bias;
+        dims[0] = a.Np;
+        dims[1] = a.Kp;
+        return TK_SUCCESS;
+    });
 }
 
 int tacker_task_logits(tacker_task_t h, const float **ptr, long *stride, int *count)

@@ -10,7 +10,7 @@
 
 // where a layer's result goes
 typedef struct DnnOutput {
-    float *raw;          // [H * W][ld], 1.1 * A * B^T
+    float *raw;          // [H * W][ld], 1.1 * A * B^T; null: nobody reads it
     const float *bias;
     void *act;           // f16, [..][act_pitch][act_C] with `border` zero pixels around: relu(raw + bias), pooled or not
     int H, W, ld;
@@ -31,6 +31,18 @@ typedef struct DnnConv {
     int ct_count;          // a group: ct_count x 16 output channels
     int segment_begin[DNN_MAX_SEGMENTS + 1];   // first chunk of each segment tzgemm cuts the reduction into; no padding chunks
 } DnnConv;
+
+#define DNN_IMAGE_SIDE (DNN_PATCH + 2)
+#define DNN_IMAGE_BYTES (DNN_IMAGE_SIDE * DNN_IMAGE_SIDE * 3 * 2)
+// The first convolution as the second one computes it for itself (conv3x3_direct_image)
+typedef struct DnnImage {
+    const float *image;    // [H][W][3]
+    float *keep;           // where the image is stored as well
+    const void *weights;   // fragments of 64 channels, `chunks` chunks of 64 k
+    const float *bias;
+    int chunks;
+    int lds;               // where in LDS the tile's image goes (DNN_IMAGE_BYTES)
+} DnnImage;
 
 typedef struct DnnFc {
     const void *x;         // f16 [64 * chunks]

@@ -155,9 +155,9 @@ struct Activation {
 class GemmLayer : public LcGemmKernel {
 public:
     // tile_end > 0: only the reference tiles [0, tile_end) are computed (the others would be padding)
-    GemmLayer(int id, const std::string &name, int M, int N, int K, const void *A, const void *B, float *C,
+    GemmLayer(VGG16 &task, int id, const std::string &name, int M, int N, int K, const void *A, const void *B, float *C,
               int tile_end = 0)
-        : M_(M), N_(N), K_(K)
+        : task_(task), M_(M), N_(N), K_(K)
     {
         this->Id = id;
         this->kernelName = name;
@@ -173,10 +173,15 @@ public:
 protected:
     virtual void before(cudaStream_t stream) = 0;   // operand staging (im2col / pack)
     virtual void fused() {}                         // tzgemm runs the layer: its raw output is all this launch writes
-    void executeImpl(cudaStream_t stream) override
+    virtual void run(cudaStream_t stream)
     {
         before(stream);
         gptb_->execute(stream);
+    }
+    void executeImpl(cudaStream_t stream) final
+    {
+        task_.layerByItself();
+        run(stream);
     }
 
 public:
@@ -187,6 +192,7 @@ public:
             executeImpl(stream);
             return;
         }
+        task_.layerByItself();
         before(stream);
         fused();
         std::unique_ptr<MixKernel> mix(createTzgemmMix(be, gptb_.get(), be_start, be_end, 0, tiles_, variant, 0, 0));
@@ -194,6 +200,7 @@ public:
     }
 
 protected:
+    VGG16 &task_;
     int M_, N_, K_, tiles_;
     std::unique_ptr<OriTZGEMMKernel> ori_;
     std::unique_ptr<GPTBKernel> gptb_;
@@ -204,9 +211,9 @@ public:
     // act_bias != nullptr: act is the raw output of the previous convolution; its bias and
     // ReLU are applied while the operand is gathered.  pooled: act is that output at twice the
     // height and width, and the 2x2 max pooling between the two layers happens on the way in too.
-    ConvKernel(int id, const std::string &name, const float *act, const float *act_bias, bool pooled, int H,
+    ConvKernel(VGG16 &task, int id, const std::string &name, const float *act, const float *act_bias, bool pooled, int H,
                int W, int C, int c_stride, int Cout, void *A, const void *Wt, float *out)
-        : GemmLayer(id, name, pad128(H * W), pad128(Cout), pad128(9 * C), A, Wt, out), act_(act),
+        : GemmLayer(task, id, name, pad128(H * W), pad128(Cout), pad128(9 * C), A, Wt, out), act_(act),
           act_bias_(act_bias), pool_(pooled ? 1 : 0), H_(H), W_(W), C_(C), cs_(c_stride), Cout_(Cout), A_(A)
     {
         this->mixable = 2;
@@ -269,26 +276,45 @@ public:
 
     void weightsHandedOut() override { direct_.reset(); }
     bool direct() const { return direct_ != nullptr; }
-    // the first layer, its image read from `image` and stored where the layer has it as a rule
-    void executeFrom(const float *image, float *keep, cudaStream_t stream) { launchDirect(image, keep, stream); }
+    // As part of a whole query.  raw: the output is written beside the activation.  image, keep: of the first layer, read
+    // from `image` and stored where the layer has it as a rule.
+    void executeInQuery(const float *image, float *keep, bool raw, cudaStream_t stream) { launchDirect(image, keep, raw, stream); }
+    // Whether the second layer can compute the first one's activation for itself: wherever a wavefront of it serves one slice of
+    // channels over segments of their own, the form its kernel for that has.  (All sizes have it there but some whose reduction is cut
+    // and that have enough tiles for a workgroup to take four slices.)
+    bool takesFirstLayer() const { return direct_ && key_.compare(0, 18, "conv3x3_direct_1_0") == 0 && threads_ <= 512; }
+    // ... and both of them, the second as part of a whole query without its raw output
+    void executeWithFirst(const ConvKernel &first, const float *image, float *keep, cudaStream_t stream)
+    {
+        DnnImage i{image, keep, first.direct_->weights, first.direct_->out.bias, first.direct_->chunks, (int)lds_};
+        DnnConv c = *direct_;
+        c.out.raw = nullptr;
+        void *args[] = {&i, &c};
+        const char *key = key_.size() > 18 ? "conv3x3_direct_image_low" : "conv3x3_direct_image";
+        TK_SAFE_CALL(tkLaunchKernel(fmap.at(key), dim3(grid_).raw(), dim3(threads_).raw(), args, lds_ + DNN_IMAGE_BYTES, stream));
+        first.next_->fresh.valid = false;
+        next_->fresh.valid = true;
+    }
 
 protected:
     void fused() override
     {
         if (next_) next_->fresh.valid = false;
     }
-    void executeImpl(cudaStream_t stream) override
+    void run(cudaStream_t stream) override
     {
         if (!direct_) {
             fused();
-            return GemmLayer::executeImpl(stream);
+            return GemmLayer::run(stream);
         }
         if (in_) in_->need(stream);
-        launchDirect(act_, nullptr, stream);
+        launchDirect(act_, nullptr, true, stream);
     }
-    void launchDirect(const float *image, float *keep, cudaStream_t stream)
+    void launchDirect(const float *image, float *keep, bool raw, cudaStream_t stream)
     {
-        void *image_args[] = {&image, &keep, direct_.get()}, *act_args[] = {direct_.get()};
+        DnnConv c = *direct_;
+        if (!raw) c.out.raw = nullptr;
+        void *image_args[] = {&image, &keep, &c}, *act_args[] = {&c};
         void **args = in_ ? act_args : image_args;
         TK_SAFE_CALL(tkLaunchKernel(fmap.at(key_), dim3(grid_).raw(), dim3(threads_).raw(), args, lds_, stream));
         next_->fresh.valid = true;
@@ -331,10 +357,10 @@ public:
     // padding) stay as allocated.
     // pool_W > 0: src is the raw output of the last convolution, [.][pool_W][pool_ld] with pool_C
     // channels, and the 2x2 max pooling in front of the classifier happens while the row is packed
-    FcKernel(int id, const std::string &name, const float *src, long src_stride, const float *src_bias,
+    FcKernel(VGG16 &task, int id, const std::string &name, const float *src, long src_stride, const float *src_bias,
              int src_relu, int in_features, int out_features, const void *Wt, void *X, float *out,
              int pool_W = 0, int pool_ld = 0, int pool_C = 0)
-        : GemmLayer(id, name, 128, pad128(out_features), pad128(in_features), X, Wt, out,
+        : GemmLayer(task, id, name, 128, pad128(out_features), pad128(in_features), X, Wt, out,
                     pad128(out_features) / TZ_REF_TILE),
           src_(src), stride_(src_stride), bias_(src_bias), relu_(src_relu), in_(in_features), out_(out_features),
           X_(X), poolW_(pool_W), poolLd_(pool_ld), poolC_(pool_C)
@@ -367,11 +393,11 @@ protected:
         if (inFresh_) inFresh_->valid = true;   // before() packed it
         if (outFresh_) outFresh_->valid = false;
     }
-    void executeImpl(cudaStream_t stream) override
+    void run(cudaStream_t stream) override
     {
         if (!direct_) {
             fused();
-            return GemmLayer::executeImpl(stream);
+            return GemmLayer::run(stream);
         }
         if (!inFresh_->holds()) before(stream);
         inFresh_->valid = true;
@@ -423,6 +449,8 @@ std::shared_ptr<StagingStream> stagingStream()
 
 }  // namespace
 
+namespace { constexpr size_t CONVOLUTIONS = 13; }
+
 struct VGG16::Impl {
     Buffers buffers;
     bool direct = false;            // layers run through the direct kernels
@@ -435,6 +463,9 @@ struct VGG16::Impl {
     int turn = 0;
     cudaStream_t lastStream = nullptr;   // the last query's
     tkEvent_t before = nullptr;          // recorded on the null stream for a query to wait for
+    bool stepped = false;                // since the last whole query the task has been used otherwise
+    bool watched = false;                // somebody has an address of a raw output, a bias or weights, or reads one
+    bool lean = false;                   // the last query has left out the raw outputs
     ~Impl()
     {
         for (tkEvent_t e : {over[0], over[1], before})
@@ -524,7 +555,7 @@ VGG16::VGG16(int taskId, const VGG16Options &o) : Task(taskId, "vgg16"), opt(o),
         void *operand = Abuf;
         if (C % 8 != 0)   // gathered, and only its data columns rewritten: needs zeros nobody else disturbs
             operand = zeroed(fl, (size_t)pad128(H * W) * Kp * 2);
-        auto *conv = new ConvKernel(id++, "Convolution_" + name, act, act_bias, pooled, H, W, C, ld, Cout, operand, Wt, out);
+        auto *conv = new ConvKernel(*this, id++, "Convolution_" + name, act, act_bias, pooled, H, W, C, ld, Cout, operand, Wt, out);
         addKernel(conv);
         if (direct) {
             // what the next layer reads: this layer's activation, pooled if a pooling follows, in a frame of
@@ -565,9 +596,9 @@ VGG16::VGG16(int taskId, const VGG16Options &o) : Task(taskId, "vgg16"), opt(o),
     float *o1 = devAlloc(fl, (size_t)128 * 4096), *o2 = devAlloc(fl, (size_t)128 * 4096);
     float *o3 = devAlloc(fl, (size_t)128 * pad128(opt.classes));
     // act is conv5_3's raw output; its pooling, bias and ReLU happen while fc1's input is packed
-    auto *fc1 = new FcKernel(id++, "Dot_fc1", act, 1, act_bias, 1, feat, 4096, W1, X1, o1, pooled ? unpooled_W : 0, ld, C);
-    auto *fc2 = new FcKernel(id++, "Dot_fc2", o1, 1, b1, 1, 4096, 4096, W2, X2, o2);
-    auto *fc3 = new FcKernel(id++, "Dot_fc3", o2, 1, b2, 1, 4096, opt.classes, W3, X3, o3);
+    auto *fc1 = new FcKernel(*this, id++, "Dot_fc1", act, 1, act_bias, 1, feat, 4096, W1, X1, o1, pooled ? unpooled_W : 0, ld, C);
+    auto *fc2 = new FcKernel(*this, id++, "Dot_fc2", o1, 1, b1, 1, 4096, 4096, W2, X2, o2);
+    auto *fc3 = new FcKernel(*this, id++, "Dot_fc3", o2, 1, b2, 1, 4096, opt.classes, W3, X3, o3);
     for (auto *fc : {fc1, fc2, fc3}) addKernel(fc);
     if (direct) {
         for (auto &a : impl->act) a.fresh.wholeQuery = &wholeQuery;
@@ -641,11 +672,45 @@ void VGG16::executeQuery(cudaStream_t stream)
         else if (stream) TK_SAFE_CALL(tkStreamWaitEvent(stream, m.before));
         if (stream || m.lastStream) TK_SAFE_CALL(tkStreamWaitEvent(stream, last));
         const WholeQuery whole(*this);
-        first->executeFrom(m.image[turn], m.input, stream);
-        for (size_t i = 1; i < kernels.size(); ++i) kernels[i]->execute(stream);
+        m.lean = !m.stepped && !m.watched;
+        size_t next = 1;
+        auto *second = static_cast<ConvKernel *>(kernels[1]);
+        if (m.lean && second->takesFirstLayer()) {
+            second->executeWithFirst(*first, m.image[turn], m.input, stream);
+            next = 2;
+        } else {
+            first->executeInQuery(m.image[turn], m.input, !m.lean, stream);
+        }
+        for (; m.lean && next < CONVOLUTIONS; ++next)
+            static_cast<ConvKernel *>(kernels[next])->executeInQuery(nullptr, nullptr, false, stream);
+        for (; next < kernels.size(); ++next) kernels[next]->execute(stream);
     }
     TK_SAFE_CALL(tkEventRecord(m.over[turn], stream));
     m.lastStream = stream;
+    m.stepped = false;
+}
+
+// The queries' kernels read each other's activations, every layer's in a buffer of its own, so what a query left out can be
+// had afterwards from what it kept: its image and the activations, which stay as they are until the next query.  On the
+// staging stream, behind the query, and waited for: the caller's stream may be recording.
+void VGG16::complete() const
+{
+    Impl &m = *impl;
+    if (!m.lean) return;
+    m.lean = false;
+    const int turn = m.turn ^ 1;   // the last query's
+    const cudaStream_t stream = m.staging->stream;
+    TK_SAFE_CALL(tkStreamWaitEvent(stream, m.over[turn]));
+    for (size_t i = 0; i < CONVOLUTIONS; ++i)
+        static_cast<ConvKernel *>(kernels[i])->executeInQuery(m.image[turn], nullptr, true, stream);
+    TK_SAFE_CALL(tkStreamSynchronize(stream));
+}
+
+void VGG16::layerByItself()
+{
+    if (wholeQuery) return;
+    complete();
+    impl->stepped = true;
 }
 
 VGG16::~VGG16()
@@ -655,6 +720,7 @@ VGG16::~VGG16()
 
 void VGG16::initExecution()
 {
+    layerByItself();
     TK_SAFE_CALL(tkMemcpy(Input[0], InputHost[0], (size_t)InputSize[0], TK_MEMCPY_H2D));
 }
 
@@ -664,15 +730,25 @@ const float *VGG16::logits(long *stride) const
     return impl->logits;
 }
 
-void VGG16::weightsHandedOut(int layer) { static_cast<GemmLayer *>(kernels.at(layer))->weightsHandedOut(); }
+void VGG16::weightsHandedOut(int layer)
+{
+    this->layer(layer);
+    static_cast<GemmLayer *>(kernels.at(layer))->weightsHandedOut();
+}
 
 void VGG16::resultHandedOut(int layer)
 {
+    this->layer(layer);
     if (layer < 13) impl->act[layer].fresh.exposed = true;
     else if (layer < 15) impl->fcInput[layer - 12].exposed = true;
 }
 
-const VGG16::Act &VGG16::layer(int idx) const { return impl->convOut.at(idx); }
+const VGG16::Act &VGG16::layer(int idx) const
+{
+    complete();
+    impl->watched = true;
+    return impl->convOut.at(idx);
+}
 
 VGG16::Act VGG16::activation(int conv_index)
 {

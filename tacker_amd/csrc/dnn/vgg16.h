@@ -58,7 +58,12 @@ public:
     // and tzgemm from now on
     struct Act { float *ptr; int H, W, C, ld; void *weights; float *bias; int Np, Kp; };
     Act activation(int conv_index);
-    const Act &layer(int idx) const;     // the same, handed to nobody
+    const Act &layer(int idx) const;     // the same, only read
+    // A whole query after a whole query leaves out what nobody reads: the convolutions' raw outputs, and the first one's launch.
+    // Before anything else is done with the task -- a layer launched by itself, an address handed out, another image
+    // staged -- complete() runs the convolutions of the last query once more, with their raw outputs.
+    void complete() const;
+    void layerByItself();                // a layer is launched, and not as part of a whole query
     VGG16Options opt;
     struct Impl;
     std::unique_ptr<Impl> impl;

@@ -7,8 +7,8 @@
 // same quarters of the same parts, ((w0 + w1) + w2) + w3, parts in order.
 //
 // Data.  An activation is f16 NHWC with a border of one zero pixel, [H + 2][W + 2][C], written by the layer before
-// with bias, ReLU and -- where a pooling follows -- the 2x2 maximum applied; beside it every layer leaves its raw
-// 1.1 * A * B^T in fp32 as the operand builders expect it.  Weights are laid out once, at the task's creation, in the
+// with bias, ReLU and -- where a pooling follows -- the 2x2 maximum applied; beside it a layer leaves its raw
+// 1.1 * A * B^T in fp32 as the operand builders expect it, where somebody may read it (54 MB a query at 224 x 224, 20 us of it).  Weights are laid out once, at the task's creation, in the
 // order the matrix instruction takes them (pack_weight_fragments): fragment (16 output channels, 32 k) is
 // 1 KiB in a row, lane l's 16 bytes at 16 l.
 #include <hip/hip_runtime.h>
@@ -24,6 +24,8 @@ typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) char lds_char;
 typedef __attribute__((address_space(3))) const half8_t lds_half8;
+typedef __attribute__((address_space(3))) half4_t lds_half4;
+typedef __attribute__((address_space(3))) _Float16 lds_half;
 typedef __attribute__((address_space(3))) float4_t lds_float4;
 typedef __attribute__((address_space(3))) float lds_float;
 
@@ -95,7 +97,7 @@ __device__ __forceinline__ void dnn_finish(lds_float4 *tile, int partials, bool 
         v *= TZ_ALPHA;
         const int y = y0 + dnn_tile_y(p), x = x0 + dnn_tile_x(p), n = n0 + 4 * q;
         if (y < o.H && x < o.W) {
-            *reinterpret_cast<float4_t *>(o.raw + (size_t)(y * o.W + x) * o.ld + n) = v;
+            if (o.raw) *reinterpret_cast<float4_t *>(o.raw + (size_t)(y * o.W + x) * o.ld + n) = v;
             if (!o.pool)
                 *reinterpret_cast<half4_t *>(reinterpret_cast<_Float16 *>(o.act) +
                                              (size_t)((y + o.border) * o.act_pitch + x + o.border) * o.act_C + n) =
@@ -141,6 +143,64 @@ __device__ __forceinline__ int dnn_tile_of(int block, int tiles)
 
 using namespace tk;
 
+// The input patch of a tile of ROWS rows of the second convolution, ROWS + 2 x 10 pixels of the first one's activation, computed
+// from the image: groups of 16 pixels, 27 k in one matrix instruction for 16 channels each, rounded as the first convolution's own
+// kernel rounds.  The image's ROWS + 4 x 12 pixels come to LDS once, in f16, where a pixel's k are three runs of nine values.
+// The tiles of a layer compute 1.6 times its pixels that way (1.9 with four rows); a launch, and its activation written and read again, are gone.
+// us, both layers: 14.0 at 224 x 224 and 6.1 at 64 x 96, where the first one took 8.6 and 5.4 and the second one 12.6 and 4.9 (17.6 and 9.8
+// without the raw outputs).  With every lane gathering its k from the image in memory, 14.4 and 6.9.
+template <int ROWS>
+__device__ __forceinline__ void dnn_patch_of_image(const DnnImage &f, lds_char *lds, lds_half *image, int y0, int x0, int H, int W,
+                                                   bool keeps, int wave, int waves, int lane)
+{
+    constexpr int PIXELS = (ROWS + 2) * DNN_PATCH, GROUPS = (PIXELS + 15) / 16, ROW = 3 * DNN_IMAGE_SIDE;
+    const int r = lane & 15, kq = lane >> 4;
+    const half8_t *weights = reinterpret_cast<const half8_t *>(f.weights) + lane;
+    half8_t w[4];
+    float4_t bias[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        w[j] = weights[(size_t)(j * f.chunks * 2) * 64];
+        bias[j] = *reinterpret_cast<const float4_t *>(f.bias + 16 * j + 4 * kq);
+    }
+    for (int i = (int)threadIdx.x; i < (ROWS + 4) * ROW; i += 64 * waves) {
+        const int row = i / ROW, column = i - row * ROW;
+        const int y = y0 - 2 + row, at = 3 * (x0 - 2) + column;
+        const bool there = y >= 0 && y < H && at >= 0 && at < 3 * W;
+        const float v = there ? f.image[y * 3 * W + at] : 0.0f;
+        image[i] = (_Float16)v;
+        if (keeps && there && row >= 2 && row < ROWS + 2 && column >= 6 && column < 6 + 3 * DNN_TILE) f.keep[y * 3 * W + at] = v;
+    }
+    int tap_at[8];   // where this lane's eight k (of 32; the last 5 are padding) of a pixel lie
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const int k = min(8 * kq + e, 26);
+        tap_at[e] = k / 9 * ROW + k % 9;
+    }
+    __syncthreads();
+    for (int group = wave; group < GROUPS; group += waves) {
+        const int p = min(16 * group + r, PIXELS - 1);
+        const int py = (p * 205) >> 11, px = p - py * DNN_PATCH;   // p / 10 for p < 1024
+        half8_t a;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) a[e] = image[py * ROW + 3 * px + tap_at[e]];
+        if (kq == 3) a[3] = a[4] = a[5] = a[6] = a[7] = (_Float16)0.0f;
+        const int y = y0 + py - 1, x = x0 + px - 1;
+        const bool inside = y >= 0 && y < H && x >= 0 && x < W;   // the border is zeros
+        const int key = ((px >> 1) + 4 * (py & 1)) & 7;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float4_t zero = {0.f, 0.f, 0.f, 0.f};
+            float4_t raw = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[j], a, zero, 0, 0, 0);
+            raw *= TZ_ALPHA;
+            half4_t h = dnn_activate(raw, bias[j]);
+            if (!inside) h = half4_t{0, 0, 0, 0};
+            // (lanes past the last pixel compute and write it again)
+            *(lds_half4 *)(lds + p * 128 + (((2 * j + (kq >> 1)) ^ key) << 4) + 8 * (kq & 1)) = h;
+        }
+    }
+}
+
 // 3x3 / pad 1 / stride 1 convolution of an activation with C a multiple of 64 channels.  A workgroup computes an 8 x 8
 // pixel tile by 16 * ct_count output channels; wavefront (cp, kw) of it 16 * NT channels over a run of the reduction:
 // one segment, a whole part (PART: its four segments one after the other, added as tzgemm adds them), or all of it
@@ -163,8 +223,8 @@ using namespace tk;
 // fragments are read from LDS while the matrix units work on those of the step before.  us a layer of VGG16 at 224 x 224,
 // first through the operand in memory and tzgemm, then reading its fragments where it uses them, now: conv2_2 26, 10.5, 9.5,
 // conv3_2 21, 9.5, 8.8, conv4_2 23, 9.7, 9.1, conv5_1 18, 8.4, 6.6; at 64 x 96 conv4_2 8.6, 6.8, conv5_1 8.2, 6.3 (the last two each).
-template <int NT, bool PART, int GROUPS>
-__device__ __forceinline__ void conv3x3_direct(const DnnConv &c, char *lds_generic)
+template <int NT, bool PART, bool IMAGE, int GROUPS>
+__device__ __forceinline__ void conv3x3_direct(const DnnConv &c, const DnnImage &first_layer, char *lds_generic)
 {
     lds_char *const lds = (lds_char *)lds_generic;
     const int lane = (int)threadIdx.x & 63;
@@ -189,8 +249,9 @@ __device__ __forceinline__ void conv3x3_direct(const DnnConv &c, char *lds_gener
 
     const int quads = 4 * c.ct_count;
     const float4_t bias = dnn_bias(c.out, group * c.ct_count * 16, quads);
+    if (IMAGE) dnn_patch_of_image<2 * GROUPS>(first_layer, lds, (lds_half *)(lds + first_layer.lds), y0, x0, H, W, group == 0, wave, waves, lane);
     // the patch: pieces of 8 pixels, every plane of a piece by one wavefront; what lies below the image's border is left out
-    const int pieces = (min(2 * GROUPS + 2, H + 2 - y0) * DNN_PATCH + 7) >> 3;
+    const int pieces = IMAGE ? 0 : (min(2 * GROUPS + 2, H + 2 - y0) * DNN_PATCH + 7) >> 3;
     const unsigned lds_base = (unsigned)(size_t)lds;
     for (int piece = wave; piece < pieces; piece += waves) {
         const int p = min(8 * piece + (lane >> 3), DNN_PATCH * DNN_PATCH - 1);
@@ -217,9 +278,13 @@ __device__ __forceinline__ void conv3x3_direct(const DnnConv &c, char *lds_gener
 #pragma unroll
     for (int u = 0; u < RING; ++u) fetch(b[u], min(first + u, final_chunk));
     __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_waitcnt(DNN_VMCNT_IMM(2 * NT * RING));
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
+    if (IMAGE) {
+        __syncthreads();
+    } else {
+        __builtin_amdgcn_s_waitcnt(DNN_VMCNT_IMM(2 * NT * RING));
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    }
 
     const int r = lane & 15;
     const int tx = dnn_tile_x(r), ty = dnn_tile_y(r);
@@ -306,7 +371,7 @@ __device__ __forceinline__ void conv3x3_direct(const DnnConv &c, char *lds_gener
     extern "C" __global__ __launch_bounds__(THREADS_) void NAME_(DnnConv c)                                            \
     {                                                                                                                 \
         extern __shared__ __align__(16) char conv_lds[];                                                              \
-        conv3x3_direct<NT_, PART_, GROUPS_>(c, conv_lds);                                                              \
+        conv3x3_direct<NT_, PART_, false, GROUPS_>(c, DnnImage{}, conv_lds);                                           \
     }
 DNN_CONV_KERNEL(conv3x3_direct_1_0, 1, false, 4, 1024)
 DNN_CONV_KERNEL(conv3x3_direct_1_1, 1, true, 4, 512)
@@ -315,6 +380,16 @@ DNN_CONV_KERNEL(conv3x3_direct_2_0, 2, false, 4, 512)
 // 104 KB of patch at 512 channels, twice the workgroups (conv5_1 at 224 x 224 8.0 -> 6.7 us, conv4_2 at 64 x 96 9.0 -> 7.3).
 DNN_CONV_KERNEL(conv3x3_direct_1_0_low, 1, false, 2, 1024)
 DNN_CONV_KERNEL(conv3x3_direct_1_1_low, 1, true, 2, 512)
+// the first two convolutions, the first one's activation as patches in LDS only
+#define DNN_IMAGE_KERNEL(NAME_, GROUPS_)                                                                               \
+    extern "C" __global__ __launch_bounds__(512, 4) void NAME_(DnnImage first_layer, DnnConv c)                        \
+    {                                                                                                                 \
+        extern __shared__ __align__(16) char conv_lds[];                                                              \
+        conv3x3_direct<1, false, true, GROUPS_>(c, first_layer, conv_lds);                                             \
+    }
+DNN_IMAGE_KERNEL(conv3x3_direct_image, 4)
+DNN_IMAGE_KERNEL(conv3x3_direct_image_low, 2)
+
 // The first convolution: the image, [H][W][3] fp32, 27 k in one matrix instruction.  A workgroup computes an 8 x 8 pixel
 // tile by 64 channels, wavefront g the pixel group g; a lane gathers its 8 k (of 32; the last 5 are padding) of its pixel.
 // keep: null, or where the image is stored as well.
@@ -503,6 +578,8 @@ extern "C" void tk_register_dnn_kernels(tk_kernel_insert_fn insert, void *ctx)
     insert("conv3x3_direct_2_0", (const void *)conv3x3_direct_2_0, ctx);
     insert("conv3x3_direct_1_0_low", (const void *)conv3x3_direct_1_0_low, ctx);
     insert("conv3x3_direct_1_1_low", (const void *)conv3x3_direct_1_1_low, ctx);
+    insert("conv3x3_direct_image", (const void *)conv3x3_direct_image, ctx);
+    insert("conv3x3_direct_image_low", (const void *)conv3x3_direct_image_low, ctx);
     insert("conv3x3_image", (const void *)conv3x3_image, ctx);
     insert("fc_direct_1", (const void *)fc_direct_1, ctx);
     insert("fc_direct_2", (const void *)fc_direct_2, ctx);

@@ -83,6 +83,56 @@ bool many_classes(int classes)
     return same(read(task.logits(nullptr), classes), read(plain.logits(nullptr), classes));
 }
 
+// What a whole query after a whole query leaves out is there as soon as anybody can see it: every raw output, behind two queries
+// of different images, as the layers through their operands and tzgemm leave it.  After the queries: nothing, another image staged, a
+// layer run by itself, its addresses handed out before or between the queries.
+bool raw_outputs_after_queries(int height, int width)
+{
+    VGG16Options opt;
+    opt.height = height, opt.width = width;
+    const auto image = [](VGG16 &t, float factor) {
+        float *host = static_cast<float *>(t.InputHost[0]);
+        for (size_t i = 0; i < t.InputSize[0] / sizeof(float); ++i) host[i] = factor * (float)((i * 2654435761u) % 1000) / 1000.0f;
+    };
+    enum { Nothing, Staged, Layer, Before, Between };
+    for (int use : {Nothing, Staged, Layer, Before, Between}) {
+        VGG16 task(1, opt), plain(2, opt);
+        use_tzgemm(plain);
+        if (use == Before) task.resultHandedOut(3);
+        for (float factor : {1.0f, 0.5f, 0.75f}) {
+            for (VGG16 *t : {&task, &plain}) {
+                image(*t, factor);
+                t->executeQuery(nullptr);
+            }
+            if (use == Between && factor == 0.5f) task.resultHandedOut(9);
+        }
+        if (use == Staged)
+            for (VGG16 *t : {&task, &plain}) {
+                image(*t, 0.25f);
+                t->initExecution();
+                t->kernels[0]->execute((cudaStream_t) nullptr);
+            }
+        if (use == Layer)
+            for (int i : {7, 1, 0, 14, 12})
+                for (VGG16 *t : {&task, &plain}) t->kernels[i]->execute((cudaStream_t) nullptr);
+        for (int again = 0; again < 2; ++again) {
+            for (int i = 0; i < 16; ++i) {
+                const VGG16::Act &a = task.layer(i), &b = plain.layer(i);
+                const size_t n = i < 13 ? size_of(a) : (size_t)a.C;
+                if (!same(read(a.ptr, n), read(b.ptr, n))) {
+                    printf("%d x %d, use %d, round %d: layer %d differs\n", height, width, use, again, i);
+                    return false;
+                }
+            }
+            for (VGG16 *t : {&task, &plain}) {   // from now on every query leaves them
+                image(*t, 0.6f);
+                t->executeQuery(nullptr);
+            }
+        }
+    }
+    return true;
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -93,6 +143,8 @@ int main(int argc, char **argv)
     if (!strcmp(check, "raw")) ok = written_between_layers(false, false) && written_between_layers(true, false);
     else if (!strcmp(check, "bias")) ok = written_between_layers(false, true) && written_between_layers(true, true);
     else if (!strcmp(check, "classes")) ok = many_classes(1000) && many_classes(8192) && many_classes(9000);
+    else if (!strcmp(check, "lean"))
+        ok = raw_outputs_after_queries(32, 32) && raw_outputs_after_queries(64, 96) && raw_outputs_after_queries(128, 160);
     else return 2;
     printf("%s %s\n", check, ok ? "ok" : "FAILED");
     return ok ? 0 : 1;

@@ -729,3 +729,9 @@ def test_checks_of_the_cxx_interface(check):
     program = os.path.join(os.path.dirname(ta.LIB_PATH), "task_checks")
     p = subprocess.run([program, check], capture_output=True, text=True, timeout=100)
     assert p.returncode == 0 and f"{check} ok" in p.stdout, p.stdout[-2000:] + p.stderr[-2000:]
+
+
+def test_what_a_query_leaves_out_is_there_once_somebody_looks():
+    # raw outputs behind two queries: with nothing done since, another image staged, layers run by themselves, an address handed
+    # out before and between the queries
+    test_checks_of_the_cxx_interface("lean")
