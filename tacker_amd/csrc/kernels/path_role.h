@@ -20,17 +20,15 @@
 //  * every column is updated in every row without asking whether it still takes part -- a column
 //    outside the shrinking pyramid holds a value nobody reads, since a column that takes part in row
 //    i only reads columns that took part in row i - 1.
-//  * the clamping at the grid's two edges is a maximum: a column off the grid is held at INT_MAX, which
-//    its neighbour's minimum then ignores -- min(prev, prev, right) and min(INT_MAX, prev, right) are one
-//    value.  min3, add, max for a column: 14 instructions a row with the two shifts.
-//  * a row of the wall is one 16-byte load a lane, AHEAD rows ahead of the row being evaluated.  The
-//    lane's four columns are read as they lie, also where the row ends between them: the elements beyond
-//    it are the neighbouring rows', inside the array for every row but the first and the last one the
-//    launch reads, and belong to columns off the grid.  Those two rows are read column by column, from
-//    indices clamped to the grid.
-// 1200 columns x 125 rows (200 windows on 200 CUs): 9 us, of which 3.4 are the launch; 25 us with two selects a
-// column for the clamping and four 4-byte loads a lane and row, 32 instructions a row.  20000 x 122 rows (1667
-// windows): 24 against 84 us.
+//  * the window is moved until all of it lies on the grid (path_window_on_grid): its columns off the grid are
+//    not read, and the wavefront has as many others instead.  The grid's edge is then the wavefront's, where the shift across
+//    lanes leaves the neighbour at INT_MAX, which the minimum ignores -- min(prev, prev, right) and min(INT_MAX, prev,
+//    right) are one value.  Nothing is clamped: a min3 and an add a column and the two shifts, 10 instructions a row.
+//  * a row of the wall is one 16-byte load a lane, AHEAD rows ahead of the row being evaluated, from a scalar row
+//    pointer that two instructions move on; whether there is such a row is asked for the last 2 AHEAD rows only.
+// 1200 columns x 125 rows (200 windows on 200 CUs): 9.05 -> 6.5 us; 20000 x 125 (3292 windows) 44.4 -> 26.9, 20000 x 118 (1000)
+// 13.6 -> 12.7, where a maximum a column held those off the grid at INT_MAX and every fetch asked for its row (14 vector
+// instructions a row and 6 scalar ones).  Narrower grids keep that form (path_window).
 #pragma once
 #include "role_common.h"
 #include "../header/path_header.h"
@@ -50,9 +48,81 @@ __device__ __forceinline__ int path_from_lane_above(int v)
     return __builtin_amdgcn_mov_dpp(v, 0x130 /* wave_shl:1 */, 0xf, 0xf, true);
 }
 
-typedef int path_int4 __attribute__((ext_vector_type(4), aligned(4)));   // a lane's columns start anywhere
+__device__ __forceinline__ int path_min3(int a, int b, int c)
+{
+    int v;   // (left to itself, the compiler shares minima of two between columns: five instructions for four)
+    asm("v_min3_i32 %0, %1, %2, %3" : "=v"(v) : "v"(a), "v"(b), "v"(c));
+    return v;
+}
 
-// one position, whole pyramid; lane = lane of the wavefront
+typedef int path_int4 __attribute__((ext_vector_type(4), aligned(4)));   // a lane's columns start anywhere
+typedef __attribute__((address_space(1))) path_int4 path_global_int4;
+typedef __attribute__((address_space(1))) char path_global_char;
+
+// One position, whole pyramid, on a grid of at least PATH_BLOCK_SIZE columns; lane = lane of the wavefront.  The wavefront's
+// columns are the window moved until it lies on the grid.  (Columns of the window that are not on the grid nobody reads, and
+// those the wavefront has instead are right for longer than the pyramid's.)
+__device__ __forceinline__ void path_window_on_grid(int iteration, const int *__restrict__ gpuWall,
+                                                    const int *__restrict__ gpuSrc, int *__restrict__ gpuResults, int cols,
+                                                    int startStep, int border, int bx, int lane)
+{
+    constexpr int C = PATH_COLS_PER_LANE, AHEAD = PATH_ROWS_AHEAD;
+    static_assert(C == 4 && C * TK_WAVE_SIZE == PATH_BLOCK_SIZE, "a lane's columns of a row are one 16-byte load");
+    const int blkX = (PATH_BLOCK_SIZE - iteration * PATH_HALO * 2) * bx - border;
+    const int first = __builtin_amdgcn_readfirstlane(min(max(blkX, 0), cols - PATH_BLOCK_SIZE));
+    unsigned at = (unsigned)(C * lane) * (unsigned)sizeof(int);
+    size_t ahead = reinterpret_cast<size_t>(gpuWall + (long long)cols * startStep + first);   // the row the next fetch takes
+    const size_t row_bytes = (size_t)cols * sizeof(int);
+    path_int4 wall[AHEAD], prev = *reinterpret_cast<const path_int4 *>(reinterpret_cast<const char *>(gpuSrc + first) + at);
+    const auto fetch = [&](path_int4 &w, size_t to_next) {
+        asm volatile("" : "+s"(ahead), "+v"(at));   // (a scalar pointer and a lane's offset, not a 64-bit vector address)
+        w = *(const path_global_int4 *)((const path_global_char *)ahead + at);
+        ahead += to_next;
+    };
+    // the neighbouring lanes' columns; beyond the wavefront's ends, which keep what they had, INT_MAX: the grid's edge, or a
+    // column outside the pyramid
+    int left = 0x7fffffff, right = 0x7fffffff;
+    const auto step = [&](const path_int4 &w) {
+        left = __builtin_amdgcn_update_dpp(left, prev[3], 0x138 /* wave_shr:1 */, 0xf, 0xf, false);
+        right = __builtin_amdgcn_update_dpp(right, prev[0], 0x130 /* wave_shl:1 */, 0xf, 0xf, false);
+        const int m1 = path_min3(prev[0], prev[1], prev[2]), m2 = path_min3(prev[1], prev[2], prev[3]);
+        const int m0 = path_min3(left, prev[0], prev[1]), m3 = path_min3(prev[2], prev[3], right);
+        // (wraps where the sum does not fit, as the reference's does)
+        prev[0] = (int)((unsigned)m0 + (unsigned)w[0]);
+        prev[3] = (int)((unsigned)m3 + (unsigned)w[3]);
+        prev[1] = (int)((unsigned)m1 + (unsigned)w[1]);
+        prev[2] = (int)((unsigned)m2 + (unsigned)w[2]);
+    };
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) fetch(wall[u], u + 1 < iteration ? row_bytes : 0);   // (the last row again where there is no other)
+    int row = 0;
+    for (; row + 2 * AHEAD <= iteration; row += AHEAD) {   // no fetch asks whether there is a row
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) {
+            step(wall[u]);
+            fetch(wall[u], row_bytes);
+            __builtin_amdgcn_sched_barrier(0);   // (eight steps and then eight fetches would wait for all of them)
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+        if (row + u < iteration) step(wall[u]);
+        if (row + AHEAD + u < iteration) fetch(wall[u], row_bytes);
+    }
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u)
+        if (row + AHEAD + u < iteration) step(wall[u]);
+    // the columns that took part in the last row: the middle of the window, where it is on the grid
+#pragma unroll
+    for (int k = 0; k < C; ++k) {
+        const int x = first + C * lane + k, tx = x - blkX;
+        if (tx >= iteration && tx <= PATH_BLOCK_SIZE - 1 - iteration) gpuResults[x] = prev[k];
+    }
+}
+
+// The same on a grid narrower than the window.  A column off the grid is held at INT_MAX by a maximum, and the first and the last row
+// are read column by column, from indices clamped to the grid: the lane's four columns are read as they lie, also where
+// the row ends between them, and the elements beyond it are the neighbouring rows', inside the array for every other row.
 __device__ __forceinline__ void path_window(int iteration, const int *__restrict__ gpuWall,
                                             const int *__restrict__ gpuSrc, int *__restrict__ gpuResults, int cols,
                                             int startStep, int border, int bx, int lane)
@@ -166,7 +236,10 @@ __device__ __forceinline__ void path_role(int iteration, const int *__restrict__
     const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
     for (long long pos = (long long)start + role_block + (long long)role_blocks * wave; pos < end;
          pos += (long long)role_blocks * waves)
-        path_window(iteration, gpuWall, gpuSrc, gpuResults, cols, startStep, border, (int)pos, lane);
+        if (cols >= PATH_BLOCK_SIZE)   // uniform
+            path_window_on_grid(iteration, gpuWall, gpuSrc, gpuResults, cols, startStep, border, (int)pos, lane);
+        else
+            path_window(iteration, gpuWall, gpuSrc, gpuResults, cols, startStep, border, (int)pos, lane);
 }
 
 }  // namespace tk

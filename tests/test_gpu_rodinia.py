@@ -173,6 +173,21 @@ def test_path_ring_of_rows_and_edges_of_the_grid(cols, iteration):
     assert np.array_equal(host(out), oracle.path(iteration, wall, src))
 
 
+@pytest.mark.parametrize("cols", [255, 256, 258, 263, 511, 1001])
+@pytest.mark.parametrize("iteration", [1, 7, 8, 9, 15, 16, 17, 24, 31, 127])
+def test_path_windows_moved_onto_the_grid(cols, iteration):
+    # grids the window just fits and somewhat wider ones, rows around once and twice the depth of the ring, sums that wrap,
+    # positions past the grid; the wall is the whole allocation
+    rng = np.random.default_rng(cols * 1000 + iteration)
+    wall = rng.integers(-2 ** 31, 2 ** 31, (iteration, cols), dtype=np.int64).astype(np.int32)
+    src = rng.integers(-2 ** 31, 2 ** 31, cols, dtype=np.int64).astype(np.int32)
+    want = oracle.path(iteration, wall, src)
+    for end in (None, ta.path_blocks(cols, iteration) + 3):
+        out = torch.full((cols,), -1, dtype=torch.int32, device="cuda:0")
+        ta.gptb_path(iteration, dev(wall), dev(src), out, end=end)
+        assert np.array_equal(host(out), want)
+
+
 def test_path_the_last_windows_of_a_very_wide_grid():
     # rows of more than 2^30 columns (the kernel launched by its handle: the entry points take walls of less than 2^31
     # cells): the last windows' columns, of which a byte offset from the row's start needs 33 bits
