@@ -17,6 +17,7 @@ public:
     void WARNING(const std::string &message) { log(LogLevel::WARNING, message); }
     [[noreturn]] void ERROR(const std::string &message);
     void DEBUG(const std::string &message);
+    bool debugging() const { return debugOn; }   // whether DEBUG prints: for callers that would put a message together for nothing
     void setConsole(bool on) { log2Console = on; }
 
 private:

@@ -17,9 +17,15 @@ namespace tkjson {
 const Value *Value::find(const std::string &key) const
 {
     if (kind != Object) return nullptr;
-    for (auto &m : members)
-        if (m.first == key) return &m.second;
-    return nullptr;
+    const auto place = places.find(key);
+    return place == places.end() ? nullptr : &members[place->second].second;
+}
+
+Value &Value::add(std::string key, Value value)
+{
+    places.emplace(key, members.size());   // (of a key twice, the first is found)
+    members.emplace_back(std::move(key), std::move(value));
+    return members.back().second;
 }
 
 namespace {
@@ -84,7 +90,7 @@ struct Parser {
                 ws();
                 if (i >= s.size() || s[i] != ':') fail("expected ':'");
                 ++i;
-                v.members.emplace_back(std::move(key), value());
+                v.add(std::move(key), value());
                 ws();
                 if (i < s.size() && s[i] == ',') { ++i; continue; }
                 if (i < s.size() && s[i] == '}') { ++i; break; }
@@ -192,8 +198,7 @@ void add_kernel_info(const std::string &kernel_name, const std::string &key, con
     if (ptr.kind != tkjson::Value::Object) ptr.kind = tkjson::Value::Object;
     tkjson::Value *k = const_cast<tkjson::Value *>(ptr.find(kernel_name));
     if (!k) {
-        ptr.members.emplace_back(kernel_name, tkjson::Value());
-        k = &ptr.members.back().second;
+        k = &ptr.add(kernel_name, tkjson::Value());
         k->kind = tkjson::Value::Object;
     }
     tkjson::Value num;
@@ -202,7 +207,7 @@ void add_kernel_info(const std::string &kernel_name, const std::string &key, con
     num.text = std::to_string(value);
     tkjson::Value *slot = const_cast<tkjson::Value *>(k->find(key));
     if (slot) *slot = num;
-    else k->members.emplace_back(key, num);
+    else k->add(key, num);
 }
 
 static void write_value(std::ostream &os, const tkjson::Value &v, int indent)
