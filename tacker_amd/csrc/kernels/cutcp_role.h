@@ -17,17 +17,18 @@
 //  * Atoms.  The neighbour list names every bin that may matter to some region: 335 bins, 1340 atoms at 4 an
 //    occupied bin, of which 450 are within 12 Angstroms of a point and 725 of some point of a half region.  A
 //    wavefront therefore looks at 64 slots (8 bins) at a time, a lane each: an atom that can reach none of the
-//    wavefront's points is dropped -- an exact zero is all it would have added -- and the others are packed, in
-//    order, into a list in LDS.
+//    wavefront's points is dropped -- an exact zero is all it would have added -- and the others are appended, in
+//    order, to a list in LDS, of which whole groups of 4 are used; what is left over waits for the next 64 slots.  Looking
+//    through 64 slots is 60 instructions, none of them a 32-bit product: the list's entries are walked with a counter.
 //  * An atom.  It is read back from that list with one 16-byte broadcast read into vector registers (an
 //    instruction with a scalar register among its operands takes 4.4 cycles of a SIMD, one without 2.3), and a
 //    point takes 5 such instructions and the reciprocal square root: where inv_cutoff2 is 1 / cutoff2 the cutoff
 //    is the clamp of s to [0, 1], a modifier of the instruction that computes it, instead of a comparison and
 //    an execution mask.
 // The atoms' order, and so every point's sum, is the same in every form of the kernel.
-// 208^3 lattice, two layers of regions: 136 us, 26 layers 1.46 ms; 290 us and 3.07 ms with every atom of the list by scalar loads and
-// a branch for each point.  Where inv_cutoff2 is not 1 / cutoff2 every point walks the list by itself: 185 us, 2.05 ms.
-// (By counters the vector units issue all the time, 1.16 in the units in which a kernel that keeps all SIMDs busy reads 1.)
+// 208^3 lattice, two layers of regions: 123 us, 26 layers 1.32 ms; 136 us and 1.44 ms with every batch filled up to whole groups
+// (a twelfth of the atoms) and the place in the list divided anew for each, in 95 instructions with five 32-bit products at a quarter of
+// the rate.  Where inv_cutoff2 is not 1 / cutoff2 every point walks the list by itself: 169 us, 1.86 ms (185, 2.01).
 #pragma once
 #include <cfloat>
 
@@ -45,6 +46,8 @@ typedef __attribute__((address_space(3))) float4_t cutcp_lds_float4;
 
 #define CUTCP_GROUP 4   // atoms read from the list at a time
 #define CUTCP_BATCH_BINS (TK_WAVE_SIZE / BIN_DEPTH)   // bins whose slots a wavefront looks at at a time
+#define CUTCP_RING (2 * TK_WAVE_SIZE)                 // atoms the list in LDS holds: those left over of less than a group, and 64
+static_assert(CUTCP_NBR_CHUNK >= 2 * CUTCP_BATCH_BINS, "a part of several is no shorter than a batch");
 
 // The neighbour list dealt to `parts` parts: part p holds the entries p, p + parts, p + 2 parts, ... (every part a
 // sample of the whole neighbourhood, so that parts cost the same wherever the atoms are).  Walked part by part
@@ -60,22 +63,36 @@ struct CutcpWalk {
         inv_each1 = 1.0f / (float)(each + 1);
     }
     __device__ __forceinline__ int begin_of(int part) const { return part * each + min(part, more); }
-    __device__ __forceinline__ int entry_at(int place) const
+    // the entry at a place, as part and number within it
+    struct Entry {
+        int part, within;
+    };
+    __device__ __forceinline__ Entry entry_at(int place) const
     {
         // divisions of numbers below 2^12 by numbers below 2^11: exact with the half added
         const int split = more * (each + 1);
         const bool first = place < split;
         const int f = first ? place : place - split;
         const int part = (int)(((float)f + 0.5f) * (first ? inv_each1 : inv_each));
-        return part + (first ? 0 : more) + (f - part * (first ? each + 1 : each)) * parts;
+        return Entry{part + (first ? 0 : more), f - part * (first ? each + 1 : each)};
     }
+    // ... a batch further (past the last one: any entry)
+    __device__ __forceinline__ void advance(Entry &e) const
+    {
+        e.within += CUTCP_BATCH_BINS;
+        const int entries = each + (e.part < more ? 1 : 0);
+        const bool next = e.within >= entries;
+        e.within -= next ? entries : 0;
+        e.part += next ? 1 : 0;
+    }
+    __device__ __forceinline__ int number_of(const Entry &e) const { return min(e.part + __mul24(e.within, parts), len - 1); }
 };
 
 // The piece `sub` of half `half` of region (xr, yr, zr): the reference's threads 64 half + lane, points e = PTS sub ..
 // PTS sub + PTS - 1 of each, over parts [part_begin, part_end) of the neighbour list.  A range that does not start
 // with part 0 goes on from the energies in memory, where the range before it left them (a float stored and reloaded
 // is unchanged, so consecutive ranges give the bits of one walk through all parts).  CLAMP: the cutoff is the clamp
-// of s.  stage: 64 x 16 bytes of LDS, this wavefront's own.
+// of s.  stage: CUTCP_RING x 16 bytes of LDS, this wavefront's own.
 template <int PTS, bool CLAMP>
 __device__ __forceinline__ void cutcp_piece(int binDim_x, int binDim_y, const float *binZeroAddr, float h, float cutoff2,
                                             float inv_cutoff2, float *regionZeroAddr, int gdx, int gdy, int xr, int yr,
@@ -105,20 +122,30 @@ __device__ __forceinline__ void cutcp_piece(int binDim_x, int binDim_y, const fl
     const float reach2 = cutoff2 * 1.0001f;
     float inv = inv_cutoff2;
     asm volatile("" : "+v"(inv));   // (in a vector register)
-    const float4_t *bins = reinterpret_cast<const float4_t *>(binZeroAddr);
     const int end = walk.begin_of(part_end);
     const int slot = lane & (BIN_DEPTH - 1);
+    // this lane's slot of the centre bin, and a bin's distance from it in bins: (k binDim_y + j) binDim_x + i, in factors of 24
+    // bits unless the bins' grid is half a million long (a 32-bit product is a quarter of the rate)
+    const float4_t *centre = reinterpret_cast<const float4_t *>(binZeroAddr) +
+                             ((((long long)bz * binDim_y + by) * binDim_x + bx) * BIN_DEPTH + slot);
+    const bool short_sides = binDim_x < (1 << 19) && binDim_y < (1 << 19);
     // The batch that starts at `place`: the list's entry of this lane's bin, then the slot this lane looks at.  A place
-    // past the end is the last entry's and not used.  Entries are fetched two batches ahead, slots one.
-    struct Entry {
+    // past the end is not used.  Entries are fetched two batches ahead, slots one.
+    struct Offset {
         int i, j, k;
     };
-    const auto entry = [&](int place) -> Entry {
-        const int n = walk.entry_at(min(place + (lane >> 3), end - 1));
-        return Entry{NbrList[n][0], NbrList[n][1], NbrList[n][2]};
+    CutcpWalk::Entry upcoming;   // of the next fetch from the list
+    const auto entry = [&]() -> Offset {
+        const unsigned at = (unsigned)__mul24(walk.number_of(upcoming), (int)sizeof(NbrList[0]));
+        const int *n = reinterpret_cast<const int *>(reinterpret_cast<const char *>(&NbrList[0][0]) + at);
+        walk.advance(upcoming);
+        return Offset{n[0], n[1], n[2]};
     };
-    const auto fetch = [&](const Entry &n) -> float4_t {
-        return bins[((long long)((bz + n.k) * binDim_y + by + n.j) * binDim_x + bx + n.i) * BIN_DEPTH + slot];
+    const auto fetch = [&](const Offset &n) -> float4_t {
+        long long bin;
+        if (short_sides) bin = __mul24(__mul24(n.k, binDim_y) + n.j, binDim_x) + n.i;   // uniform
+        else bin = ((long long)n.k * binDim_y + n.j) * binDim_x + n.i;
+        return centre[bin * BIN_DEPTH];
     };
     // the lanes whose slot is an atom that a bin holds: its atoms end with the first charge of zero
     const auto held = [&](const float4_t &a, int place) -> unsigned long long {
@@ -131,39 +158,24 @@ __device__ __forceinline__ void cutcp_piece(int binDim_x, int binDim_y, const fl
     const int begin = walk.begin_of(part_begin);
     unsigned long long all = ~0ull;   // the lanes that have met finite charges only
     float4_t next = {0.f, 0.f, 0.f, 0.f};
-    Entry ahead = {0, 0, 0};
-    if (begin < end) {
-        next = fetch(entry(begin));
-        ahead = entry(begin + CUTCP_BATCH_BINS);
-    }
-    for (int place = begin; place < end; place += CUTCP_BATCH_BINS) {
-        const float4_t a = next;
-        next = fetch(ahead);
-        ahead = entry(place + 2 * CUTCP_BATCH_BINS);
-        // how far the atom is from the box (no number, and so out of reach, where a coordinate is none)
-        const float ex = a.x - __builtin_amdgcn_fmed3f(a.x, box_x0, box_x1);
-        const float ey = a.y - __builtin_amdgcn_fmed3f(a.y, box_y0, box_y1);
-        const float ez = a.z - __builtin_amdgcn_fmed3f(a.z, box_z0, box_z1);
-        const float e2 = ex * ex + ey * ey + ez * ez;
-        // beyond a point's cutoff the clamp makes s zero, and the term with it unless the charge is infinite or no number
-        // (whole masks, so that no branch and no mask made into numbers and back comes of it)
-        const unsigned long long usable = CLAMP ? finite(a) : ~0ull;
-        all &= usable;
-        const unsigned long long kept = held(a, place) & __ballot(e2 < reach2) & usable;
-        const bool keep = __builtin_amdgcn_inverse_ballot_w64(kept);
-        const int count = __popcll(kept);
-        const int at = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(kept >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)kept, 0u));
-        // the wavefront's reads of the list before are behind it: LDS serves a wavefront in order
-        if (keep) stage[at] = a;
-        // ... and up to a whole number of groups, charges of zero out of everybody's reach
-        if (lane < (-count & (CUTCP_GROUP - 1))) stage[count + lane] = float4_t{1e18f, 1e18f, 1e18f, 0.f};
+    Offset ahead = {0, 0, 0};
+    const auto start = [&]() {   // at the first batch
+        upcoming = walk.entry_at(min(begin + (lane >> 3), end - 1));
+        next = fetch(entry());
+        ahead = entry();
+    };
+    if (begin < end) start();
+    int first = 0, behind = 0;   // the list: atoms first .. behind - 1, atom n at n modulo its size; first is a multiple of a group
+    const auto fence = [] {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    const auto use_groups = [&]() {   // the whole groups there are
         float4_t ga[CUTCP_GROUP], gb[CUTCP_GROUP];
-        const auto read = [&](float4_t (&g)[CUTCP_GROUP], int first) {
+        const auto read = [&](float4_t (&g)[CUTCP_GROUP], int at) {
 #pragma unroll
-            for (int u = 0; u < CUTCP_GROUP; ++u) g[u] = stage[(first & (TK_WAVE_SIZE - 1)) + u];
+            for (int u = 0; u < CUTCP_GROUP; ++u) g[u] = stage[(at & (CUTCP_RING - 1)) + u];
             __builtin_amdgcn_sched_barrier(0);   // on its way while the group before it is used
         };
         const auto use = [&](const float4_t (&g)[CUTCP_GROUP]) {
@@ -185,23 +197,54 @@ __device__ __forceinline__ void cutcp_piece(int binDim_x, int binDim_y, const fl
             }
             __builtin_amdgcn_sched_barrier(0);
         };
-        if (count > 0) read(ga, 0);
-        for (int i = 0; i < count; i += 2 * CUTCP_GROUP) {
-            read(gb, i + CUTCP_GROUP);
+        if (first + CUTCP_GROUP <= behind) read(ga, first);
+        while (first + CUTCP_GROUP <= behind) {   // uniform
+            read(gb, first + CUTCP_GROUP);
             use(ga);
-            if (i + CUTCP_GROUP >= count) break;   // uniform
-            read(ga, i + 2 * CUTCP_GROUP);
+            first += CUTCP_GROUP;
+            if (first + CUTCP_GROUP > behind) break;
+            read(ga, first + CUTCP_GROUP);
             use(gb);
+            first += CUTCP_GROUP;
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
+    };
+    for (int place = begin; place < end; place += CUTCP_BATCH_BINS) {
+        const float4_t a = next;
+        next = fetch(ahead);
+        ahead = entry();
+        // how far the atom is from the box (no number, and so out of reach, where a coordinate is none)
+        const float ex = a.x - __builtin_amdgcn_fmed3f(a.x, box_x0, box_x1);
+        const float ey = a.y - __builtin_amdgcn_fmed3f(a.y, box_y0, box_y1);
+        const float ez = a.z - __builtin_amdgcn_fmed3f(a.z, box_z0, box_z1);
+        const float e2 = ex * ex + ey * ey + ez * ez;
+        // beyond a point's cutoff the clamp makes s zero, and the term with it unless the charge is infinite or no number
+        // (whole masks, so that no branch and no mask made into numbers and back comes of it)
+        const unsigned long long usable = CLAMP ? finite(a) : ~0ull;
+        all &= usable;
+        const unsigned long long kept = held(a, place) & __ballot(e2 < reach2) & usable;
+        const bool keep = __builtin_amdgcn_inverse_ballot_w64(kept);
+        const int at = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(kept >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)kept, (unsigned)behind));
+        // the wavefront's reads of the list before are behind it: LDS serves a wavefront in order
+        if (keep) stage[at & (CUTCP_RING - 1)] = a;
+        behind += __popcll(kept);
+        if (place + CUTCP_BATCH_BINS >= end) {   // uniform: the last ones, up to a whole group with charges of zero out of everybody's reach
+            const int pad = (first - behind) & (CUTCP_GROUP - 1);
+            if (lane < pad) stage[(behind + lane) & (CUTCP_RING - 1)] = float4_t{1e18f, 1e18f, 1e18f, 0.f};
+            behind += pad;
+        }
+        fence();
+        use_groups();
+        fence();
     }
     // The atoms left out are compared with the cutoff, on a walk of their own: a sum they are part of is infinite or no
     // number whenever they are added.  (As a second form of the loop above, chosen for every 64 slots, this cost 1.5 us of
     // 26 at 36 regions and 2.3 of 45 at 361.)
     if (CLAMP && all != ~0ull) {   // uniform
+        start();
         for (int place = begin; place < end; place += CUTCP_BATCH_BINS) {
-            const float4_t a = fetch(entry(place));
+            const float4_t a = next;
+            next = fetch(ahead);
+            ahead = entry();
             unsigned long long those = held(a, place) & ~finite(a);
             while (those != 0) {
                 const int from = __builtin_ctzll(those);
@@ -229,15 +272,15 @@ __device__ __forceinline__ void cutcp_piece(int binDim_x, int binDim_y, const fl
 // How the regions are cut into units of a wavefront each: half regions with all four points a thread, or pieces of
 // a quarter or a half of those.  A smaller piece is more wavefronts -- one that has its SIMD to itself issues at
 // half the rate of two -- and evener shares, and has fewer atoms in reach (725 of a half region, 620 of a quarter of
-// it); against it stand what a wavefront spends on looking for them, about 100 instructions for every 64 slots, and
-// the three instructions and the read an atom costs before its points.  Measured with 1, 2 and 4 points, us:
-// 128 regions 35 / 42 / 61, 288 47 / 50 / 64, 512 84 / 62 / 82, 676 86 / 77 / 75, 1352 150 / 147 / 160, 17576
-// 1501 / 1506 / 1466.
+// it); against it stand what a wavefront spends on looking for them, about 60 instructions for every 64 slots, and
+// the four instructions and the read an atom costs before its points.  Measured with 1, 2 and 4 points, us: 128 regions
+// 31.6 / 38.0 / 56.9, 289 36.3 / 40.8 / 51.0, 338 43.2 / 46.0 / 64.4, 392 50.2 / 47.2 / 68.0, 676 66.1 / 59.4 / 69.4, 1352
+// 119 / 123 / 147, 2704 285 / 226 / 261, 4056 382 / 321 / 326, 5408 517 / 456 / 444, 17576 1628 / 1352 / 1337.
 struct CutcpPieces {
     int pts, subs;
     __device__ __forceinline__ CutcpPieces(int regions, int waves)
     {
-        pts = regions * 8 <= min(waves, 2 * 4 * TK_CU_NUM) ? 1 : (regions <= 8 * TK_CU_NUM ? 2 : 4);
+        pts = regions * 8 <= min(waves, 11 * TK_CU_NUM) ? 1 : (regions <= 16 * TK_CU_NUM ? 2 : 4);
         subs = 4 / pts;
     }
     __device__ __forceinline__ int first_of(int region) const { return region * 2 * subs; }
@@ -275,11 +318,11 @@ __device__ __forceinline__ void cutcp_phase(const CutcpPieces pieces, int region
     }
 }
 
-// the LDS of the role's wavefronts: 64 atoms each.  role_wave: the calling wavefront's number within the role
+// the LDS of the role's wavefronts: CUTCP_RING atoms each.  role_wave: the calling wavefront's number within the role
 template <int WAVES>
 __device__ __forceinline__ cutcp_lds_float4 *cutcp_stage_of_wave(int role_wave)
 {
-    __shared__ __align__(16) float4_t cutcp_stage[WAVES][TK_WAVE_SIZE];
+    __shared__ __align__(16) float4_t cutcp_stage[WAVES][CUTCP_RING];
     return (cutcp_lds_float4 *)&cutcp_stage[role_wave][0];
 }
 

@@ -107,6 +107,51 @@ def test_any_tiling_of_the_positions_gives_the_one_kernel(seed):
     assert np.array_equal(got == -3.0, want == -3.0) and close(got, want)
 
 
+@pytest.mark.parametrize("length", [1, 7, 8, 9, 31, 32, 33, 47, 64, 65, 97, 334])
+def test_neighbour_lists_of_any_length(length):
+    # eight bins are looked at at a time and the atoms found used four at a time: lists that end inside a batch, of one part and
+    # of several (from 33 on), bins of none to eight atoms
+    atoms, inp, prep = case(points=(24, 16, 16), natoms=400 + 37 * (length % 8), seed=length)
+    full = inp.nbr
+    try:
+        inp.nbr = np.ascontiguousarray(np.random.default_rng(length).permutation(full)[:length])
+        inp.load_neighbours()
+        prep["nbr"] = inp.nbr
+        for inv in (1 / 144.0, 0.0065):
+            want = oracle.cutcp(prep, H, C2, inv, inp.regions)
+            e = [torch.zeros_like(inp.energies) for _ in range(3)]
+            ta.ori_cutcp(inp, C2, inv, e[0])
+            ta.gptb_cutcp(inp, C2, inv, e[1])
+            ta.gptb_cutcp(inp, C2, inv, e[2], launch_grid=2, launch_block=64)
+            assert close(host(e[0]), want)
+            assert np.array_equal(bits(e[1]), bits(e[0])) and np.array_equal(bits(e[2]), bits(e[0]))
+    finally:
+        inp.nbr = full
+        inp.load_neighbours()
+
+
+def test_a_grid_of_bins_too_long_for_products_of_24_bits():
+    # the same two rows of bins, 4 and 600000 bins apart
+    atoms, inp, _ = case(points=(8, 8, 8), natoms=20, seed=3)
+    full = inp.nbr
+    rows = np.random.default_rng(5).uniform(0.5, 3, (2, 4, 8, 4)).astype(np.float32)
+    got = []
+    try:
+        inp.nbr = np.array([[0, 0, 0], [1, 0, 0], [2, 0, 0], [0, 1, 0], [1, 1, 0], [3, 1, 0]], np.int32)
+        inp.load_neighbours()
+        for length in (4, 600000):
+            inp.bins = torch.zeros((2, length, 8, 4), device="cuda:0")
+            inp.bins[:, :4] = dev(rows)
+            inp.binDim, inp.bin_zero = (length, 2, 1), inp.bins.data_ptr()
+            e = torch.zeros_like(inp.energies)
+            ta.gptb_cutcp(inp, C2, 1 / 144.0, e)
+            got.append(bits(e))
+        assert np.array_equal(got[0], got[1]) and np.abs(got[0].view(np.float32)).min() > 1
+    finally:
+        inp.nbr = full
+        inp.load_neighbours()
+
+
 @pytest.mark.parametrize("inv", [1 / 144.0, 0.0065, 0.008])
 @pytest.mark.parametrize("regions,natoms", [((1, 1, 1), 1), ((2, 1, 1), 64), ((1, 3, 2), 2000), ((9, 8, 3), 900), ((8, 9, 7), 1500)])
 def test_cut_of_the_regions_and_meaning_of_the_cutoff(inv, regions, natoms):
