@@ -78,7 +78,9 @@ __device__ __forceinline__ void mriq_voxels(int k_begin, int k_end, const float 
     }
     const int lane = mriq_lane();
     const float4_t *table = reinterpret_cast<const float4_t *>(ck);
-    constexpr int U = 4;
+    // (a voxel alone needs eight records to have enough chains: 2048 x 65536, one voxel a lane and one or two wavefronts a
+    // SIMD, 51.9 us with four, 46.6 with eight; beside tzgemm 1024^3 57.2 and 48.9)
+    constexpr int U = V == 1 ? 8 : 4;
     // U records at a time, written stage by stage (all phases, then all sines and cosines,
     // then the accumulation in ascending k): the U * V chains are independent until the last
     // stage, and the order of the source is already the interleaved one -- the compiler's
