@@ -634,8 +634,8 @@ void VGG16::captured()
 //  * On the null stream its launches wait for all that by themselves.
 //  * On a stream that is not ordered with it, the device waits for an event recorded there, which is over by the time the
 //    image is in place where the null stream is idle: 0 to 1 us a query.
-//  * On a stream that is, the host waits, after the image has been staged: 178 us a query at 224 x 224 where the null stream
-//    takes 163.  An event there, behind the stream's own last query, takes 315.
+//  * On a stream that is, the host waits, after the image has been staged: 158 us a query at 224 x 224 where the null stream
+//    takes 144.  An event there, behind the stream's own last query, took 315 where the null stream took 163.
 // Graphs and single layers on a caller's stream that is not ordered with the null stream are the caller's to order
 // with a query on another stream.
 void VGG16::executeQuery(cudaStream_t stream)
