@@ -250,8 +250,22 @@ public:
             while (ct > 1 && (Cout_ % (16 * ct) != 0 || (segments > 1 && ct * segments > 16) ||
                               (long)d.tiles * (Cout_ / (16 * ct)) * 4 < (long)cuCount() * 3))
                 ct /= 2;
-            slices = ct % 2 == 0 && ct / 2 * segments >= 8 ? 2 : 1;
             part = segments > 16;
+            // More workgroups than CUs, but not twice as many, leave a few CUs with two in turn: as half as many with twice the channels
+            // every CU has one.  Where 16 wavefronts cannot take a segment each any more, each takes a part.  us of the layers before and
+            // after: conv4_2 at 192 x 160 (288 workgroups of 16 wavefronts -> 144 of 8) 12.8 / 10.1, conv3_2 at 192 x 192 (288 -> 144) 10.3 / 8.0,
+            // at 224 x 192 (336 -> 168) 11.1 / 8.3, at 160 x 128 (320 -> 160) 8.8 / 8.4, conv1_2 with the first layer in it at 96 x 96
+            // 10.0 / 8.0; conv4_2 at 224 x 160 (384 -> 192) 11.9 / 11.6.
+            const long workgroups = (long)d.tiles * (Cout_ / (16 * ct));
+            if (!part && workgroups > cuCount() && workgroups < 2L * cuCount() && ct < 8 && Cout_ % (32 * ct) == 0) {
+                if (segments == 1 || 2 * ct * segments <= 16) {
+                    ct *= 2;
+                } else if (2 * ct * (segments / 4) <= 8 && C_ > 64) {   // (C = 64: the form that takes the first layer)
+                    ct *= 2;
+                    part = true;
+                }
+            }
+            slices = !part && ct % 2 == 0 && ct / 2 * segments >= 8 ? 2 : 1;
             d.runs = part ? segments / 4 : segments;
             key_ = std::string("conv3x3_direct_") + (slices == 2 ? "2" : "1") + (part ? "_1" : "_0");
             // Tiles of four rows where an image has no more, and where those of eight make workgroups for half of the CUs or

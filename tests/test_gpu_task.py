@@ -439,6 +439,12 @@ def test_a_layer_in_tiles_of_four_rows_gives_the_bits_of_its_operand_and_tzgemm(
     test_a_layer_by_itself_gives_the_bits_of_its_operand_and_tzgemm(H, W)
 
 
+@pytest.mark.parametrize("H,W", [(96, 96), (192, 96), (224, 96), (160, 160), (224, 160), (192, 192)])
+def test_a_layer_whose_groups_would_be_more_than_the_cus_gives_the_bits_of_its_operand_and_tzgemm(H, W):
+    # 288 workgroups of uncut reductions (conv1_2, conv3_2) and of 8 and 16 segments (conv3_2, conv4_2: parts instead), 336, 384
+    test_a_layer_by_itself_gives_the_bits_of_its_operand_and_tzgemm(H, W)
+
+
 @pytest.mark.parametrize("H,W,own_stream", [(32, 32, False), (224, 224, False), (96, 64, True), (224, 224, True)])
 def test_an_image_may_change_as_soon_as_the_query_is_launched(H, W, own_stream):
     # images are staged while the query before runs, into two device images in turn: the host's one is overwritten the
