@@ -84,6 +84,9 @@ TK_API int tkMemcpyFromSymbol(void *dst, const char *symbol, size_t bytes, size_
 
 TK_API int tkStreamCreate(tkStream_t *s);
 TK_API int tkStreamCreateNonBlocking(tkStream_t *s); /* not ordered with the null stream */
+/* waits for s, which is not being recorded, also while the calling thread records another stream (a plain wait for any
+ * stream or event is refused then) */
+TK_API int tkStreamSynchronizeBesideCapture(tkStream_t s);
 TK_API int tkStreamIsBlocking(tkStream_t s, unsigned *blocking); /* cudaStreamGetFlags: ordered with the null stream? */
 TK_API int tkStreamDestroy(tkStream_t s);
 TK_API int tkStreamSynchronize(tkStream_t s);

@@ -717,7 +717,7 @@ void VGG16::complete() const
     TK_SAFE_CALL(tkStreamWaitEvent(stream, m.over[turn]));
     for (size_t i = 0; i < CONVOLUTIONS; ++i)
         static_cast<ConvKernel *>(kernels[i])->executeInQuery(m.image[turn], nullptr, true, stream);
-    TK_SAFE_CALL(tkStreamSynchronize(stream));
+    TK_SAFE_CALL(tkStreamSynchronizeBesideCapture(stream));
 }
 
 void VGG16::layerByItself()

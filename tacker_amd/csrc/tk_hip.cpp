@@ -183,6 +183,15 @@ int tkMemcpyFromSymbol(void *dst, const char *symbol, size_t bytes, size_t offse
 
 int tkStreamCreate(tkStream_t *s) { return FOLD(hipStreamCreate((hipStream_t *)s)); }
 int tkStreamCreateNonBlocking(tkStream_t *s) { return FOLD(hipStreamCreateWithFlags((hipStream_t *)s, hipStreamNonBlocking)); }
+int tkStreamSynchronizeBesideCapture(tkStream_t s)
+{
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    int rc = FOLD(hipThreadExchangeStreamCaptureMode(&mode));
+    if (rc) return rc;
+    rc = FOLD(hipStreamSynchronize((hipStream_t)s));
+    const int back = FOLD(hipThreadExchangeStreamCaptureMode(&mode));
+    return rc ? rc : back;
+}
 int tkStreamIsBlocking(tkStream_t s, unsigned *blocking)
 {
     const int rc = FOLD(hipStreamGetFlags((hipStream_t)s, blocking));

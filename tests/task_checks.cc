@@ -1,8 +1,10 @@
 // Checks of the VGG16 task's C++ interface: what no C entry point reaches.  Usage: task_checks <check>; exit code 0 if it holds.
 #include <cstdio>
 #include <cstring>
+#include <exception>
 #include <vector>
 
+#include "Creator.h"
 #include "dnn/vgg16.h"
 #include "../include/tacker_amd.h"
 
@@ -83,6 +85,12 @@ bool many_classes(int classes)
     return same(read(task.logits(nullptr), classes), read(plain.logits(nullptr), classes));
 }
 
+void image(VGG16 &t, float factor)
+{
+    float *host = static_cast<float *>(t.InputHost[0]);
+    for (size_t i = 0; i < t.InputSize[0] / sizeof(float); ++i) host[i] = factor * (float)((i * 2654435761u) % 1000) / 1000.0f;
+}
+
 // What a whole query after a whole query leaves out is there as soon as anybody can see it: every raw output, behind two queries
 // of different images, as the layers through their operands and tzgemm leave it.  After the queries: nothing, another image staged, a
 // layer run by itself, its addresses handed out before or between the queries.
@@ -90,10 +98,6 @@ bool raw_outputs_after_queries(int height, int width)
 {
     VGG16Options opt;
     opt.height = height, opt.width = width;
-    const auto image = [](VGG16 &t, float factor) {
-        float *host = static_cast<float *>(t.InputHost[0]);
-        for (size_t i = 0; i < t.InputSize[0] / sizeof(float); ++i) host[i] = factor * (float)((i * 2654435761u) % 1000) / 1000.0f;
-    };
     enum { Nothing, Staged, Layer, Before, Between };
     for (int use : {Nothing, Staged, Layer, Before, Between}) {
         VGG16 task(1, opt), plain(2, opt);
@@ -133,6 +137,99 @@ bool raw_outputs_after_queries(int height, int width)
     return true;
 }
 
+bool same_outputs(const char *what, VGG16 &task, VGG16 &plain)
+{
+    for (int i = 0; i < 16; ++i) {
+        const VGG16::Act &a = task.layer(i), &b = plain.layer(i);
+        const size_t n = i < 13 ? size_of(a) : (size_t)a.C;
+        if (!same(read(a.ptr, n), read(b.ptr, n))) {
+            printf("%s: layer %d differs\n", what, i);
+            return false;
+        }
+    }
+    return true;
+}
+
+struct Stream {
+    cudaStream_t s = nullptr;
+    explicit Stream(bool blocking) { TK_SAFE_CALL(blocking ? tkStreamCreate(&s) : tkStreamCreateNonBlocking(&s)); }
+    ~Stream() { tkErrCheck(tkStreamDestroy(s)); }
+};
+
+// A part of a query that a caller records -- layers 1 .. 15, or layer `fused` beside a best-effort kernel and those behind it
+// -- on a new task, behind one query or behind two (which runs what they left out, while the stream is being recorded), and
+// replays: straight away, or behind other queries.  It reads what the last query left.
+bool recorded_part(int fused, bool others)
+{
+    VGG16Options opt;
+    opt.height = 64, opt.width = 96;
+    GPTBKernel *be = fused ? createKernel("stencil") : nullptr;
+    const auto part = [&](VGG16 &t, cudaStream_t stream) {
+        for (int i = fused ? fused : 1; i < 16; ++i) {
+            auto *layer = static_cast<LcGemmKernel *>(t.kernels[i]);
+            if (i == fused) layer->executeMixed(be, 0, 256, stream);
+            else layer->execute(stream);
+        }
+    };
+    for (int queries : {1, 2}) {
+        VGG16 task(1, opt), plain(2, opt);
+        for (int i = 0; i < 16; ++i) plain.resultHandedOut(i);   // its queries leave nothing out
+        Stream stream(true);
+        for (int q = 0; q < queries; ++q) task.executeQuery(nullptr);
+        plain.executeQuery(nullptr);
+        TK_SAFE_CALL(tkDeviceSynchronize());
+        tkGraphExec_t graph = nullptr;
+        TK_SAFE_CALL(tkStreamBeginCapture(stream.s));
+        part(task, stream.s);
+        TK_SAFE_CALL(tkStreamEndCapture(stream.s, &graph));
+        bool ok = true;
+        for (int replay = 0; replay < 4; ++replay) {
+            if (others)
+                for (VGG16 *t : {&task, &plain}) {
+                    image(*t, 0.25f * (float)(4 - replay));
+                    t->executeQuery(nullptr);
+                }
+            TK_SAFE_CALL(tkGraphLaunch(graph, stream.s));
+            part(plain, nullptr);
+            const size_t n = (size_t)opt.classes;
+            if (!same(read(task.logits(nullptr), n), read(plain.logits(nullptr), n))) {
+                printf("fused %d, recorded behind %d queries, replay %d: not its logits\n", fused, queries, replay);
+                ok = false;
+            }
+        }
+        ok = ok && same_outputs("recorded part", task, plain);
+        TK_SAFE_CALL(tkGraphExecDestroy(graph));
+        if (!ok) return false;
+    }
+    return true;
+}
+
+// A whole query recorded, before or behind queries; it is launched on an image that was written on the device, and what it leaves stays.
+bool recorded_query(bool first)
+{
+    VGG16Options opt;
+    opt.height = 64, opt.width = 96;
+    VGG16 task(1, opt), plain(2, opt);
+    use_tzgemm(plain);
+    Stream stream(true);
+    tkGraphExec_t graph = nullptr;
+    if (first) graph = task.captureQuery(stream.s);
+    for (float factor : {1.0f, 0.5f}) {
+        image(task, factor);
+        task.executeQuery(nullptr);
+    }
+    if (!first) graph = task.captureQuery(stream.s);
+    image(plain, 0.75f);
+    plain.executeQuery(nullptr);
+    const float *host = static_cast<float *>(plain.InputHost[0]);
+    write(static_cast<float *>(task.Input[0]), std::vector<float>(host, host + plain.InputSize[0] / sizeof(float)));
+    TK_SAFE_CALL(tkGraphLaunch(graph, stream.s));
+    TK_SAFE_CALL(tkDeviceSynchronize());
+    const bool ok = same_outputs("recorded query", task, plain);
+    TK_SAFE_CALL(tkGraphExecDestroy(graph));
+    return ok;
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -140,12 +237,20 @@ int main(int argc, char **argv)
     const char *check = argc > 1 ? argv[1] : "";
     if (tacker_init(0, nullptr)) return 2;
     bool ok = false;
-    if (!strcmp(check, "raw")) ok = written_between_layers(false, false) && written_between_layers(true, false);
-    else if (!strcmp(check, "bias")) ok = written_between_layers(false, true) && written_between_layers(true, true);
-    else if (!strcmp(check, "classes")) ok = many_classes(1000) && many_classes(8192) && many_classes(9000);
-    else if (!strcmp(check, "lean"))
-        ok = raw_outputs_after_queries(32, 32) && raw_outputs_after_queries(64, 96) && raw_outputs_after_queries(128, 160);
-    else return 2;
+    try {
+        if (!strcmp(check, "raw")) ok = written_between_layers(false, false) && written_between_layers(true, false);
+        else if (!strcmp(check, "bias")) ok = written_between_layers(false, true) && written_between_layers(true, true);
+        else if (!strcmp(check, "classes")) ok = many_classes(1000) && many_classes(8192) && many_classes(9000);
+        else if (!strcmp(check, "lean"))
+            ok = raw_outputs_after_queries(32, 32) && raw_outputs_after_queries(64, 96) && raw_outputs_after_queries(128, 160);
+        else if (!strcmp(check, "recorded_layers")) ok = recorded_part(0, true);
+        else if (!strcmp(check, "recorded_fused")) ok = recorded_part(5, true);
+        else if (!strcmp(check, "recorded_behind_queries")) ok = recorded_part(0, false) && recorded_part(5, false);
+        else if (!strcmp(check, "recorded_query")) ok = recorded_query(true) && recorded_query(false);
+        else return 2;
+    } catch (const std::exception &e) {
+        printf("%s\n", e.what());
+    }
     printf("%s %s\n", check, ok ? "ok" : "FAILED");
     return ok ? 0 : 1;
 }

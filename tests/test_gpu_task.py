@@ -741,3 +741,8 @@ def test_what_a_query_leaves_out_is_there_once_somebody_looks():
     # raw outputs behind two queries: with nothing done since, another image staged, layers run by themselves, an address handed
     # out before and between the queries
     test_checks_of_the_cxx_interface("lean")
+
+
+def test_layers_can_be_recorded_behind_queries():
+    # behind two queries the outputs they left out are computed while the caller's stream is being recorded
+    test_checks_of_the_cxx_interface("recorded_behind_queries")
