@@ -63,6 +63,7 @@ void Task::executeQuery(cudaStream_t stream)
 tkGraphExec_t Task::captureQuery(cudaStream_t stream)
 {
     tkGraphExec_t graph = nullptr;
+    recording();
     TK_SAFE_CALL(tkStreamBeginCapture(stream));
     const WholeQuery whole(*this);
     try {

@@ -34,6 +34,8 @@ public:
         explicit WholeQuery(Task &t) : task(t) { task.wholeQuery = true; }
         ~WholeQuery() { task.wholeQuery = false; }
     };
+    // the kernels' execute() is about to be recorded
+    virtual void recording() {}
     // the kernels' execute() has been recorded, not run: what a task remembers of its last run no longer holds
     virtual void captured() {}
 

@@ -180,7 +180,7 @@ protected:
     }
     void executeImpl(cudaStream_t stream) final
     {
-        task_.layerByItself();
+        task_.layerByItself(stream);
         run(stream);
     }
 
@@ -192,7 +192,7 @@ public:
             executeImpl(stream);
             return;
         }
-        task_.layerByItself();
+        task_.layerByItself(stream);
         before(stream);
         fused();
         std::unique_ptr<MixKernel> mix(createTzgemmMix(be, gptb_.get(), be_start, be_end, 0, tiles_, variant, 0, 0));
@@ -478,7 +478,7 @@ struct VGG16::Impl {
     cudaStream_t lastStream = nullptr;   // the last query's
     tkEvent_t before = nullptr;          // recorded on the null stream for a query to wait for
     bool stepped = false;                // since the last whole query the task has been used otherwise
-    bool watched = false;                // somebody has an address of a raw output, a bias or weights, or reads one
+    bool watched = false;                // somebody has an address of a raw output, a bias or weights, or has recorded a launch that has
     bool lean = false;                   // the last query has left out the raw outputs
     ~Impl()
     {
@@ -720,11 +720,24 @@ void VGG16::complete() const
     TK_SAFE_CALL(tkStreamSynchronizeBesideCapture(stream));
 }
 
-void VGG16::layerByItself()
+void VGG16::layerByItself(cudaStream_t stream)
 {
     if (wholeQuery) return;
     complete();
     impl->stepped = true;
+    // A launch that is recorded reads the outputs of the layers before it whenever the caller replays it.  (The null stream cannot be
+    // recorded, also not by its other name; a stream that gives no answer is taken to be.)
+    int capturing = 1;
+    if (!impl->watched && stream && stream != reinterpret_cast<cudaStream_t>(1) &&
+        (tkStreamIsCapturing(stream, &capturing) || capturing))
+        impl->watched = true;
+}
+
+// A recorded query writes every output whenever it is launched, behind no call of the task's.
+void VGG16::recording()
+{
+    complete();
+    impl->watched = true;
 }
 
 VGG16::~VGG16()
@@ -734,7 +747,7 @@ VGG16::~VGG16()
 
 void VGG16::initExecution()
 {
-    layerByItself();
+    layerByItself(nullptr);
     TK_SAFE_CALL(tkMemcpy(Input[0], InputHost[0], (size_t)InputSize[0], TK_MEMCPY_H2D));
 }
 

@@ -48,6 +48,7 @@ public:
     void executeQuery(cudaStream_t stream) override;
     void weightsHandedOut(int layer);    // a caller has the address of layer 0 .. 15's weights and may write them
     void resultHandedOut(int layer);     // ... of its raw output or its bias
+    void recording() override;           // queries leave nothing out from now on
     void captured() override;            // nothing of what was recorded has run: no activation is known to be up to date
     // device pointer / length of the logits (column 0 of the last GEMM's output, stride ld)
     const float *logits(long *stride) const;
@@ -61,9 +62,10 @@ public:
     const Act &layer(int idx) const;     // the same, only read
     // A whole query after a whole query leaves out what nobody reads: the convolutions' raw outputs, and the first one's launch.
     // Before anything else is done with the task -- a layer launched by itself, an address handed out, another image
-    // staged -- complete() runs the convolutions of the last query once more, with their raw outputs.
+    // staged -- complete() runs the convolutions of the last query once more, with their raw outputs.  Once a layer or a query has been
+    // recorded, nothing is left out any more: a graph is launched without asking the task.
     void complete() const;
-    void layerByItself();                // a layer is launched, and not as part of a whole query
+    void layerByItself(cudaStream_t stream);   // a layer is launched, or recorded, and not as part of a whole query
     VGG16Options opt;
     struct Impl;
     std::unique_ptr<Impl> impl;

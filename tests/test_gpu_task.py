@@ -743,6 +743,8 @@ def test_what_a_query_leaves_out_is_there_once_somebody_looks():
     test_checks_of_the_cxx_interface("lean")
 
 
-def test_layers_can_be_recorded_behind_queries():
-    # behind two queries the outputs they left out are computed while the caller's stream is being recorded
-    test_checks_of_the_cxx_interface("recorded_behind_queries")
+@pytest.mark.parametrize("check", ["recorded_behind_queries", "recorded_layers", "recorded_fused", "recorded_query"])
+def test_what_a_caller_records_reads_what_the_last_query_left(check):
+    # layers 1 .. 15, a fused layer and those behind it, a whole query: recorded behind queries (whose outputs left out are computed
+    # while the caller's stream is being recorded), replayed straight away and behind others
+    test_checks_of_the_cxx_interface(check)
