@@ -479,7 +479,8 @@ struct VGG16::Impl {
     tkEvent_t before = nullptr;          // recorded on the null stream for a query to wait for
     bool stepped = false;                // since the last whole query the task has been used otherwise
     bool watched = false;                // somebody has an address of a raw output, a bias or weights, or has recorded a launch that has
-    bool lean = false;                   // the last query has left out the raw outputs
+    bool lean = false;                   // the last query has left out the raw outputs ...
+    int leanTurn = 0;                    // ... and read this image
     ~Impl()
     {
         for (tkEvent_t e : {over[0], over[1], before})
@@ -666,8 +667,13 @@ void VGG16::executeQuery(cudaStream_t stream)
         if (capturing) throw std::runtime_error("vgg16: a query copies its image and cannot be recorded; captureQuery records its kernels");
     }
     const int turn = m.turn;
-    m.turn ^= 1;
     const tkEvent_t last = m.over[turn ^ 1];
+    // what comes after this query waits for what there is of it
+    const auto launched = [&]() {
+        m.turn ^= 1;
+        m.lastStream = stream;
+        return tkEventRecord(m.over[turn], stream);
+    };
     auto *first = m.direct ? dynamic_cast<ConvKernel *>(kernels.front()) : nullptr;
     if (!first || !first->direct()) {
         // the copy on the null stream waits for the streams ordered with it; for the others the host does
@@ -687,20 +693,25 @@ void VGG16::executeQuery(cudaStream_t stream)
         if (stream || m.lastStream) TK_SAFE_CALL(tkStreamWaitEvent(stream, last));
         const WholeQuery whole(*this);
         m.lean = !m.stepped && !m.watched;
-        size_t next = 1;
-        auto *second = static_cast<ConvKernel *>(kernels[1]);
-        if (m.lean && second->takesFirstLayer()) {
-            second->executeWithFirst(*first, m.image[turn], m.input, stream);
-            next = 2;
-        } else {
-            first->executeInQuery(m.image[turn], m.input, !m.lean, stream);
+        m.leanTurn = turn;
+        try {
+            size_t next = 1;
+            auto *second = static_cast<ConvKernel *>(kernels[1]);
+            if (m.lean && second->takesFirstLayer()) {
+                second->executeWithFirst(*first, m.image[turn], m.input, stream);
+                next = 2;
+            } else {
+                first->executeInQuery(m.image[turn], m.input, !m.lean, stream);
+            }
+            for (; m.lean && next < CONVOLUTIONS; ++next)
+                static_cast<ConvKernel *>(kernels[next])->executeInQuery(nullptr, nullptr, false, stream);
+            for (; next < kernels.size(); ++next) kernels[next]->execute(stream);
+        } catch (...) {
+            (void)launched();
+            throw;
         }
-        for (; m.lean && next < CONVOLUTIONS; ++next)
-            static_cast<ConvKernel *>(kernels[next])->executeInQuery(nullptr, nullptr, false, stream);
-        for (; next < kernels.size(); ++next) kernels[next]->execute(stream);
     }
-    TK_SAFE_CALL(tkEventRecord(m.over[turn], stream));
-    m.lastStream = stream;
+    TK_SAFE_CALL(launched());
     m.stepped = false;
 }
 
@@ -711,13 +722,12 @@ void VGG16::complete() const
 {
     Impl &m = *impl;
     if (!m.lean) return;
-    m.lean = false;
-    const int turn = m.turn ^ 1;   // the last query's
     const cudaStream_t stream = m.staging->stream;
-    TK_SAFE_CALL(tkStreamWaitEvent(stream, m.over[turn]));
+    TK_SAFE_CALL(tkStreamWaitEvent(stream, m.over[m.leanTurn]));
     for (size_t i = 0; i < CONVOLUTIONS; ++i)
-        static_cast<ConvKernel *>(kernels[i])->executeInQuery(m.image[turn], nullptr, true, stream);
+        static_cast<ConvKernel *>(kernels[i])->executeInQuery(m.image[m.leanTurn], nullptr, true, stream);
     TK_SAFE_CALL(tkStreamSynchronizeBesideCapture(stream));
+    m.lean = false;   // (and no sooner: where one of these fails, the next call tries again)
 }
 
 void VGG16::layerByItself(cudaStream_t stream)

@@ -2,11 +2,15 @@
 #include <cstdio>
 #include <cstring>
 #include <exception>
+#include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "Creator.h"
 #include "dnn/vgg16.h"
 #include "../include/tacker_amd.h"
+
+extern std::unordered_map<std::string, void *> fmap;
 
 namespace {
 
@@ -230,6 +234,49 @@ bool recorded_query(bool first)
     return ok;
 }
 
+// A launch that fails, in a query or while what queries left out is computed, is an error of that call: the next one has the
+// outputs of the image the query read, or goes on from there.
+bool after_a_failed_launch(bool query)
+{
+    VGG16Options opt;
+    opt.height = 64, opt.width = 96;
+    const auto fails = [](const char *prefix, auto call) {   // with the kernels of that prefix out of reach
+        const auto kept = fmap;
+        for (auto &k : kept)
+            if (k.first.compare(0, strlen(prefix), prefix) == 0) fmap.erase(k.first);
+        bool failed = false;
+        try {
+            call();
+        } catch (const std::exception &) {
+            failed = true;
+        }
+        fmap = kept;
+        return failed;
+    };
+    for (int queries : {1, 2}) {
+        VGG16 task(1, opt), plain(2, opt);
+        use_tzgemm(plain);
+        for (int q = 0; q < queries; ++q)
+            for (VGG16 *t : {&task, &plain}) {
+                image(*t, 1.0f / (float)(1 + q));
+                t->executeQuery(nullptr);
+            }
+        if (query) {
+            image(task, 0.75f);
+            if (!fails("fc_direct", [&] { task.executeQuery(nullptr); })) return false;
+            for (VGG16 *t : {&task, &plain}) {
+                image(*t, 0.6f);
+                t->executeQuery(nullptr);
+            }
+        } else {
+            for (int again = 0; again < 2; ++again)
+                if (!fails("conv3x3_direct", [&] { task.layer(3); })) return false;
+        }
+        if (!same_outputs("after a failed launch", task, plain)) return false;
+    }
+    return true;
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -247,6 +294,7 @@ int main(int argc, char **argv)
         else if (!strcmp(check, "recorded_fused")) ok = recorded_part(5, true);
         else if (!strcmp(check, "recorded_behind_queries")) ok = recorded_part(0, false) && recorded_part(5, false);
         else if (!strcmp(check, "recorded_query")) ok = recorded_query(true) && recorded_query(false);
+        else if (!strcmp(check, "failed_launch")) ok = after_a_failed_launch(true) && after_a_failed_launch(false);
         else return 2;
     } catch (const std::exception &e) {
         printf("%s\n", e.what());

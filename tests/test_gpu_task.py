@@ -748,3 +748,8 @@ def test_what_a_caller_records_reads_what_the_last_query_left(check):
     # layers 1 .. 15, a fused layer and those behind it, a whole query: recorded behind queries (whose outputs left out are computed
     # while the caller's stream is being recorded), replayed straight away and behind others
     test_checks_of_the_cxx_interface(check)
+
+
+def test_what_a_query_leaves_out_after_a_launch_that_failed():
+    # a kernel that cannot be found, in a query or while what queries left out is computed: the error is that call's alone
+    test_checks_of_the_cxx_interface("failed_launch")
