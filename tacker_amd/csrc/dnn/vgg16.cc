@@ -758,6 +758,8 @@ VGG16::~VGG16()
 void VGG16::initExecution()
 {
     layerByItself(nullptr);
+    // (the last query's first kernel, which may still wait on a stream that the copy is not ordered with, stores its own image there)
+    TK_SAFE_CALL(tkEventSynchronize(impl->over[impl->turn ^ 1]));
     TK_SAFE_CALL(tkMemcpy(Input[0], InputHost[0], (size_t)InputSize[0], TK_MEMCPY_H2D));
 }
 

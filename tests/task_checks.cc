@@ -234,6 +234,47 @@ bool recorded_query(bool first)
     return ok;
 }
 
+// Queries on a stream that is not ordered with the null stream, and straight behind the last one, while it is running: its outputs
+// looked at, another image staged, a layer run by itself.
+bool straight_behind_queries(int height, int width)
+{
+    VGG16Options opt;
+    opt.height = height, opt.width = width;
+    VGG16 plain(2, opt);
+    use_tzgemm(plain);
+    enum { Look, Stage, Layer };
+    for (bool watched : {false, true})
+        for (int use : {Look, Stage, Layer})
+            for (int queries : {1, 2, 3, 4}) {
+                VGG16 task(1, opt);
+                if (watched) task.resultHandedOut(3);
+                Stream stream(false);
+                for (int q = 0; q < queries; ++q) {
+                    image(task, 1.0f / (float)(1 + q));
+                    task.executeQuery(stream.s);
+                }
+                image(task, 0.3f);
+                std::vector<float> first;
+                if (use == Look) first = read(task.layer(0).ptr, size_of(task.layer(0)));
+                if (use == Stage) task.initExecution();
+                if (use == Layer) task.kernels[3]->execute(stream.s);
+                TK_SAFE_CALL(tkStreamSynchronize(stream.s));
+                image(plain, 1.0f / (float)queries);
+                plain.executeQuery(nullptr);
+                char what[100];
+                snprintf(what, sizeof(what), "%d x %d, use %d behind %d queries, watched %d", height, width, use, queries, watched);
+                if (!same_outputs(what, task, plain)) return false;
+                if (use == Look && !same(first, read(plain.layer(0).ptr, size_of(plain.layer(0))))) return false;
+                const float *staged = static_cast<float *>(task.Input[0]), *host = static_cast<float *>(task.InputHost[0]);
+                const size_t n = task.InputSize[0] / sizeof(float);
+                if (use == Stage && !same(read(staged, n), std::vector<float>(host, host + n))) {
+                    printf("%s: not the image staged\n", what);
+                    return false;
+                }
+            }
+    return true;
+}
+
 // A launch that fails, in a query or while what queries left out is computed, is an error of that call: the next one has the
 // outputs of the image the query read, or goes on from there.
 bool after_a_failed_launch(bool query)
@@ -294,6 +335,7 @@ int main(int argc, char **argv)
         else if (!strcmp(check, "recorded_fused")) ok = recorded_part(5, true);
         else if (!strcmp(check, "recorded_behind_queries")) ok = recorded_part(0, false) && recorded_part(5, false);
         else if (!strcmp(check, "recorded_query")) ok = recorded_query(true) && recorded_query(false);
+        else if (!strcmp(check, "straight_behind")) ok = straight_behind_queries(64, 96) && straight_behind_queries(224, 224);
         else if (!strcmp(check, "failed_launch")) ok = after_a_failed_launch(true) && after_a_failed_launch(false);
         else return 2;
     } catch (const std::exception &e) {

@@ -753,3 +753,8 @@ def test_what_a_caller_records_reads_what_the_last_query_left(check):
 def test_what_a_query_leaves_out_after_a_launch_that_failed():
     # a kernel that cannot be found, in a query or while what queries left out is computed: the error is that call's alone
     test_checks_of_the_cxx_interface("failed_launch")
+
+
+def test_what_comes_straight_behind_queries_on_a_stream_of_their_own():
+    # outputs looked at, another image staged, a layer run by itself, with the last query still running and both of its images in use
+    test_checks_of_the_cxx_interface("straight_behind")
