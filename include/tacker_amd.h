@@ -628,10 +628,11 @@ typedef void *tacker_task_manager_t;
 TK_API tacker_task_t tacker_task_create(const char *model, int height, int width);
 TK_API int tacker_task_destroy(tacker_task_t task);
 /* Task::initExecution + every kernel's execute(stream) (the warm-up loop of
- * src/main.cu:290-297) */
+ * src/main.cu:290-297); what VGG16 leaves out then: tacker_task_activation */
 TK_API int tacker_task_execute(tacker_task_t task, tkStream_t stream);
 /* Task::initExecution alone (src/Task.h:24 of the reference; VGG16's copies the query's input to
- * the device, synchronously) */
+ * the device, synchronously, behind the last tacker_task_execute; the first time behind one it may take 0.2 ms
+ * more, see tacker_task_activation) */
 TK_API int tacker_task_stage_input(tacker_task_t task);
 /* The task's launches recorded from `stream` into one graph (no counterpart in the reference, which
  * launches a query kernel by kernel): every kernel's execute(stream) between tkStreamBeginCapture
@@ -646,9 +647,10 @@ TK_API int tacker_task_kernel_info(tacker_task_t task, int index, char *name, in
 /* VGG16 only: the buffer layer conv_index writes (0..12 the convolutions, 13..15 the three fully
  * connected layers, whose result is one row: H = W = 1): device pointer and dims = {H, W, channels,
  * channel stride}.  It holds the raw GEMM output 1.1 * A * B^T; the layer that reads it adds the bias
- * and rectifies.  A whole query after a whole query leaves the convolutions' buffers out as long as nobody has
- * asked for an address here or below: the first call behind such a query runs its convolutions once more, with
- * them, and waits (0.2 ms), and from then on every query writes them (141 -> 152 us at 224 x 224).
+ * and rectifies.  A tacker_task_execute with nothing else done with the task since the last one, or since it was
+ * made, leaves the convolutions' buffers out.  The first call behind such a query that asks for an address (here
+ * or below), stages an image, captures the task or launches a layer by itself runs its convolutions once more, with
+ * them, and waits (0.2 ms); from then on every query of the task writes them (141 -> 152 us at 224 x 224).
  * logits = the first `count` floats of the last layer's buffer */
 TK_API int tacker_task_activation(tacker_task_t task, int conv_index, float **ptr, int dims[4]);
 TK_API int tacker_task_logits(tacker_task_t task, const float **ptr, long *stride, int *count);

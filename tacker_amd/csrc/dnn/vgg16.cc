@@ -478,7 +478,8 @@ struct VGG16::Impl {
     cudaStream_t lastStream = nullptr;   // the last query's
     tkEvent_t before = nullptr;          // recorded on the null stream for a query to wait for
     bool stepped = false;                // since the last whole query the task has been used otherwise
-    bool watched = false;                // somebody has an address of a raw output, a bias or weights, or has recorded a launch that has
+    bool watched = false;                // no query leaves anything out: somebody has an address of a raw output, a bias or weights, or has
+                                         // recorded a launch that has, or something was left out that somebody needed
     bool lean = false;                   // the last query has left out the raw outputs ...
     int leanTurn = 0;                    // ... and read this image
     ~Impl()
@@ -728,6 +729,7 @@ void VGG16::complete() const
         static_cast<ConvKernel *>(kernels[i])->executeInQuery(m.image[m.leanTurn], nullptr, true, stream);
     TK_SAFE_CALL(tkStreamSynchronizeBesideCapture(stream));
     m.lean = false;   // (and no sooner: where one of these fails, the next call tries again)
+    m.watched = true;   // (a caller who does something else between queries does it again: this, 0.2 ms, once in a task's life)
 }
 
 void VGG16::layerByItself(cudaStream_t stream)
@@ -781,6 +783,8 @@ void VGG16::resultHandedOut(int layer)
     if (layer < 13) impl->act[layer].fresh.exposed = true;
     else if (layer < 15) impl->fcInput[layer - 12].exposed = true;
 }
+
+bool VGG16::leavesOutputsOut() const { return impl->direct && !impl->watched && !impl->stepped; }
 
 const VGG16::Act &VGG16::layer(int idx) const
 {

@@ -60,11 +60,13 @@ public:
     struct Act { float *ptr; int H, W, C, ld; void *weights; float *bias; int Np, Kp; };
     Act activation(int conv_index);
     const Act &layer(int idx) const;     // the same, only read
-    // A whole query after a whole query leaves out what nobody reads: the convolutions' raw outputs, and the first one's launch.
-    // Before anything else is done with the task -- a layer launched by itself, an address handed out, another image
-    // staged -- complete() runs the convolutions of the last query once more, with their raw outputs.  Once a layer or a query has been
-    // recorded, nothing is left out any more: a graph is launched without asking the task.
+    // A whole query with nothing else done since the last one, or since the task was made, leaves out what nobody reads: the
+    // convolutions' raw outputs, and the first one's launch.  Before anything else is done with the task -- a layer launched by
+    // itself, an address handed out, another image staged -- complete() runs the convolutions of the last query once more, with
+    // their raw outputs, and from then on no query leaves anything out.  The same holds once a layer or a query has been recorded:
+    // a graph is launched without asking the task.
     void complete() const;
+    bool leavesOutputsOut() const;             // the next whole query does
     void layerByItself(cudaStream_t stream);   // a layer is launched, or recorded, and not as part of a whole query
     VGG16Options opt;
     struct Impl;

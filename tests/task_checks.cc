@@ -234,6 +234,34 @@ bool recorded_query(bool first)
     return ok;
 }
 
+// A task that somebody uses otherwise between its queries pays for what they left out once.
+bool paid_once()
+{
+    VGG16Options opt;
+    opt.height = opt.width = 32;
+    enum { Look, Stage, Layer, Record };
+    for (int use : {Look, Stage, Layer, Record}) {
+        VGG16 task(1, opt);
+        bool left = task.leavesOutputsOut();   // a new task's
+        for (int round = 0; round < 2; ++round) {
+            for (int q = 0; q < 3; ++q) task.executeQuery(nullptr);
+            left = left && task.leavesOutputsOut() == (round == 0);
+            if (use == Look) task.layer(2);
+            if (use == Stage) task.initExecution();
+            if (use == Layer) task.kernels[14]->execute((cudaStream_t) nullptr);
+            if (use == Record) {
+                Stream stream(false);
+                TK_SAFE_CALL(tkGraphExecDestroy(task.captureQuery(stream.s)));
+            }
+        }
+        if (!left || task.leavesOutputsOut()) {
+            printf("use %d\n", use);
+            return false;
+        }
+    }
+    return true;
+}
+
 // Queries on a stream that is not ordered with the null stream, and straight behind the last one, while it is running: its outputs
 // looked at, another image staged, a layer run by itself.
 bool straight_behind_queries(int height, int width)
@@ -335,6 +363,7 @@ int main(int argc, char **argv)
         else if (!strcmp(check, "recorded_fused")) ok = recorded_part(5, true);
         else if (!strcmp(check, "recorded_behind_queries")) ok = recorded_part(0, false) && recorded_part(5, false);
         else if (!strcmp(check, "recorded_query")) ok = recorded_query(true) && recorded_query(false);
+        else if (!strcmp(check, "paid_once")) ok = paid_once();
         else if (!strcmp(check, "straight_behind")) ok = straight_behind_queries(64, 96) && straight_behind_queries(224, 224);
         else if (!strcmp(check, "failed_launch")) ok = after_a_failed_launch(true) && after_a_failed_launch(false);
         else return 2;

@@ -758,3 +758,8 @@ def test_what_a_query_leaves_out_after_a_launch_that_failed():
 def test_what_comes_straight_behind_queries_on_a_stream_of_their_own():
     # outputs looked at, another image staged, a layer run by itself, with the last query still running and both of its images in use
     test_checks_of_the_cxx_interface("straight_behind")
+
+
+def test_a_task_used_otherwise_between_queries_pays_for_it_once():
+    # outputs looked at, an image staged, a layer launched, a query recorded: from then on queries leave nothing out
+    test_checks_of_the_cxx_interface("paid_once")
