@@ -243,8 +243,8 @@ public:
         d.tiles = d.tiles_x * ((H_ + DNN_TILE - 1) / DNN_TILE);
         d.per_group = reciprocal(d.tiles);
         d.per_row = reciprocal(d.tiles_x);
-        int ct = 8, slices = 1;
-        bool part = false;
+        int ct = 8, &slices = slices_;
+        bool &part = part_, &low = low_;
         if (in) {
             const int segments = reductionCut(M_, N_, K_, 9 * C_ / TZ_BLOCK_K, d.segment_begin);
             while (ct > 1 && (Cout_ % (16 * ct) != 0 || (segments > 1 && ct * segments > 16) ||
@@ -267,15 +267,15 @@ public:
             }
             slices = !part && ct % 2 == 0 && ct / 2 * segments >= 8 ? 2 : 1;
             d.runs = part ? segments / 4 : segments;
-            key_ = std::string("conv3x3_direct_") + (slices == 2 ? "2" : "1") + (part ? "_1" : "_0");
             // Tiles of four rows where an image has no more, and where those of eight make workgroups for half of the CUs or
             // fewer: us with tiles of eight and four rows, conv5_1 at 224 x 224 (128 workgroups of 8 x 8) 8.0 / 6.7, conv4_2 at
             // 64 x 96 (64) 9.0 / 7.3, conv3_2 there (96) 6.2 / 5.2.
-            if (slices == 1 && (H_ <= DNN_TILE / 2 || (ct == 1 && 2L * d.tiles * (Cout_ / 16) <= cuCount()))) {
-                key_ += "_low";
+            low = slices == 1 && (H_ <= DNN_TILE / 2 || (ct == 1 && 2L * d.tiles * (Cout_ / 16) <= cuCount()));
+            if (low) {
                 d.tiles = d.tiles_x * ((H_ + DNN_TILE / 2 - 1) / (DNN_TILE / 2));
                 d.per_group = reciprocal(d.tiles);
             }
+            key_ = std::string("conv3x3_direct_") + (slices == 2 ? "2" : "1") + (part ? "_1" : "_0") + (low ? "_low" : "");
             lds_ = std::max((size_t)(C_ / 64) * DNN_PLANE_BYTES, (size_t)ct * d.runs * DNN_PARTIAL_BYTES);
         } else {
             ct = Cout_ / 16;
@@ -293,10 +293,11 @@ public:
     // As part of a whole query.  raw: the output is written beside the activation.  image, keep: of the first layer, read
     // from `image` and stored where the layer has it as a rule.
     void executeInQuery(const float *image, float *keep, bool raw, cudaStream_t stream) { launchDirect(image, keep, raw, stream); }
-    // Whether the second layer can compute the first one's activation for itself: wherever a wavefront of it serves one slice of
-    // channels over segments of their own, the form its kernel for that has.  (All sizes have it there but some whose reduction is cut
-    // and that have enough tiles for a workgroup to take four slices.)
-    bool takesFirstLayer() const { return direct_ && key_.compare(0, 18, "conv3x3_direct_1_0") == 0 && threads_ <= 512; }
+    // Whether the second layer can compute the first one's activation for itself: where a wavefront of it serves one slice of
+    // channels over segments of their own, the form its kernel for that has.  That is so at all sizes on 256 CUs: a reduction that
+    // is cut is one of at most 128 pixel tiles, too few for a workgroup to take the four slices that make two a wavefront.  On
+    // fewer CUs it may not be, and the first layer then has its launch.
+    bool takesFirstLayer() const { return direct_ && slices_ == 1 && !part_ && threads_ <= 512; }
     // ... and both of them, the second as part of a whole query without its raw output
     void executeWithFirst(const ConvKernel &first, const float *image, float *keep, cudaStream_t stream)
     {
@@ -304,7 +305,7 @@ public:
         DnnConv c = *direct_;
         c.out.raw = nullptr;
         void *args[] = {&i, &c};
-        const char *key = key_.size() > 18 ? "conv3x3_direct_image_low" : "conv3x3_direct_image";
+        const char *key = low_ ? "conv3x3_direct_image_low" : "conv3x3_direct_image";
         TK_SAFE_CALL(tkLaunchKernel(fmap.at(key), dim3(grid_).raw(), dim3(threads_).raw(), args, lds_ + DNN_IMAGE_BYTES, stream));
         first.next_->fresh.valid = false;
         next_->fresh.valid = true;
@@ -358,6 +359,8 @@ private:
     std::unique_ptr<DnnConv> direct_;
     Activation *in_ = nullptr, *next_ = nullptr;
     std::string key_;
+    int slices_ = 1;                     // of 16 channels a wavefront takes
+    bool part_ = false, low_ = false;    // ... over a whole part of the reduction; tiles of four rows
     unsigned grid_ = 0, threads_ = 0;
     size_t lds_ = 0;
 };
@@ -698,7 +701,7 @@ void VGG16::executeQuery(cudaStream_t stream)
         try {
             size_t next = 1;
             auto *second = static_cast<ConvKernel *>(kernels[1]);
-            if (m.lean && second->takesFirstLayer()) {
+            if (m.lean && !opt.firstLayerApart && second->takesFirstLayer()) {
                 second->executeWithFirst(*first, m.image[turn], m.input, stream);
                 next = 2;
             } else {

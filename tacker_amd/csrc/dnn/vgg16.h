@@ -38,6 +38,7 @@ struct VGG16Options {
     int height = 224, width = 224;   // input resolution (multiples of 32)
     int classes = 1000;
     unsigned long long seed = 1337ULL;
+    bool firstLayerApart = false;    // the first convolution has its own launch in every query, as on a device of few CUs
 };
 
 class VGG16 : public Task {
