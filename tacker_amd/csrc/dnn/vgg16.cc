@@ -252,15 +252,19 @@ public:
                 ct /= 2;
             part = segments > 16;
             // More workgroups than CUs, but not twice as many, leave a few CUs with two in turn: as half as many with twice the channels
-            // every CU has one.  Where 16 wavefronts cannot take a segment each any more, each takes a part.  us of the layers before and
-            // after: conv4_2 at 192 x 160 (288 workgroups of 16 wavefronts -> 144 of 8) 12.8 / 10.1, conv3_2 at 192 x 192 (288 -> 144) 10.3 / 8.0,
-            // at 224 x 192 (336 -> 168) 11.1 / 8.3, at 160 x 128 (320 -> 160) 8.8 / 8.4, conv1_2 with the first layer in it at 96 x 96
-            // 10.0 / 8.0; conv4_2 at 224 x 160 (384 -> 192) 11.9 / 11.6.
+            // every CU has one.  us of the layers before and after: conv4_2 at 320 x 416 (280 workgroups -> 140) 27.5 / 20.5, at
+            // 160 x 416 (336) 13.8 / 9.8, conv3_2 at 192 x 192 (288) 10.3 / 8.0, at 224 x 192 (336) 11.1 / 8.3, at 160 x 128 (320) 8.8 / 8.4, at
+            // 224 x 416 (364) 13.2 / 12.9, conv1_2 with the first layer in it at 96 x 96 10.0 / 8.0.
+            // Where 16 wavefronts cannot take a segment each any more, each takes a part, if a workgroup had 16 channels only: conv4_2
+            // at 160 x 160 (288) 11.4 / 9.1, at 128 x 288 (320) 11.1 / 10.9, at 224 x 160 (384) 10.6 / 10.7 and conv4_3 there 11.1 / 10.9, at
+            // 96 x 416 (448) 11.1 / 10.9, conv5_1 at 288 x 416 (384) 11.9 / 9.2.  Of two slices of eight segments and of four of four it makes
+            // eight longer wavefronts out of 16 and loses: conv4_2 at 224 x 288 (320) 13.0 / 14.0, at 160 x 352 (288) 12.5 / 13.9, at
+            // 352 x 352 (288) 19.3 / 22.7.
             const long workgroups = (long)d.tiles * (Cout_ / (16 * ct));
             if (!part && workgroups > cuCount() && workgroups < 2L * cuCount() && ct < 8 && Cout_ % (32 * ct) == 0) {
                 if (segments == 1 || 2 * ct * segments <= 16) {
                     ct *= 2;
-                } else if (2 * ct * (segments / 4) <= 8 && C_ > 64) {   // (C = 64: the form that takes the first layer)
+                } else if (ct == 1 && C_ > 64) {   // (C = 64: the form that takes the first layer)
                     ct *= 2;
                     part = true;
                 }

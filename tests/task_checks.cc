@@ -263,6 +263,17 @@ bool paid_once()
     return true;
 }
 
+// every output of a query as the layers through their operands and tzgemm leave it
+bool outputs(int height, int width)
+{
+    VGG16Options opt;
+    opt.height = height, opt.width = width;
+    VGG16 task(1, opt), plain(2, opt);
+    use_tzgemm(plain);
+    for (VGG16 *t : {&task, &plain}) t->executeQuery(nullptr);
+    return same_outputs("a query", task, plain);
+}
+
 // Queries on a stream that is not ordered with the null stream, and straight behind the last one, while it is running: its outputs
 // looked at, another image staged, a layer run by itself.
 bool straight_behind_queries(int height, int width, int most)
@@ -365,6 +376,7 @@ int main(int argc, char **argv)
         else if (!strcmp(check, "recorded_fused")) ok = recorded_part(5, true);
         else if (!strcmp(check, "recorded_behind_queries")) ok = recorded_part(0, false) && recorded_part(5, false);
         else if (!strcmp(check, "recorded_query")) ok = recorded_query(true) && recorded_query(false);
+        else if (!strcmp(check, "sizes")) ok = outputs(160, 160) && outputs(160, 352) && outputs(352, 352) && outputs(96, 416);
         else if (!strcmp(check, "paid_once")) ok = paid_once();
         else if (!strcmp(check, "straight_behind")) ok = straight_behind_queries(64, 96, 4) && straight_behind_queries(224, 224, 2);
         else if (!strcmp(check, "failed_launch")) ok = after_a_failed_launch(true) && after_a_failed_launch(false);

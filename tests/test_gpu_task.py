@@ -763,3 +763,8 @@ def test_what_comes_straight_behind_queries_on_a_stream_of_their_own():
 def test_a_task_used_otherwise_between_queries_pays_for_it_once():
     # outputs looked at, an image staged, a layer launched, a query recorded: from then on queries leave nothing out
     test_checks_of_the_cxx_interface("paid_once")
+
+
+def test_queries_whose_layers_make_a_few_more_workgroups_than_there_are_cus():
+    # conv4 in 288 workgroups of 16 channels and 16 segments, 32 and 8, 64 and 4, and in 448 of 16 and 12: twice the channels or not
+    test_checks_of_the_cxx_interface("sizes")
