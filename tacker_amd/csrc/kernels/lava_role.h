@@ -17,10 +17,13 @@
 // exponential 8.4, and MFMAs take the same slots), so three things count.
 //  * How many instructions a pair takes.  The force on i is a sum of w (xi - xj), w = qj vij; it is computed as
 //    (xi - c) sum w - sum vij [qj (xj - c)], which leaves four multiply-adds a pair (v and the force together)
-//    where the difference, its product and the sum of w took eight instructions.  c is about the middle of the home box (lava_centre),
-//    so that the two terms are of the size of the force and nothing cancels: against 64 bits the result is as far off as with
-//    the differences (2-norm of the whole output, 2^3 / 5^3 / 9^3 / 24^3 boxes: 5.0 / 7.3 / 7.6 / 7.9e-8 both ways; of
-//    the forces alone 5.4 / 7.3 / 7.7 / 7.9e-8 against 5.2 / 7.3 / 7.6 / 7.9e-8).
+//    where the difference, its product and the sum of w take eight instructions.  c is about the middle of the home box, on a
+//    coarse grid (LavaCentre).  The two terms are of the size of |x - c| sum w, so this is as exact as the differences only
+//    where no pair much closer than that matters more than the rest: where a2 |x - c|^2 <= 1/2 (LAVA_CENTRED), and weights differ
+//    little across the box.  Forces against 64 bits, 2-norm over the middle box of 3^3, 60 systems, differences / this form
+//    where it is taken: unit boxes around the origin, v = |x|^2 / 2, alpha 0.35 12.3 / 12.0e-8, 0.5 13.3 / 13.0e-8; x and v in
+//    0.1 ... 1 in every box, alpha 0.35 8.0 / 8.1e-8, 0.5 7.9 / 8.1e-8.  Where it is not taken it would be off by more: unit boxes,
+//    alpha 1 25.8 / 30.7e-8, 2 58 / 86e-8 (with a centre off the grid, which cost 8 % at 0.5).  Those boxes take the differences.
 //  * What is computed per neighbour and not per pair.  A wavefront prepares the 100 neighbours of a part once, a lane
 //    each: {scale v, -scale x, -scale y, -scale z} and {q, q (x - cx), q (y - cy), q (z - cz)} go to LDS and
 //    come back as two 16-byte broadcast reads a step.  (By a vector load for every step and row of lanes, and four multiplies
@@ -28,7 +31,7 @@
 //  * How full the lanes are.  The wavefront is four rows of 16 lanes: row g takes neighbours g, g + 4, g + 8, ... (25 of the
 //    100), a lane LAVA_MAX_P = 6 of the first 96 home particles: 150 steps without an empty slot.  The last four
 //    particles are four lanes side by side, 16 neighbours at a time: 7 steps, where a seventh particle a lane would take 25.
-// A pair is 8 such instructions and the exponential.  At the end of a part the four rows' sums are added,
+// A pair is 8 such instructions and the exponential, 12 from the differences.  At the end of a part the four rows' sums are added,
 // (g0 + g2) + (g1 + g3), by lane swaps that add two values at once, which leaves component v, y, x, z of the
 // total in row 0, 1, 2, 3; the total goes on from the output array.  24^3 boxes: 837 us (35 cycles a SIMD and step of 64 pairs), where twelve instructions
 // a pair, neighbours by vector loads and seven particles a lane took 1325; 18^3 372 / 577, 9^3 78 / 116, 3^3 36.5 / 46.
@@ -58,6 +61,7 @@ typedef __attribute__((address_space(4))) const box_str lava_const_box;
 #define LAVA_MAX_P 6                                    // home particles per lane when one wavefront serves a box
 #define LAVA_WAVES_PER_SIMD 4                           // wavefronts of this role a SIMD holds (registers)
 #define LAVA_STEPS (NUMBER_PAR_PER_BOX / LAVA_ROWS)     // neighbours a row takes per box
+#define LAVA_CENTRED 0.72f                              // a2 log2(e) |x - c|^2 up to which forces are computed about the centre
 #define LAVA_REST 4                                     // home particles behind the lanes' own ...
 #define LAVA_REST_FROM (NUMBER_PAR_PER_BOX - LAVA_REST)
 #define LAVA_REST_STEP (TK_WAVE_SIZE / LAVA_REST)       // ... and the neighbours they take a step
@@ -94,26 +98,205 @@ __device__ __forceinline__ float lava_add_along_row(float v)
     return v + __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x120 + N, 0xf, 0xf, false));
 }
 
-// About the middle of the home box, the same for every wavefront that serves a part of it: the median of three thirds' means,
-// which one particle far away -- or one that is no number -- does not move, and 0 where that is not finite either.
-__device__ __forceinline__ void lava_centre(const float4_t *rA, int lane, float (&centre)[3])
+template <int N>
+__device__ __forceinline__ float lava_max_along_row(float v)
 {
-    const float4_t lo = rA[lane], hi = rA[min(lane + TK_WAVE_SIZE, NUMBER_PAR_PER_BOX - 1)];
-    const bool two = lane + TK_WAVE_SIZE < NUMBER_PAR_PER_BOX;
+    return __builtin_fmaxf(v, __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x120 + N, 0xf, 0xf, false)));
+}
+
+// The median of three thirds' means of a value that every home particle has -- lo of particle `lane`, hi of particle 64 + lane --
+// which one particle far away, or one that is no number, does not move; 0 where that is not finite either.
+__device__ __forceinline__ float lava_middle(float lo, float hi, int lane)
+{
+    float v = lo + (lane + TK_WAVE_SIZE < NUMBER_PAR_PER_BOX ? hi : 0.f);
+    v = lava_add_along_row<8>(v);
+    v = lava_add_along_row<4>(v);
+    v = lava_add_along_row<2>(v);
+    v = lava_add_along_row<1>(v);
+    float row[LAVA_ROWS];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        float v = lo[c + 1] + (two ? hi[c + 1] : 0.f);
-        v = lava_add_along_row<8>(v);
-        v = lava_add_along_row<4>(v);
-        v = lava_add_along_row<2>(v);
-        v = lava_add_along_row<1>(v);
-        float row[LAVA_ROWS];
+    for (int g = 0; g < LAVA_ROWS; ++g)
+        row[g] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), LAVA_LANES * g));
+    // particles 0 - 15 and 64 - 79, 16 - 31 and 80 - 95, 32 - 63 and 96 - 99
+    const float m = __builtin_amdgcn_fmed3f(row[0] * (1.f / 32), row[1] * (1.f / 32), (row[2] + row[3]) * (1.f / 36));
+    return __builtin_fabsf(m) <= FLT_MAX ? m : 0.f;
+}
+
+// the largest of a value of every lane
+__device__ __forceinline__ float lava_largest(float v)
+{
+    v = lava_max_along_row<8>(v);
+    v = lava_max_along_row<4>(v);
+    v = lava_max_along_row<2>(v);
+    v = lava_max_along_row<1>(v);
+    float most = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), 0));
 #pragma unroll
-        for (int g = 0; g < LAVA_ROWS; ++g)
-            row[g] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), LAVA_LANES * g));
-        // particles 0 - 15 and 64 - 79, 16 - 31 and 80 - 95, 32 - 63 and 96 - 99
-        const float m = __builtin_amdgcn_fmed3f(row[0] * (1.f / 32), row[1] * (1.f / 32), (row[2] + row[3]) * (1.f / 36));
-        centre[c] = __builtin_fabsf(m) <= FLT_MAX ? m : 0.f;
+    for (int g = 1; g < LAVA_ROWS; ++g)
+        most = __builtin_fmaxf(most, __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), LAVA_LANES * g)));
+    return most;
+}
+
+// a value that all lanes have, in a scalar register
+__device__ __forceinline__ float lava_scalar(float v) { return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v))); }
+
+// About the middle of the home box, which its forces are computed about, the same for every wavefront that serves a part of it.
+struct LavaCentre {
+    float at[3];
+    bool use;   // the box allows it
+    __device__ __forceinline__ LavaCentre(const float4_t *rA, float scale, int lane)
+    {
+        const float4_t lo = rA[lane], hi = rA[min(lane + TK_WAVE_SIZE, NUMBER_PAR_PER_BOX - 1)];
+        float across = 0.f;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            at[c] = lava_middle(lo[c + 1], hi[c + 1], lane);
+            across = __builtin_fmaxf(across, __builtin_fmaxf(__builtin_fabsf(lo[c + 1] - at[c]), __builtin_fabsf(hi[c + 1] - at[c])));
+        }
+        // on a grid of an eighth to a quarter of the box's half width: x - c is then exact for most coordinates, and its
+        // rounding was what the form about the centre lost most by
+        const int grid = __builtin_amdgcn_frexp_expf(lava_largest(across)) - 3;
+        float lo2 = 0.f, hi2 = 0.f;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            at[c] = lava_scalar(__builtin_ldexpf(__builtin_rintf(__builtin_ldexpf(at[c], -grid)), grid));
+            lo2 += (lo[c + 1] - at[c]) * (lo[c + 1] - at[c]);
+            hi2 += (hi[c + 1] - at[c]) * (hi[c + 1] - at[c]);
+        }
+        use = -scale * lava_largest(__builtin_fmaxf(lo2, hi2)) <= LAVA_CENTRED;   // (not where a2 is no number)
+    }
+};
+
+// The forces of the staged part on P home particles a lane -- and on the last four, if `rest` -- added to their totals: about
+// the centre c (CENTRED), or from the differences of the coordinates.
+template <int P, bool CENTRED>
+__device__ __forceinline__ void lava_part(const float4_t (&home)[P], const float (&centre)[3], int row, float twice, bool rest,
+                                          const lava_lds_float4 *rest_home, int lane, const lava_lds_float4 *stage,
+                                          float (&total)[P], float &last_total)
+{
+    float4_t f[P];   // sums of w, and of vij q (x - c) -- or of w (xi - xj) -- component by component
+#pragma unroll
+    for (int k = 0; k < P; ++k) f[k] = float4_t{0.f, 0.f, 0.f, 0.f};
+    const lava_lds_float4 *at = stage + 2 * row;
+    float4_t a = at[0], b = at[1];
+    // Six particles a lane are chains enough for the compiler to interleave as it likes (24^3 boxes 829 us, with the step's
+    // read held in front of it 871); with fewer, the reads stay in front of a step's work and every step is written out (3^3 boxes
+    // 36.5 us; 42.1 in a loop of five steps, 43.2 as the compiler likes).
+#pragma unroll P < LAVA_MAX_P ? LAVA_STEPS : 5
+    for (int t = 0; t < LAVA_STEPS; ++t) {
+        at += 2 * LAVA_ROWS;
+        const lava_lds_float4 *next = t + 1 < LAVA_STEPS ? at : stage;   // (the last read is not used)
+        const float4_t na = next[0], nb = next[1];
+        if (P < LAVA_MAX_P) __builtin_amdgcn_sched_barrier(0);
+        // scale (vi + vj - (xi xj + yi yj + zi zj)) = -r2 a2 log2(e), stage by stage over the lane's
+        // particles: their chains are independent, and in this order none waits for its own last result
+        float w[P];
+#pragma unroll
+        for (int k = 0; k < P; ++k) w[k] = home[k][0] + a[0];
+#pragma unroll
+        for (int c = 1; c < 4; ++c)
+#pragma unroll
+            for (int k = 0; k < P; ++k) w[k] = __builtin_fmaf(home[k][c], a[c], w[k]);
+#pragma unroll
+        for (int k = 0; k < P; ++k) w[k] = __builtin_amdgcn_exp2f(w[k]);
+        if (CENTRED) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+#pragma unroll
+                for (int k = 0; k < P; ++k) f[k][c] = __builtin_fmaf(w[k], b[c], f[k][c]);
+        } else {
+#pragma unroll
+            for (int k = 0; k < P; ++k) w[k] *= b[0];
+#pragma unroll
+            for (int k = 0; k < P; ++k) f[k][0] += w[k];
+#pragma unroll
+            for (int c = 1; c < 4; ++c)
+#pragma unroll
+                for (int k = 0; k < P; ++k) f[k][c] = __builtin_fmaf(w[k], home[k][c] - b[c], f[k][c]);
+        }
+        if (P < LAVA_MAX_P) __builtin_amdgcn_sched_barrier(0);
+        a = na;
+        b = nb;
+    }
+#pragma unroll
+    for (int k = 0; k < P; ++k) {
+        if (CENTRED) {
+#pragma unroll
+            for (int c = 1; c < 4; ++c) f[k][c] = __builtin_fmaf(home[k][c] - centre[c - 1], f[k][0], -f[k][c]);
+        }
+        total[k] += twice * lava_fold_rows(lava_fold_halves(f[k][0], f[k][1]), lava_fold_halves(f[k][2], f[k][3]));
+    }
+    if (!rest) return;   // uniform
+    const float4_t last = rest_home[lane & (LAVA_REST - 1)];
+    float4_t g = {0.f, 0.f, 0.f, 0.f};
+    const auto pair = [&](int j) {
+        const float4_t a = stage[2 * j], b = stage[2 * j + 1];
+        float w = last[0] + a[0];
+#pragma unroll
+        for (int c = 1; c < 4; ++c) w = __builtin_fmaf(last[c], a[c], w);
+        w = __builtin_amdgcn_exp2f(w);
+        if (!CENTRED) w *= b[0];
+        g[0] = CENTRED ? __builtin_fmaf(w, b[0], g[0]) : g[0] + w;
+#pragma unroll
+        for (int c = 1; c < 4; ++c) g[c] = __builtin_fmaf(w, CENTRED ? b[c] : last[c] - b[c], g[c]);
+    };
+    const int from = lane / LAVA_REST;
+#pragma unroll
+    for (int j = 0; j + LAVA_REST_STEP <= NUMBER_PAR_PER_BOX; j += LAVA_REST_STEP) pair(j + from);
+    if (from < NUMBER_PAR_PER_BOX % LAVA_REST_STEP) pair(NUMBER_PAR_PER_BOX / LAVA_REST_STEP * LAVA_REST_STEP + from);
+    if (CENTRED) {
+#pragma unroll
+        for (int c = 1; c < 4; ++c) g[c] = __builtin_fmaf(last[c] - centre[c - 1], g[0], -g[c]);
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) g[c] = lava_add_along_row<4>(lava_add_along_row<8>(g[c]));
+    last_total += twice * lava_fold_rows(lava_fold_halves(g[0], g[1]), lava_fold_halves(g[2], g[3]));
+}
+
+// Parts [part_begin, part_end) of box `bx`, added to the totals of its home particles as lava_part does.
+template <int P, bool CENTRED>
+__device__ __forceinline__ void lava_parts(const float scale, const lava_const_box *boxes, const FOUR_VECTOR *d_rv_gpu,
+                                           const float *d_qv_gpu, int bx, int part_begin, int part_end, const float4_t (&home)[P],
+                                           const float (&centre)[3], int row, float twice, bool rest, int lane,
+                                           lava_lds_float4 *stage, float (&total)[P], float &last_total)
+{
+    const lava_lds_float4 *rest_home = stage + 2 * NUMBER_PAR_PER_BOX;
+    // A neighbour is named by its number alone (its offset in the list is not read): two loads behind one another, and the
+    // particles behind them.  The number is fetched three parts ahead, the offset two, the particles one; where there is no such part,
+    // the home box's own are read.
+    const auto box_of = [&](int part) -> int { return part == 0 || part >= part_end ? bx : boxes[bx].nei[part - 1].number; };
+    const int second = min(lane + TK_WAVE_SIZE, NUMBER_PAR_PER_BOX - 1);   // a lane's second neighbour (past the last: not used)
+    float4_t r0, r1;
+    float q0, q1;
+    const auto fetch = [&](long first_j) {
+        const float4_t *rB = reinterpret_cast<const float4_t *>(d_rv_gpu + first_j);
+        const float *qB = d_qv_gpu + first_j;
+        r0 = rB[lane];
+        r1 = rB[second];
+        q0 = qB[lane];
+        q1 = qB[second];
+    };
+    fetch(boxes[box_of(part_begin)].offset);
+    long next_j = boxes[box_of(part_begin + 1)].offset;
+    int after_next = box_of(part_begin + 2);
+    for (int part = part_begin; part < part_end; ++part) {
+        const auto put = [&](int j, const float4_t &r, float q) {
+            stage[2 * j] = float4_t{scale * r[0], -scale * r[1], -scale * r[2], -scale * r[3]};
+            stage[2 * j + 1] = CENTRED ? float4_t{q, q * (r[1] - centre[0]), q * (r[2] - centre[1]), q * (r[3] - centre[2])}
+                                       : float4_t{q, r[1], r[2], r[3]};
+        };
+        // the wavefront's reads of the part before are behind it: LDS serves a wavefront in order
+        put(lane, r0, q0);
+        if (lane < NUMBER_PAR_PER_BOX - TK_WAVE_SIZE) put(lane + TK_WAVE_SIZE, r1, q1);
+        fetch(next_j);
+        next_j = boxes[after_next].offset;
+        after_next = box_of(part + 3);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+
+        lava_part<P, CENTRED>(home, centre, row, twice, rest, rest_home, lane, stage, total, last_total);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
     }
 }
 
@@ -150,105 +333,9 @@ __device__ __forceinline__ void lava_box(const float scale, const box_str *d_box
         rest_home[lane] = r;
     }
     last_total = fA[4 * (LAVA_REST_FROM + (lane & (LAVA_REST - 1)))];
-    float centre[3];
-    lava_centre(rA, lane, centre);
-    // A neighbour is named by its number alone (its offset in the list is not read): two loads behind one another, and the
-    // particles behind them.  The number is fetched three parts ahead, the offset two, the particles one; where there is no such part,
-    // the home box's own are read.
-    const auto box_of = [&](int part) -> int { return part == 0 || part >= part_end ? bx : boxes[bx].nei[part - 1].number; };
-    const int second = min(lane + TK_WAVE_SIZE, NUMBER_PAR_PER_BOX - 1);   // a lane's second neighbour (past the last: not used)
-    float4_t r0, r1;
-    float q0, q1;
-    const auto fetch = [&](long first_j) {
-        const float4_t *rB = reinterpret_cast<const float4_t *>(d_rv_gpu + first_j);
-        const float *qB = d_qv_gpu + first_j;
-        r0 = rB[lane];
-        r1 = rB[second];
-        q0 = qB[lane];
-        q1 = qB[second];
-    };
-    fetch(boxes[box_of(part_begin)].offset);
-    long next_j = boxes[box_of(part_begin + 1)].offset;
-    int after_next = box_of(part_begin + 2);
-    for (int part = part_begin; part < part_end; ++part) {
-        const auto put = [&](int j, const float4_t &r, float q) {
-            stage[2 * j] = float4_t{scale * r[0], -scale * r[1], -scale * r[2], -scale * r[3]};
-            stage[2 * j + 1] = float4_t{q, q * (r[1] - centre[0]), q * (r[2] - centre[1]), q * (r[3] - centre[2])};
-        };
-        // the wavefront's reads of the part before are behind it: LDS serves a wavefront in order
-        put(lane, r0, q0);
-        if (lane < NUMBER_PAR_PER_BOX - TK_WAVE_SIZE) put(lane + TK_WAVE_SIZE, r1, q1);
-        fetch(next_j);
-        next_j = boxes[after_next].offset;
-        after_next = box_of(part + 3);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-
-        float4_t f[P];   // sums of w, and of vij q (x - c) component by component
-#pragma unroll
-        for (int k = 0; k < P; ++k) f[k] = float4_t{0.f, 0.f, 0.f, 0.f};
-        const lava_lds_float4 *at = stage + 2 * row;
-        float4_t a = at[0], b = at[1];
-        // Six particles a lane are chains enough for the compiler to interleave as it likes (24^3 boxes 829 us, with the step's
-        // read held in front of it 871); with fewer, the reads stay in front of a step's work and every step is written out (3^3 boxes
-        // 36.5 us; 42.1 in a loop of five steps, 43.2 as the compiler likes).
-#pragma unroll P < LAVA_MAX_P ? LAVA_STEPS : 5
-        for (int t = 0; t < LAVA_STEPS; ++t) {
-            at += 2 * LAVA_ROWS;
-            const lava_lds_float4 *next = t + 1 < LAVA_STEPS ? at : stage;   // (the last read is not used)
-            const float4_t na = next[0], nb = next[1];
-            if (P < LAVA_MAX_P) __builtin_amdgcn_sched_barrier(0);
-            // scale (vi + vj - (xi xj + yi yj + zi zj)) = -r2 a2 log2(e), stage by stage over the lane's
-            // particles: their chains are independent, and in this order none waits for its own last result
-            float w[P];
-#pragma unroll
-            for (int k = 0; k < P; ++k) w[k] = home[k][0] + a[0];
-#pragma unroll
-            for (int c = 1; c < 4; ++c)
-#pragma unroll
-                for (int k = 0; k < P; ++k) w[k] = __builtin_fmaf(home[k][c], a[c], w[k]);
-#pragma unroll
-            for (int k = 0; k < P; ++k) w[k] = __builtin_amdgcn_exp2f(w[k]);
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
-#pragma unroll
-                for (int k = 0; k < P; ++k) f[k][c] = __builtin_fmaf(w[k], b[c], f[k][c]);
-            if (P < LAVA_MAX_P) __builtin_amdgcn_sched_barrier(0);
-            a = na;
-            b = nb;
-        }
-#pragma unroll
-        for (int k = 0; k < P; ++k) {
-#pragma unroll
-            for (int c = 1; c < 4; ++c) f[k][c] = __builtin_fmaf(home[k][c] - centre[c - 1], f[k][0], -f[k][c]);
-            total[k] += twice * lava_fold_rows(lava_fold_halves(f[k][0], f[k][1]), lava_fold_halves(f[k][2], f[k][3]));
-        }
-        if (rest) {   // uniform
-            const float4_t last = rest_home[lane & (LAVA_REST - 1)];
-            float4_t g = {0.f, 0.f, 0.f, 0.f};
-            const auto pair = [&](int j) {
-                const float4_t a = stage[2 * j], b = stage[2 * j + 1];
-                float w = last[0] + a[0];
-#pragma unroll
-                for (int c = 1; c < 4; ++c) w = __builtin_fmaf(last[c], a[c], w);
-                w = __builtin_amdgcn_exp2f(w);
-#pragma unroll
-                for (int c = 0; c < 4; ++c) g[c] = __builtin_fmaf(w, b[c], g[c]);
-            };
-            const int from = lane / LAVA_REST;
-#pragma unroll
-            for (int j = 0; j + LAVA_REST_STEP <= NUMBER_PAR_PER_BOX; j += LAVA_REST_STEP) pair(j + from);
-            if (from < NUMBER_PAR_PER_BOX % LAVA_REST_STEP) pair(NUMBER_PAR_PER_BOX / LAVA_REST_STEP * LAVA_REST_STEP + from);
-#pragma unroll
-            for (int c = 1; c < 4; ++c) g[c] = __builtin_fmaf(last[c] - centre[c - 1], g[0], -g[c]);
-#pragma unroll
-            for (int c = 0; c < 4; ++c) g[c] = lava_add_along_row<4>(lava_add_along_row<8>(g[c]));
-            last_total += twice * lava_fold_rows(lava_fold_halves(g[0], g[1]), lava_fold_halves(g[2], g[3]));
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-    }
+    const LavaCentre centre(rA, scale, lane);
+    if (centre.use) lava_parts<P, true>(scale, boxes, d_rv_gpu, d_qv_gpu, bx, part_begin, part_end, home, centre.at, row, twice, rest, lane, stage, total, last_total);
+    else lava_parts<P, false>(scale, boxes, d_rv_gpu, d_qv_gpu, bx, part_begin, part_end, home, centre.at, row, twice, rest, lane, stage, total, last_total);
 #pragma unroll
     for (int k = 0; k < P; ++k) fA[4 * ((sub * P + k) * LAVA_LANES + (lane & (LAVA_LANES - 1)))] = total[k];
     if (rest && (lane & (LAVA_LANES - 1)) < LAVA_REST) fA[4 * (LAVA_REST_FROM + (lane & (LAVA_REST - 1)))] = last_total;

@@ -363,6 +363,79 @@ def test_lava_forces_against_64_bits(boxes1d, offset, far):
         assert np.linalg.norm(got[:, part] - want[:, part]) <= bound * np.linalg.norm(want[:, part])
 
 
+def lava_differences(boxes, q, alpha):
+    """forces on the middle one of 27 boxes in fp32, w (xi - xj) pair by pair, in the kernel's order of sums"""
+    f, up = np.float32, lambda *a: [np.asarray(v, np.float64) for v in a]
+
+    def fma(a, b, c):
+        a, b, c = up(a, b, c)
+        return (a * b + c).astype(f)
+    scale = f(-(f(2) * f(alpha) * f(alpha)) * f(np.log2(np.e)))
+    home, total = boxes[13], np.zeros((100, 3), f)
+    for part in [13] + [b for b in range(27) if b != 13]:
+        near = boxes[part]
+        w = (home[:, :1] * scale + near[:, 0] * scale).astype(f)
+        for c in (1, 2, 3):
+            w = fma(home[:, c:c + 1], -scale * near[:, c], w)
+        w = np.exp2(w.astype(np.float64)).astype(f) * q[part]
+        d, rows = home[:, None, 1:] - near[None, :, 1:], np.zeros((4, 100, 3), f)
+        for j in range(100):
+            rows[j % 4] = fma(w[:, j, None], d[:, j], rows[j % 4])
+        total = total + f(2) * ((rows[0] + rows[2]) + (rows[1] + rows[3]))
+    return total
+
+
+@pytest.mark.parametrize("v,alpha", [("half |x|^2", 0.35), ("half |x|^2", 0.5), ("half |x|^2", 1), ("half |x|^2", 2), ("half |x|^2", 3),
+                                     ("any", 0.5), ("any", 1)])
+def test_lava_forces_are_as_exact_as_sums_of_differences(v, alpha):
+    # the farther a2 = 2 alpha^2 reaches below the size of a box, the more a force about a common centre would lose against
+    # the differences: 1.2 times their error at alpha 1, 1.5 at 2.  Two evaluations with the same roundings but the exponential's
+    # last bit differ by a few per cent over 8 systems of 300 forces.
+    errors = []
+    for seed in range(8):
+        rng = np.random.default_rng(seed)
+        q = rng.uniform(0.1, 1, (27, 100)).astype(np.float32)
+        boxes = rng.uniform(0.1, 1, (27, 100, 4)).astype(np.float32)
+        if v != "any":
+            at = np.array([(x, y, z) for z in (-1, 0, 1) for y in (-1, 0, 1) for x in (-1, 0, 1)])
+            boxes[:, :, 1:] = at[:, None] + rng.uniform(-0.5, 0.5, (27, 100, 3))
+            boxes[:, :, 0] = (boxes[:, :, 1:].astype(np.float64) ** 2).sum(-1) / 2
+        out = torch.zeros((2700, 4), device="cuda:0")
+        ta.gptb_lava(alpha, dev(boxes.reshape(-1, 4)), dev(q.reshape(-1)), out)
+        p, home = boxes.astype(np.float64), boxes[13].astype(np.float64)
+        w = q.astype(np.float64)[:, None] * np.exp(-2 * float(np.float32(alpha)) ** 2 * (
+            home[None, :, :1] + p[:, None, :, 0] - np.stack([home[:, 1:] @ b[:, 1:].T for b in p])))
+        exact = 2 * (w[..., None] * (home[None, :, None, 1:] - p[:, None, :, 1:])).sum((0, 2))
+        errors.append([np.linalg.norm(got - exact) / np.linalg.norm(exact)
+                       for got in (host(out)[1300:1400, 1:], lava_differences(boxes, q, alpha))])
+    got, differences = np.sqrt(np.mean(np.square(errors), 0))
+    print(f"v {v}, alpha {alpha}: {got:.3e}, by differences {differences:.3e}")
+    assert got <= 1.1 * differences
+
+
+@pytest.mark.parametrize("boxes1d,launch_grid", [(2, 1), (3, 40), (5, 256), (9, 700)])
+def test_lava_every_cut_gives_the_same_bits_in_either_form(boxes1d, launch_grid):
+    # alpha at which some boxes take the form about their centre and others, wider ones, the differences
+    rv, qv = lava_inputs(boxes1d, seed=60 + boxes1d)
+    wide = np.arange(len(rv)) // 100 % 3 == 1
+    rv[wide, 1:] = 3 * rv[wide, 1:] - 1
+    rv[wide, 0] = (rv[wide, 1:] ** 2).sum(1) / 2
+    d_r, d_q = dev(rv), dev(qv)
+    out = [torch.zeros((rv.shape[0], 4), device="cuda:0") for _ in range(5)]
+    ta.gptb_lava(0.5, d_r, d_q, out[0])
+    ta.ori_lava(0.5, d_r, d_q, out[1])
+    ta.gptb_lava(0.5, d_r, d_q, out[2], launch_grid=launch_grid, launch_block=256)
+    ta.gptb_lava(0.5, d_r, d_q, out[3], launch_grid=launch_grid, launch_block=64)
+    n = ta.lava_blocks(boxes1d)
+    cuts = [0, n // 5, n // 2 + 1, n]
+    for a, b in zip(cuts, cuts[1:]):
+        ta.gptb_lava(0.5, d_r, d_q, out[4], a, b)
+    for o in out[1:]:
+        assert np.array_equal(bits(o), bits(out[0]))
+    if boxes1d <= 3:
+        assert lava_close(host(out[0]), oracle.lava(0.5, boxes1d, rv, qv))
+
+
 @pytest.mark.parametrize("seed", range(4))
 def test_lava_any_ascending_tiling_of_the_positions(seed):
     rng = np.random.default_rng(400 + seed)
