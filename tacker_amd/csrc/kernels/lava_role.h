@@ -23,7 +23,10 @@
 //    little across the box.  Forces against 64 bits, 2-norm over the middle box of 3^3, 60 systems, differences / this form
 //    where it is taken: unit boxes around the origin, v = |x|^2 / 2, alpha 0.35 12.3 / 12.0e-8, 0.5 13.3 / 13.0e-8; x and v in
 //    0.1 ... 1 in every box, alpha 0.35 8.0 / 8.1e-8, 0.5 7.9 / 8.1e-8.  Where it is not taken it would be off by more: unit boxes,
-//    alpha 1 25.8 / 30.7e-8, 2 58 / 86e-8 (with a centre off the grid, which cost 8 % at 0.5).  Those boxes take the differences.
+//    alpha 1 25.8 / 30.7e-8, 2 58 / 86e-8 (with a centre off the grid, which cost 8 % at 0.5).  Those boxes take the differences, and
+//    so does one in which v differ so much (LAVA_CENTRED_V) that a particle's weight on itself, which no force comes from, could
+//    be larger than all the others' together: with one v of -30 among 0.1 ... 1 the form about the centre is off by 3.9e-4, they by 5.9e-7.
+//    A total that is not finite is computed once more from them.
 //  * What is computed per neighbour and not per pair.  A wavefront prepares the 100 neighbours of a part once, a lane
 //    each: {scale v, -scale x, -scale y, -scale z} and {q, q (x - cx), q (y - cy), q (z - cz)} go to LDS and
 //    come back as two 16-byte broadcast reads a step.  (By a vector load for every step and row of lanes, and four multiplies
@@ -33,8 +36,9 @@
 //    particles are four lanes side by side, 16 neighbours at a time: 7 steps, where a seventh particle a lane would take 25.
 // A pair is 8 such instructions and the exponential, 12 from the differences.  At the end of a part the four rows' sums are added,
 // (g0 + g2) + (g1 + g3), by lane swaps that add two values at once, which leaves component v, y, x, z of the
-// total in row 0, 1, 2, 3; the total goes on from the output array.  24^3 boxes: 837 us (35 cycles a SIMD and step of 64 pairs), where twelve instructions
-// a pair, neighbours by vector loads and seven particles a lane took 1325; 18^3 372 / 577, 9^3 78 / 116, 3^3 36.5 / 46.
+// total in row 0, 1, 2, 3; the total goes on from the output array.  24^3 boxes: 835 us (35 cycles a SIMD and step of 64 pairs), from
+// the differences 1130, where neighbours by vector loads and seven particles a lane took 1325; 18^3 361 / 475 / 577, 9^3 71 / 80 / 116,
+// 3^3 37 / 41 / 46.
 //
 // Few boxes: a box is then split over several wavefronts (P home particles a lane instead of 6, every particle
 // summed exactly as before), see LavaUnits.
@@ -62,6 +66,7 @@ typedef __attribute__((address_space(4))) const box_str lava_const_box;
 #define LAVA_WAVES_PER_SIMD 4                           // wavefronts of this role a SIMD holds (registers)
 #define LAVA_STEPS (NUMBER_PAR_PER_BOX / LAVA_ROWS)     // neighbours a row takes per box
 #define LAVA_CENTRED 0.72f                              // a2 log2(e) |x - c|^2 up to which forces are computed about the centre
+#define LAVA_CENTRED_V 4.f                              // ... and a2 log2(e) times how far v - c x may differ: a weight on itself of 2^4 of the usual
 #define LAVA_REST 4                                     // home particles behind the lanes' own ...
 #define LAVA_REST_FROM (NUMBER_PAR_PER_BOX - LAVA_REST)
 #define LAVA_REST_STEP (TK_WAVE_SIZE / LAVA_REST)       // ... and the neighbours they take a step
@@ -163,6 +168,15 @@ struct LavaCentre {
             hi2 += (hi[c + 1] - at[c]) * (hi[c + 1] - at[c]);
         }
         use = -scale * lava_largest(__builtin_fmaxf(lo2, hi2)) <= LAVA_CENTRED;   // (not where a2 is no number)
+        // what the v of its particles make of their weights beside the others': v - c x
+        lo2 = lo[0], hi2 = hi[0];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            lo2 = __builtin_fmaf(-at[c], lo[c + 1], lo2);
+            hi2 = __builtin_fmaf(-at[c], hi[c + 1], hi2);
+        }
+        const float most = lava_largest(__builtin_fmaxf(lo2, hi2)), least = -lava_largest(__builtin_fmaxf(-lo2, -hi2));
+        use = use && -scale * (most - least) <= LAVA_CENTRED_V;
     }
 };
 
@@ -334,11 +348,33 @@ __device__ __forceinline__ void lava_box(const float scale, const box_str *d_box
     }
     last_total = fA[4 * (LAVA_REST_FROM + (lane & (LAVA_REST - 1)))];
     const LavaCentre centre(rA, scale, lane);
-    if (centre.use) lava_parts<P, true>(scale, boxes, d_rv_gpu, d_qv_gpu, bx, part_begin, part_end, home, centre.at, row, twice, rest, lane, stage, total, last_total);
-    else lava_parts<P, false>(scale, boxes, d_rv_gpu, d_qv_gpu, bx, part_begin, part_end, home, centre.at, row, twice, rest, lane, stage, total, last_total);
+    const auto slot = [&](int k) -> float & { return fA[4 * ((sub * P + k) * LAVA_LANES + (lane & (LAVA_LANES - 1)))]; };
+    float &last_slot = fA[4 * (LAVA_REST_FROM + (lane & (LAVA_REST - 1)))];
+    const bool last_here = rest && (lane & (LAVA_LANES - 1)) < LAVA_REST;
+    unsigned todo = ~0u;   // bit k, or P: this total is still to be computed
+    if (centre.use) {
+        lava_parts<P, true>(scale, boxes, d_rv_gpu, d_qv_gpu, bx, part_begin, part_end, home, centre.at, row, twice, rest, lane, stage, total, last_total);
+        // What is not finite is computed once more from the differences, from where it began: they are finite where a charge and a distance
+        // whose product is not meet a weight of zero, and have signs where weights are infinite.
+        todo = 0;
+        const auto keep = [&](int k, float &in_memory, float &value) {
+            if (__builtin_fabsf(value) <= FLT_MAX) {
+                in_memory = value;
+            } else {
+                value = in_memory;
+                todo |= 1u << k;
+            }
+        };
 #pragma unroll
-    for (int k = 0; k < P; ++k) fA[4 * ((sub * P + k) * LAVA_LANES + (lane & (LAVA_LANES - 1)))] = total[k];
-    if (rest && (lane & (LAVA_LANES - 1)) < LAVA_REST) fA[4 * (LAVA_REST_FROM + (lane & (LAVA_REST - 1)))] = last_total;
+        for (int k = 0; k < P; ++k) keep(k, slot(k), total[k]);
+        if (last_here) keep(P, last_slot, last_total);
+        if (__builtin_amdgcn_ballot_w64(todo != 0) == 0) return;
+    }
+    lava_parts<P, false>(scale, boxes, d_rv_gpu, d_qv_gpu, bx, part_begin, part_end, home, centre.at, row, twice, rest, lane, stage, total, last_total);
+#pragma unroll
+    for (int k = 0; k < P; ++k)
+        if (todo >> k & 1) slot(k) = total[k];
+    if (last_here && (todo >> P & 1)) last_slot = last_total;
 }
 
 // wavefronts a box is split over with P home particles a lane

@@ -386,17 +386,20 @@ def lava_differences(boxes, q, alpha):
 
 
 @pytest.mark.parametrize("v,alpha", [("half |x|^2", 0.35), ("half |x|^2", 0.5), ("half |x|^2", 1), ("half |x|^2", 2), ("half |x|^2", 3),
-                                     ("any", 0.5), ("any", 1)])
+                                     ("any", 0.5), ("any", 1), ("heavy", 0.5)])
 def test_lava_forces_are_as_exact_as_sums_of_differences(v, alpha):
     # the farther a2 = 2 alpha^2 reaches below the size of a box, the more a force about a common centre would lose against
     # the differences: 1.2 times their error at alpha 1, 1.5 at 2.  Two evaluations with the same roundings but the exponential's
-    # last bit differ by a few per cent over 8 systems of 300 forces.
+    # last bit differ by a few per cent over 8 systems of 300 forces.  A particle whose v makes its weight on itself, which no
+    # force comes from, larger than all the others' (heavy) would make it lose at any alpha.
     errors = []
     for seed in range(8):
         rng = np.random.default_rng(seed)
         q = rng.uniform(0.1, 1, (27, 100)).astype(np.float32)
         boxes = rng.uniform(0.1, 1, (27, 100, 4)).astype(np.float32)
-        if v != "any":
+        if v == "heavy":
+            boxes[13, 5, 0] = -30
+        if v == "half |x|^2":
             at = np.array([(x, y, z) for z in (-1, 0, 1) for y in (-1, 0, 1) for x in (-1, 0, 1)])
             boxes[:, :, 1:] = at[:, None] + rng.uniform(-0.5, 0.5, (27, 100, 3))
             boxes[:, :, 0] = (boxes[:, :, 1:].astype(np.float64) ** 2).sum(-1) / 2
@@ -411,6 +414,34 @@ def test_lava_forces_are_as_exact_as_sums_of_differences(v, alpha):
     got, differences = np.sqrt(np.mean(np.square(errors), 0))
     print(f"v {v}, alpha {alpha}: {got:.3e}, by differences {differences:.3e}")
     assert got <= 1.1 * differences
+
+
+@pytest.mark.parametrize("what", ["far", "infinite weight", "large charges"])
+@pytest.mark.parametrize("boxes1d,alpha", [(3, 0.5), (3, 0.1), (8, 0.5)])
+def test_lava_what_is_not_finite_is_what_the_differences_give(boxes1d, alpha, what):
+    # a particle of another box so far away that its charge times its distance is infinite, with a weight of zero; one whose
+    # weight is infinite; charges whose sum is.  boxes1d 8: a wavefront serves a part of a box
+    rng = np.random.default_rng(12)
+    boxes, q = (rng.uniform(0.1, 1, (boxes1d ** 3, 100, k)).astype(np.float32).squeeze() for k in (4, 1))
+    if what == "far":
+        boxes[0, 7, :2], q[0, 7] = (np.inf, 1e30), 1e10
+    elif what == "infinite weight":
+        boxes[0, 7, 0] = -1e6
+    else:
+        q[0, :40] = 3e37
+    out = torch.zeros((100 * boxes1d ** 3, 4), device="cuda:0")
+    ta.gptb_lava(alpha, dev(boxes.reshape(-1, 4)), dev(q.reshape(-1)), out)
+    # the middle one of the 3 x 3 x 3 boxes in the corner where box 0 is
+    block = [x + boxes1d * (y + boxes1d * z) for z in range(3) for y in range(3) for x in range(3)]
+    got = host(out)[100 * block[13]:100 * block[13] + 100]
+    with np.errstate(all="ignore"):
+        want = lava_differences(boxes[block], q[block], alpha)
+    assert np.array_equal(np.isnan(got[:, 1:]), np.isnan(want))
+    finite = np.isfinite(want)
+    assert np.array_equal(got[:, 1:][~finite], want[~finite], equal_nan=True)
+    assert finite.all() if what == "far" else not finite.all()
+    # 2 ulp of the exponential at arguments below 4, and 2700 terms
+    np.testing.assert_allclose(got[:, 1:][finite], want[finite], rtol=2e-4, atol=2e-3 * (1 if what == "far" else 1e37))
 
 
 @pytest.mark.parametrize("boxes1d,launch_grid", [(2, 1), (3, 40), (5, 256), (9, 700)])
