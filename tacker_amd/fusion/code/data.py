@@ -38,7 +38,8 @@ REFERENCE_KERNEL_INFO = {
 
 # gfx950 roles.  register = VGPRs per lane of the role compiled alone (the
 # compiler's kernel-resource-usage remarks), shared_memory = LDS bytes
-# per role instance, blocksize = threads of one role instance (a multiple of the
+# per role instance in a fused launch (mri-q's and mri-fhd's own GPTB kernels
+# hold it for workgroups of 16 wavefronts: 16384 and 20480), blocksize = threads of one role instance (a multiple of the
 # 64-wide wavefront), solo_ptb_blks = role instances per CU of the plain GPTB
 # launch, ori_blks = blocks of the reference-shaped natural grid at the
 # benchmark's problem size.
@@ -51,10 +52,10 @@ KERNEL_INFO = {
     "lbm": {"register": 64, "shared_memory": 0, "blocksize": 256, "solo_ptb_blks": 16,
             "ori_blks": 18000},
     # 1024 blocks of 256 voxels x 16 chunks of 128 k records
-    "mriq": {"register": 40, "shared_memory": 0, "blocksize": 256, "solo_ptb_blks": 8,
+    "mriq": {"register": 100, "shared_memory": 4096, "blocksize": 256, "solo_ptb_blks": 8,
              "ori_blks": 16384},
     # 1024 blocks of 256 voxels x 16 chunks of 128 k records
-    "mrif": {"register": 44, "shared_memory": 0, "blocksize": 256, "solo_ptb_blks": 8,
+    "mrif": {"register": 110, "shared_memory": 5120, "blocksize": 256, "solo_ptb_blks": 8,
              "ori_blks": 16384},
     # 32 x 258 blocks of 128 rows x 16 columns of C x 64 parts of 64 k steps (4096 x 4128 x 4064)
     "sgemm": {"register": 64, "shared_memory": 0, "blocksize": 128, "solo_ptb_blks": 16,
@@ -63,7 +64,7 @@ KERNEL_INFO = {
     "fft": {"register": 40, "shared_memory": 8192, "blocksize": 256, "solo_ptb_blks": 8,
             "ori_blks": 10240},
     # 26 x 26 x 2 regions of 8 x 8 x 8 lattice points (two wavefronts each) x 11 parts of 32 neighbour bins
-    "cutcp": {"register": 94, "shared_memory": 2048, "blocksize": 128, "solo_ptb_blks": 16,
+    "cutcp": {"register": 94, "shared_memory": 4096, "blocksize": 128, "solo_ptb_blks": 16,
               "ori_blks": 14872},
     # 2560000 blocks of 256 records; a stream that wants many workgroups in flight (4.0 TB/s with 8 a CU,
     # 4.95 with 32)
@@ -76,10 +77,10 @@ KERNEL_INFO = {
     # 216000 boxes of 100 particles (a wavefront each) x 27 parts (the home box and its neighbour slots);
     # boxes on the faces have fewer neighbours: the more owner wavefronts, the evener their shares
     # (42.4 ms with 4 workgroups a CU, 35.8 with 32)
-    "lava": {"register": 119, "shared_memory": 0, "blocksize": 256, "solo_ptb_blks": 32,
+    "lava": {"register": 127, "shared_memory": 13056, "blocksize": 256, "solo_ptb_blks": 32,
              "ori_blks": 5832000},
     # 200 windows of 256 columns (6 result columns each), a wavefront each
-    "path": {"register": 77, "shared_memory": 0, "blocksize": 256, "solo_ptb_blks": 1,
+    "path": {"register": 78, "shared_memory": 0, "blocksize": 256, "solo_ptb_blks": 1,
              "ori_blks": 200},
     # 16384 blocks of 128 x 8 points x 4 parts of the unrolled x points
     "cp": {"register": 40, "shared_memory": 0, "blocksize": 128, "solo_ptb_blks": 16,
