@@ -13,7 +13,7 @@
 // The kernel has the shape of MRI-Q (a voxel block times a run of k records) and
 // shares its walk over block positions (mriq_role.h): x = blocks of 256 voxels,
 // y = chunks of MRIF_K_CHUNK records, one owner thread group per voxel block.
-// As there, the hardware sine and cosine take the phase in revolutions, the records come through LDS, and the
+// The hardware sine and cosine take the phase in revolutions, the records come through a wavefront's LDS, and the
 // multiply-adds are fused the way the reference's source contracts under nvcc's
 // default -fmad=true: the product on the left of each sum or difference is
 // folded into it, fma(RhoPhiR, cos, -(RhoPhiI*sin)) and fma(RhoPhiI, cos,
@@ -25,6 +25,11 @@
 __constant__ mrif_kValues c_mrif[MRIF_MAX_K];
 
 namespace tk {
+
+template <int N>
+struct mrif_count {
+    static constexpr int value = N;
+};
 
 static_assert(MRIF_K_CHUNK == MRIQ_K_CHUNK && KERNEL_FH_THREADS_PER_BLOCK == KERNEL_Q_THREADS_PER_BLOCK,
               "MRI-FHD shares MRI-Q's position grid: same voxel block and k chunk");
@@ -48,8 +53,8 @@ __device__ __forceinline__ void mrif_voxels(int k_begin, int k_end, const float 
         sOutR[v] = outR[i];
         sOutI[v] = outI[i];
     }
-    // U records at a time, stage by stage, as in mriq_voxels: the U * V chains are independent
-    // until the accumulation, which runs in ascending k.
+    // U records at a time, written stage by stage (all phases, then all sines and cosines, then the accumulation in ascending k): the
+    // U * V chains are independent until the last stage, and the source's order is the interleaved one already.
     constexpr int U = 4;
     const auto add = [&](const float4_t *k, const float *imaginary, auto records) {
         constexpr int N = decltype(records)::value;
@@ -93,7 +98,7 @@ __device__ __forceinline__ void mrif_voxels(int k_begin, int k_end, const float 
         };
         const auto use = [&](const float4_t (&r)[U], const float4_t &imaginary) {
             const float im[U] = {imaginary[0], imaginary[1], imaginary[2], imaginary[3]};
-            add(r, im, mriq_count<U>());
+            add(r, im, mrif_count<U>());
             __builtin_amdgcn_sched_barrier(0);
         };
         float4_t ka[U], kb[U], ia, ib;
@@ -108,7 +113,7 @@ __device__ __forceinline__ void mrif_voxels(int k_begin, int k_end, const float 
         for (; i < count; ++i) {   // (the table's last records)
             const float4_t one[1] = {stage[i]};
             const float im[1] = {stage_imaginary[i]};
-            add(one, im, mriq_count<1>());
+            add(one, im, mrif_count<1>());
         }
         mriq_stage_fence();
     }
@@ -120,15 +125,23 @@ __device__ __forceinline__ void mrif_voxels(int k_begin, int k_end, const float 
 }
 
 struct MrifBody {
+    static constexpr int AT_ONCE = 4;
+    static constexpr bool SHARES = false;   // a block's voxels over more wavefronts than they fill
     static constexpr int STAGE_QUADS = TK_WAVE_SIZE + TK_WAVE_SIZE / 4;
     static __device__ __forceinline__ int chunk() { return MRIF_K_CHUNK; }
-    template <int V>
+    static __device__ __forceinline__ int parts(int, int) { return KERNEL_FH_THREADS_PER_BLOCK / TK_WAVE_SIZE; }
+    template <int V, int T>
     static __device__ __forceinline__ void voxels(int k_begin, int k_end, const float *__restrict__ x,
                                                   const float *__restrict__ y, const float *__restrict__ z,
                                                   float *__restrict__ outR, float *__restrict__ outI,
-                                                  const int (&xIndex)[V], mriq_lds_float4 *stage)
+                                                  const int (&base)[V], mriq_lds_float4 *stage)
     {
-        mrif_voxels<V>(k_begin, k_end, x, y, z, outR, outI, xIndex, stage);
+        if constexpr (T == 4) {
+            int xIndex[V];
+#pragma unroll
+            for (int v = 0; v < V; ++v) xIndex[v] = base[v] + mriq_lane();
+            mrif_voxels<V>(k_begin, k_end, x, y, z, outR, outI, xIndex, stage);
+        }
     }
 };
 

@@ -13,13 +13,12 @@
 // gfx950: what bounds it is VALU issue.  The hardware sine and cosine take their argument in revolutions and reduce
 // it themselves, at any size: the phase k.x goes to them as it is, cos(2 pi p) = v_cos(p).  (Over the whole range of
 // floats they are within 1.3e-7 of sine and cosine; behind a v_fract, which rounds a negative phase to a whole turn's
-// last bit, within 2.7e-7 at |p| < 300 and the same above.)  The dot product and the two accumulations are fused
-// multiply-adds in the reference's order (((Kx*x) + Ky*y) + Kz*z; Q + PhiMag*c) -- what nvcc makes of the reference's
-// source with its default -fmad=true -- so a (k, x) pair is 5 such instructions and the two transcendentals.  The five
-// take 2.5 to 2.8 cycles of a SIMD with two wavefronts at work if all their operands are vector registers and 4.4 with a
-// scalar one (v_fract 4.3, sine and cosine 8.5 each), so a wavefront brings the records, 64 at a time, through LDS of its
-// own and reads each back with one 16-byte broadcast.  2048 records and 262144 voxels: 130 us alone, 145 beside tzgemm
-// 2048^3; 153 and 161 with the records in scalar registers and a v_fract.  (Without the v_fract alone: 152 and 153.)
+// last bit, within 2.7e-7 at |p| < 300 and the same above.)  A (k, x) pair is the two transcendentals, 8.45 cycles of a SIMD each, two fused
+// multiply-adds of 2.75 (Q + PhiMag*c, as nvcc contracts the reference's source with its default -fmad=true) and a 256th of a matrix
+// instruction, 4 cycles that the vector units need not wait for while other wavefronts have something for them: the phase (mriq_put_point below).
+// With the phase as three multiply-adds in the reference's order, ((Kx*x) + Ky*y) + Kz*z, 2032 records and 262144 voxels took 130 us alone and
+// 144 to 151 beside tzgemm 2048^3, so 104 and 118, and with the transcendentals first 104 and 112; 700 records and 65536 voxels beside tzgemm 1024^3
+// 21.2 to 22.1, now 18.5.
 // The result differs from a float64 evaluation by about 1e-6 per term, far inside the 1e-3 + 1e-4 |Q| bar.
 #pragma once
 #include "role_common.h"
@@ -28,11 +27,6 @@
 __constant__ mriq_kValues ck[MRIQ_MAX_K];
 
 namespace tk {
-
-template <int N>
-struct mriq_count {
-    static constexpr int value = N;
-};
 
 typedef __attribute__((address_space(3))) float4_t mriq_lds_float4;
 
@@ -54,160 +48,267 @@ __device__ __forceinline__ void mriq_stage_fence()
 
 __device__ __forceinline__ int mriq_lane() { return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
 
-// V voxels per thread at once, k records [k_begin, k_end).  The k loop is a chain of
-// dependent operations per voxel (dot product, sin/cos, accumulate) and a fused
-// launch leaves the role at most two waves per SIMD, so the independent work that hides
-// instruction latency has to come from inside the thread; V voxels also share each
-// read of a k record.  stage: this wavefront's LDS.
-template <int V>
-__device__ __forceinline__ void mriq_voxels(int k_begin, int k_end, const float *__restrict__ x,
-                                            const float *__restrict__ y, const float *__restrict__ z,
-                                            float *__restrict__ Qr, float *__restrict__ Qi,
-                                            const int (&xIndex)[V], mriq_lds_float4 *stage)
+// A phase k.x by the matrix units.  A float is the sum of three bf16 pieces, each the rest rounded to nearest, and products of
+// pieces are exact in the matrix instruction's fp32 sum, so eight of the nine products of pieces of a coordinate (not the one of the two last,
+// 2^-32 of it) for three coordinates are 24 of the 32 slots of one v_mfma_f32_16x16x32_bf16, which gives 256 phases in 16 cycles of a SIMD
+// where three multiply-adds in fp32 take 32, and leaves the vector units to others part of the time.
+//
+// In LDS a point -- a record's K or a voxel -- is three tokens of four bf16, {x, y, z, 0} of its first, second and third pieces.  Lanes
+// 16 g .. 16 g + 15 hold slots 8 g .. 8 g + 7 of an operand, two tokens; which ones decides how the products add up.  The sum
+// runs from group 0 to 3, so the largest product comes last, with the smallest: phases then have less error than the chain of three
+// multiply-adds (2-norm against 64 bits: |K|, |x| up to 0.5 4.2e-9 for 5.1e-9, up to 20 7.7e-6 for 8.3e-6; with the largest first 6.7e-9 and 11e-6).
+typedef __bf16 mriq_bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 mriq_bf16x8 __attribute__((ext_vector_type(8)));
+typedef float mriq_float2 __attribute__((ext_vector_type(2)));
+typedef unsigned mriq_uint2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) mriq_uint2 mriq_lds_token;
+#define MRIQ_TOKENS 3   // of a point
+#define MRIQ_TILE 16    // records, and voxels, of a matrix instruction
+
+struct MriqSlots {
+    // tokens of lane group g, one digit of 8 bits a group
+    static __device__ __forceinline__ int pick(unsigned digits, int group) { return (int)(digits >> (8 * group)) & 3; }
+    int record[2], voxel[2];
+    __device__ __forceinline__ explicit MriqSlots(int group)
+        : record{pick(0x00000001u, group), pick(0x02010201u, group)}, voxel{pick(0x00010202u, group), pick(0x01000001u, group)} {}
+};
+
+// the next pieces of two values, which lose them
+__device__ __forceinline__ unsigned mriq_pieces(float &a, float &b)
 {
-    if (k_begin >= k_end) return;
-    float sX[V], sY[V], sZ[V], sQr[V], sQi[V];
+    const unsigned p = __builtin_bit_cast(unsigned, __builtin_convertvector(mriq_float2{a, b}, mriq_bf16x2));
+    a -= __uint_as_float(p << 16);
+    b -= __uint_as_float(p & 0xffff0000u);
+    return p;
+}
+
+__device__ __forceinline__ void mriq_put_point(mriq_lds_token *tokens, float x, float y, float z)
+{
+    float nothing = 0.f;
 #pragma unroll
-    for (int v = 0; v < V; ++v) {
-        const int i = xIndex[v];
-        sX[v] = x[i];
-        sY[v] = y[i];
-        sZ[v] = z[i];
-        sQr[v] = Qr[i];
-        sQi[v] = Qi[i];
-    }
-    const int lane = mriq_lane();
-    const float4_t *table = reinterpret_cast<const float4_t *>(ck);
-    // (a voxel alone needs eight records to have enough chains: 2048 x 65536, one voxel a lane and one or two wavefronts a
-    // SIMD, 51.9 us with four, 46.6 with eight; beside tzgemm 1024^3 57.2 and 48.9)
-    constexpr int U = V == 1 ? 8 : 4;
-    // U records at a time, written stage by stage (all phases, then all sines and cosines,
-    // then the accumulation in ascending k): the U * V chains are independent until the last
-    // stage, and the order of the source is already the interleaved one -- the compiler's
-    // scheduler does not have to find it (for one of the instances in a fused kernel it did
-    // not, and that loop ran one dependent chain at a time).
-    const auto add = [&](const float4_t *k, auto records) {
-        constexpr int N = decltype(records)::value;
-        float c[N][V], s[N][V];
-#pragma unroll
-        for (int u = 0; u < N; ++u)
-#pragma unroll
-            for (int v = 0; v < V; ++v)   // revolutions
-                c[u][v] = __builtin_fmaf(k[u].z, sZ[v], __builtin_fmaf(k[u].y, sY[v], k[u].x * sX[v]));
-#pragma unroll
-        for (int u = 0; u < N; ++u)
-#pragma unroll
-            for (int v = 0; v < V; ++v) {
-                s[u][v] = __builtin_amdgcn_sinf(c[u][v]);
-                c[u][v] = __builtin_amdgcn_cosf(c[u][v]);
-            }
-#pragma unroll
-        for (int u = 0; u < N; ++u)
-#pragma unroll
-            for (int v = 0; v < V; ++v) {
-                sQr[v] = __builtin_fmaf(k[u].w, c[u][v], sQr[v]);
-                sQi[v] = __builtin_fmaf(k[u].w, s[u][v], sQi[v]);
-            }
-    };
-    float4_t ahead = table[min(k_begin + lane, k_end - 1)];
-    for (int k0 = k_begin; k0 < k_end; k0 += TK_WAVE_SIZE) {
-        stage[lane] = ahead;
-        ahead = table[min(k0 + TK_WAVE_SIZE + lane, k_end - 1)];
-        mriq_stage_fence();
-        const int count = min(TK_WAVE_SIZE, k_end - k0);
-        const auto read = [&](float4_t (&r)[U], int first) {
-#pragma unroll
-            for (int u = 0; u < U; ++u) r[u] = stage[(first & (TK_WAVE_SIZE - 1)) + u];
-            __builtin_amdgcn_sched_barrier(0);   // on its way while the records before it are used
-        };
-        float4_t ka[U], kb[U];
-        read(ka, 0);
-        int i = 0;
-        for (; i + 2 * U <= count; i += 2 * U) {
-            read(kb, i + U);
-            add(ka, mriq_count<U>());
-            __builtin_amdgcn_sched_barrier(0);
-            read(ka, i + 2 * U);
-            add(kb, mriq_count<U>());
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        // The table's last records: up to 15 one by one with a voxel alone, up to 7 with more.  They cost 0.4 to 1.1 us of a launch: 262144
-        // voxels, 2032 records 130.3 us and 2047 131.4, 128 and 143 10.9 and 12.5; 65536 voxels 46.1 and 46.9, 5.9 and 6.7.  (The records
-        // in scalar registers took 152.9 and 154.4, 12.3 and 13.1, 69.0 and 69.9, 6.8 and 7.4 there.)
-        for (; i < count; ++i) {
-            const float4_t one[1] = {stage[i]};
-            add(one, mriq_count<1>());
-        }
-        mriq_stage_fence();
-    }
-#pragma unroll
-    for (int v = 0; v < V; ++v) {
-        Qr[xIndex[v]] = sQr[v];
-        Qi[xIndex[v]] = sQi[v];
+    for (int i = 0; i < MRIQ_TOKENS; ++i) {
+        const unsigned xy = mriq_pieces(x, y);
+        tokens[i] = mriq_uint2{xy, mriq_pieces(z, nothing)};
     }
 }
 
-// What a thread does for V voxels and a run of k records: the part of the kernel that the
+__device__ __forceinline__ mriq_bf16x8 mriq_slots(const mriq_lds_token *point, const int (&tokens)[2])
+{
+    const mriq_uint2 a = point[tokens[0]], b = point[tokens[1]];
+    return __builtin_bit_cast(mriq_bf16x8, uint4_t{a.x, a.y, b.x, b.y});
+}
+
+// the halves of a wavefront, and the rows of 16 lanes, added by lane swaps that add two values at once
+__device__ __forceinline__ float mriq_fold_halves(float a, float b)
+{
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);   // lower half: sum of a's, upper half: of b's
+}
+__device__ __forceinline__ float mriq_fold_rows(float a, float b)
+{
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);   // even rows: sum of a's pair, odd rows: of b's
+}
+
+// V times T tiles of 16 voxels of a wavefront, from voxel base[v] on, k records [k_begin, k_end) from a multiple of MRIQ_K_CHUNK.  The wavefront
+// brings 64 records at a time through its LDS.  A lane has voxel 16 t + lane % 16 of every tile t of 16 and, of 16 records, the four
+// 4 (lane / 16) ..: its sums over a chunk of records are added to the other three lane groups' at the chunk's end, and that to Q, so any
+// split at chunks gives the same bits.  The last records of the table come in a whole tile of 16, with weights of zero behind them.
+// stage: this wavefront's LDS.
+template <int V, int T>
+__device__ __forceinline__ void mriq_voxels(int k_begin, int k_end, const float *__restrict__ x,
+                                            const float *__restrict__ y, const float *__restrict__ z,
+                                            float *__restrict__ Qr, float *__restrict__ Qi,
+                                            const int (&base)[V], mriq_lds_float4 *stage)
+{
+    static_assert(T == 1 || T == 2 || T == 4, "the folds leave a lane one voxel's sums");
+    if (k_begin >= k_end) return;
+    constexpr int GROUPS = TK_WAVE_SIZE / MRIQ_TILE, TILES = T * V, AHEAD = TILES == 1 ? 1 : 2;
+    const int lane = mriq_lane();
+    const int group = lane / MRIQ_TILE, column = lane % MRIQ_TILE;
+    const MriqSlots slots(group);
+    mriq_lds_token *const points = (mriq_lds_token *)stage;
+    __attribute__((address_space(3))) float *const weights =
+        (__attribute__((address_space(3))) float *)(points + MRIQ_TOKENS * TK_WAVE_SIZE);
+    // the tile whose sum the folds leave here
+    const int own_tile = T == 4 ? (group == 1 ? 2 : (group == 2 ? 1 : group)) : (T == 2 ? group / 2 : 0);
+
+    mriq_bf16x8 voxel[TILES];
+    int own[V];   // this lane's voxel of each 64, whose sums the folds leave here
+    float totalR[V], totalI[V];
+    const float4_t *table = reinterpret_cast<const float4_t *>(ck);
+    float4_t ahead = table[min(k_begin + lane, k_end - 1)];
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        const int i = base[v] + lane % (T * MRIQ_TILE);
+        own[v] = base[v] + MRIQ_TILE * own_tile + column;
+        totalR[v] = Qr[own[v]];
+        totalI[v] = Qi[own[v]];
+        mriq_put_point(points + MRIQ_TOKENS * lane, x[i], y[i], z[i]);
+        mriq_stage_fence();
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+            voxel[T * v + t] = mriq_slots(points + MRIQ_TOKENS * (MRIQ_TILE * t + column), slots.voxel);
+        mriq_stage_fence();
+    }
+    float r[TILES], i[TILES];
+    const auto phases = [&](const mriq_bf16x8 &k, int t) {
+        const float4_t zero = {0.f, 0.f, 0.f, 0.f};
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(k, voxel[t], zero, 0, 0, 0);
+    };
+    // two tiles at a time, the matrix instructions of the next two in front of their sines.  (The next records' first ones in front of the last
+    // tiles' sines as well, and records read another step ahead: 122 us for 112 beside tzgemm 2048^3.)
+    const auto add = [&](const mriq_bf16x8 &k, const float4_t &w) {
+        float4_t now[AHEAD];
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) now[u] = phases(k, u);
+#pragma unroll
+        for (int t = 0; t < TILES; t += AHEAD) {
+            float4_t next[AHEAD];
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u) next[u] = t + AHEAD < TILES ? phases(k, t + AHEAD + u) : now[u];
+            float c[AHEAD][4], s[AHEAD][4];
+            if (T == 4) transcendentals_begin();   // (with fewer tiles the compiler's order is worth more: 65536 voxels 27.0 us for 30.9)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int u = 0; u < AHEAD; ++u) {   // revolutions
+                    c[u][e] = __builtin_amdgcn_cosf(now[u][e]);
+                    s[u][e] = __builtin_amdgcn_sinf(now[u][e]);
+                }
+            if (T == 4) transcendentals_end();
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int u = 0; u < AHEAD; ++u) {
+                    r[t + u] = __builtin_fmaf(w[e], c[u][e], r[t + u]);
+                    i[t + u] = __builtin_fmaf(w[e], s[u][e], i[t + u]);
+                }
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u) now[u] = next[u];
+        }
+    };
+    for (int chunk = k_begin; chunk < k_end; chunk += MRIQ_K_CHUNK) {
+        const int chunk_end = min(chunk + MRIQ_K_CHUNK, k_end);
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) r[t] = i[t] = 0.f;
+        for (int k0 = chunk; k0 < chunk_end; k0 += TK_WAVE_SIZE) {
+            mriq_put_point(points + MRIQ_TOKENS * lane, ahead.x, ahead.y, ahead.z);
+            weights[lane] = k0 + lane < k_end ? ahead.w : 0.f;
+            ahead = table[min(k0 + TK_WAVE_SIZE + lane, k_end - 1)];
+            mriq_stage_fence();
+            const int tiles = (min(TK_WAVE_SIZE, chunk_end - k0) + MRIQ_TILE - 1) / MRIQ_TILE;
+            const auto record = [&](int tile) { return mriq_slots(points + MRIQ_TOKENS * (MRIQ_TILE * tile + column), slots.record); };
+            const auto weight = [&](int tile) { return ((mriq_lds_float4 *)weights)[GROUPS * tile + group]; };
+            mriq_bf16x8 k = record(0);
+            float4_t w = weight(0);
+            for (int tile = 0; tile < tiles; ++tile) {
+                const int next = (tile + 1) % GROUPS;   // (the last read is not used)
+                const mriq_bf16x8 next_k = record(next);
+                const float4_t next_w = weight(next);
+                add(k, w);
+                k = next_k;
+                w = next_w;
+            }
+            mriq_stage_fence();
+        }
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            const auto fold = [&](const float (&of)[TILES]) {   // (g0 + g2) + (g1 + g3)
+                const float *tile = of + T * v;
+                const float a = mriq_fold_halves(tile[0], tile[T > 1 ? 1 : 0]);
+                return mriq_fold_rows(a, T == 4 ? mriq_fold_halves(tile[T == 4 ? 2 : 0], tile[T == 4 ? 3 : 0]) : a);
+            };
+            totalR[v] += fold(r);
+            totalI[v] += fold(i);
+        }
+    }
+    if (T < 4 && group != own_tile * (GROUPS / T)) return;   // (with fewer tiles than lane groups several have the same voxel)
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        Qr[own[v]] = totalR[v];
+        Qi[own[v]] = totalI[v];
+    }
+}
+
+// What a wavefront does for V times T tiles of 16 voxels and a run of k records: the part of the kernel that the
 // walk over block positions below does not know about.  MRI-FHD (mrif_role.h) walks the
 // same position grid with another body.
 struct MriqBody {
-    static constexpr int STAGE_QUADS = TK_WAVE_SIZE;   // float4s of LDS a wavefront needs
+    static constexpr bool SHARES = true;   // a block's voxels over more wavefronts than they fill
+    static constexpr int AT_ONCE = 2;   // units of 64 voxels: eight tiles of a wavefront, 32 registers of pieces
+    static constexpr int STAGE_QUADS = TK_WAVE_SIZE * (8 * MRIQ_TOKENS + 4) / 16;   // float4s of LDS a wavefront needs: 64 points and weights
     static __device__ __forceinline__ int chunk() { return MRIQ_K_CHUNK; }
-    template <int V>
+    // Wavefronts a block of 256 voxels is shared out over, where `simds` SIMDs serve `blocks` blocks: 4 of 64 voxels each, or twice or four
+    // times as many where that leaves less for the SIMD that has most, in three turns or fewer (a smaller unit prepares the records
+    // for fewer voxels).  us, 1024 records beside a GEMM of four tiles, 64 / 32 / 16 voxels a wavefront, * = taken: 8192 voxels
+    // 19.8 / 13.9 / 11.8*, 24576 20.1 / 14.9* / 15.2, 49152 20.4* / 20.8 / 27.5, 65536 31.9 / 27.0* / 30.9, 81920 32.2 / 27.2* / 40.3,
+    // 98304 32.4* / 38.8 / 43.6, 131072 43.6* / 45.1 / 56.1, 262144 68.0* / 81.6 / 107.6.
+    static __device__ __forceinline__ int parts(int blocks, int simds)
+    {
+        int p = KERNEL_Q_THREADS_PER_BLOCK / TK_WAVE_SIZE;
+        while (p < KERNEL_Q_THREADS_PER_BLOCK / MRIQ_TILE) {
+            const int most = (blocks * p + simds - 1) / simds, halves = (blocks * 2 * p + simds - 1) / simds;
+            if (halves >= 2 * most || halves > 3) break;
+            p *= 2;
+        }
+        return p;
+    }
+    template <int V, int T>
     static __device__ __forceinline__ void voxels(int k_begin, int k_end, const float *__restrict__ x,
                                                   const float *__restrict__ y, const float *__restrict__ z,
                                                   float *__restrict__ Qr, float *__restrict__ Qi,
-                                                  const int (&xIndex)[V], mriq_lds_float4 *stage)
+                                                  const int (&base)[V], mriq_lds_float4 *stage)
     {
-        mriq_voxels<V>(k_begin, k_end, x, y, z, Qr, Qi, xIndex, stage);
+        mriq_voxels<V, T>(k_begin, k_end, x, y, z, Qr, Qi, base, stage);
     }
 };
 
-// the natural kernel's thread: one voxel, every record.  tid: thread of the workgroup, of WAVES wavefronts
+// the natural kernel's wavefront: 64 voxels, every record.  tid: thread of the workgroup, of WAVES wavefronts
 template <int WAVES, class Body = MriqBody>
 __device__ __forceinline__ void mriq_voxel(int numK, const float *__restrict__ x,
                                            const float *__restrict__ y, const float *__restrict__ z,
                                            float *__restrict__ Qr, float *__restrict__ Qi, int xIndex, int tid)
 {
-    const int one[1] = {xIndex};
-    Body::template voxels<1>(0, numK, x, y, z, Qr, Qi, one,
-                             mriq_stage_of_wave<WAVES, Body::STAGE_QUADS>(__builtin_amdgcn_readfirstlane(tid / TK_WAVE_SIZE)));
+    const int one[1] = {xIndex - tid % TK_WAVE_SIZE};
+    Body::template voxels<1, 4>(0, numK, x, y, z, Qr, Qi, one,
+                                mriq_stage_of_wave<WAVES, Body::STAGE_QUADS>(__builtin_amdgcn_readfirstlane(tid / TK_WAVE_SIZE)));
 }
 
-// One phase of a launch: voxel blocks [block_lo, block_hi) each take records
-// [k_begin, k_end).  A thread serves the blocks it owns -- first_owned, first_owned +
-// stride, ... -- up to MRIQ_VOXELS_PER_THREAD at a time.
-#define MRIQ_VOXELS_PER_THREAD 4
-template <class Body>
-__device__ __forceinline__ void mriq_phase(int block_lo, int block_hi, int k_begin, int k_end,
+// One phase of a launch: units [lo, hi) of T tiles each take records [k_begin, k_end).  A wavefront serves the units it
+// owns -- first_owned, first_owned + stride, ... -- up to AT_ONCE at a time.
+template <class Body, int T, int AT_ONCE>
+__device__ __forceinline__ void mriq_phase(int lo, int hi, int k_begin, int k_end,
                                            const float *__restrict__ x, const float *__restrict__ y,
                                            const float *__restrict__ z, float *__restrict__ Qr,
-                                           float *__restrict__ Qi, int first_owned, int stride, int t,
+                                           float *__restrict__ Qi, int first_owned, int stride,
                                            mriq_lds_float4 *stage)
 {
-    constexpr int V = MRIQ_VOXELS_PER_THREAD;
-    if (block_lo >= block_hi || k_begin >= k_end) return;
-    int b = first_owned;
-    if (b < block_lo) b += (block_lo - b + stride - 1) / stride * stride;
-    for (; b < block_hi; b += V * stride) {
-        int idx[V];
+    constexpr int V = AT_ONCE;
+    if (lo >= hi || k_begin >= k_end) return;
+    int u = first_owned;
+    if (u < lo) u += (lo - u + stride - 1) / stride * stride;
+    for (; u < hi; u += V * stride) {
+        int base[V];
         int count = 0;
 #pragma unroll
         for (int v = 0; v < V; ++v) {
-            const int bv = b + v * stride;
-            if (bv < block_hi) count = v + 1;
-            idx[v] = (bv < block_hi ? bv : b) * KERNEL_Q_THREADS_PER_BLOCK + t;
+            const int uv = u + v * stride;
+            if (uv < hi) count = v + 1;
+            base[v] = (uv < hi ? uv : u) * (T * MRIQ_TILE);
         }
         if (count == V) {
-            Body::template voxels<V>(k_begin, k_end, x, y, z, Qr, Qi, idx, stage);
-        } else {
-            if (count >= 2) {
-                const int two[2] = {idx[0], idx[1]};
-                Body::template voxels<2>(k_begin, k_end, x, y, z, Qr, Qi, two, stage);
+            Body::template voxels<V, T>(k_begin, k_end, x, y, z, Qr, Qi, base, stage);
+        } else if constexpr (V > 1) {
+            if constexpr (V > 2) {
+                if (count >= 2) {
+                    const int two[2] = {base[0], base[1]};
+                    Body::template voxels<2, T>(k_begin, k_end, x, y, z, Qr, Qi, two, stage);
+                }
             }
             if (count & 1) {
-                const int one[1] = {idx[count - 1]};
-                Body::template voxels<1>(k_begin, k_end, x, y, z, Qr, Qi, one, stage);
+                const int one[1] = {base[count - 1]};
+                Body::template voxels<1, T>(k_begin, k_end, x, y, z, Qr, Qi, one, stage);
             }
         }
     }
@@ -224,12 +325,12 @@ __device__ __forceinline__ void mriq_phase(int block_lo, int block_hi, int k_beg
 // one k loop.
 //
 // A range [start, end) is a partial first row of the position grid, whole rows, and a
-// partial last row.  Every voxel block has one owner thread group for the whole launch
-// (slot-major over the role's workgroups, so a short range still spreads over all CUs),
+// partial last row.  A block is 4 units of 64 voxels, or where that leaves wavefronts without one 8 or 16 smaller
+// ones.  Every unit has one owner wavefront for the whole launch (first_piece),
 // and the owner walks the three parts in order: the chunks of a voxel are added in
-// ascending position order without any synchronisation between threads.  Whole rows that
+// ascending position order without any synchronisation between wavefronts.  Whole rows that
 // follow each other are one run of the k loop.
-// WAVES: wavefronts of a workgroup that there is LDS for; those of a larger workgroup leave the blocks to them.
+// WAVES: wavefronts of a workgroup that there is LDS for; those of a larger workgroup leave the units to them.
 template <int WAVES, class Body = MriqBody>
 __device__ __forceinline__ void mriq_role(int numK, const float *__restrict__ x,
                                           const float *__restrict__ y, const float *__restrict__ z,
@@ -237,41 +338,30 @@ __device__ __forceinline__ void mriq_role(int numK, const float *__restrict__ x,
                                           int grid_dimension_x, int grid_dimension_y, int role_block,
                                           int role_blocks, int start, int end, int tid, int role_threads)
 {
-    const int blocks_at_once = min(role_threads, WAVES * TK_WAVE_SIZE) / KERNEL_Q_THREADS_PER_BLOCK;
-    const int slot = tid / KERNEL_Q_THREADS_PER_BLOCK;
-    const int t = tid % KERNEL_Q_THREADS_PER_BLOCK;
-    if (slot >= blocks_at_once || start >= end) return;
-    mriq_lds_float4 *stage = mriq_stage_of_wave<WAVES, Body::STAGE_QUADS>(__builtin_amdgcn_readfirstlane(tid / TK_WAVE_SIZE));
+    constexpr int UNITS = KERNEL_Q_THREADS_PER_BLOCK / TK_WAVE_SIZE;   // of 64 voxels a block
+    const int waves = min(role_threads / TK_WAVE_SIZE, WAVES);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / TK_WAVE_SIZE);
+    if (wave >= waves || start >= end) return;
+    mriq_lds_float4 *stage = mriq_stage_of_wave<WAVES, Body::STAGE_QUADS>(wave);
     const int gx = grid_dimension_x;
     const int gy = grid_dimension_y;
-    const int stride = role_blocks * blocks_at_once;
-    const int first_owned = slot * role_blocks + role_block;
-    const auto chunk_begin = [&](int row) { return min((row % gy) * Body::chunk(), numK); };
-    const auto chunk_end = [&](int row) { return min((row % gy + 1) * Body::chunk(), numK); };
-
-    const int first_row = start / gx;
-    const int last_row = (end - 1) / gx;   // row of the last position
-    if (first_row == last_row) {
-        mriq_phase<Body>(start - first_row * gx, end - first_row * gx, chunk_begin(first_row), chunk_end(first_row),
-                   x, y, z, Qr, Qi, first_owned, stride, t, stage);
-        return;
-    }
-    int row = first_row;
-    if (start != first_row * gx) {   // partial first row
-        mriq_phase<Body>(start - first_row * gx, gx, chunk_begin(row), chunk_end(row), x, y, z, Qr, Qi,
-                   first_owned, stride, t, stage);
-        ++row;
-    }
-    const int whole_end = (end == (last_row + 1) * gx) ? last_row + 1 : last_row;   // whole rows [row, whole_end)
-    while (row < whole_end) {
+    const int stride = role_blocks * waves;
+    const int parts = Body::parts(gx, min(role_blocks * min(waves, 4), 4 * TK_CU_NUM));   // (a CU has four SIMDs)
+    const int first_owned = first_piece(gx * parts, 4 * TK_CU_NUM, wave, waves, role_block, role_blocks);
+    for (int pos = start; pos < end;) {
+        const int row = pos / gx, chunk = row % gy;
+        const int lo = pos - row * gx, hi = min(gx, lo + (end - pos));
         // rows up to the next multiple of grid_dimension_y are consecutive chunks
-        const int run_end = min(whole_end, (row / gy + 1) * gy);
-        mriq_phase<Body>(0, gx, chunk_begin(row), chunk_end(run_end - 1), x, y, z, Qr, Qi, first_owned, stride, t, stage);
-        row = run_end;
+        const int rows = lo == 0 && hi == gx ? min((end - pos) / gx, gy - chunk) : 1;
+        pos += rows == 1 ? hi - lo : rows * gx;
+        const int k_begin = min(chunk * Body::chunk(), numK), k_end = min((chunk + rows) * Body::chunk(), numK);
+#define MRIQ_PHASE(T_, AT_ONCE_) \
+    mriq_phase<Body, T_, AT_ONCE_>(lo * parts, hi * parts, k_begin, k_end, x, y, z, Qr, Qi, first_owned, stride, stage)
+        if (Body::SHARES && parts == 4 * UNITS) MRIQ_PHASE(1, 1);
+        else if (Body::SHARES && parts == 2 * UNITS) MRIQ_PHASE(2, 1);
+        else MRIQ_PHASE(4, Body::AT_ONCE);
+#undef MRIQ_PHASE
     }
-    if (whole_end == last_row)       // partial last row
-        mriq_phase<Body>(0, end - last_row * gx, chunk_begin(last_row), chunk_end(last_row), x, y, z, Qr, Qi,
-                   first_owned, stride, t, stage);
 }
 
 }  // namespace tk

@@ -166,6 +166,41 @@ __device__ __forceinline__ void role_wave_done(unsigned *words)
     if (lane == 0) __hip_atomic_fetch_sub(words + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
+// Around a run of transcendental instructions (or others that the vector unit takes 8 cycles for), in kernels that are bound by its issue.
+// A SIMD starts a 2-cycle instruction every 2 cycles only while two of its wavefronts have one: a wavefront by itself
+// starts one every 4.  A transcendental holds the unit for 8 cycles whoever else is ready, so where wavefronts get to their
+// transcendentals one after the other there are seldom two at the short ones.  With their transcendentals in front of everything
+// else they get them over with, and then have the short ones together.  Cycles of a SIMD for 8 exponentials and 32 multiply-adds of a wavefront,
+// two / three / four wavefronts a SIMD: 192 / 191 / 191, so 135 / 152 / 133; 16 and 40: 288 / 288 / 288, so 213 / 237 / 211.
+// (In longer runs as in shorter ones; in front of the multiply-adds instead it does nothing.)  A GEMM's wavefronts beside them go first all the
+// same (TK_GEMM_WAVE_PRIORITY).
+__device__ __forceinline__ void transcendentals_begin()
+{
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(1);
+    __builtin_amdgcn_sched_barrier(0);
+}
+__device__ __forceinline__ void transcendentals_end()
+{
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// The first of `pieces` pieces of work that wavefront `wave` of a role owns, which are dealt to wavefronts in turn.  Up to `spread` of them one to
+// a workgroup, so that a CU has as few as can be; more of them four to a workgroup (a SIMD each), then four to the next one, and so on
+// through the role's workgroups before a fifth: in a launch of more workgroups than are at work at a time nearly all those at work
+// then have four, where with one to a workgroup three SIMDs of four are idle.  us so / one to a workgroup: mri-q's 4096 pieces in 2048
+// workgroups of 4 wavefronts 111 / 157, 1024 pieces 40.9 / 39.8; cutcp's 5408 pieces in 4096 workgroups of 2 wavefronts 99.5 / 111.5, 2592 pieces
+// 35.9 / 39.0, 2048 pieces 36.2 / 34.0, 1352 pieces 33.7 / 29.8; lavaMD's 1296 pieces in 8192 workgroups of 4 wavefronts 40.8 / 42.6.
+__device__ __forceinline__ int first_piece(int pieces, int spread, int wave, int waves, int role_block, int role_blocks)
+{
+    if (pieces <= spread) return wave * role_blocks + role_block;
+    const int quads = waves / 4, quad = wave / 4;
+    if (quad < quads) return (quad * role_blocks + role_block) * 4 + wave % 4;
+    return quads * role_blocks * 4 + role_block * (waves % 4) + wave % 4;   // (a workgroup's last one to three)
+}
+
 // Where a workgroup of a workgroup-split fused launch belongs.
 // The launch has gridDim.x = groups * (a + b) workgroups.  Hardware hands
 // consecutive workgroup ids to the 8 XCDs round-robin, so roles are assigned by

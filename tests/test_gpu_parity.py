@@ -536,6 +536,28 @@ def test_mri_record_counts_signs_and_large_phases(kernel, numK):
         assert np.array_equal(got[0], first[0]) and np.array_equal(got[1], first[1])
 
 
+# voxels a wavefront takes on 256 CUs: 16, 16, 32, 64 (one and two at a time, or none), 32 in three turns, 64
+@pytest.mark.parametrize("numX", [256, 8192, 24576, 49152, 65536 + 256, 65536 + 7680, 131072 + 256])
+@pytest.mark.parametrize("numK", [5, 145])
+def test_mriq_voxels_a_wavefront_takes_do_not_change_a_bit(numX, numK):
+    k, phiR, phiI, xyz = mriq_inputs(numK, numX, seed=numX + numK)
+    kv = np.concatenate([k, oracle.mriq_phimag(phiR, phiI)[:, None]], 1).astype(np.float32)
+    ta.mriq_set_kvalues(kv)
+    d = [dev(v) for v in xyz]
+    got = []
+    for form, kw in (("ori", {}), ("gptb", {}), ("gptb", {"launch_grid": 256}), ("gptb", {"launch_grid": 7})):
+        re, im = torch.full((numX,), 0.25, device="cuda:0"), torch.full((numX,), -0.5, device="cuda:0")
+        getattr(ta, f"{form}_mriq")(numK, *d, re, im, **kw)
+        got.append((host(re), host(im)))
+        assert np.array_equal(got[-1][0], got[0][0]) and np.array_equal(got[-1][1], got[0][1])
+    at = np.unique(np.linspace(0, numX - 1, 4096).astype(int))
+    turn = np.exp(2j * np.pi * (kv[:, :3].astype(np.float64) @ xyz.astype(np.float64)[:, at]))
+    want = kv[:, 3].astype(np.float64) @ turn + (0.25 - 0.5j)
+    # a phase is below 1, within 2^-24 of it three times over, sine and cosine within 2e-7; numK terms are summed in fp32
+    bound = (np.abs(kv[:, 3]) * (2 * np.pi * 3 * 2.0 ** -24 + 4e-7)).sum() + numK * np.abs(kv[:, 3]).sum() * 2.0 ** -24
+    assert np.abs(got[0][0][at] - want.real).max() <= bound and np.abs(got[0][1][at] - want.imag).max() <= bound
+
+
 def test_mriq_block_positions_are_voxel_blocks_by_k_chunks():
     # numK 300 -> chunks of 128, 128 and 44 records; 4 voxel blocks -> 12 block positions
     numK, numX = 300, 1024
