@@ -21,14 +21,15 @@
 //    order, to a list in LDS, of which whole groups of 4 are used; what is left over waits for the next 64 slots.  Looking
 //    through 64 slots is 60 instructions, none of them a 32-bit product: the list's entries are walked with a counter.
 //  * An atom.  It is read back from that list with one 16-byte broadcast read into vector registers (an
-//    instruction with a scalar register among its operands takes 4.4 cycles of a SIMD, one without 2.3), and a
-//    point takes 5 such instructions and the reciprocal square root: where inv_cutoff2 is 1 / cutoff2 the cutoff
+//    instruction with a scalar register among its operands takes 4.2 cycles of a SIMD, one without 2.1), and a
+//    point takes 7 such instructions and the reciprocal square root, 8 cycles, which goes first
+//    (transcendentals_begin): where inv_cutoff2 is 1 / cutoff2 the cutoff
 //    is the clamp of s to [0, 1], a modifier of the instruction that computes it, instead of a comparison and
 //    an execution mask.
 // The atoms' order, and so every point's sum, is the same in every form of the kernel.
-// 208^3 lattice, two layers of regions: 123 us, 26 layers 1.32 ms; 136 us and 1.44 ms with every batch filled up to whole groups
+// 208^3 lattice, two layers of regions: 99 us (123 with the square roots where they fall and a workgroup's pieces far apart); 136 us with every batch filled up to whole groups
 // (a twelfth of the atoms) and the place in the list divided anew for each, in 95 instructions with five 32-bit products at a quarter of
-// the rate.  Where inv_cutoff2 is not 1 / cutoff2 every point walks the list by itself: 169 us, 1.86 ms (185, 2.01).
+// the rate.  Where inv_cutoff2 is not 1 / cutoff2 every point walks the list by itself: 169 us where the clamp took 123 (185 before).
 #pragma once
 #include <cfloat>
 
@@ -179,22 +180,33 @@ __device__ __forceinline__ void cutcp_piece(int binDim_x, int binDim_y, const fl
             __builtin_amdgcn_sched_barrier(0);   // on its way while the group before it is used
         };
         const auto use = [&](const float4_t (&g)[CUTCP_GROUP]) {
+            float r2[CUTCP_GROUP][PTS], inverse[CUTCP_GROUP][PTS];
 #pragma unroll
             for (int u = 0; u < CUTCP_GROUP; ++u) {
-                const float4_t c = g[u];
-                const float dx = c.x - x;
-                const float dz = c.z - z;
+                const float dx = g[u].x - x;
+                const float dz = g[u].z - z;
                 const float dxdz2 = __builtin_fmaf(dx, dx, dz * dz);
 #pragma unroll
                 for (int e = 0; e < PTS; ++e) {
-                    const float dy = c.y - y[e];
-                    const float r2 = __builtin_fmaf(dy, dy, dxdz2);
-                    float s = __builtin_fmaf(-r2, inv, 1.f);
-                    if (CLAMP) s = __builtin_amdgcn_fmed3f(s, 0.f, 1.f);
-                    const float add = __builtin_fmaf(c.w * __builtin_amdgcn_rsqf(r2), s * s, energy[e]);
-                    energy[e] = CLAMP || r2 < cutoff2 ? add : energy[e];
+                    const float dy = g[u].y - y[e];
+                    r2[u][e] = __builtin_fmaf(dy, dy, dxdz2);
                 }
             }
+            transcendentals_begin();
+#pragma unroll
+            for (int u = 0; u < CUTCP_GROUP; ++u)
+#pragma unroll
+                for (int e = 0; e < PTS; ++e) inverse[u][e] = __builtin_amdgcn_rsqf(r2[u][e]);
+            transcendentals_end();
+#pragma unroll
+            for (int u = 0; u < CUTCP_GROUP; ++u)
+#pragma unroll
+                for (int e = 0; e < PTS; ++e) {
+                    float s = __builtin_fmaf(-r2[u][e], inv, 1.f);
+                    if (CLAMP) s = __builtin_amdgcn_fmed3f(s, 0.f, 1.f);
+                    const float add = __builtin_fmaf(g[u].w * inverse[u][e], s * s, energy[e]);
+                    energy[e] = CLAMP || r2[u][e] < cutoff2 ? add : energy[e];
+                }
             __builtin_amdgcn_sched_barrier(0);
         };
         if (first + CUTCP_GROUP <= behind) read(ga, first);
@@ -273,14 +285,14 @@ __device__ __forceinline__ void cutcp_piece(int binDim_x, int binDim_y, const fl
 // a quarter or a half of those.  A smaller piece is more wavefronts -- one that has its SIMD to itself issues at
 // half the rate of two -- and evener shares, and has fewer atoms in reach (725 of a half region, 620 of a quarter of
 // it); against it stand what a wavefront spends on looking for them, about 60 instructions for every 64 slots, and
-// the four instructions and the read an atom costs before its points.  Measured with 1, 2 and 4 points, us: 128 regions
-// 31.6 / 38.0 / 56.9, 289 36.3 / 40.8 / 51.0, 338 43.2 / 46.0 / 64.4, 392 50.2 / 47.2 / 68.0, 676 66.1 / 59.4 / 69.4, 1352
-// 119 / 123 / 147, 2704 285 / 226 / 261, 4056 382 / 321 / 326, 5408 517 / 456 / 444, 17576 1628 / 1352 / 1337.
+// the four instructions and the read an atom costs before its points.  Measured with 1 and 2 points, us: 361 regions
+// 39.5 / 45.5, 400 42.5 / 45.7, 450 49.4 / 51.3, 484 44.7 / 46.9, 576 53.9 / 48.1, 722 73.1 / 63.6; with 2 and 4, before the square roots went first, 4056
+// 321 / 326, 5408 456 / 444, 17576 1352 / 1337.
 struct CutcpPieces {
     int pts, subs;
     __device__ __forceinline__ CutcpPieces(int regions, int waves)
     {
-        pts = regions * 8 <= min(waves, 11 * TK_CU_NUM) ? 1 : (regions <= 16 * TK_CU_NUM ? 2 : 4);
+        pts = regions * 8 <= min(waves, 16 * TK_CU_NUM) ? 1 : (regions <= 16 * TK_CU_NUM ? 2 : 4);
         subs = 4 / pts;
     }
     __device__ __forceinline__ int first_of(int region) const { return region * 2 * subs; }
@@ -350,9 +362,9 @@ __device__ __forceinline__ void cutcp_role(int binDim_x, int binDim_y, const flo
     const int gx = grid_dimension_x * grid_dimension_y * gdz;                  // regions = columns
     if (gx <= 0) return;
     const int stride = role_blocks * waves;
-    const int first_owned = wave * role_blocks + role_block;
     const CutcpWalk walk(len, gy);
     const CutcpPieces pieces(gx, stride);
+    const int first_owned = first_piece(pieces.first_of(gx), 8 * TK_CU_NUM, wave, waves, role_block, role_blocks);
     cutcp_lds_float4 *stage = cutcp_stage_of_wave<WAVES>(__builtin_amdgcn_readfirstlane(wave));
     // the range as phases: a partial row, or whole rows that follow each other up to the last part
     for (int pos = start; pos < end;) {

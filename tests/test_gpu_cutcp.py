@@ -107,6 +107,27 @@ def test_any_tiling_of_the_positions_gives_the_one_kernel(seed):
     assert np.array_equal(got == -3.0, want == -3.0) and close(got, want)
 
 
+# one point a thread in pieces dealt one and two to a workgroup (up to and from 256 regions on 256 CUs), two points (from 513)
+@pytest.mark.parametrize("regions", [(16, 16, 1), (257, 1, 1), (16, 16, 2), (19, 27, 1)])
+def test_pieces_of_every_size_give_the_same_bits(regions):
+    rng = np.random.default_rng(sum(regions))
+    atoms = atoms_in_box(6000, 1.0, seed=9)
+    atoms[:, :3] *= [(8 * r - 1) * H for r in regions]
+    inp = ta.CutcpInput(atoms, (0, 0, 0), *(8 * r for r in regions), H, CUTOFF, regions=regions)
+    e_ori, e_gptb, e_small, e_cut = (torch.zeros_like(inp.energies) for _ in range(4))
+    ta.ori_cutcp(inp, C2, INV_C2, e_ori)
+    ta.gptb_cutcp(inp, C2, INV_C2, e_gptb)
+    ta.gptb_cutcp(inp, C2, INV_C2, e_small, launch_grid=40, launch_block=256)
+    cuts = [0, int(rng.integers(1, inp.blocks())), inp.blocks()]
+    for a, b in zip(cuts, cuts[1:]):
+        ta.gptb_cutcp(inp, C2, INV_C2, e_cut, a, b)
+    for e in (e_gptb, e_small, e_cut):
+        assert np.array_equal(bits(e), bits(e_ori))
+    if regions[2] == 1:
+        prep = oracle.cutcp_prepare(atoms, (0, 0, 0), *(8 * r for r in regions), H, CUTOFF)
+        assert close(host(e_ori), oracle.cutcp(prep, H, C2, INV_C2, inp.regions))
+
+
 @pytest.mark.parametrize("length", [1, 7, 8, 9, 31, 32, 33, 47, 64, 65, 97, 334])
 def test_neighbour_lists_of_any_length(length):
     # eight bins are looked at at a time and the atoms found used four at a time: lists that end inside a batch, of one part and
