@@ -467,6 +467,66 @@ def test_lava_every_cut_gives_the_same_bits_in_either_form(boxes1d, launch_grid)
         assert lava_close(host(out[0]), oracle.lava(0.5, boxes1d, rv, qv))
 
 
+# 13^3 = 2197 boxes are the smallest cube whose exponents come from the matrix units; every third box is too wide for the form about its centre
+@pytest.mark.parametrize("boxes1d,launch_grid", [(13, 700), (13, 64), (17, 2048)])
+def test_lava_large_domains_give_the_same_bits_however_they_are_cut(boxes1d, launch_grid):
+    rv, qv = lava_inputs(boxes1d, seed=70 + boxes1d)
+    wide = np.arange(len(rv)) // 100 % 3 == 1
+    rv[wide, 1:] = 3 * rv[wide, 1:] - 1
+    rv[wide, 0] = (rv[wide, 1:] ** 2).sum(1) / 2
+    d_r, d_q = dev(rv), dev(qv)
+    out = [torch.zeros((rv.shape[0], 4), device="cuda:0") for _ in range(5)]
+    ta.gptb_lava(0.5, d_r, d_q, out[0])
+    ta.ori_lava(0.5, d_r, d_q, out[1])
+    ta.gptb_lava(0.5, d_r, d_q, out[2], launch_grid=launch_grid, launch_block=256)
+    ta.gptb_lava(0.5, d_r, d_q, out[3], launch_grid=launch_grid, launch_block=64)
+    n = ta.lava_blocks(boxes1d)
+    cuts = [0, n // 5, n // 2 + 1, n]
+    for a, b in zip(cuts, cuts[1:]):
+        ta.gptb_lava(0.5, d_r, d_q, out[4], a, b)
+    for o in out[1:]:
+        assert np.array_equal(bits(o), bits(out[0]))
+
+
+@pytest.mark.parametrize("what", ["plain", "far", "infinite weight", "large charges", "at the end of the range"])
+def test_lava_exponents_from_the_matrix_units(what):
+    # the middle one of the 3 x 3 x 3 boxes in a corner of 13^3: against 64 bits with no more error than the differences, and what is not
+    # finite -- or too large for bf16, whose range ends 2^-9 sooner -- is what they give
+    boxes1d, alpha, errors = 13, 0.5, []
+    block = [x + boxes1d * (y + boxes1d * z) for z in range(3) for y in range(3) for x in range(3)]
+    for seed in range(8 if what == "plain" else 1):
+        rng = np.random.default_rng(seed)
+        boxes, q = (rng.uniform(0.1, 1, (boxes1d ** 3, 100, k)).astype(np.float32).squeeze() for k in (4, 1))
+        if what == "far":
+            boxes[0, 7, :2], q[0, 7] = (np.inf, 1e30), 1e10
+        elif what == "infinite weight":
+            boxes[0, 97, 0] = -1e6
+        elif what == "large charges":
+            q[0, :40] = 3e37
+        elif what == "at the end of the range":
+            boxes[0, 50, 0] = np.finfo(np.float32).max
+        out = torch.zeros((100 * boxes1d ** 3, 4), device="cuda:0")
+        ta.gptb_lava(alpha, dev(boxes.reshape(-1, 4)), dev(q.reshape(-1)), out)
+        got = host(out)[100 * block[13]:100 * block[13] + 100]
+        with np.errstate(all="ignore"):
+            want = lava_differences(boxes[block], q[block], alpha)
+        if what == "plain":
+            p, w = boxes[block].astype(np.float64), q[block].astype(np.float64)
+            w = w[:, None] * np.exp(-2 * alpha ** 2 * (p[13][None, :, :1] + p[:, None, :, 0] - np.stack([p[13][:, 1:] @ b[:, 1:].T for b in p])))
+            exact = 2 * (w[..., None] * (p[13][None, :, None, 1:] - p[:, None, :, 1:])).sum((0, 2))
+            np.testing.assert_allclose(got[:, 0], w.sum((0, 2)), rtol=2e-6)
+            errors.append([np.linalg.norm(v - exact) / np.linalg.norm(exact) for v in (got[:, 1:], want)])
+            continue
+        finite = np.isfinite(want)
+        assert np.array_equal(got[:, 1:][~finite], want[~finite], equal_nan=True)
+        assert finite.all() == (what in ("far", "at the end of the range"))
+        np.testing.assert_allclose(got[:, 1:][finite], want[finite], rtol=2e-4, atol=2e-3 * (1 if finite.all() else 1e37))
+    if what == "plain":
+        got, differences = np.sqrt(np.mean(np.square(errors), 0))
+        print(f"{got:.3e}, by differences {differences:.3e}")
+        assert got <= 1.1 * differences     # (the two evaluations' roundings are independent: a few per cent over 8 systems)
+
+
 @pytest.mark.parametrize("seed", range(4))
 def test_lava_any_ascending_tiling_of_the_positions(seed):
     rng = np.random.default_rng(400 + seed)
