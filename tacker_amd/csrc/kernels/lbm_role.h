@@ -13,10 +13,15 @@
 // race is always resolved in favour of the in-range writer, so results are
 // reproducible.
 //
-// gfx950 design: a block is one x-row (y,z); a lane takes two x-adjacent cells (one
-// if the row length is odd), so each of the 20 loads and 19 stores of a wave is one
-// contiguous row segment of 8 bytes per lane.  No LDS, no barrier.
-// A role of T threads processes T / roundup64(lanes per row) rows at once.
+// gfx950 design: a block is one x-row (y,z), and rows that follow each other in the position grid follow each other in
+// memory.  What a cell does depends on its linear index alone, so a range of blocks is a run of cells, whatever the
+// rows' length: a wave takes 128 of them, two a lane, and each of its 20 loads and 19 stores is one contiguous piece of
+// 8 bytes per lane.  No LDS, no barrier.  What bounds it is memory; us beside a GEMM, on grids that are not in the memory-side cache, with a wave a
+// row (60 to 12 lanes of it at work, a cell a lane where the length is odd, whole lines at neither end) / so: 120 x 120 x 150 cells beside 4096 x 4096 x
+// 1024 117.7 / 116.1, 128^3 beside 1024 x 4096 x 512 93.2 / 77.2, 127 x 128 x 128 beside 2048 x 1024 x 1024 155.6 / 98.9, 64 x 100 x 64
+// beside 1024^3 25.0 / 21.1, 97^3 beside 128^3 43.5 / 32.6, 33 x 61 x 97 beside 1024 x 1024 x 512 16.6 / 11.5.  (The first three with other ways
+// of dealing the pieces: no slabs an XCD 126, 90, 107; a wave's second piece a round further 121, 91, 120; a run of its own for every workgroup
+// 132, 93, 112; one piece at a time 130, 76, 113; with nontemporal stores 121, 83, 108.)
 #pragma once
 #include "role_common.h"
 #include "../header/lbm_header.h"
@@ -187,12 +192,12 @@ __device__ __forceinline__ void lbm_cell_pair(const float *__restrict__ src, flo
 #undef TK_LBM_SCATTER2
 }
 
-// N rows at once, for a role that has few waves on its CU (inside a fused kernel): all 20 N loads
-// of the rows are issued before the first collision, so a wave has N times the bytes in flight.
-// Each destination word has one writer whichever rows are taken together, so the result is the
-// same as row by row.
+// N pairs a lane at once, for a role that has few waves on its CU (inside a fused kernel): all 20 N loads
+// are issued before the first collision, so a wave has N times the bytes in flight.
+// Each destination word has one writer whichever cells are taken together, so the result is the
+// same as one pair after the other.
 template <int N>
-__device__ __forceinline__ void lbm_cell_pair_rows(const float *__restrict__ src, float *__restrict__ dst,
+__device__ __forceinline__ void lbm_cell_pairs(const float *__restrict__ src, float *__restrict__ dst,
                                                    int cells, const int (&c)[N], int sx, int sxy)
 {
     lbm_pair_t in[N][20];
@@ -203,8 +208,8 @@ __device__ __forceinline__ void lbm_cell_pair_rows(const float *__restrict__ src
 #undef TK_LBM_LOAD
         in[r][LBM_FLAGS] = lbm_load_pair(src + cells * LBM_FLAGS + c[r]);
     }
-    // a row is collided and scattered while the loads of the rows behind it are still on their way;
-    // the scheduling fences keep the rows' arithmetic apart (interleaved it needs more registers
+    // a pair is collided and scattered while the loads of those behind it are still on their way;
+    // the scheduling fences keep the pairs' arithmetic apart (interleaved it needs more registers
     // than a fused kernel has)
 #pragma unroll
     for (int r = 0; r < N; ++r) {
@@ -232,9 +237,9 @@ __device__ __forceinline__ void lbm_cell_pair_rows(const float *__restrict__ src
 }
 
 // grid_dimension_x = sy, grid_dimension_y = sz, block_dimension_x = sx
-// (src/ori_kernel/lbm_kernel.cu:218-222).  ROWS_PER_WAVE = N > 1: a wave takes N of its rows at a
-// time (see lbm_cell_pair_rows); which rows a wave owns is the same either way.
-template <int ROWS_PER_WAVE = 1>
+// (src/ori_kernel/lbm_kernel.cu:218-222).  PAIRS > 1: a wave takes that many pieces of 128 cells, which follow each other, at a
+// time (see lbm_cell_pairs).
+template <int PAIRS = 1>
 __device__ __forceinline__ void lbm_role(const float *__restrict__ src, float *__restrict__ dst,
                                          int grid_dimension_x, int grid_dimension_y,
                                          int block_dimension_x, int role_block, int role_blocks,
@@ -242,53 +247,45 @@ __device__ __forceinline__ void lbm_role(const float *__restrict__ src, float *_
 {
     const int sx = block_dimension_x, sy = grid_dimension_x, sz = grid_dimension_y;
     const int sxy = sx * sy;
-    const int cells = sxy * sz;
-    // even row length: a lane takes two cells, odd: one
-    const int per_lane = (sx & 1) ? 1 : 2;
-    const int row_lanes = (sx + per_lane - 1) / per_lane;
-    const int lanes_per_row = ((row_lanes + TK_WAVE_SIZE - 1) / TK_WAVE_SIZE) * TK_WAVE_SIZE;
-    int rows_at_once = role_threads / lanes_per_row;
-    int row_slot, x_first, x_step;
-    if (rows_at_once >= 1) {
-        row_slot = tid / lanes_per_row;
-        x_first = (tid % lanes_per_row) * per_lane;
-        x_step = lanes_per_row * per_lane;
-        if (row_slot >= rows_at_once) return;
-    } else {   // row longer than the role: the role's threads sweep it
-        rows_at_once = 1;
-        row_slot = 0;
-        x_first = tid * per_lane;
-        x_step = role_threads * per_lane;
-    }
-    const unsigned stride = (unsigned)role_blocks * rows_at_once;
-    unsigned pos = (unsigned)start + role_block * rows_at_once + row_slot;
-    if (ROWS_PER_WAVE > 1 && per_lane == 2) {
-        constexpr int N = ROWS_PER_WAVE > 1 ? ROWS_PER_WAVE : 2;
-        // while N more rows of this wave lie in the range (and the position does not wrap)
-        for (; (unsigned long long)pos + (unsigned long long)(N - 1) * stride < (unsigned)end; pos += N * stride) {
-            int row[N];
-#pragma unroll
-            for (int r = 0; r < N; ++r) {
-                const unsigned p = pos + (unsigned)r * stride;
-                row[r] = (int)(p % sy) * sx + (int)((p / sy) % sz) * sxy;
-            }
-            for (int x = x_first; x < sx; x += x_step) {
-                int c[N];
-#pragma unroll
-                for (int r = 0; r < N; ++r) c[r] = x + row[r];
-                lbm_cell_pair_rows<N>(src, dst, cells, c, sx, sxy);
-            }
+    const int rows = sy * sz, cells = sx * rows;
+    const int lane = tid & (TK_WAVE_SIZE - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / TK_WAVE_SIZE), waves = role_threads / TK_WAVE_SIZE;
+    constexpr int PIECE = 2 * TK_WAVE_SIZE;
+    // Every XCD (workgroups go to them in turn) takes a slab of the run, in order: the lines that two waves' scattered pieces share
+    // are completed in one L2.
+    const int xcds = role_blocks % TK_XCD_NUM == 0 ? TK_XCD_NUM : 1;
+    // what of the range lies before the end of the grid, and again from its beginning
+    for (int pos = start; pos < end;) {
+        const int row = pos % rows, here = min(end - pos, rows - row);
+        pos += here;
+        const int first = row * sx, count = here * sx;
+        const int pieces = (count + PIECE - 1) / PIECE;
+        const int slab = (pieces + xcds - 1) / xcds, lo = role_block % xcds * slab, hi = min(pieces, lo + slab);
+        const int groups = role_blocks / xcds, group = role_block / xcds;
+        // this lane's pair of a piece: the run's last lane takes its last two cells where it has an odd one left (both of a cell's
+        // writers have the same bits), those behind it none
+        const auto cell_of = [&](int piece) { return first + min(piece * PIECE + 2 * lane, count - 2); };
+        const auto there = [&](int piece) { return piece * PIECE + 2 * lane < count; };
+        if (count == 1) {
+            if (role_block == 0 && tid == 0) lbm_cell(src, dst, cells, first, sx, sxy);
+            continue;
         }
-    }
-    for (; pos < (unsigned)end; pos += stride) {
-        const int y = pos % sy;
-        const int z = (pos / sy) % sz;
-        if (per_lane == 2) {
-            for (int x = x_first; x < sx; x += x_step)
-                lbm_cell_pair(src, dst, cells, x + y * sx + z * sxy, sx, sxy);
-        } else {
-            for (int x = x_first; x < sx; x += x_step)
-                lbm_cell(src, dst, cells, x + y * sx + z * sxy, sx, sxy);
+        const auto one = [&](int piece) {
+            if (there(piece)) lbm_cell_pair(src, dst, cells, cell_of(piece), sx, sxy);
+        };
+        if (hi - lo <= groups * waves * PAIRS) {   // few: one at a time, over all workgroups before a second wave of one
+            for (int piece = lo + wave * groups + group; piece < hi; piece += groups * waves) one(piece);
+            continue;
+        }
+        for (int piece = lo + (group * waves + wave) * PAIRS; piece < hi; piece += groups * waves * PAIRS) {
+            if (PAIRS > 1 && piece + PAIRS < hi) {   // (the last piece may be a part of one)
+                int c[PAIRS];
+#pragma unroll
+                for (int r = 0; r < PAIRS; ++r) c[r] = first + (piece + r) * PIECE + 2 * lane;
+                lbm_cell_pairs<PAIRS>(src, dst, cells, c, sx, sxy);
+            } else {
+                for (int r = 0; r < PAIRS && piece + r < hi; ++r) one(piece + r);
+            }
         }
     }
 }

@@ -448,6 +448,39 @@ def test_lbm_ori_and_gptb_bit_exact(dims):
     assert np.array_equal(host(d3).view(np.uint32), want.view(np.uint32))
 
 
+# pieces of 128 cells: less than one, one and a cell more, rows of one cell, an odd run, several rounds in few and many workgroups
+@pytest.mark.parametrize("dims", [(1, 1, 5), (1, 43, 3), (3, 43, 1), (129, 1, 1), (127, 9, 7), (25, 40, 61)])
+@pytest.mark.parametrize("kw", [{}, {"launch_grid": 1, "launch_block": 64}, {"launch_grid": 3, "launch_block": 256},
+                                {"launch_grid": 16, "launch_block": 128}])
+def test_lbm_runs_of_cells(dims, kw):
+    sx, sy, sz = dims
+    src = lbm_inputs(sx, sy, sz, obstacle_p=0.2, accel_p=0.1)
+    rows = sy * sz
+    dst = np.full_like(src, -5.0)
+    # the whole grid, a part of it, one row, past its end and round to its beginning
+    for a, b in ((0, rows), (rows // 3, rows - rows // 4), (rows // 2, rows // 2 + 1), (rows - 1, rows + 2)):
+        d = dev(dst)
+        ta.gptb_lbm(dev(src), d, sx, sy, sz, start=a, end=b, **kw)
+        want = oracle.lbm(src, dst, sx, sy, sz, a, min(b, rows))
+        if b > rows:
+            want = oracle.lbm(src, want, sx, sy, sz, 0, min(b - rows, rows))
+        assert np.array_equal(host(d).view(np.uint32), want.view(np.uint32)), (a, b)
+
+
+# two pieces at a time: beside a GEMM with workgroups to spare, one with a tile for each, and the large form
+@pytest.mark.parametrize("dims,gemm", [((127, 71, 70), (256, 256, 128)), ((127, 71, 70), (2048, 2048, 128)), ((90, 121, 128), (4096, 4096, 128))])
+def test_mix_tzgemm_lbm_many_pieces(dims, gemm):
+    A, B = gemm_inputs(*gemm, seed=6)
+    dA, dB = dev(A), dev(B)
+    want_c, got_c = (torch.zeros(gemm[:2], device="cuda:0") for _ in range(2))
+    ta.gptb_tzgemm(dA, dB, want_c)
+    src = lbm_inputs(*dims)
+    d = torch.zeros(src.size, device="cuda:0")
+    ta.mix_tzgemm_lbm(dev(src), d, *dims, dA, dB, got_c)
+    assert np.array_equal(host(got_c).view(np.uint32), host(want_c).view(np.uint32))
+    assert np.array_equal(host(d).view(np.uint32), oracle.lbm(src, np.zeros_like(src), *dims).view(np.uint32))
+
+
 def test_lbm_ranges():
     sx, sy, sz = 16, 4, 3
     src = lbm_inputs(sx, sy, sz)
