@@ -146,6 +146,10 @@ struct StencilQuadMarch {
     float *__restrict__ Anext;
     int nx, ny, lane;
     size_t plane;
+    // Bytes from the start of a plane to what this lane reads and writes of it: the quad's rows, those below and above, the outside column.
+    // (In vector registers they are all the addresses there are beside a plane's own.  us with each row's address by itself / so, beside a GEMM:
+    // 512 x 300 x 64 and 1024^3 28.5 / 26.5, 480 x 400 x 62 and 2048 x 1024 x 1024 44.5 / 43.0, 512 x 500 x 60 and 1024 x 1024 x 512 34.0 / 33.7.)
+    unsigned row_at[ROWS], dn_at, up_at, edge_at;
     // z index of step 0 of the march and its direction (+1 up, -1 down): step L of a run is
     // plane z0 + dz*L.  Runs that are neighbours in z march in opposite directions, so the
     // two planes they share are read by both at the same moment (both at their start or
@@ -163,27 +167,26 @@ struct StencilQuadMarch {
     {
         const int x = x0 + 4 * lane;
         const bool xin = x < nx;
-        const size_t z = (size_t)(z0 + dz * P);
-        const float *col = A0 + (size_t)x + (size_t)nx * j0 + plane * z;
+        const char *at = reinterpret_cast<const char *>(A0 + plane * (size_t)(z0 + dz * P));
         const bool have = P <= nplanes + 1;
 #pragma unroll
         for (int r = 0; r < ROWS; ++r) {
             float4_t v = {0.f, 0.f, 0.f, 0.f};
-            if (have && xin && (j0 + r) < ny) v = *reinterpret_cast<const float4_t *>(col + (size_t)nx * r);
+            if (have && xin && (j0 + r) < ny) v = *reinterpret_cast<const float4_t *>(at + row_at[r]);
             own[P % RING][r] = v;
         }
         if (P >= 1 && P <= Z) {
             const bool centre = P <= nplanes;
             float4_t d = {0.f, 0.f, 0.f, 0.f}, u = {0.f, 0.f, 0.f, 0.f};
-            if (centre && xin && j0 > 0) d = *reinterpret_cast<const float4_t *>(col - (size_t)nx);
-            if (centre && xin && (j0 + ROWS) < ny) u = *reinterpret_cast<const float4_t *>(col + (size_t)nx * ROWS);
+            if (centre && xin && j0 > 0) d = *reinterpret_cast<const float4_t *>(at + dn_at);
+            if (centre && xin && (j0 + ROWS) < ny) u = *reinterpret_cast<const float4_t *>(at + up_at);
             dn[P % 3] = d;
             up[P % 3] = u;
             float e = 0.f;
             const int er = lane & 3;
             const int ex = (lane & 4) ? x0 + 256 : x0 - 1;
             if (centre && lane < 8 && ex >= 0 && ex < nx && (j0 + er) < ny)
-                e = A0[(size_t)ex + (size_t)nx * (j0 + er) + plane * z];
+                e = *reinterpret_cast<const float *>(at + edge_at);
             edge[P % 3] = e;
         }
     }
@@ -195,7 +198,7 @@ struct StencilQuadMarch {
     {
         if (C > nplanes) return;
         const int x = x0 + 4 * lane;
-        float *out = Anext + (size_t)x + (size_t)nx * j0 + plane * (size_t)(z0 + dz * C);
+        char *out = reinterpret_cast<char *>(Anext + plane * (size_t)(z0 + dz * C));
         const bool mine = (block_ok >> (lane >> 4)) & 1u;
 #pragma unroll
         for (int r = 0; r < ROWS; ++r) {
@@ -221,7 +224,7 @@ struct StencilQuadMarch {
             const int j = j0 + r;
             const bool row_ok = mine && j > 0 && j < ny - 1 && x < nx;
             if (row_ok) {
-                float *o = out + (size_t)nx * r;
+                float *o = reinterpret_cast<float *>(out + row_at[r]);
                 if (x > 0 && x + 3 < nx - 1) {
                     *reinterpret_cast<float4_t *>(o) = v;
                 } else {   // the quad touches the first or the last column of the grid
@@ -252,6 +255,12 @@ struct StencilQuadMarch {
     {
         z0 = upward ? k_first - 1 : k_first + nplanes;
         dz = upward ? 1 : -1;
+        const unsigned first = 4u * (unsigned)(x0 + 4 * lane + nx * j0), row = 4u * (unsigned)nx;
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) row_at[r] = first + row * r;
+        dn_at = first - row;
+        up_at = first + row * ROWS;
+        edge_at = 4u * (unsigned)(((lane & 4) ? x0 + 256 : x0 - 1) + nx * (j0 + (lane & 3)));
         issue<0>(k_first, nplanes, x0, j0);
         issue<1>(k_first, nplanes, x0, j0);
         issue<2>(k_first, nplanes, x0, j0);
@@ -434,7 +443,7 @@ __device__ __forceinline__ void stencil_role_wide(float c0, float c1, const floa
         const unsigned nr = runs_before(q1) - run_first;
         const unsigned first_row = lo / gdx;
         const unsigned rows = (hi - 1) / gdx - first_row + 1;
-        const unsigned tasks = rows * quads_per_row * nr;
+        unsigned tasks = rows * quads_per_row * nr;
         // this wave's tasks of the piece: global task numbers base + local, = me modulo stride
         unsigned local = (me + stride - base % stride) % stride;
         // Which (row, run, quad) task number `local` is.  Any one-to-one numbering gives the same grid;
@@ -449,19 +458,28 @@ __device__ __forceinline__ void stencil_role_wide(float c0, float c1, const floa
         // of the shared planes came from another XCD's share and were fetched twice.)
         const unsigned uw = (unsigned)waves;
         const bool slabs = rows % (8u * uw) == 0u;
+        // Tasks that are less than one for every wave -- the last round, or all there are -- are halves or quarters of a run each where there
+        // are waves enough, up to eight a CU (more read each other's planes again for nothing: the 2048 runs of 512 x 512 x 64 cut for a launch of
+        // 8192 waves 45.9 us for 35.4).  us with whole runs / so: 512 x 512 x 64 beside tzgemm 128^3, 2048 runs for 2016 waves, 45.8 / 40.6;
+        // 400 x 300 x 40 beside 1024^3, 750 for 2048, 19.2 / 16.0.
+        const unsigned last_round = tasks / stride * stride, left = tasks - last_round;
+        const unsigned at_work = min(stride, 8u * TK_CU_NUM), cuts = left * 4 <= at_work ? 4 : (left * 2 <= at_work ? 2 : 1);
+        tasks = last_round + left * cuts;
         for (; local < tasks; local += stride) {
+            const unsigned cut = local < last_round ? 0 : (local - last_round) / max(left, 1u);
+            const unsigned of = local < last_round ? 1 : cuts, task = local - cut * left;
             unsigned row, qx;
             int run;
             if (slabs) {
-                const unsigned slot = local / uw, xcd = slot % 8u, idx = slot / 8u;
+                const unsigned slot = task / uw, xcd = slot % 8u, idx = slot / 8u;
                 const unsigned rows_x = rows / 8u, row_groups = rows_x / uw;
                 const unsigned rest = idx / row_groups;
-                row = first_row + xcd * rows_x + (idx % row_groups) * uw + local % uw;
+                row = first_row + xcd * rows_x + (idx % row_groups) * uw + task % uw;
                 run = (int)((run_first + rest % nr) % rg.runs);
                 qx = rest / nr;
             } else {
-                row = first_row + local % rows;
-                const unsigned rest = local / rows;
+                row = first_row + task % rows;
+                const unsigned rest = task / rows;
                 run = (int)((run_first + rest % nr) % rg.runs);
                 qx = rest / nr;
             }
@@ -473,9 +491,11 @@ __device__ __forceinline__ void stencil_role_wide(float c0, float c1, const floa
                 if (bx < gdx && pos >= lo && pos < hi) block_ok |= 1u << b;
             }
             if (block_ok == 0) continue;
-            const int k_first = 1 + run * STENCIL_Z_RUN;
-            m.run(c0, c1, k_first, min(STENCIL_Z_RUN, nz - 1 - k_first), (int)(qx * 4 * 2 * STENCIL_TILE_X),
-                  (int)(row % (unsigned)grid_dimension_y) * STENCIL_TILE_Y, block_ok, (run & 1) == 0);
+            const int k_first = 1 + run * STENCIL_Z_RUN, planes = min(STENCIL_Z_RUN, nz - 1 - k_first);
+            const int each = (planes + (int)of - 1) / (int)of, skip = (int)cut * each;
+            if (skip >= planes) continue;
+            m.run(c0, c1, k_first + skip, min(each, planes - skip), (int)(qx * 4 * 2 * STENCIL_TILE_X),
+                  (int)(row % (unsigned)grid_dimension_y) * STENCIL_TILE_Y, block_ok, ((run * (int)of + (int)cut) & 1) == 0);
         }
         base += tasks;
     }
@@ -496,13 +516,13 @@ __device__ __forceinline__ void stencil_role(float c0, float c1, const float *__
         tasks += (g.hi - g.lo) * (g.r1 - g.r0);
     }
     const unsigned role_waves = (unsigned)role_blocks * (unsigned)(role_threads >> 6);
-    // Rows that are 16-byte aligned take the wide form -- unless the range is short: when every
+    // Rows that are 16-byte aligned take the wide form, which holds a plane's addresses in 32 bits -- unless the range is short: when every
     // wave gets at most two runs, the narrow form's "all loads of a run at once" ends after one
     // trip to memory where the march makes five, and latency is all that counts.  Its dword
     // accesses move bytes at half the wide form's rate, so beyond STENCIL_SHORT_RANGE_TASKS runs
     // (a quarter of the 512 x 512 x 64 sweep, where the two forms take the same time on 256 CUs)
     // the march wins whatever the launch.
-    if ((nx & 3) == 0 && (tasks > 2 * role_waves || tasks > STENCIL_SHORT_RANGE_TASKS))
+    if ((nx & 3) == 0 && (size_t)nx * ny < (1u << 29) && (tasks > 2 * role_waves || tasks > STENCIL_SHORT_RANGE_TASKS))
         stencil_role_wide(c0, c1, A0, Anext, nx, ny, nz, grid_dimension_x, grid_dimension_y, rg, role_block,
                           role_blocks, tid, role_threads);
     else

@@ -415,6 +415,24 @@ def test_stencil_slab_numbering_of_the_wide_form_is_one_sweep(ny, grid):
     assert ta.spin_fail_flag() == 0
 
 
+# the wide form's last round: 36 runs of up to 8 planes (the second ones of a column have 3) for 20, 24, 30, 32 and 1 waves -- 16 whole ones,
+# 12 halves, 6 quarters, 4 quarters, none; and 750 runs, all in halves, in a launch of many waves
+@pytest.mark.parametrize("shape,grid", [((13, 36, 260), 20), ((13, 36, 260), 24), ((13, 36, 260), 30), ((13, 36, 260), 32),
+                                        ((13, 36, 260), 1), ((40, 300, 400), 0)])
+def test_stencil_last_round_in_shorter_runs(shape, grid):
+    A0 = stencil_inputs(*shape, seed=sum(shape) + grid)
+    nz, ny, nx = shape
+    total = ta.stencil_blocks(nx, ny, nz)
+    want = oracle.stencil(C0, C1, A0, np.full_like(A0, -5.0))
+    kw = {"launch_grid": grid, "launch_block": 64} if grid else {}
+    d0 = dev(A0)
+    for cuts in ([0, total], [0, total // 3, total]):
+        d1 = dev(np.full_like(A0, -5.0))
+        for a, b in zip(cuts, cuts[1:]):
+            ta.gptb_stencil(C0, C1, d0, d1, start=a, end=b, **kw)
+        assert np.array_equal(host(d1).view(np.uint32), want.view(np.uint32))
+
+
 def test_stencil_iterations_ping_pong():
     A0 = stencil_inputs(6, 16, 128)
     a, b = dev(A0), dev(A0)
