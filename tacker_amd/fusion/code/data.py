@@ -49,13 +49,13 @@ KERNEL_INFO = {
     "stencil": {"register": 48, "shared_memory": 0, "blocksize": 256, "solo_ptb_blks": 8,
                 "ori_blks": 8192},
     # 67.4 us with 16 workgroups a CU, 69.9 with 8 (profile_gptb.py)
-    "lbm": {"register": 64, "shared_memory": 0, "blocksize": 256, "solo_ptb_blks": 16,
+    "lbm": {"register": 57, "shared_memory": 0, "blocksize": 256, "solo_ptb_blks": 16,
             "ori_blks": 18000},
     # 1024 blocks of 256 voxels x 16 chunks of 128 k records
-    "mriq": {"register": 100, "shared_memory": 4096, "blocksize": 256, "solo_ptb_blks": 8,
+    "mriq": {"register": 123, "shared_memory": 7168, "blocksize": 256, "solo_ptb_blks": 8,
              "ori_blks": 16384},
     # 1024 blocks of 256 voxels x 16 chunks of 128 k records
-    "mrif": {"register": 110, "shared_memory": 5120, "blocksize": 256, "solo_ptb_blks": 8,
+    "mrif": {"register": 107, "shared_memory": 5120, "blocksize": 256, "solo_ptb_blks": 8,
              "ori_blks": 16384},
     # 32 x 258 blocks of 128 rows x 16 columns of C x 64 parts of 64 k steps (4096 x 4128 x 4064)
     "sgemm": {"register": 64, "shared_memory": 0, "blocksize": 128, "solo_ptb_blks": 16,
@@ -64,7 +64,7 @@ KERNEL_INFO = {
     "fft": {"register": 40, "shared_memory": 8192, "blocksize": 256, "solo_ptb_blks": 8,
             "ori_blks": 10240},
     # 26 x 26 x 2 regions of 8 x 8 x 8 lattice points (two wavefronts each) x 11 parts of 32 neighbour bins
-    "cutcp": {"register": 94, "shared_memory": 4096, "blocksize": 128, "solo_ptb_blks": 16,
+    "cutcp": {"register": 113, "shared_memory": 4096, "blocksize": 128, "solo_ptb_blks": 16,
               "ori_blks": 14872},
     # 2560000 blocks of 256 records; a stream that wants many workgroups in flight (4.0 TB/s with 8 a CU,
     # 4.95 with 32)
@@ -77,7 +77,7 @@ KERNEL_INFO = {
     # 216000 boxes of 100 particles (a wavefront each) x 27 parts (the home box and its neighbour slots);
     # boxes on the faces have fewer neighbours: the more owner wavefronts, the evener their shares
     # (42.4 ms with 4 workgroups a CU, 35.8 with 32)
-    "lava": {"register": 127, "shared_memory": 13056, "blocksize": 256, "solo_ptb_blks": 32,
+    "lava": {"register": 128, "shared_memory": 15872, "blocksize": 256, "solo_ptb_blks": 32,
              "ori_blks": 5832000},
     # 200 windows of 256 columns (6 result columns each), a wavefront each
     "path": {"register": 78, "shared_memory": 0, "blocksize": 256, "solo_ptb_blks": 1,
