@@ -48,7 +48,7 @@ KERNEL_INFO = {
     # 1024 blocks of 64 x 4 columns x 8 runs of 8 centre planes
     "stencil": {"register": 48, "shared_memory": 0, "blocksize": 256, "solo_ptb_blks": 8,
                 "ori_blks": 8192},
-    # 67.4 us with 16 workgroups a CU, 69.9 with 8 (profile_gptb.py)
+    # 55.6 us with 16 workgroups a CU, 57.7 with 8 (profile_gptb.py)
     "lbm": {"register": 57, "shared_memory": 0, "blocksize": 256, "solo_ptb_blks": 16,
             "ori_blks": 18000},
     # 1024 blocks of 256 voxels x 16 chunks of 128 k records
@@ -76,7 +76,7 @@ KERNEL_INFO = {
               "ori_blks": 524288},
     # 216000 boxes of 100 particles (a wavefront each) x 27 parts (the home box and its neighbour slots);
     # boxes on the faces have fewer neighbours: the more owner wavefronts, the evener their shares
-    # (42.4 ms with 4 workgroups a CU, 35.8 with 32)
+    # (12.4 ms with 4 workgroups a CU, 11.2 with 32)
     "lava": {"register": 128, "shared_memory": 15872, "blocksize": 256, "solo_ptb_blks": 32,
              "ori_blks": 5832000},
     # 200 windows of 256 columns (6 result columns each), a wavefront each
