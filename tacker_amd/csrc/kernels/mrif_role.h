@@ -131,7 +131,7 @@ struct MrifBody {
     static __device__ __forceinline__ int chunk() { return MRIF_K_CHUNK; }
     static __device__ __forceinline__ int parts(int, int) { return KERNEL_FH_THREADS_PER_BLOCK / TK_WAVE_SIZE; }
     template <int V, int T>
-    static __device__ __forceinline__ void voxels(int k_begin, int k_end, const float *__restrict__ x,
+    static __device__ __forceinline__ bool voxels(int k_begin, int k_end, const float *__restrict__ x,
                                                   const float *__restrict__ y, const float *__restrict__ z,
                                                   float *__restrict__ outR, float *__restrict__ outI,
                                                   const int (&base)[V], mriq_lds_float4 *stage)
@@ -142,7 +142,10 @@ struct MrifBody {
             for (int v = 0; v < V; ++v) xIndex[v] = base[v] + mriq_lane();
             mrif_voxels<V>(k_begin, k_end, x, y, z, outR, outI, xIndex, stage);
         }
+        return false;
     }
+    static __device__ __forceinline__ void far_voxels(int, int, const float *, const float *, const float *, float *, float *, int, int,
+                                                      mriq_lds_float4 *) {}   // (phases are multiply-adds at any size)
 };
 
 // Block positions [start, end) of the (voxel blocks) x (k chunks) grid, as mriq_role.

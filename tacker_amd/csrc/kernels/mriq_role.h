@@ -92,6 +92,13 @@ __device__ __forceinline__ void mriq_put_point(mriq_lds_token *tokens, float x, 
     }
 }
 
+// Pieces hold a value exactly from 2^-109 to 3.39e38, and to 2^-134 below.  Beside a coordinate of 2^64 or more, where that may show in a phase or a
+// piece round to infinity, phases are the chain of multiply-adds.  (Elsewhere 2^-134 is less than 2^-67 of a turn.)
+__device__ __forceinline__ bool mriq_far(float x, float y, float z)
+{
+    return (__builtin_fabsf(x) >= 0x1p64f) | (__builtin_fabsf(y) >= 0x1p64f) | (__builtin_fabsf(z) >= 0x1p64f);
+}
+
 __device__ __forceinline__ mriq_bf16x8 mriq_slots(const mriq_lds_token *point, const int (&tokens)[2])
 {
     const mriq_uint2 a = point[tokens[0]], b = point[tokens[1]];
@@ -114,17 +121,19 @@ __device__ __forceinline__ float mriq_fold_rows(float a, float b)
 // brings 64 records at a time through its LDS.  A lane has voxel 16 t + lane % 16 of every tile t of 16 and, of 16 records, the four
 // 4 (lane / 16) ..: its sums over a chunk of records are added to the other three lane groups' at the chunk's end, and that to Q, so any
 // split at chunks gives the same bits.  The last records of the table come in a whole tile of 16, with weights of zero behind them.
-// stage: this wavefront's LDS.
-template <int V, int T>
-__device__ __forceinline__ void mriq_voxels(int k_begin, int k_end, const float *__restrict__ x,
+// stage: this wavefront's LDS.  Where a voxel or a record was far, nothing is written and the result is true: then FAR computes the voxels, 16 at a time,
+// and differs in the phases of what is far alone, so that a voxel's bits do not depend on those beside it.
+template <int V, int T, bool FAR = false>
+__device__ __forceinline__ bool mriq_voxels(int k_begin, int k_end, const float *__restrict__ x,
                                             const float *__restrict__ y, const float *__restrict__ z,
                                             float *__restrict__ Qr, float *__restrict__ Qi,
                                             const int (&base)[V], mriq_lds_float4 *stage)
 {
     static_assert(T == 1 || T == 2 || T == 4, "the folds leave a lane one voxel's sums");
-    if (k_begin >= k_end) return;
+    if (k_begin >= k_end) return false;
     constexpr int GROUPS = TK_WAVE_SIZE / MRIQ_TILE, TILES = T * V, AHEAD = TILES == 1 ? 1 : 2;
-    const int lane = mriq_lane();
+    int lane = mriq_lane();
+    if (FAR) asm volatile("" : "+v"(lane));   // (what follows from it is not kept through a launch, in registers that it does not have)
     const int group = lane / MRIQ_TILE, column = lane % MRIQ_TILE;
     const MriqSlots slots(group);
     mriq_lds_token *const points = (mriq_lds_token *)stage;
@@ -134,6 +143,7 @@ __device__ __forceinline__ void mriq_voxels(int k_begin, int k_end, const float 
     const int own_tile = T == 4 ? (group == 1 ? 2 : (group == 2 ? 1 : group)) : (T == 2 ? group / 2 : 0);
 
     mriq_bf16x8 voxel[TILES];
+    unsigned long long far = 0;   // lanes that met a far voxel or record
     int own[V];   // this lane's voxel of each 64, whose sums the folds leave here
     float totalR[V], totalI[V];
     const float4_t *table = reinterpret_cast<const float4_t *>(ck);
@@ -145,6 +155,7 @@ __device__ __forceinline__ void mriq_voxels(int k_begin, int k_end, const float 
         totalR[v] = Qr[own[v]];
         totalI[v] = Qi[own[v]];
         mriq_put_point(points + MRIQ_TOKENS * lane, x[i], y[i], z[i]);
+        if (!FAR) far |= __builtin_amdgcn_ballot_w64(mriq_far(x[i], y[i], z[i]));
         mriq_stage_fence();
 #pragma unroll
         for (int t = 0; t < T; ++t)
@@ -158,7 +169,8 @@ __device__ __forceinline__ void mriq_voxels(int k_begin, int k_end, const float 
     };
     // two tiles at a time, the matrix instructions of the next two in front of their sines.  (The next records' first ones in front of the last
     // tiles' sines as well, and records read another step ahead: 122 us for 112 beside tzgemm 2048^3.)
-    const auto add = [&](const mriq_bf16x8 &k, const float4_t &w) {
+    // first: the lane's first record of the four.
+    const auto add = [&](const mriq_bf16x8 &k, const float4_t &w, int first) {
         float4_t now[AHEAD];
 #pragma unroll
         for (int u = 0; u < AHEAD; ++u) now[u] = phases(k, u);
@@ -167,6 +179,15 @@ __device__ __forceinline__ void mriq_voxels(int k_begin, int k_end, const float 
             float4_t next[AHEAD];
 #pragma unroll
             for (int u = 0; u < AHEAD; ++u) next[u] = t + AHEAD < TILES ? phases(k, t + AHEAD + u) : now[u];
+            if (FAR) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int at = base[0] + column;
+                    const float4_t of = table[min(first + e, k_end - 1)];
+                    if (mriq_far(x[at], y[at], z[at]) || mriq_far(of.x, of.y, of.z))
+                        now[0][e] = __builtin_fmaf(of.z, z[at], __builtin_fmaf(of.y, y[at], of.x * x[at]));
+                }
+            }
             float c[AHEAD][4], s[AHEAD][4];
             if (T == 4) transcendentals_begin();   // (with fewer tiles the compiler's order is worth more: 65536 voxels 27.0 us for 30.9)
 #pragma unroll
@@ -194,6 +215,7 @@ __device__ __forceinline__ void mriq_voxels(int k_begin, int k_end, const float 
         for (int t = 0; t < TILES; ++t) r[t] = i[t] = 0.f;
         for (int k0 = chunk; k0 < chunk_end; k0 += TK_WAVE_SIZE) {
             mriq_put_point(points + MRIQ_TOKENS * lane, ahead.x, ahead.y, ahead.z);
+            if (!FAR) far |= __builtin_amdgcn_ballot_w64(mriq_far(ahead.x, ahead.y, ahead.z));
             weights[lane] = k0 + lane < k_end ? ahead.w : 0.f;
             ahead = table[min(k0 + TK_WAVE_SIZE + lane, k_end - 1)];
             mriq_stage_fence();
@@ -206,7 +228,7 @@ __device__ __forceinline__ void mriq_voxels(int k_begin, int k_end, const float 
                 const int next = (tile + 1) % GROUPS;   // (the last read is not used)
                 const mriq_bf16x8 next_k = record(next);
                 const float4_t next_w = weight(next);
-                add(k, w);
+                add(k, w, k0 + MRIQ_TILE * tile + 4 * group);
                 k = next_k;
                 w = next_w;
             }
@@ -223,12 +245,14 @@ __device__ __forceinline__ void mriq_voxels(int k_begin, int k_end, const float 
             totalI[v] += fold(i);
         }
     }
-    if (T < 4 && group != own_tile * (GROUPS / T)) return;   // (with fewer tiles than lane groups several have the same voxel)
+    if (!FAR && far != 0) return true;
+    if (T < 4 && group != own_tile * (GROUPS / T)) return false;   // (with fewer tiles than lane groups several have the same voxel)
 #pragma unroll
     for (int v = 0; v < V; ++v) {
         Qr[own[v]] = totalR[v];
         Qi[own[v]] = totalI[v];
     }
+    return false;
 }
 
 // What a wavefront does for V times T tiles of 16 voxels and a run of k records: the part of the kernel that the
@@ -255,12 +279,24 @@ struct MriqBody {
         return p;
     }
     template <int V, int T>
-    static __device__ __forceinline__ void voxels(int k_begin, int k_end, const float *__restrict__ x,
+    static __device__ __forceinline__ bool voxels(int k_begin, int k_end, const float *__restrict__ x,
                                                   const float *__restrict__ y, const float *__restrict__ z,
                                                   float *__restrict__ Qr, float *__restrict__ Qi,
                                                   const int (&base)[V], mriq_lds_float4 *stage)
     {
-        mriq_voxels<V, T>(k_begin, k_end, x, y, z, Qr, Qi, base, stage);
+        return mriq_voxels<V, T>(k_begin, k_end, x, y, z, Qr, Qi, base, stage);
+    }
+    // `count` voxels from `first` on, some of which may be far (called in one place of a kernel: four more of them cost the others 1 to 2 %)
+    static __device__ __forceinline__ void far_voxels(int k_begin, int k_end, const float *__restrict__ x,
+                                                      const float *__restrict__ y, const float *__restrict__ z,
+                                                      float *__restrict__ Qr, float *__restrict__ Qi, int first, int count,
+                                                      mriq_lds_float4 *stage)
+    {
+#pragma unroll 1
+        for (int t = 0; t < count; t += MRIQ_TILE) {
+            const int one[1] = {first + t};
+            mriq_voxels<1, 1, true>(k_begin, k_end, x, y, z, Qr, Qi, one, stage);
+        }
     }
 };
 
@@ -271,21 +307,22 @@ __device__ __forceinline__ void mriq_voxel(int numK, const float *__restrict__ x
                                            float *__restrict__ Qr, float *__restrict__ Qi, int xIndex, int tid)
 {
     const int one[1] = {xIndex - tid % TK_WAVE_SIZE};
-    Body::template voxels<1, 4>(0, numK, x, y, z, Qr, Qi, one,
-                                mriq_stage_of_wave<WAVES, Body::STAGE_QUADS>(__builtin_amdgcn_readfirstlane(tid / TK_WAVE_SIZE)));
+    mriq_lds_float4 *stage = mriq_stage_of_wave<WAVES, Body::STAGE_QUADS>(__builtin_amdgcn_readfirstlane(tid / TK_WAVE_SIZE));
+    if (Body::template voxels<1, 4>(0, numK, x, y, z, Qr, Qi, one, stage))
+        Body::far_voxels(0, numK, x, y, z, Qr, Qi, one[0], TK_WAVE_SIZE, stage);
 }
 
 // One phase of a launch: units [lo, hi) of T tiles each take records [k_begin, k_end).  A wavefront serves the units it
-// owns -- first_owned, first_owned + stride, ... -- up to AT_ONCE at a time.
+// owns -- first_owned, first_owned + stride, ... -- up to AT_ONCE at a time, up to the first ones that are far.  Which that is, or hi or more.
 template <class Body, int T, int AT_ONCE>
-__device__ __forceinline__ void mriq_phase(int lo, int hi, int k_begin, int k_end,
+__device__ __forceinline__ int mriq_phase(int lo, int hi, int k_begin, int k_end,
                                            const float *__restrict__ x, const float *__restrict__ y,
                                            const float *__restrict__ z, float *__restrict__ Qr,
                                            float *__restrict__ Qi, int first_owned, int stride,
                                            mriq_lds_float4 *stage)
 {
     constexpr int V = AT_ONCE;
-    if (lo >= hi || k_begin >= k_end) return;
+    if (lo >= hi || k_begin >= k_end) return hi;
     int u = first_owned;
     if (u < lo) u += (lo - u + stride - 1) / stride * stride;
     for (; u < hi; u += V * stride) {
@@ -298,20 +335,21 @@ __device__ __forceinline__ void mriq_phase(int lo, int hi, int k_begin, int k_en
             base[v] = (uv < hi ? uv : u) * (T * MRIQ_TILE);
         }
         if (count == V) {
-            Body::template voxels<V, T>(k_begin, k_end, x, y, z, Qr, Qi, base, stage);
+            if (Body::template voxels<V, T>(k_begin, k_end, x, y, z, Qr, Qi, base, stage)) break;
         } else if constexpr (V > 1) {
             if constexpr (V > 2) {
                 if (count >= 2) {
                     const int two[2] = {base[0], base[1]};
-                    Body::template voxels<2, T>(k_begin, k_end, x, y, z, Qr, Qi, two, stage);
+                    if (Body::template voxels<2, T>(k_begin, k_end, x, y, z, Qr, Qi, two, stage)) break;
                 }
             }
             if (count & 1) {
                 const int one[1] = {base[count - 1]};
-                Body::template voxels<1, T>(k_begin, k_end, x, y, z, Qr, Qi, one, stage);
+                if (Body::template voxels<1, T>(k_begin, k_end, x, y, z, Qr, Qi, one, stage)) break;
             }
         }
     }
+    return u;
 }
 
 // Block positions of the GPTB form are a grid of grid_dimension_x voxel blocks (256 voxels
@@ -355,11 +393,15 @@ __device__ __forceinline__ void mriq_role(int numK, const float *__restrict__ x,
         const int rows = lo == 0 && hi == gx ? min((end - pos) / gx, gy - chunk) : 1;
         pos += rows == 1 ? hi - lo : rows * gx;
         const int k_begin = min(chunk * Body::chunk(), numK), k_end = min((chunk + rows) * Body::chunk(), numK);
+        int u;
 #define MRIQ_PHASE(T_, AT_ONCE_) \
-    mriq_phase<Body, T_, AT_ONCE_>(lo * parts, hi * parts, k_begin, k_end, x, y, z, Qr, Qi, first_owned, stride, stage)
+    u = mriq_phase<Body, T_, AT_ONCE_>(lo * parts, hi * parts, k_begin, k_end, x, y, z, Qr, Qi, first_owned, stride, stage)
         if (Body::SHARES && parts == 4 * UNITS) MRIQ_PHASE(1, 1);
         else if (Body::SHARES && parts == 2 * UNITS) MRIQ_PHASE(2, 1);
         else MRIQ_PHASE(4, Body::AT_ONCE);
+        const int voxels = MRIQ_TILE * (parts == 4 * UNITS ? 1 : (parts == 2 * UNITS ? 2 : 4));
+        for (; __builtin_expect(u < hi * parts, 0); u += stride)
+            Body::far_voxels(k_begin, k_end, x, y, z, Qr, Qi, u * voxels, voxels, stage);
 #undef MRIQ_PHASE
     }
 }

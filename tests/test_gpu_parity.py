@@ -587,6 +587,37 @@ def test_mri_record_counts_signs_and_large_phases(kernel, numK):
         assert np.array_equal(got[0], first[0]) and np.array_equal(got[1], first[1])
 
 
+# What three pieces of 16 bits do not hold: coordinates from 3.396e38 on, which round to infinity, and the last bits of tiny ones.  Their phases
+# are moderate beside tiny and huge ones.
+@pytest.mark.parametrize("numX", [256, 65536, 131072 + 256])     # 16, 32 and 64 voxels a wavefront on 256 CUs
+def test_mriq_coordinates_at_the_ends_of_the_range(numX):
+    rng = np.random.default_rng(numX)
+    largest = float(np.finfo(np.float32).max)
+    kv = np.concatenate([np.ldexp(rng.uniform(-2, 2, (200, 3)), rng.integers(-130, -122, (200, 3))), rng.uniform(0, 2, (200, 1))], 1).astype(np.float32)
+    xyz = rng.uniform(-0.5, 0.5, (3, numX)).astype(np.float32)
+    xyz[0, 5::7], xyz[2, 2::5], xyz[2, 3::11] = largest, -largest * (1 - 2.0 ** -9), largest * (1 - 2.0 ** -12)
+    kv[150, 1], xyz[1] = 1.2345 * 2.0 ** 80, np.ldexp(xyz[1], -78)     # and a record
+    bad = np.arange(numX) % 97 == 1
+    xyz[0, bad] = np.resize(np.float32([np.inf, -np.inf, np.nan]), bad.sum())
+    finite = np.where(bad, 0, xyz).astype(np.float64)
+    want = kv[:, 3].astype(np.float64) @ np.exp(2j * np.pi * (kv[:, :3].astype(np.float64) @ finite))
+    reach = np.abs(kv[:, :3]).astype(np.float64) @ np.abs(finite)
+    # as above: a phase is within 2^-24 of |K||x| three times over, sine and cosine within 2e-7, and the terms are summed in fp32
+    bound = (np.abs(kv[:, 3:]) * (2 * np.pi * 3 * 2.0 ** -24 * reach + 4e-7)).sum(0) + len(kv) * np.abs(kv[:, 3]).sum() * 2.0 ** -24
+    assert np.median(bound) < 2e-2 and bound.max() < 0.2
+    ta.mriq_set_kvalues(kv)
+    d = [dev(v) for v in xyz]
+    first = None
+    for form, kw in (("ori", {}), ("gptb", {}), ("gptb", {"launch_grid": 7})):
+        re, im = torch.zeros(numX, device="cuda:0"), torch.zeros(numX, device="cuda:0")
+        getattr(ta, f"{form}_mriq")(len(kv), *d, re, im, **kw)
+        re, im = host(re), host(im)
+        assert np.isnan(re[bad]).all() and np.isnan(im[bad]).all()
+        assert np.all(np.abs(re - want.real)[~bad] <= bound[~bad]) and np.all(np.abs(im - want.imag)[~bad] <= bound[~bad])
+        first = first or (re, im)
+        assert np.array_equal(re, first[0], equal_nan=True) and np.array_equal(im, first[1], equal_nan=True)
+
+
 # voxels a wavefront takes on 256 CUs: 16, 16, 32, 64 (one and two at a time, or none), 32 in three turns, 64
 @pytest.mark.parametrize("numX", [256, 8192, 24576, 49152, 65536 + 256, 65536 + 7680, 131072 + 256])
 @pytest.mark.parametrize("numK", [5, 145])
