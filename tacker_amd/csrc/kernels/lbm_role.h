@@ -251,17 +251,32 @@ __device__ __forceinline__ void lbm_role(const float *__restrict__ src, float *_
     const int lane = tid & (TK_WAVE_SIZE - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / TK_WAVE_SIZE), waves = role_threads / TK_WAVE_SIZE;
     constexpr int PIECE = 2 * TK_WAVE_SIZE;
+    if (__builtin_expect(role_threads < TK_WAVE_SIZE, 0)) {   // workgroups of less than a wavefront: a cell a thread
+#pragma unroll 1
+        for (int i = role_block * role_threads + tid; i < min(end - start, rows) * sx; i += role_blocks * role_threads) {
+            int c = start % rows * sx + i;
+            c = c < cells ? c : c - cells;
+            asm volatile("" : "+v"(c)::"memory");   // (nothing of it in registers that the others do without)
+            lbm_cell(src, dst, cells, c, sx, sxy);
+        }
+        return;
+    }
     // Every XCD (workgroups go to them in turn) takes a slab of the run, in order: the lines that two waves' scattered pieces share
     // are completed in one L2.
-    const int xcds = role_blocks % TK_XCD_NUM == 0 ? TK_XCD_NUM : 1;
+    const int xcd_bits = role_blocks % TK_XCD_NUM == 0 ? __builtin_ctz(TK_XCD_NUM) : 0;
+    const int groups = role_blocks >> xcd_bits, group = role_block >> xcd_bits, xcd = role_block - (group << xcd_bits);
+    const auto slab_of = [&](int pieces) { return (pieces + (1 << xcd_bits) - 1) >> xcd_bits; };
+    // A launch by itself has 16 wavefronts a SIMD, most of which have nothing to do in a short range: they leave before anything else.  Alone, us with a
+    // wave a row / with three divisions in front of that / so: 281 rows of 120 cells 5.0 / 8.2 / 4.5, 1125 7.3 / 9.6 / 6.4, 2250 9.8 / 11.7 / 9.3, 18000
+    // 57.2 / 54.4 / 54.4; 64 rows of 97 cells, which were taken a cell a lane, 3.7 / 7.9 / 4.2, 1125 6.8 / 9.1 / 5.5.
+    if (wave * groups + group >= slab_of((min(end - start, rows) * sx + PIECE - 1) / PIECE)) return;
     // what of the range lies before the end of the grid, and again from its beginning
     for (int pos = start; pos < end;) {
-        const int row = pos % rows, here = min(end - pos, rows - row);
+        const int row = pos < rows ? pos : pos % rows, here = min(end - pos, rows - row);
         pos += here;
         const int first = row * sx, count = here * sx;
         const int pieces = (count + PIECE - 1) / PIECE;
-        const int slab = (pieces + xcds - 1) / xcds, lo = role_block % xcds * slab, hi = min(pieces, lo + slab);
-        const int groups = role_blocks / xcds, group = role_block / xcds;
+        const int slab = slab_of(pieces), lo = xcd * slab, hi = min(pieces, lo + slab);
         // this lane's pair of a piece: the run's last lane takes its last two cells where it has an odd one left (both of a cell's
         // writers have the same bits), those behind it none
         const auto cell_of = [&](int piece) { return first + min(piece * PIECE + 2 * lane, count - 2); };
@@ -273,20 +288,27 @@ __device__ __forceinline__ void lbm_role(const float *__restrict__ src, float *_
         const auto one = [&](int piece) {
             if (there(piece)) lbm_cell_pair(src, dst, cells, cell_of(piece), sx, sxy);
         };
-        if (hi - lo <= groups * waves * PAIRS) {   // few: one at a time, over all workgroups before a second wave of one
-            for (int piece = lo + wave * groups + group; piece < hi; piece += groups * waves) one(piece);
-            continue;
-        }
-        for (int piece = lo + (group * waves + wave) * PAIRS; piece < hi; piece += groups * waves * PAIRS) {
-            if (PAIRS > 1 && piece + PAIRS < hi) {   // (the last piece may be a part of one)
-                int c[PAIRS];
+        // Pieces that all waves take at a time: PAIRS each, as long as there are enough for all, and what is left one each, so that a last
+        // round of few does not take as long as one of all.  us beside 2048^3 with what is left dealt PAIRS a wave / so: 120 x 120 x 150, a quarter
+        // of a round left, 110.3 / 104.4, 4500 of its rows 45.3 / 38.2.
+        const int round = groups * waves * PAIRS;
+        int from = lo;
+        if (PAIRS > 1)
+            for (; from + round <= hi; from += round) {
+                const int piece = from + (group * waves + wave) * PAIRS;
+                if ((piece + PAIRS) * PIECE <= count) {
+                    int c[PAIRS];
 #pragma unroll
-                for (int r = 0; r < PAIRS; ++r) c[r] = first + (piece + r) * PIECE + 2 * lane;
-                lbm_cell_pairs<PAIRS>(src, dst, cells, c, sx, sxy);
-            } else {
-                for (int r = 0; r < PAIRS && piece + r < hi; ++r) one(piece + r);
+                    for (int r = 0; r < PAIRS; ++r) c[r] = first + (piece + r) * PIECE + 2 * lane;
+                    lbm_cell_pairs<PAIRS>(src, dst, cells, c, sx, sxy);
+                } else {   // (the run's last piece may be a part of one)
+                    for (int r = 0; r < PAIRS; ++r) one(piece + r);
+                }
             }
-        }
+        // What is left one at a time, over all workgroups before a second wave of one; where that is more than a round, a
+        // workgroup's pieces side by side, so that the last ones are those of few workgroups.
+        const bool few = PAIRS > 1 || hi - from < round;
+        for (int piece = from + (few ? wave * groups + group : group * waves + wave); piece < hi; piece += groups * waves) one(piece);
     }
 }
 

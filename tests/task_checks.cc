@@ -1,4 +1,4 @@
-// Checks of the VGG16 task's C++ interface: what no C entry point reaches.  Usage: task_checks <check>; exit code 0 if it holds.
+// Checks of the C++ interface, the VGG16 task's and launch sizes of lbm: what no C entry point reaches.  Usage: task_checks <check>; exit code 0 if it holds.
 #include <cstdio>
 #include <cstring>
 #include <exception>
@@ -8,6 +8,7 @@
 
 #include "Creator.h"
 #include "dnn/vgg16.h"
+#include "ori_kernel/lbm_kernel.h"
 #include "../include/tacker_amd.h"
 
 extern std::unordered_map<std::string, void *> fmap;
@@ -358,6 +359,31 @@ bool after_a_failed_launch(bool query)
     return true;
 }
 
+// Ranges of lbm in workgroups of less than a wavefront, of a wavefront and a half, and of eight, are those of ordinary ones.
+bool lbm_workgroups()
+{
+    OriLBMKernel ori(1);
+    const int rows = ori.sizeY() * ori.sizeZ();
+    const size_t floats = (size_t)ori.sizeX() * rows * 19;
+    const std::vector<float> nothing(floats, -5.0f);
+    for (const auto &range : {std::pair<int, int>(0, rows), {0, 1}, {rows / 2, rows / 2 + 77}, {rows - 3, rows + 2}}) {
+        std::vector<float> want;
+        for (int block : {256, 32, 48, 96, 512}) {
+            write(ori.params()->dst, nothing);
+            GPTBKernel k(2, "lbm", "gptb_lbm", &ori, dim3(block < 64 ? 1000 : 75, 1, 1), dim3(block, 1, 1), range.first, range.second);
+            k.execute(nullptr);
+            const std::vector<float> got = read(ori.params()->dst, floats);
+            if (want.empty()) want = got;
+            if (!same(got, want)) {
+                printf("rows %d to %d, workgroups of %d\n", range.first, range.second, block);
+                return false;
+            }
+        }
+        if (same(want, nothing)) return false;
+    }
+    return true;
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -380,6 +406,7 @@ int main(int argc, char **argv)
         else if (!strcmp(check, "paid_once")) ok = paid_once();
         else if (!strcmp(check, "straight_behind")) ok = straight_behind_queries(64, 96, 4) && straight_behind_queries(224, 224, 2);
         else if (!strcmp(check, "failed_launch")) ok = after_a_failed_launch(true) && after_a_failed_launch(false);
+        else if (!strcmp(check, "lbm_workgroups")) ok = lbm_workgroups();
         else return 2;
     } catch (const std::exception &e) {
         printf("%s\n", e.what());

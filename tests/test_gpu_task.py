@@ -750,6 +750,11 @@ def test_what_a_caller_records_reads_what_the_last_query_left(check):
     test_checks_of_the_cxx_interface(check)
 
 
+def test_lbm_in_workgroups_of_any_size():
+    # less than a wavefront, one and a half, eight: the host's own check is in front of the C entry points alone
+    test_checks_of_the_cxx_interface("lbm_workgroups")
+
+
 def test_what_a_query_leaves_out_after_a_launch_that_failed():
     # a kernel that cannot be found, in a query or while what queries left out is computed: the error is that call's alone
     test_checks_of_the_cxx_interface("failed_launch")
