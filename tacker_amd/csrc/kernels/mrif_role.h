@@ -129,7 +129,7 @@ struct MrifBody {
     static constexpr bool SHARES = false;   // a block's voxels over more wavefronts than they fill
     static constexpr int STAGE_QUADS = TK_WAVE_SIZE + TK_WAVE_SIZE / 4;
     static __device__ __forceinline__ int chunk() { return MRIF_K_CHUNK; }
-    static __device__ __forceinline__ int parts(int, int) { return KERNEL_FH_THREADS_PER_BLOCK / TK_WAVE_SIZE; }
+    static __device__ __forceinline__ int parts(int, int, int) { return KERNEL_FH_THREADS_PER_BLOCK / TK_WAVE_SIZE; }
     template <int V, int T>
     static __device__ __forceinline__ bool voxels(int k_begin, int k_end, const float *__restrict__ x,
                                                   const float *__restrict__ y, const float *__restrict__ z,

@@ -267,11 +267,12 @@ struct MriqBody {
     // times as many where that leaves less for the SIMD that has most, in three turns or fewer (a smaller unit prepares the records
     // for fewer voxels).  us, 1024 records beside a GEMM of four tiles, 64 / 32 / 16 voxels a wavefront, * = taken: 8192 voxels
     // 19.8 / 13.9 / 11.8*, 24576 20.1 / 14.9* / 15.2, 49152 20.4* / 20.8 / 27.5, 65536 31.9 / 27.0* / 30.9, 81920 32.2 / 27.2* / 40.3,
-    // 98304 32.4* / 38.8 / 43.6, 131072 43.6* / 45.1 / 56.1, 262144 68.0* / 81.6 / 107.6.
-    static __device__ __forceinline__ int parts(int blocks, int simds)
+    // 98304 32.4* / 38.8 / 43.6, 131072 43.6* / 45.1 / 56.1, 262144 68.0* / 81.6 / 107.6.  A table of one chunk is over before units of 16 voxels are
+    // worth it: 128 records, 8192 voxels beside 256^3 6.4 / 6.3* / 6.5, alone 4.5 / 3.9* / 4.0; 256 records beside 128^3 7.0 / 5.6 / 5.6*.
+    static __device__ __forceinline__ int parts(int blocks, int chunks, int simds)
     {
         int p = KERNEL_Q_THREADS_PER_BLOCK / TK_WAVE_SIZE;
-        while (p < KERNEL_Q_THREADS_PER_BLOCK / MRIQ_TILE) {
+        while (p < KERNEL_Q_THREADS_PER_BLOCK / (chunks > 1 ? MRIQ_TILE : 2 * MRIQ_TILE)) {
             const int most = (blocks * p + simds - 1) / simds, halves = (blocks * 2 * p + simds - 1) / simds;
             if (halves >= 2 * most || halves > 3) break;
             p *= 2;
@@ -337,10 +338,10 @@ __device__ __forceinline__ int mriq_phase(int lo, int hi, int k_begin, int k_end
         if (count == V) {
             if (Body::template voxels<V, T>(k_begin, k_end, x, y, z, Qr, Qi, base, stage)) break;
         } else if constexpr (V > 1) {
-            if constexpr (V > 2) {
+            if constexpr (V > 2) {   // (a body that takes as many has nothing far: the first two would be added twice)
                 if (count >= 2) {
                     const int two[2] = {base[0], base[1]};
-                    if (Body::template voxels<2, T>(k_begin, k_end, x, y, z, Qr, Qi, two, stage)) break;
+                    Body::template voxels<2, T>(k_begin, k_end, x, y, z, Qr, Qi, two, stage);
                 }
             }
             if (count & 1) {
@@ -384,8 +385,9 @@ __device__ __forceinline__ void mriq_role(int numK, const float *__restrict__ x,
     const int gx = grid_dimension_x;
     const int gy = grid_dimension_y;
     const int stride = role_blocks * waves;
-    const int parts = Body::parts(gx, min(role_blocks * min(waves, 4), 4 * TK_CU_NUM));   // (a CU has four SIMDs)
+    const int parts = Body::parts(gx, gy, min(role_blocks * min(waves, 4), 4 * TK_CU_NUM));   // (a CU has four SIMDs)
     const int first_owned = first_piece(gx * parts, 4 * TK_CU_NUM, wave, waves, role_block, role_blocks);
+    if (first_owned >= gx * parts) return;   // (most, in small launches: 128 records, 8192 voxels alone 5.0 us, so 4.0)
     for (int pos = start; pos < end;) {
         const int row = pos / gx, chunk = row % gy;
         const int lo = pos - row * gx, hi = min(gx, lo + (end - pos));

@@ -618,7 +618,7 @@ def test_mriq_coordinates_at_the_ends_of_the_range(numX):
         assert np.array_equal(re, first[0], equal_nan=True) and np.array_equal(im, first[1], equal_nan=True)
 
 
-# voxels a wavefront takes on 256 CUs: 16, 16, 32, 64 (one and two at a time, or none), 32 in three turns, 64
+# voxels a wavefront takes on 256 CUs: 16 (32 where the table is one chunk) twice, 32, 64 (one and two at a time, or none), 32 in three turns, 64
 @pytest.mark.parametrize("numX", [256, 8192, 24576, 49152, 65536 + 256, 65536 + 7680, 131072 + 256])
 @pytest.mark.parametrize("numK", [5, 145])
 def test_mriq_voxels_a_wavefront_takes_do_not_change_a_bit(numX, numK):
