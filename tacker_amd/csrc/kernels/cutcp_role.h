@@ -192,6 +192,8 @@ __device__ __forceinline__ void cutcp_piece(int binDim_x, int binDim_y, const fl
                     r2[u][e] = __builtin_fmaf(dy, dy, dxdz2);
                 }
             }
+            // (Where a wavefront has its SIMD to itself they might as well not go first: in an instance of its own for up to 4 * TK_CU_NUM pieces, 48 points
+            // 23.8 us for 24.0, but 72 to 104 points 2 to 3 % more, with more code around theirs.)
             transcendentals_begin();
 #pragma unroll
             for (int u = 0; u < CUTCP_GROUP; ++u)
@@ -353,7 +355,7 @@ __device__ __forceinline__ void cutcp_role(int binDim_x, int binDim_y, const flo
                                            int start, int end, int tid, int role_threads)
 {
     const int waves = min(role_threads / TK_WAVE_SIZE, WAVES);
-    const int wave = tid / TK_WAVE_SIZE;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / TK_WAVE_SIZE);
     if (wave >= waves || start >= end) return;
     const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
     const int len = NbrListLen;
@@ -362,10 +364,11 @@ __device__ __forceinline__ void cutcp_role(int binDim_x, int binDim_y, const flo
     const int gx = grid_dimension_x * grid_dimension_y * gdz;                  // regions = columns
     if (gx <= 0) return;
     const int stride = role_blocks * waves;
-    const CutcpWalk walk(len, gy);
     const CutcpPieces pieces(gx, stride);
     const int first_owned = first_piece(pieces.first_of(gx), 8 * TK_CU_NUM, wave, waves, role_block, role_blocks);
-    cutcp_lds_float4 *stage = cutcp_stage_of_wave<WAVES>(__builtin_amdgcn_readfirstlane(wave));
+    if (first_owned >= pieces.first_of(gx)) return;   // (most, in small lattices: 48 points 24.7 us, so 24.0, 104 points 29.6 and 28.8)
+    const CutcpWalk walk(len, gy);
+    cutcp_lds_float4 *stage = cutcp_stage_of_wave<WAVES>(wave);
     // the range as phases: a partial row, or whole rows that follow each other up to the last part
     for (int pos = start; pos < end;) {
         const int row = pos / gx;
