@@ -444,7 +444,7 @@ def test_lava_what_is_not_finite_is_what_the_differences_give(boxes1d, alpha, wh
     np.testing.assert_allclose(got[:, 1:][finite], want[finite], rtol=2e-4, atol=2e-3 * (1 if what == "far" else 1e37))
 
 
-@pytest.mark.parametrize("boxes1d,launch_grid", [(2, 1), (3, 40), (5, 256), (9, 700)])
+@pytest.mark.parametrize("boxes1d,launch_grid", [(2, 1), (3, 40), (5, 256), (9, 700), (12, 700)])
 def test_lava_every_cut_gives_the_same_bits_in_either_form(boxes1d, launch_grid):
     # alpha at which some boxes take the form about their centre and others, wider ones, the differences
     rv, qv = lava_inputs(boxes1d, seed=60 + boxes1d)
@@ -631,6 +631,49 @@ def test_pairs_among_the_three(first, second, variant):
     ta.gptb_create(ori1, 0, 0, 1, n1 - 1).execute()
     ta.gptb_create(ori2, 0, 0, 0, n2 // 2).execute()
     assert np.array_equal(got[0].view(np.uint32), bits(out1)) and np.array_equal(got[1].view(np.uint32), bits(out2))
+    assert ta.spin_fail_flag() == 0
+
+
+def _lava_large():
+    # 13^3 boxes, whose exponents come from the matrix units; every third one is too wide for the form about its centre.  What a launch by itself gives
+    rv, qv = lava_inputs(13, seed=77)
+    wide = np.arange(len(rv)) // 100 % 3 == 1
+    rv[wide, 1:] = 3 * rv[wide, 1:] - 1
+    rv[wide, 0] = (rv[wide, 1:] ** 2).sum(1) / 2
+    d_r, d_q, alone, out = dev(rv), dev(qv), *(torch.zeros((len(rv), 4), device="cuda:0") for _ in range(2))
+    ta.gptb_lava(0.5, d_r, d_q, alone)
+    n = ta.lava_blocks(13)
+    return ta.gptb_create(ta.ori_lava_create(0.5, d_r, d_q, out), 0, 0, 0, n), n, out, alone
+
+
+@pytest.mark.parametrize("variant", [None, "wave_256", "wave_512", "wg_1_1", "wg_1_2"])
+def test_lava_large_domains_beside_tzgemm(variant):
+    A, B = gemm_inputs(512, 512, 128, seed=52)
+    a, b, c, solo_c = dev(A), dev(B), *(torch.zeros((512, 512), device="cuda:0") for _ in range(2))
+    ta.gptb_tzgemm(a, b, solo_c)
+    lava, n, out, alone = _lava_large()
+    tz = ta.gptb_create(ta.ori_tzgemm_create(a, b, c), 0, 0, 0, 64)
+    for cuts in ((0, n), (0, n // 3, n)):
+        out.zero_()
+        c.zero_()
+        for i, (lo, hi) in enumerate(zip(cuts, cuts[1:])):
+            ta.mix_create(lava, tz, lo, hi, 20 * i, 64 if hi == n else 20, variant=variant).execute()
+        assert np.array_equal(bits(out), bits(alone)) and np.array_equal(host(c), host(solo_c))
+    assert ta.spin_fail_flag() == 0
+
+
+@pytest.mark.parametrize("first,second", [p for p in RODINIA_PAIRS if "lava" in p])
+@pytest.mark.parametrize("variant", [None, "wg_1_1", "wg_1_2", "wg_2_1", "ord_1_1", "ord_1_2", "ord_2_1"])
+def test_lava_large_domains_beside_the_others(first, second, variant):
+    lava, n, out, alone = _lava_large()
+    ori, m, other, want = _small(second if first == "lava" else first)
+    partner = ta.gptb_create(ori, 0, 0, 0, m)
+    for cuts in ((0, n), (0, n // 3, n)):
+        out.zero_()
+        for lo, hi in zip(cuts, cuts[1:]):
+            if first == "lava": ta.be_pair_create(lava, partner, lo, hi, 0, m, variant=variant).execute()
+            else: ta.be_pair_create(partner, lava, 0, m, lo, hi, variant=variant).execute()
+        assert np.array_equal(bits(out), bits(alone)) and _same(other, want)
     assert ta.spin_fail_flag() == 0
 
 
