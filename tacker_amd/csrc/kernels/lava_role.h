@@ -761,10 +761,12 @@ __device__ __forceinline__ void lava_role(par_str d_par_gpu, dim_str d_dim_gpu, 
     const int cols = grid_dimension_x;   // positions per row, including boxes past number_boxes
     const int stride = role_blocks * waves;
     const LavaUnits units(gx, stride, d_dim_gpu.number_boxes >= LAVA_TILES_FROM);
-    // many units: those of a workgroup follow each other, so that the fine ones of the last round start last; few:
-    // those that follow each other lie in different workgroups, so that a short range uses every CU there is
+    // Many units: those of a workgroup follow each other, so that the fine ones of the last round start last; fewer: as first_piece says.  (By the
+    // units of the range instead of the domain's, which spreads short ranges over more workgroups, they are slower: 64 and 512 boxes of 11^3 6.9 and
+    // 9.5 us, so 7.9 and 10.5.)
     const int first_owned = units.first_of(gx) >= LAVA_WAVES_PER_SIMD * 4 * TK_CU_NUM ? role_block * waves + wave
                                                                                       : first_piece(units.first_of(gx), 4 * TK_CU_NUM, wave, waves, role_block, role_blocks);
+    if (first_owned >= units.first_of(gx)) return;   // (most, in a launch of 32 wavefronts a SIMD: 64 and 512 boxes of 11^3 10.1 and 12.7 us, so 6.9 and 9.5)
     // the range as phases: a partial row, or whole rows that follow each other up to the last part
     for (int pos = start; pos < end;) {
         const int row = pos / cols;
