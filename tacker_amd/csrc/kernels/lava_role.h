@@ -39,7 +39,7 @@
 //    pay for: 3^3 boxes 49 us for 37, 8^3 68 for 57, 12^3 146 for 138, 13^3 141 for 143, 16^3 225 for 257, 24^3 705 for 772.  (The bits
 //    differ in the last place, so that the domain alone decides.)
 // A pair is 8 short instructions and the exponential otherwise, 12 from the differences; the exponentials go first (transcendentals_begin) where a
-// wavefront does not have its SIMD to itself.  At the end of a part the four rows' sums are added,
+// lane has several.  At the end of a part the four rows' sums are added,
 // (g0 + g2) + (g1 + g3), by lane swaps that add two values at once, which leaves component v, y, x, z of the
 // total in row 0, 1, 2, 3; the total goes on from the output array.  24^3 boxes: 708 us (772 without the matrix units, 833 with neither, 1325 with
 // neighbours by vector loads and seven particles a lane); 18^3 321 / - / 359 / 577, 9^3 72 / - / 71 / 116, 3^3 36.6 / - / 36.8 / 46.
@@ -493,7 +493,9 @@ __device__ __forceinline__ void lava_part(const float4_t (&home)[P], const float
         const float4_t na = next[0], nb = next[1];
         if (P < LAVA_MAX_P) __builtin_amdgcn_sched_barrier(0);
         // scale (vi + vj - (xi xj + yi yj + zi zj)) = -r2 a2 log2(e), stage by stage over the lane's
-        // particles: their chains are independent, and in this order none waits for its own last result
+        // particles: their chains are independent, and in this order none waits for its own last result.  With one particle a lane there is one
+        // exponential, and holding it in front of the rest gains nothing where wavefronts share a SIMD (8^3 boxes 56.8 us for 57.2, 9^3 72.1 for 72.2, 11^3
+        // 117.5 for 116.4) and costs where they do not (2^3 to 5^3 14.5 to 40.2 for 13.7 to 38.0); with two, 12^3 boxes 133.4 for 135.4.
         float w[P];
 #pragma unroll
         for (int k = 0; k < P; ++k) w[k] = home[k][0] + a[0];
@@ -501,10 +503,10 @@ __device__ __forceinline__ void lava_part(const float4_t (&home)[P], const float
         for (int c = 1; c < 4; ++c)
 #pragma unroll
             for (int k = 0; k < P; ++k) w[k] = __builtin_fmaf(home[k][c], a[c], w[k]);
-        if (P == LAVA_MAX_P) transcendentals_begin();   // (fewer are for domains that leave a wavefront its SIMD)
+        if (P > 1) transcendentals_begin();
 #pragma unroll
         for (int k = 0; k < P; ++k) w[k] = __builtin_amdgcn_exp2f(w[k]);
-        if (P == LAVA_MAX_P) transcendentals_end();
+        if (P > 1) transcendentals_end();
         if (CENTRED) {
 #pragma unroll
             for (int c = 0; c < 4; ++c)
@@ -694,21 +696,19 @@ struct LavaUnits {
     // `waves` wavefronts serve `boxes` boxes.  Whole rounds of as many boxes as wavefronts are at work at a time
     // take a box each; what is left over -- all of it when the domain is small -- is cut: a box is 0.1 to 0.3 ms of
     // one wavefront, with up to 4 of them on a SIMD, and a last round of few boxes would leave most of the chip idle that
-    // long.  Finer cuts spread better, but every wavefront prepares the neighbours again and a read serves fewer pairs.  us
-    // with everything left over in units of 6 / 3 / 2 / 1 particles a lane, in a launch of more wavefronts than are at work
-    // at a time, which the dispatcher evens out:
-    //     8^3 (512 boxes) 117 / 63 / 66 / 60,  9^3 (729) 116 / 86 / 79 / 70,  11^3 (1331) 160 / 120 / 120 / 113,
-    //     12^3 (1728) 163 / 153 / 137 / 140,  13^3 (2197) 218 / 149 / 157 / 172,  15^3 (3375) 296 / 229 / 224 / 255,
-    //     24^3 (3 x 4096 + 1536) 833 / 823 / 818 / 829.
-    // In a launch of fewer, whose wavefronts each have their units from the start, the finest cut that gives nobody two.
+    // long.  Finer cuts spread better, but every wavefront prepares the neighbours again and a read serves fewer pairs.  Taken is the finest cut
+    // that gives no wavefront at work two units (*).  us with everything left over in units of 6 / 3 / 2 / 1 particles a lane, in a launch of more
+    // wavefronts than are at work at a time:
+    //     8^3 (512 boxes) 110 / 65 / 64 / 57*,  9^3 (729) 109 / 81 / 66* / 72,  10^3 (1000) 110 / 82 / 85* / 95,  11^3 (1331) 144 / 109 / 105* / 116,
+    //     12^3 (1728) 145 / 129* / 135 / 144;  with exponents from the matrix units, 6 or 3: 13^3 (2197) 133* / 143,  15^3 (3375) 210* / 219,
+    //     18^3 (4096 + 1736) 335 / 319*,  24^3 (3 x 4096 + 1536) 731 / 737*.
     __device__ __forceinline__ LavaUnits(int boxes, int waves, bool tiles_) : tiles(tiles_)
     {
         const int at_once = min(waves, LAVA_WAVES_PER_SIMD * 4 * TK_CU_NUM);
-        const bool evened = waves > at_once;
         whole = boxes / at_once * at_once;
         const int left = boxes - whole;
-        if (tiles) p = evened || left * lava_subs(3) <= at_once ? 3 : LAVA_MAX_P;
-        else p = left * (evened ? 3 : lava_subs(1)) <= at_once ? 1 : (left * (evened ? 2 : lava_subs(2)) <= at_once ? 2 : (evened || left * lava_subs(3) <= at_once ? 3 : LAVA_MAX_P));
+        p = left * lava_subs(LAVA_TILES_P) <= at_once ? LAVA_TILES_P : LAVA_MAX_P;
+        if (!tiles && left * lava_subs(2) <= at_once) p = left * lava_subs(1) <= at_once ? 1 : 2;
         subs = p == 1 ? lava_subs(1) : (p == 2 ? lava_subs(2) : (p == 3 ? lava_subs(3) : 1));
     }
     __device__ __forceinline__ int first_of(int box) const { return box <= whole ? box : whole + (box - whole) * subs; }
