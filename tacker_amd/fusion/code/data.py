@@ -39,7 +39,7 @@ REFERENCE_KERNEL_INFO = {
 # gfx950 roles.  register = VGPRs per lane of the role compiled alone (the
 # compiler's kernel-resource-usage remarks), shared_memory = LDS bytes
 # per role instance in a fused launch (mri-q's and mri-fhd's own GPTB kernels
-# hold it for workgroups of 16 wavefronts: 16384 and 20480), blocksize = threads of one role instance (a multiple of the
+# hold it for workgroups of 16 wavefronts: 28672 and 20480), blocksize = threads of one role instance (a multiple of the
 # 64-wide wavefront), solo_ptb_blks = role instances per CU of the plain GPTB
 # launch, ori_blks = blocks of the reference-shaped natural grid at the
 # benchmark's problem size.
@@ -48,11 +48,11 @@ KERNEL_INFO = {
     # 1024 blocks of 64 x 4 columns x 8 runs of 8 centre planes
     "stencil": {"register": 48, "shared_memory": 0, "blocksize": 256, "solo_ptb_blks": 8,
                 "ori_blks": 8192},
-    # 55.6 us with 16 workgroups a CU, 57.7 with 8 (profile_gptb.py)
-    "lbm": {"register": 57, "shared_memory": 0, "blocksize": 256, "solo_ptb_blks": 16,
+    # 55.0 us with 16 workgroups a CU, 56.3 with 8 (profile_gptb.py)
+    "lbm": {"register": 59, "shared_memory": 0, "blocksize": 256, "solo_ptb_blks": 16,
             "ori_blks": 18000},
     # 1024 blocks of 256 voxels x 16 chunks of 128 k records
-    "mriq": {"register": 123, "shared_memory": 7168, "blocksize": 256, "solo_ptb_blks": 8,
+    "mriq": {"register": 120, "shared_memory": 7168, "blocksize": 256, "solo_ptb_blks": 8,
              "ori_blks": 16384},
     # 1024 blocks of 256 voxels x 16 chunks of 128 k records
     "mrif": {"register": 107, "shared_memory": 5120, "blocksize": 256, "solo_ptb_blks": 8,
@@ -64,7 +64,7 @@ KERNEL_INFO = {
     "fft": {"register": 40, "shared_memory": 8192, "blocksize": 256, "solo_ptb_blks": 8,
             "ori_blks": 10240},
     # 26 x 26 x 2 regions of 8 x 8 x 8 lattice points (two wavefronts each) x 11 parts of 32 neighbour bins
-    "cutcp": {"register": 113, "shared_memory": 4096, "blocksize": 128, "solo_ptb_blks": 16,
+    "cutcp": {"register": 109, "shared_memory": 4096, "blocksize": 128, "solo_ptb_blks": 16,
               "ori_blks": 14872},
     # 2560000 blocks of 256 records; a stream that wants many workgroups in flight (4.0 TB/s with 8 a CU,
     # 4.95 with 32)
@@ -76,7 +76,7 @@ KERNEL_INFO = {
               "ori_blks": 524288},
     # 216000 boxes of 100 particles (a wavefront each) x 27 parts (the home box and its neighbour slots);
     # boxes on the faces have fewer neighbours: the more owner wavefronts, the evener their shares
-    # (12.4 ms with 4 workgroups a CU, 11.2 with 32)
+    # (12.5 ms with 4 workgroups a CU, 11.0 with 32)
     "lava": {"register": 128, "shared_memory": 15872, "blocksize": 256, "solo_ptb_blks": 32,
              "ori_blks": 5832000},
     # 200 windows of 256 columns (6 result columns each), a wavefront each
