@@ -27,7 +27,7 @@
 //    is the clamp of s to [0, 1], a modifier of the instruction that computes it, instead of a comparison and
 //    an execution mask.
 // The atoms' order, and so every point's sum, is the same in every form of the kernel.
-// 208^3 lattice, two layers of regions: 99 us (123 with the square roots where they fall and a workgroup's pieces far apart); 136 us with every batch filled up to whole groups
+// 208^3 lattice, two layers of regions: 99 to 103 us (123 with the square roots where they fall and a workgroup's pieces far apart); 136 us with every batch filled up to whole groups
 // (a twelfth of the atoms) and the place in the list divided anew for each, in 95 instructions with five 32-bit products at a quarter of
 // the rate.  Where inv_cutoff2 is not 1 / cutoff2 every point walks the list by itself: 169 us where the clamp took 123 (185 before).
 #pragma once

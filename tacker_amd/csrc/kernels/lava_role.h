@@ -36,13 +36,13 @@
 //    particles are four lanes side by side, 16 neighbours at a time: 7 steps, where a seventh particle a lane would take 25.
 //  * What else could compute.  In domains of LAVA_TILES_FROM boxes or more the exponents come from the matrix units (below), and
 //    a pair is four multiply-adds and the exponential.  Preparing a neighbour is 45 instructions then, which few home particles a wavefront do not
-//    pay for: 3^3 boxes 49 us for 37, 8^3 68 for 57, 12^3 146 for 138, 13^3 141 for 143, 16^3 225 for 257, 24^3 705 for 772.  (The bits
-//    differ in the last place, so that the domain alone decides.)
+//    pay for: with three a lane 3^3 boxes 49 us for 37, 8^3 68 for 57, 12^3 146 for 138, 13^3 141 for 143, with six 16^3 225 for 257, 24^3 705 for 772.  (The bits
+//    differ in the last place, so that the domain alone decides, and neither the launch nor the number of CUs; the figures are of 256.)
 // A pair is 8 short instructions and the exponential otherwise, 12 from the differences; the exponentials go first (transcendentals_begin) where a
 // lane has several.  At the end of a part the four rows' sums are added,
 // (g0 + g2) + (g1 + g3), by lane swaps that add two values at once, which leaves component v, y, x, z of the
-// total in row 0, 1, 2, 3; the total goes on from the output array.  24^3 boxes: 708 us (772 without the matrix units, 833 with neither, 1325 with
-// neighbours by vector loads and seven particles a lane); 18^3 321 / - / 359 / 577, 9^3 72 / - / 71 / 116, 3^3 36.6 / - / 36.8 / 46.
+// total in row 0, 1, 2, 3; the total goes on from the output array.  24^3 boxes: 690 to 740 us (772 without the matrix units, 833 with neither, 1325 with
+// neighbours by vector loads and seven particles a lane); 18^3 319 / - / 359 / 577, 9^3 65 / - / 71 / 116, 3^3 36.1 / - / 36.6 / 46.
 //
 // Few boxes: a box is then split over several wavefronts (P home particles a lane instead of 6, every particle
 // summed exactly as before), see LavaUnits.
@@ -483,7 +483,7 @@ __device__ __forceinline__ void lava_part(const float4_t (&home)[P], const float
     for (int k = 0; k < P; ++k) f[k] = float4_t{0.f, 0.f, 0.f, 0.f};
     const lava_lds_float4 *at = stage + 2 * row;
     float4_t a = at[0], b = at[1];
-    // Six particles a lane are chains enough for the compiler to interleave as it likes (24^3 boxes 829 us, with the step's
+    // Six particles a lane are chains enough for the compiler to interleave as it likes (24^3 boxes, when they took this loop, 829 us, with the step's
     // read held in front of it 871); with fewer, the reads stay in front of a step's work and every step is written out (3^3 boxes
     // 36.5 us; 42.1 in a loop of five steps, 43.2 as the compiler likes).
 #pragma unroll P < LAVA_MAX_P ? LAVA_STEPS : 5

@@ -289,8 +289,8 @@ __device__ __forceinline__ void lbm_role(const float *__restrict__ src, float *_
             if (there(piece)) lbm_cell_pair(src, dst, cells, cell_of(piece), sx, sxy);
         };
         // Pieces that all waves take at a time: PAIRS each, as long as there are enough for all, and what is left one each, so that a last
-        // round of few does not take as long as one of all.  us beside 2048^3 with what is left dealt PAIRS a wave / so: 120 x 120 x 150, a quarter
-        // of a round left, 110.3 / 104.4, 4500 of its rows 45.3 / 38.2.
+        // round of few does not take as long as one of all.  us beside 2048^3 with what is left dealt PAIRS a wave / so: 120 x 120 x 150, an eighth
+        // of a round left, 110.3 / 104.4, 4500 of its rows, a thirtieth left, 45.3 / 38.2.
         const int round = groups * waves * PAIRS;
         int from = lo;
         if (PAIRS > 1)

@@ -17,7 +17,7 @@
 // multiply-adds of 2.75 (Q + PhiMag*c, as nvcc contracts the reference's source with its default -fmad=true) and a 256th of a matrix
 // instruction, 4 cycles that the vector units need not wait for while other wavefronts have something for them: the phase (mriq_put_point below).
 // With the phase as three multiply-adds in the reference's order, ((Kx*x) + Ky*y) + Kz*z, 2032 records and 262144 voxels took 130 us alone and
-// 144 to 151 beside tzgemm 2048^3, so 104 and 118, and with the transcendentals first 104 and 112; 700 records and 65536 voxels beside tzgemm 1024^3
+// 144 to 160 beside tzgemm 2048^3, so 104 and 118 to 122, and with the transcendentals first 104 to 106 and 112 to 121; 700 records and 65536 voxels beside tzgemm 1024^3
 // 21.2 to 22.1, now 18.5.
 // The result differs from a float64 evaluation by about 1e-6 per term, far inside the 1e-3 + 1e-4 |Q| bar.
 #pragma once

@@ -172,8 +172,10 @@ __device__ __forceinline__ void role_wave_done(unsigned *words)
 // transcendentals one after the other there are seldom two at the short ones.  With their transcendentals in front of everything
 // else they get them over with, and then have the short ones together.  Cycles of a SIMD for 8 exponentials and 32 multiply-adds of a wavefront,
 // two / three / four wavefronts a SIMD: 192 / 191 / 191, so 135 / 152 / 133; 16 and 40: 288 / 288 / 288, so 213 / 237 / 211.
-// (In longer runs as in shorter ones; in front of the multiply-adds instead it does nothing.)  A GEMM's wavefronts beside them go first all the
-// same (TK_GEMM_WAVE_PRIORITY).
+// (In longer runs as in shorter ones; in front of the multiply-adds instead it does nothing.)  A GEMM's wavefronts in the same workgroup go first all
+// the same (TK_GEMM_WAVE_PRIORITY); those of workgroup-split forms, and the partners in pairs of best-effort kernels, have the usual priority and stand back for
+// these instructions.  us without / with them beside 2048^3, tzgemm on workgroups of its own: 1 : 2 mri-q 253 / 193, cutcp 321 / 258, lavaMD 15^3 590 / 393; 1 : 1 294 /
+// 255, 382 / 383, 688 / 638.  (With the kernels' other changes of that time.)
 __device__ __forceinline__ void transcendentals_begin()
 {
     __builtin_amdgcn_sched_barrier(0);
@@ -191,7 +193,7 @@ __device__ __forceinline__ void transcendentals_end()
 // a workgroup, so that a CU has as few as can be; more of them four to a workgroup (a SIMD each), then four to the next one, and so on
 // through the role's workgroups before a fifth: in a launch of more workgroups than are at work at a time nearly all those at work
 // then have four, where with one to a workgroup three SIMDs of four are idle.  us so / one to a workgroup: mri-q's 4096 pieces in 2048
-// workgroups of 4 wavefronts 111 / 157, 1024 pieces 40.9 / 39.8; cutcp's 5408 pieces in 4096 workgroups of 2 wavefronts 99.5 / 111.5, 2592 pieces
+// workgroups of 4 wavefronts 111 / 157, 1024 pieces 40.9 / 39.8; mri-fhd's 1024 pieces alone 70.0 / 72.4 and beside tzgemm 1024^3 78.0 / 78.4, 4096 172 / 173 and 186 / 184; cutcp's 5408 pieces in 4096 workgroups of 2 wavefronts 99.5 / 111.5, 2592 pieces
 // 35.9 / 39.0, 2048 pieces 36.2 / 34.0, 1352 pieces 33.7 / 29.8; lavaMD's 1296 pieces in 8192 workgroups of 4 wavefronts 40.8 / 42.6.
 __device__ __forceinline__ int first_piece(int pieces, int spread, int wave, int waves, int role_block, int role_blocks)
 {
