@@ -485,8 +485,9 @@ def test_lbm_runs_of_cells(dims, kw):
         assert np.array_equal(host(d).view(np.uint32), want.view(np.uint32)), (a, b)
 
 
-# two pieces at a time: beside a GEMM with workgroups to spare, one with a tile for each, and the large form
-@pytest.mark.parametrize("dims,gemm", [((127, 71, 70), (256, 256, 128)), ((127, 71, 70), (2048, 2048, 128)), ((90, 121, 128), (4096, 4096, 128))])
+# two pieces at a time: beside a GEMM with a tile for each workgroup (one round of 4096 pieces, the last one not whole, and others), one with workgroups to
+# spare, and the large form
+@pytest.mark.parametrize("dims,gemm", [((151, 217, 16), (2048, 2048, 128)), ((127, 71, 70), (256, 256, 128)), ((127, 71, 70), (2048, 2048, 128)), ((90, 121, 128), (4096, 4096, 128))])
 def test_mix_tzgemm_lbm_many_pieces(dims, gemm):
     A, B = gemm_inputs(*gemm, seed=6)
     dA, dB = dev(A), dev(B)
@@ -616,6 +617,11 @@ def test_mriq_coordinates_at_the_ends_of_the_range(numX):
         assert np.all(np.abs(re - want.real)[~bad] <= bound[~bad]) and np.all(np.abs(im - want.imag)[~bad] <= bound[~bad])
         first = first or (re, im)
         assert np.array_equal(re, first[0], equal_nan=True) and np.array_equal(im, first[1], equal_nan=True)
+    A, B = gemm_inputs(256, 256, 128, seed=7)
+    for variant in (None, "wave_256", "wg_1_1", "wg_1_2"):
+        re, im, c = torch.zeros(numX, device="cuda:0"), torch.zeros(numX, device="cuda:0"), torch.zeros((256, 256), device="cuda:0")
+        ta.mix_tzgemm_mriq(len(kv), *d, re, im, dev(A), dev(B), c, variant=variant)
+        assert np.array_equal(host(re), first[0], equal_nan=True) and np.array_equal(host(im), first[1], equal_nan=True)
 
 
 # voxels a wavefront takes on 256 CUs: 16 (32 where the table is one chunk) twice, 32, 64 (one and two at a time, or none), 32 in three turns, 64
