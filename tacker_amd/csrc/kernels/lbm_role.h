@@ -21,7 +21,8 @@
 // 1024 117.7 / 116.1, 128^3 beside 1024 x 4096 x 512 93.2 / 77.2, 127 x 128 x 128 beside 2048 x 1024 x 1024 155.6 / 98.9, 64 x 100 x 64
 // beside 1024^3 25.0 / 21.1, 97^3 beside 128^3 43.5 / 32.6, 33 x 61 x 97 beside 1024 x 1024 x 512 16.6 / 11.5.  (The first three with other ways
 // of dealing the pieces: no slabs an XCD 126, 90, 107; a wave's second piece a round further 121, 91, 120; a run of its own for every workgroup
-// 132, 93, 112; one piece at a time 130, 76, 113; with nontemporal stores 121, 83, 108.)
+// 132, 93, 112; one piece at a time 130, 76, 113; with nontemporal stores 121, 83, 108.  The first of the three moves by up to 8 % with what else is in
+// the library: the same source 116 in the whole one and 126 in one of this pair alone.)
 #pragma once
 #include "role_common.h"
 #include "../header/lbm_header.h"
