@@ -237,6 +237,8 @@ __device__ __forceinline__ void lbm_cell_pairs(const float *__restrict__ src, fl
     __builtin_amdgcn_sched_barrier(0);
 }
 
+#define LBM_FEW_CELLS (2 * TK_CU_NUM * TK_WAVE_SIZE)
+
 // grid_dimension_x = sy, grid_dimension_y = sz, block_dimension_x = sx
 // (src/ori_kernel/lbm_kernel.cu:218-222).  PAIRS > 1: a wave takes that many pieces of 128 cells, which follow each other, at a
 // time (see lbm_cell_pairs).
@@ -268,9 +270,13 @@ __device__ __forceinline__ void lbm_role(const float *__restrict__ src, float *_
     const int groups = role_blocks >> xcd_bits, group = role_block >> xcd_bits, xcd = role_block - (group << xcd_bits);
     const auto slab_of = [&](int pieces) { return (pieces + (1 << xcd_bits) - 1) >> xcd_bits; };
     // A launch by itself has 16 wavefronts a SIMD, most of which have nothing to do in a short range: they leave before anything else.  Alone, us with a
-    // wave a row / with three divisions in front of that / so: 281 rows of 120 cells 5.0 / 8.2 / 4.5, 1125 7.3 / 9.6 / 6.4, 2250 9.8 / 11.7 / 9.3, 18000
-    // 57.2 / 54.4 / 54.4; 64 rows of 97 cells, which were taken a cell a lane, 3.7 / 7.9 / 4.2, 1125 6.8 / 9.1 / 5.5.
-    if (wave * groups + group >= slab_of((min(end - start, rows) * sx + PIECE - 1) / PIECE)) return;
+    // wave a row / with three divisions in front of that / so: 281 rows of 120 cells 5.0 / 8.2 / 4.5, 1125 7.3 / 9.6 / 6.7, 2250 9.8 / 11.7 / 9.3, 18000
+    // 57.2 / 54.4 / 54.4; 1125 rows of 97 cells 6.8 / 9.1 / 5.7.
+    // Where there are cells for few wavefronts they are taken a cell a lane, which is over sooner than two: 64 rows of 120 4.4 / 3.5, 64 rows of 97 4.3 / 3.4,
+    // 281 of 97 4.4 / 3.8; with twice as many cells 5.0 / 5.8.  (Beside a GEMM it is as often the slower way.)
+    const int most = min(end - start, rows) * sx, cell = (wave * role_blocks + role_block) * TK_WAVE_SIZE + lane;
+    const bool cell_a_lane = PAIRS == 1 && most <= min(LBM_FEW_CELLS, role_blocks * waves * TK_WAVE_SIZE);
+    if (cell_a_lane ? cell - lane >= most : wave * groups + group >= slab_of((most + PIECE - 1) / PIECE)) return;
     // what of the range lies before the end of the grid, and again from its beginning
     for (int pos = start; pos < end;) {
         const int row = pos < rows ? pos : pos % rows, here = min(end - pos, rows - row);
@@ -282,8 +288,8 @@ __device__ __forceinline__ void lbm_role(const float *__restrict__ src, float *_
         // writers have the same bits), those behind it none
         const auto cell_of = [&](int piece) { return first + min(piece * PIECE + 2 * lane, count - 2); };
         const auto there = [&](int piece) { return piece * PIECE + 2 * lane < count; };
-        if (count == 1) {
-            if (role_block == 0 && tid == 0) lbm_cell(src, dst, cells, first, sx, sxy);
+        if (cell_a_lane || count == 1) {
+            if (cell < count) lbm_cell(src, dst, cells, first + cell, sx, sxy);
             continue;
         }
         const auto one = [&](int piece) {

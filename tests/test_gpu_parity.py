@@ -466,8 +466,9 @@ def test_lbm_ori_and_gptb_bit_exact(dims):
     assert np.array_equal(host(d3).view(np.uint32), want.view(np.uint32))
 
 
-# pieces of 128 cells: less than one, one and a cell more, rows of one cell, an odd run, several rounds in few and many workgroups
-@pytest.mark.parametrize("dims", [(1, 1, 5), (1, 43, 3), (3, 43, 1), (129, 1, 1), (127, 9, 7), (25, 40, 61)])
+# pieces of 128 cells: less than one, one and a cell more, rows of one cell, an odd run, several rounds in few and many workgroups; up to 32768 cells a lane
+# takes one where there are wavefronts enough
+@pytest.mark.parametrize("dims", [(1, 1, 5), (1, 43, 3), (3, 43, 1), (129, 1, 1), (127, 9, 7), (25, 40, 61), (128, 16, 16), (331, 11, 9)])
 @pytest.mark.parametrize("kw", [{}, {"launch_grid": 1, "launch_block": 64}, {"launch_grid": 3, "launch_block": 256},
                                 {"launch_grid": 16, "launch_block": 128}])
 def test_lbm_runs_of_cells(dims, kw):
